@@ -1,15 +1,22 @@
 // Binned power spectra over R2C half spectra: the mode sums behind jaxpm
 // utils.py:76-128 (power_spectrum) and its bin table utils.py:14-73.
 //
-// Each wave walks one (kx, ky) row of the half spectrum, lanes on
-// consecutive kz (coalesced).  Per mode it forms |k| exactly as the
-// reference bins it (float64 sum of squares, rounded to float32, float32
-// square root), finds the bin by binary search over the float64 edges, and
-// adds the mode and its Hermitian mirror (X(-k) = conj X(k), not stored in
-// the half spectrum) to per-bin sums.  Lanes of one bin are summed across
-// the wave first (one LDS float64 atomic per bin run), each workgroup writes
-// its partial sums, and a second kernel adds the partials in a fixed order,
-// so results repeat bitwise.
+// The half spectrum is walked flat, 64 consecutive modes a wave (coalesced,
+// and no lane idles at the end of a row of nz/2 + 1 modes).  Per mode the
+// wave forms |k| exactly as the reference bins it (float64 sum of squares,
+// rounded to float32, float32 square root), finds the bin by binary search
+// over the edges, and adds the mode and its Hermitian mirror (X(-k) = conj
+// X(k), not stored in the half spectrum) to per-bin sums.  |k| grows along a
+// row, so the lanes of one bin are neighbours: a segmented scan across the
+// wave sums them and the last lane of each run adds the sum to the wave's
+// own bins in LDS.  The waves' bins are then added in a fixed order, within
+// the workgroup and, by a second kernel, over the workgroups.
+//
+// Bound by float64 instruction issue (the scans and the divisions by |k|),
+// not by the 8 bytes a mode.  256^3, poles 0 2 4: 1671 + 127 us when each
+// run of a bin was summed by its own full-wave reductions, the wave numbers
+// divided per mode, and the partial sums added by one thread per slot; now
+// 120 + 14 us.
 #include <cmath>
 
 #include "common.hpp"
@@ -18,52 +25,45 @@ namespace jpm {
 
 constexpr int kPkMaxPoles = 8;
 constexpr int kPkMaxSlots = 8192;   // accumulators x bins, float64 in LDS (64 KiB)
-constexpr int kPkBlock = 256;
-constexpr int kPkMaxBlocks = 512;
+constexpr int kPkMaxWaves = 4;      // per workgroup, each with its own bins
+constexpr int kPkLdsSlots = 4096;   // slots of all waves of a workgroup, when more than one
+constexpr int kPkMaxBlocks = 2048;
 
 struct PkParams {
   int nx, ny, nz, nzh;
+  uint32_t modes;  // nx ny nzh
+  FastDiv div_nzh, div_ny;
+  double inv[3];   // 1 / n_d
   double fac[3];   // 2 pi n_d / L_d: cell wave number to h/Mpc
   double los[3];   // unit line of sight (multipoles only)
-  int nedges, nbins, nslots, npoles;
-  int cross, aniso;
+  int nedges, nbins, nslots, npoles, lmax;
   int poles[kPkMaxPoles];
 };
 
 // numpy.fft.fftfreq(n)[i] = i' * (1.0 / n), i' the signed index.
-__device__ __forceinline__ double fftfreq(int i, int n) {
+__device__ __forceinline__ double fftfreq(int i, int n, double inv) {
   const int s = i <= (n - 1) / 2 ? i : i - n;
-  return double(s) * (1.0 / double(n));
+  return double(s) * inv;
 }
 
-// Correctly rounded float32 square root: a float64 root rounded to float32,
-// then moved to the neighbour whose rounding interval holds f.  The interval
-// ends (midpoints between adjacent floats, 25 significant bits) square
-// exactly in float64.
-__device__ __forceinline__ float sqrt_rn(float f) {
-  if (!(f > 0.0f)) return 0.0f;
-  float s = float(sqrt(double(f)));
-  const double hi = 0.5 * (double(s) + double(nextafterf(s, INFINITY)));
-  if (double(f) > hi * hi) return nextafterf(s, INFINITY);
-  const double lo = 0.5 * (double(s) + double(nextafterf(s, 0.0f)));
-  if (double(f) < lo * lo) return nextafterf(s, 0.0f);
-  return s;
-}
-
-// Legendre polynomial by Bonnet's recurrence.
-__device__ __forceinline__ double legendre(int ell, double mu) {
-  if (ell == 0) return 1.0;
+// (2 l + 1) P_l(mu) of every pole, by Bonnet's recurrence up to the largest.
+template <int NP>
+__device__ __forceinline__ void legendre_weights(const PkParams &p, double mu, double w[NP]) {
+#pragma unroll
+  for (int q = 0; q < NP; ++q) w[q] = p.poles[q] == 0 ? 1.0 : 3.0 * mu;
   double p0 = 1.0, p1 = mu;
-  for (int n = 1; n < ell; ++n) {
+  for (int n = 1; n < p.lmax; ++n) {
     const double p2 = (double(2 * n + 1) * mu * p1 - double(n) * p0) / double(n + 1);
     p0 = p1;
     p1 = p2;
+#pragma unroll
+    for (int q = 0; q < NP; ++q)
+      if (p.poles[q] == n + 1) w[q] = double(2 * n + 3) * p1;
   }
-  return p1;
 }
 
 // np.digitize(x, edges) for increasing edges: the number of edges <= x.
-__device__ __forceinline__ int digitize(const double *__restrict__ edges, int n, double x) {
+__device__ __forceinline__ int digitize(const double *edges, int n, double x) {
   int lo = 0, hi = n;
   while (lo < hi) {
     const int mid = (lo + hi) >> 1;
@@ -75,123 +75,178 @@ __device__ __forceinline__ int digitize(const double *__restrict__ edges, int n,
   return lo;
 }
 
-__device__ __forceinline__ double wave_sum(double v) {
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off);
+// v of the lane that the DPP control names (lanes without one keep 0).
+template <int CTRL, int ROWS>
+__device__ __forceinline__ double dpp_move(double v) {
+  const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(v), CTRL, ROWS, 0xf, false);
+  const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(v), CTRL, ROWS, 0xf, false);
+  return __hiloint2double(hi, lo);
+}
+
+// Sum of v over the lanes from `head` to this one (head <= lane, the same for
+// every lane of a run): row shifts by 1, 2, 4, 8 within rows of 16 lanes,
+// then the last lane of row 0 / 2 into row 1 / 3 and of lane 31 into the
+// upper half.
+__device__ __forceinline__ double segment_scan(double v, int lane, int head) {
+  const int r = lane & 15;
+  double t;
+  t = dpp_move<0x111, 0xf>(v);
+  v += (r >= 1 && lane - 1 >= head) ? t : 0.0;
+  t = dpp_move<0x112, 0xf>(v);
+  v += (r >= 2 && lane - 2 >= head) ? t : 0.0;
+  t = dpp_move<0x114, 0xf>(v);
+  v += (r >= 4 && lane - 4 >= head) ? t : 0.0;
+  t = dpp_move<0x118, 0xf>(v);
+  v += (r >= 8 && lane - 8 >= head) ? t : 0.0;
+  t = dpp_move<0x142, 0xa>(v);   // row_bcast:15
+  v += ((lane & 16) && head < (lane & 48)) ? t : 0.0;
+  t = dpp_move<0x143, 0xc>(v);   // row_bcast:31
+  v += (lane >= 32 && head < 32) ? t : 0.0;
   return v;
 }
 
 // Slots per bin: 0 mode count, 1 sum of |k|, 2+q Re sum for pole q, and for
-// cross spectra 2+npoles+q the Im sum.  acc is [slot][bin].
-__global__ __launch_bounds__(kPkBlock) void pk_bin_kernel(const float2 *__restrict__ s1,
-                                                          const float2 *__restrict__ s2,
-                                                          const double *__restrict__ edges, PkParams p,
-                                                          double *__restrict__ partial) {
+// cross spectra 2+npoles+q the Im sum.  acc is [wave][slot][bin], then the
+// edges.
+template <int NP, bool CROSS, bool ANISO>
+__global__ __launch_bounds__(kPkMaxWaves * 64) void pk_bin_kernel(const float2 *__restrict__ s1,
+                                                                  const float2 *__restrict__ s2,
+                                                                  const double *__restrict__ edges, PkParams p,
+                                                                  double *__restrict__ partial) {
   extern __shared__ double acc[];
-  for (int e = threadIdx.x; e < p.nslots; e += blockDim.x) acc[e] = 0.0;
+  const int waves = int(blockDim.x >> 6), lane = int(threadIdx.x & 63u), wave = int(threadIdx.x >> 6);
+  double *ed = acc + waves * p.nslots;
+  for (int e = int(threadIdx.x); e < waves * p.nslots; e += int(blockDim.x)) acc[e] = 0.0;
+  for (int e = int(threadIdx.x); e < p.nedges; e += int(blockDim.x)) ed[e] = edges[e];
   __syncthreads();
-  const int lane = threadIdx.x & 63;
-  const int wave = threadIdx.x >> 6;
-  const int waves = blockDim.x >> 6;
-  const int64_t rows = int64_t(p.nx) * p.ny;
-  for (int64_t row = int64_t(blockIdx.x) * waves + wave; row < rows; row += int64_t(gridDim.x) * waves) {
-    const int i = int(row / p.ny);
-    const int j = int(row - int64_t(i) * p.ny);
-    const double kx = p.fac[0] * fftfreq(i, p.nx);
-    const double ky = p.fac[1] * fftfreq(j, p.ny);
-    // the Hermitian mirror's components (Nyquist entries mirror onto themselves)
-    const double kxm = p.fac[0] * fftfreq(i == 0 ? 0 : p.nx - i, p.nx);
-    const double kym = p.fac[1] * fftfreq(j == 0 ? 0 : p.ny - j, p.ny);
-    const float2 *r1 = s1 + row * p.nzh;
-    const float2 *r2 = s2 + row * p.nzh;
-    for (int k0 = 0; k0 < p.nzh; k0 += 64) {
-      const int k = k0 + lane;
-      const bool valid = k < p.nzh;
-      int bin = 0;
-      double cnt = 0.0, ks = 0.0;
-      double re[kPkMaxPoles], im[kPkMaxPoles];
+  double *mine = acc + wave * p.nslots;
+  const uint32_t stride = gridDim.x * uint32_t(waves) * 64u;
+  for (uint32_t base = (blockIdx.x * uint32_t(waves) + uint32_t(wave)) * 64u; base < p.modes; base += stride) {
+    const uint32_t m = base + uint32_t(lane);
+    const bool valid = m < p.modes;
+    int bin = -1;
+    bool pair = false;
+    double ks = 0.0, re[NP], im[NP];
 #pragma unroll
-      for (int q = 0; q < kPkMaxPoles; ++q) re[q] = im[q] = 0.0;
-      if (valid) {
-        const double kz = p.fac[2] * fftfreq(k, p.nz);
-        const double ksq = kx * kx + ky * ky + kz * kz;
-        const float kf = sqrt_rn(float(ksq));
-        bin = digitize(edges, p.nedges, double(kf));
-        const bool pair = k > 0 && 2 * k != p.nz;   // mirror not stored
-        const float2 a = r1[k];
-        const float2 b = p.cross ? r2[k] : a;
-        const double xr = double(a.x) * double(b.x) + double(a.y) * double(b.y);
-        const double xi = double(a.y) * double(b.x) - double(a.x) * double(b.y);
-        cnt = pair ? 2.0 : 1.0;
-        ks = cnt * double(kf);
-        double mu = 1.0, mum = 1.0;
-        if (p.aniso) {
-          const double kzm = p.fac[2] * fftfreq(k == 0 ? 0 : p.nz - k, p.nz);
-          const double num = kx * p.los[0] + ky * p.los[1] + kz * p.los[2];
-          const double numm = kxm * p.los[0] + kym * p.los[1] + kzm * p.los[2];
-          mu = kf == 0.0f ? 0.0 : num / double(kf);
-          mum = kf == 0.0f ? 0.0 : numm / double(kf);
+    for (int q = 0; q < NP; ++q) re[q] = im[q] = 0.0;
+    if (valid) {
+      const float2 a = s1[m];
+      const float2 b = CROSS ? s2[m] : a;
+      const uint32_t row = p.div_nzh.div(m);
+      const int k = int(m - row * uint32_t(p.nzh));
+      const uint32_t iu = p.div_ny.div(row);
+      const int i = int(iu), j = int(row - iu * uint32_t(p.ny));
+      const double kx = p.fac[0] * fftfreq(i, p.nx, p.inv[0]);
+      const double ky = p.fac[1] * fftfreq(j, p.ny, p.inv[1]);
+      const double kz = p.fac[2] * fftfreq(k, p.nz, p.inv[2]);
+      const float kf = __fsqrt_rn(float(kx * kx + ky * ky + kz * kz));
+      bin = digitize(ed, p.nedges, double(kf));
+      pair = k > 0 && 2 * k != p.nz;   // mirror not stored
+      const double xr = double(a.x) * double(b.x) + double(a.y) * double(b.y);
+      const double xi = CROSS ? double(a.y) * double(b.x) - double(a.x) * double(b.y) : 0.0;
+      ks = (pair ? 2.0 : 1.0) * double(kf);
+      // the mirror carries conj: Re adds, Im subtracts
+      if (!ANISO) {
+#pragma unroll
+        for (int q = 0; q < NP; ++q) {
+          re[q] = pair ? 2.0 * xr : xr;
+          im[q] = pair ? 0.0 : xi;
+        }
+      } else {
+        const double tx = kx * p.los[0], ty = ky * p.los[1], tz = kz * p.los[2];
+        double w[NP], wm[NP];
+        legendre_weights<NP>(p, kf == 0.0f ? 0.0 : (tx + ty + tz) / double(kf), w);
+        // The mirror of (kx, ky, kz) is its negative, and P_l(-mu) =
+        // (-1)^l P_l(mu), except that Nyquist components mirror onto
+        // themselves.
+        const bool nx2 = 2 * i == p.nx, ny2 = 2 * j == p.ny;
+        if (nx2 || ny2) {
+          const double numm = (nx2 ? tx : -tx) + (ny2 ? ty : -ty) - tz;
+          legendre_weights<NP>(p, kf == 0.0f ? 0.0 : numm / double(kf), wm);
+        } else {
+#pragma unroll
+          for (int q = 0; q < NP; ++q) wm[q] = (p.poles[q] & 1) ? -w[q] : w[q];
         }
 #pragma unroll
-        for (int q = 0; q < kPkMaxPoles; ++q) {
-          if (q < p.npoles) {
-            const int ell = p.poles[q];
-            const double w = double(2 * ell + 1) * legendre(ell, mu);
-            const double wm = pair ? double(2 * ell + 1) * legendre(ell, mum) : 0.0;
-            re[q] = (w + wm) * xr;   // the mirror carries conj: Re adds, Im subtracts
-            im[q] = (w - wm) * xi;
-          }
+        for (int q = 0; q < NP; ++q) {
+          if (!pair) wm[q] = 0.0;
+          re[q] = (w[q] + wm[q]) * xr;
+          im[q] = (w[q] - wm[q]) * xi;
         }
       }
-      uint64_t todo = __ballot(valid);
-      while (todo) {
-        const int leader = __ffsll((unsigned long long)todo) - 1;
-        const int lb = __shfl(bin, leader);
-        const bool mine = valid && bin == lb;
-        todo &= ~uint64_t(__ballot(mine));
-        double v = wave_sum(mine ? cnt : 0.0);
-        if (lane == leader) atomicAdd(&acc[lb], v);
-        v = wave_sum(mine ? ks : 0.0);
-        if (lane == leader) atomicAdd(&acc[p.nbins + lb], v);
+    }
+    // runs of one bin (neighbouring lanes), each summed into its last lane
+    const int prev = __shfl_up(bin, 1);
+    const unsigned long long heads = __ballot(lane == 0 || bin != prev) | 1ull;
+    const unsigned long long below = heads & ((2ull << lane) - 1ull);
+    const int head = 63 - __clzll((long long)below);
+    const bool last = lane == 63 || ((heads >> (lane + 1)) & 1ull);
+    const unsigned long long run = ((2ull << lane) - 1ull) & ~((1ull << head) - 1ull);
+    const unsigned long long pairs = __ballot(pair);
+    ks = segment_scan(ks, lane, head);
 #pragma unroll
-        for (int q = 0; q < kPkMaxPoles; ++q) {
-          if (q < p.npoles) {
-            v = wave_sum(mine ? re[q] : 0.0);
-            if (lane == leader) atomicAdd(&acc[(2 + q) * p.nbins + lb], v);
-            if (p.cross) {
-              v = wave_sum(mine ? im[q] : 0.0);
-              if (lane == leader) atomicAdd(&acc[(2 + p.npoles + q) * p.nbins + lb], v);
-            }
-          }
+    for (int q = 0; q < NP; ++q) {
+      re[q] = segment_scan(re[q], lane, head);
+      if (CROSS) im[q] = segment_scan(im[q], lane, head);
+    }
+    if (last && bin >= 0) {
+      unsafeAtomicAdd(&mine[bin], double(__popcll(run) + __popcll(run & pairs)));
+      unsafeAtomicAdd(&mine[p.nbins + bin], ks);
+#pragma unroll
+      for (int q = 0; q < NP; ++q) {
+        if (q < p.npoles) {
+          unsafeAtomicAdd(&mine[(2 + q) * p.nbins + bin], re[q]);
+          if (CROSS) unsafeAtomicAdd(&mine[(2 + p.npoles + q) * p.nbins + bin], im[q]);
         }
       }
     }
   }
   __syncthreads();
-  double *mine = partial + int64_t(blockIdx.x) * p.nslots;
-  for (int e = threadIdx.x; e < p.nslots; e += blockDim.x) mine[e] = acc[e];
+  double *out = partial + size_t(blockIdx.x) * size_t(p.nslots);
+  for (int e = int(threadIdx.x); e < p.nslots; e += int(blockDim.x)) {
+    double v = acc[e];
+    for (int w = 1; w < waves; ++w) v += acc[w * p.nslots + e];
+    out[e] = v;
+  }
 }
 
-__global__ void pk_reduce_kernel(const double *__restrict__ partial, int blocks, int nslots,
-                                 double *__restrict__ out) {
-  const int e = blockIdx.x * blockDim.x + threadIdx.x;
-  if (e >= nslots) return;
-  double s = 0.0;
-  for (int b = 0; b < blocks; ++b) s += partial[int64_t(b) * nslots + e];
-  out[e] = s;
+// out[e] = the sum of slot e over the workgroups: one wave per slot, each lane
+// a stride of 64 of them, then a fixed tree.
+__global__ void __launch_bounds__(64) pk_reduce_kernel(const double *__restrict__ partial, int blocks, int nslots,
+                                                       double *__restrict__ out) {
+  const int e = int(blockIdx.x);
+  double v = 0.0;
+  for (int b = int(threadIdx.x); b < blocks; b += 64) v += partial[size_t(b) * size_t(nslots) + size_t(e)];
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off);
+  if (threadIdx.x == 0) out[e] = v;
 }
 
-static int pk_blocks(int nx, int ny) {
-  const int64_t rows = int64_t(nx) * ny;
-  int64_t b = (rows + (kPkBlock / 64) - 1) / (kPkBlock / 64);
+// Waves of a workgroup: as many as have room for their own bins.
+static int pk_waves(int nslots) {
+  int w = kPkMaxWaves;
+  while (w > 1 && w * nslots > kPkLdsSlots) w >>= 1;
+  return w;
+}
+
+static int pk_blocks(int nx, int ny, int nz, int nslots) {
+  const int64_t per = 64 * pk_waves(nslots);
+  const int64_t b = (half_cells(nx, ny, nz) + per - 1) / per;
   return int(b < kPkMaxBlocks ? (b < 1 ? 1 : b) : kPkMaxBlocks);
+}
+
+template <int NP>
+static auto pk_kernel(bool cross, bool aniso) {
+  return cross ? (aniso ? pk_bin_kernel<NP, true, true> : pk_bin_kernel<NP, true, false>)
+               : (aniso ? pk_bin_kernel<NP, false, true> : pk_bin_kernel<NP, false, false>);
 }
 
 int pk_slots(int nedges, int npoles, int cross) { return (2 + npoles * (cross ? 2 : 1)) * (nedges + 1); }
 
 size_t power_spectrum_ws(int nx, int ny, int nz, int nedges, int npoles, int cross) {
   if (nx <= 0 || ny <= 0 || nz <= 0 || nedges < 0 || npoles < 1) return 0;
-  return size_t(pk_blocks(nx, ny)) * size_t(pk_slots(nedges, npoles, cross)) * sizeof(double);
+  const int nslots = pk_slots(nedges, npoles, cross);
+  return size_t(pk_blocks(nx, ny, nz, nslots)) * size_t(nslots) * sizeof(double);
 }
 
 int power_spectrum(hipStream_t s, int nx, int ny, int nz, const void *spec1, const void *spec2, double fx, double fy,
@@ -214,6 +269,12 @@ int power_spectrum(hipStream_t s, int nx, int ny, int nz, const void *spec1, con
   p.ny = ny;
   p.nz = nz;
   p.nzh = nz / 2 + 1;
+  p.modes = uint32_t(half_cells(nx, ny, nz));
+  p.div_nzh = FastDiv(uint32_t(p.nzh));
+  p.div_ny = FastDiv(uint32_t(ny));
+  p.inv[0] = 1.0 / double(nx);
+  p.inv[1] = 1.0 / double(ny);
+  p.inv[2] = 1.0 / double(nz);
   p.fac[0] = fx;
   p.fac[1] = fy;
   p.fac[2] = fz;
@@ -224,25 +285,31 @@ int power_spectrum(hipStream_t s, int nx, int ny, int nz, const void *spec1, con
   p.nbins = nedges + 1;
   p.nslots = nslots;
   p.npoles = npoles;
-  p.cross = cross;
-  p.aniso = 0;
   for (int q = 0; q < npoles; ++q) {
     JPM_REQUIRE(poles[q] >= 0 && poles[q] <= 64, "power spectrum: multipole %d outside [0, 64]", poles[q]);
     p.poles[q] = poles[q];
-    if (poles[q] != 0) p.aniso = 1;
+    if (poles[q] > p.lmax) p.lmax = poles[q];
   }
-  const int blocks = pk_blocks(nx, ny);
+  const bool aniso = p.lmax > 0;
+  const int blocks = pk_blocks(nx, ny, nz, nslots), waves = pk_waves(nslots);
   double *partial = static_cast<double *>(ws);
+  const size_t lds = (size_t(waves) * size_t(nslots) + size_t(nedges)) * sizeof(double);
+  auto kern = npoles == 1   ? pk_kernel<1>(cross, aniso)
+              : npoles == 2 ? pk_kernel<2>(cross, aniso)
+              : npoles == 3 ? pk_kernel<3>(cross, aniso)
+                            : pk_kernel<kPkMaxPoles>(cross, aniso);
+  if (lds > 65536)
+    JPM_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(kern), hipFuncAttributeMaxDynamicSharedMemorySize,
+                                int(lds)));
   {
     JPM_TIMED(s, "pk_bin_kernel");
-    hipLaunchKernelGGL(pk_bin_kernel, dim3(blocks), dim3(kPkBlock), size_t(nslots) * sizeof(double), s,
-                       static_cast<const float2 *>(spec1), static_cast<const float2 *>(cross ? spec2 : spec1),
-                       edges, p, partial);
+    hipLaunchKernelGGL(kern, dim3(blocks), dim3(64 * waves), lds, s, static_cast<const float2 *>(spec1),
+                       static_cast<const float2 *>(cross ? spec2 : spec1), edges, p, partial);
     JPM_LAUNCHED("pk_bin_kernel");
   }
   {
     JPM_TIMED(s, "pk_reduce_kernel");
-    hipLaunchKernelGGL(pk_reduce_kernel, dim3((nslots + 255) / 256), dim3(256), 0, s, partial, blocks, nslots, out);
+    hipLaunchKernelGGL(pk_reduce_kernel, dim3(nslots), dim3(64), 0, s, partial, blocks, nslots, out);
     JPM_LAUNCHED("pk_reduce_kernel");
   }
   return JPM_OK;

@@ -52,6 +52,32 @@ def test_power_spectrum_cross_multipoles(gpu, shape, box):
             np.testing.assert_allclose(got, rp, rtol=1e-5, atol=1e-5 * np.abs(rp).max())
 
 
+@pytest.mark.parametrize("shape,bins,poles", [((6, 5, 126), 9, [0, 2, 4]), ((5, 3, 127), 400, [0, 1, 2, 3, 4]),
+                                              ((4, 6, 128), 700, [0, 2, 4, 6]), ((3, 2, 1), 3, [0, 3]),
+                                              ((2, 4, 2), 5, [0, 2]), ((7, 9, 33), 1300, [0, 2])])
+def test_power_spectrum_wave_and_slot_edges(gpu, shape, bins, poles):
+    """Rows of 63, 64, 65, 1, 2 and 17 modes against waves of 64, mode counts
+    that end inside a wave, and slot counts that give a workgroup 4, 2 and 1
+    waves.  Within 1e-5 of the largest value, as the float32 transforms are
+    the only difference; a bin of few modes has no smaller error."""
+    from jaxpm_amd import utils
+    r = np.random.default_rng(44)
+    a = r.normal(size=shape).astype(np.float32)
+    b = (0.6 * a + r.normal(size=shape)).astype(np.float32)
+    edges = np.linspace(0.01, 1.02 * np.pi * np.sqrt(3.0), bins)
+    los = (0.3, -1.0, 2.0)
+    for mesh2 in (None, b):
+        print(f"pk edges {shape} bins={bins} poles={poles} cross={mesh2 is not None}", flush=True)
+        k, p = utils.power_spectrum(dev(a), None if mesh2 is None else dev(mesh2), kedges=edges, multipoles=poles,
+                                    los=los)
+        rk, rp = ou.power_spectrum(a, mesh2, kedges=edges, multipoles=poles, los=los)
+        got = p.cpu().numpy()
+        assert np.array_equal(np.isnan(k), np.isnan(rk)) and np.array_equal(np.isnan(got), np.isnan(rp))
+        ok = ~np.isnan(rk)
+        np.testing.assert_allclose(k[ok], rk[ok], rtol=1e-12)
+        np.testing.assert_allclose(got[:, ok], rp[:, ok], rtol=1e-5, atol=1e-5 * np.abs(rp[:, ok]).max())
+
+
 def test_transfer_coherence(gpu):
     from jaxpm_amd import utils
     r = np.random.default_rng(42)
