@@ -16,7 +16,7 @@
 // not by the 8 bytes a mode.  256^3, poles 0 2 4: 1671 + 127 us when each
 // run of a bin was summed by its own full-wave reductions, the wave numbers
 // divided per mode, and the partial sums added by one thread per slot; now
-// 120 + 14 us.
+// 123 + 14 us.
 #include <cmath>
 
 #include "common.hpp"
@@ -139,7 +139,9 @@ __global__ __launch_bounds__(kPkMaxWaves * 64) void pk_bin_kernel(const float2 *
       const double kx = p.fac[0] * fftfreq(i, p.nx, p.inv[0]);
       const double ky = p.fac[1] * fftfreq(j, p.ny, p.inv[1]);
       const double kz = p.fac[2] * fftfreq(k, p.nz, p.inv[2]);
-      const float kf = __fsqrt_rn(float(kx * kx + ky * ky + kz * kz));
+      // sqrtf rounds correctly here, as NumPy's float32 root does (with the
+      // compiler's default options; the __fsqrt_rn intrinsic does not)
+      const float kf = sqrtf(float(kx * kx + ky * ky + kz * kz));
       bin = digitize(ed, p.nedges, double(kf));
       pair = k > 0 && 2 * k != p.nz;   // mirror not stored
       const double xr = double(a.x) * double(b.x) + double(a.y) * double(b.y);
