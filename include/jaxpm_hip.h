@@ -554,6 +554,17 @@ int jpm_density_plane_f32(void *stream, const float *pos, int64_t n,
                           int box_nx, int box_ny, double center, double width,
                           int res, float *plane);
 
+/* jpm_density_plane_f32 with a workspace of
+ * jpm_density_plane_workspace_size(n, res) bytes, in which many particles are
+ * sorted by plane tile and summed without atomics on the pixels.  Where that
+ * size is 0 (few particles, or a plane of more than 4096^2 pixels) ws may be
+ * NULL and the call is jpm_density_plane_f32. */
+size_t jpm_density_plane_workspace_size(int64_t n, int res);
+int jpm_density_plane_ws_f32(void *stream, const float *pos, int64_t n,
+                             int box_nx, int box_ny, double center,
+                             double width, int res, float *plane, void *ws,
+                             size_t ws_bytes);
+
 /* Adjoint of jpm_density_plane_f32 for a plane cotangent g[res][res], which
  * is overwritten (divided by the normalisation): gpos[n][3] = the position
  * cotangent (z and the particles outside the slab get 0). */

@@ -128,6 +128,8 @@ SIGNATURES = {
     "jpm_cic_paint_2d_f32": (_i, [_vp, _i, _i, _vp, _i64, _i, _vp, _vp]),
     "jpm_cic_paint_2d_vjp_f32": (_i, [_vp, _i, _i, _vp, _i64, _i, _vp, _vp, _vp, _i, _vp]),
     "jpm_density_plane_f32": (_i, [_vp, _vp, _i64, _i, _i, _d, _d, _i, _vp]),
+    "jpm_density_plane_workspace_size": (_sz, [_i64, _i]),
+    "jpm_density_plane_ws_f32": (_i, [_vp, _vp, _i64, _i, _i, _d, _d, _i, _vp, _vp, _sz]),
     "jpm_density_plane_vjp_f32": (_i, [_vp, _vp, _i64, _i, _i, _d, _d, _i, _vp, _vp]),
     "jpm_gaussian_smoothing_workspace_size": (_sz, [_i, _i]),
     "jpm_gaussian_smoothing_f32": (_i, [_vp, _i, _i, _vp, _vp, _d, _vp, _sz]),

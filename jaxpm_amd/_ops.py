@@ -472,11 +472,14 @@ def paint_2d_vjp(g, pos2, weight=None, want_pos=True, want_weight=False):
 
 
 def density_plane(pos, box_shape, center, width, res):
-    """A new res x res plane (jpm_density_plane_f32) of positions (n, 3)."""
+    """A new res x res plane (jpm_density_plane_ws_f32) of positions (n, 3)."""
     pos = _f32(pos, "positions")
+    n = pos.numel() // 3
     plane = torch.empty((res, res), dtype=torch.float32, device=pos.device)
-    call("jpm_density_plane_f32", stream(), ptr(pos), pos.numel() // 3, int(box_shape[0]), int(box_shape[1]),
-         float(center), float(width), int(res), ptr(plane))
+    wsb = size("jpm_density_plane_workspace_size", n, int(res))
+    ws = torch.empty(wsb, dtype=torch.uint8, device=pos.device) if wsb else None
+    call("jpm_density_plane_ws_f32", stream(), ptr(pos), n, int(box_shape[0]), int(box_shape[1]), float(center),
+         float(width), int(res), ptr(plane), ptr(ws), wsb)
     return plane
 
 

@@ -63,25 +63,6 @@ __device__ __forceinline__ uint32_t tile_key(int cx, int cy, int cz, const TileG
 
 // --------------------------------------------------------------- count
 
-// Runs of equal keys among the 64 lanes of a wavefront: `heads` has bit l set
-// when lane l starts a run (its key differs from lane l-1's, or l is lane 0);
-// a head's run ends where the next head begins or at the last active lane
-// (active lanes are always a prefix of the wavefront).
-__device__ __forceinline__ unsigned long long run_heads(uint32_t key, bool active) {
-  const int lane = threadIdx.x & 63;
-  const uint32_t prev = __shfl_up(key, 1);
-  const bool head = active && (lane == 0 || key != prev);
-  return __ballot(head);
-}
-
-__device__ __forceinline__ uint32_t run_length(unsigned long long heads, unsigned long long act) {
-  const int lane = threadIdx.x & 63;
-  const unsigned long long above = heads & ~((2ull << lane) - 1ull);
-  const int next = above ? __ffsll((long long)above) - 1 : 64;
-  const int last_active = 63 - __clzll((long long)act);
-  return uint32_t(min(next, last_active + 1) - lane);
-}
-
 // The particle range [p0, p1) of count/scatter workgroup `blk` of simulation s.
 __device__ __forceinline__ void block_range(const SimRef &s, uint32_t blk, uint32_t slice, uint32_t &p0,
                                             uint32_t &p1) {
@@ -329,6 +310,15 @@ tile_table_kernel(const uint32_t *__restrict__ count, uint32_t K, uint32_t chunk
       desc[cb] = d;
     }
   }
+}
+
+int tile_table(hipStream_t s, const uint32_t *count, uint32_t K, uint32_t chunk, uint32_t *tstart, uint32_t *cursor,
+               uint32_t *nchunk, uint32_t *choff, uint32_t *totals, ChunkDesc *desc) {
+  JPM_REQUIRE(K >= 1 && K <= kTableMaxK, "%u tiles exceed the tile table's %u", K, kTableMaxK);
+  hipLaunchKernelGGL(tile_table_kernel, dim3((K + kTableThreads - 1) / kTableThreads), dim3(kTableThreads), 0, s,
+                     count, K, chunk, tstart, cursor, nchunk, choff, totals, desc);
+  JPM_LAUNCHED("tile_table_kernel");
+  return JPM_OK;
 }
 
 // -------------------------------------------------------------- scatter
@@ -1114,10 +1104,9 @@ static int sort_into(hipStream_t s, const G &g, const SortDims &d, uint32_t M, b
   }
   // 2. tile starts, scatter cursors, chunk table
   if (d.K <= kTableMaxK) {
-    hipLaunchKernelGGL(tile_table_kernel, dim3((d.K + kTableThreads - 1) / kTableThreads), dim3(kTableThreads), 0, s,
-                       count, d.K, d.chunk, tstart, cursor,
-                       nchunk, choff, totals, reinterpret_cast<ChunkDesc *>(base + w.desc));
-    JPM_LAUNCHED("tile_table_kernel");
+    rc = tile_table(s, count, d.K, d.chunk, tstart, cursor, nchunk, choff, totals,
+                    reinterpret_cast<ChunkDesc *>(base + w.desc));
+    if (rc) return rc;
   } else {
     JPM_HIP(hipMemcpyAsync(tstart, count, size_t(d.K) * 4, hipMemcpyDeviceToDevice, s));
     rc = exclusive_scan(s, tstart, d.K, sums, totals);

@@ -119,7 +119,8 @@ int permute_rows(hipStream_t, int64_t, const uint32_t *, const float *, float *,
 int paint_2d(hipStream_t, int, int, const float *, int64_t, int, const float *, float *);
 int paint_2d_vjp(hipStream_t, int, int, const float *, int64_t, int, const float *, const float *, float *, int,
                  float *);
-int density_plane(hipStream_t, const float *, int64_t, int, int, double, double, int, float *);
+size_t density_plane_ws(int64_t, int);
+int density_plane(hipStream_t, const float *, int64_t, int, int, double, double, int, float *, void *, size_t);
 int density_plane_vjp(hipStream_t, const float *, int64_t, int, int, double, double, int, float *, float *);
 size_t gaussian_smoothing_ws(int, int);
 int gaussian_smoothing(hipStream_t, int, int, const float *, float *, double, void *, size_t);
@@ -872,7 +873,14 @@ int jpm_cic_paint_2d_vjp_f32(void *stream, int nx, int ny, const float *pos, int
 
 int jpm_density_plane_f32(void *stream, const float *pos, int64_t n, int box_nx, int box_ny, double center,
                           double width, int res, float *plane) {
-  JPM_GUARD(density_plane(as_stream(stream), pos, n, box_nx, box_ny, center, width, res, plane));
+  JPM_GUARD(density_plane(as_stream(stream), pos, n, box_nx, box_ny, center, width, res, plane, nullptr, 0));
+}
+
+size_t jpm_density_plane_workspace_size(int64_t n, int res) { return density_plane_ws(n, res); }
+
+int jpm_density_plane_ws_f32(void *stream, const float *pos, int64_t n, int box_nx, int box_ny, double center,
+                             double width, int res, float *plane, void *ws, size_t ws_bytes) {
+  JPM_GUARD(density_plane(as_stream(stream), pos, n, box_nx, box_ny, center, width, res, plane, ws, ws_bytes));
 }
 
 int jpm_density_plane_vjp_f32(void *stream, const float *pos, int64_t n, int box_nx, int box_ny, double center,

@@ -5,10 +5,10 @@
 // 2-D transforms.
 //
 // A plane is small next to the particle arrays (1024^2 cells are 4 MB, 256^3
-// particles 201 MB), so the paints stream the particles once and add their
-// four deposits with float atomics, which L2 absorbs; the density plane
-// reads only the particles and skips those outside the slab, whose deposits
-// are zeros.
+// particles 201 MB), so the 2-D paint streams the particles once and adds
+// its four deposits with float atomics; so does the density plane of few
+// particles.  Many particles go through a counting sort into 64 x 64-pixel
+// tiles first and are summed in LDS windows (plane_select_kernel and below).
 #include "tiles.hpp"
 
 namespace jpm {
@@ -99,6 +99,205 @@ density_plane_kernel(const float *__restrict__ pos, uint32_t n, float bnx, float
 #pragma unroll
     for (int o = 0; o < 4; ++o) atomicAdd(&plane[c.idx[o]], c.w[o]);
   }
+}
+
+// The density plane of many particles, without global atomics on pixels:
+//   select   one pass over the particles: those of the slab become records
+//            (their plane coordinates, 8 bytes), compacted, and are counted
+//            per 64 x 64-pixel tile
+//   (tile table: tile starts and chunk descriptors)
+//   scatter  the records into tile order
+//   accum    one workgroup per chunk of a tile's records: a 65 x 65 window of
+//            float64 sums in LDS (ds_add_f64), stored as floats
+//   reduce   each pixel sums its tile's windows and, on a low edge, the +1
+//            halos of the lower neighbours, and divides by the normalisation
+// One float atomic per corner runs at about 25 G/s whatever the order of the
+// particles (lines shared by the 8 XCDs' L2s).  256^3 particles, a quarter in
+// the slab, 1024^2 pixels, lattice order: 673 -> 134 us, of which the select
+// pass over the positions 76.
+constexpr int kPt = 64, kPw = kPt + 1, kPwCells = kPw * kPw;
+constexpr uint32_t kPlaneSelect = 4096;     // particles per select workgroup, records per scatter workgroup
+constexpr uint32_t kPlaneChunk = 8192;      // records per window
+constexpr uint32_t kPlaneMaxTiles = 4096;   // 4096^2 pixels: the LDS histogram is 16 KiB
+constexpr int64_t kPlaneSortMin = 3 << 18;
+
+struct PlaneTiles {
+  int res, t;   // pixels and tiles per axis
+  FastDiv div_t;
+};
+
+__device__ __forceinline__ int plane_cell(float u, int res) { return wrapi(cell_int(floorf(u)), res); }
+
+__device__ __forceinline__ uint32_t plane_tile(float2 r, const PlaneTiles &t) {
+  return uint32_t(plane_cell(r.x, t.res) / kPt) * uint32_t(t.t) + uint32_t(plane_cell(r.y, t.res) / kPt);
+}
+
+__device__ __forceinline__ int plane_len(int i, const PlaneTiles &t) {
+  return i == t.t - 1 ? t.res - i * kPt : kPt;
+}
+
+__global__ void __launch_bounds__(64) plane_clear_kernel(uint32_t *__restrict__ a, uint32_t n) {
+  for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) a[i] = 0u;
+}
+
+// nsel[0] selected particles, count[t] of them in tile t (both start at 0).
+__global__ void __launch_bounds__(256)
+plane_select_kernel(const float *__restrict__ pos, uint32_t n, float bnx, float lo, float hi, PlaneTiles t,
+                    uint32_t *__restrict__ nsel, uint32_t *__restrict__ count, float2 *__restrict__ recs) {
+  __shared__ float2 stage[kPlaneSelect];
+  __shared__ uint32_t cnt, base;
+  extern __shared__ uint32_t hist[];
+  const uint32_t T = uint32_t(t.t) * uint32_t(t.t);
+  if (threadIdx.x == 0) cnt = 0;
+  for (uint32_t k = threadIdx.x; k < T; k += 256) hist[k] = 0;
+  __syncthreads();
+  const int lane = threadIdx.x & 63;
+  const uint32_t p0 = blockIdx.x * kPlaneSelect;
+  constexpr int kPer = 4;   // particles of a thread whose loads are in flight together
+  for (uint32_t b = 0; b < kPlaneSelect; b += 256 * kPer) {
+    float x[kPer], y[kPer], z[kPer];
+#pragma unroll
+    for (int i = 0; i < kPer; ++i) {
+      const uint32_t p = p0 + b + uint32_t(i) * 256 + threadIdx.x;
+      const size_t at = 3 * size_t(p < n ? p : n - 1);
+      x[i] = pos[at];
+      y[i] = pos[at + 1];
+      z[i] = p < n ? pos[at + 2] : NAN;
+    }
+#pragma unroll
+    for (int i = 0; i < kPer; ++i) {
+      const bool in = z[i] > lo && z[i] <= hi;
+      const unsigned long long act = __ballot(in);
+      uint32_t at = 0;
+      if (lane == 0 && act) at = atomicAdd(&cnt, uint32_t(__popcll(act)));
+      at = __shfl(at, 0) + uint32_t(__popcll(act & ((1ull << lane) - 1ull)));
+      if (in) stage[at] = make_float2(plane_coord(x[i], bnx, float(t.res)), plane_coord(y[i], bnx, float(t.res)));
+    }
+  }
+  __syncthreads();
+  const uint32_t m = cnt;
+  if (threadIdx.x == 0 && m) base = atomicAdd(nsel, m);
+  __syncthreads();
+  for (uint32_t b = 0; b < m; b += 256) {
+    const uint32_t q = b + threadIdx.x;
+    const bool active = q < m;
+    uint32_t key = 0xffffffffu;
+    if (active) {
+      const float2 r = stage[q];
+      recs[base + q] = r;
+      key = plane_tile(r, t);
+    }
+    const unsigned long long act = __ballot(active);
+    const unsigned long long heads = run_heads(key, active);
+    if (active && ((heads >> lane) & 1ull)) atomicAdd(&hist[key], run_length(heads, act));
+  }
+  __syncthreads();
+  for (uint32_t k = threadIdx.x; k < T; k += 256)
+    if (hist[k]) atomicAdd(&count[k], hist[k]);
+}
+
+__global__ void __launch_bounds__(512)
+plane_scatter_kernel(const float2 *__restrict__ recs, const uint32_t *__restrict__ nsel, PlaneTiles t,
+                     uint32_t *__restrict__ cursor, float2 *__restrict__ sorted) {
+  extern __shared__ uint32_t cur[];
+  const uint32_t n = *nsel, p0 = blockIdx.x * kPlaneSelect;
+  if (p0 >= n) return;
+  constexpr int kPer = int(kPlaneSelect) / 512;
+  const uint32_t T = uint32_t(t.t) * uint32_t(t.t);
+  const int lane = threadIdx.x & 63;
+  for (uint32_t k = threadIdx.x; k < T; k += 512) cur[k] = 0;
+  float2 r[kPer];
+  uint32_t key[kPer];
+#pragma unroll
+  for (int i = 0; i < kPer; ++i) {
+    const uint32_t p = p0 + uint32_t(i) * 512 + threadIdx.x;
+    r[i] = recs[p < n ? p : n - 1];
+  }
+#pragma unroll
+  for (int i = 0; i < kPer; ++i) {
+    const uint32_t p = p0 + uint32_t(i) * 512 + threadIdx.x;
+    key[i] = p < n ? plane_tile(r[i], t) : 0xffffffffu;
+  }
+  __syncthreads();
+#pragma unroll
+  for (int i = 0; i < kPer; ++i) {
+    const bool active = key[i] != 0xffffffffu;
+    const unsigned long long act = __ballot(active);
+    const unsigned long long heads = run_heads(key[i], active);
+    if (active && ((heads >> lane) & 1ull)) atomicAdd(&cur[key[i]], run_length(heads, act));
+  }
+  __syncthreads();
+  for (uint32_t k = threadIdx.x; k < T; k += 512)
+    if (cur[k]) cur[k] = atomicAdd(&cursor[k], cur[k]);
+  __syncthreads();
+#pragma unroll
+  for (int i = 0; i < kPer; ++i) {
+    const bool active = key[i] != 0xffffffffu;
+    const unsigned long long act = __ballot(active);
+    const unsigned long long heads = run_heads(key[i], active);
+    uint32_t base = 0;
+    if (active && ((heads >> lane) & 1ull)) base = atomicAdd(&cur[key[i]], run_length(heads, act));
+    const unsigned long long below = heads & ((2ull << lane) - 1ull);
+    const int my_head = below ? 63 - __clzll((long long)below) : 0;
+    base = __shfl(base, my_head);
+    if (active) sorted[base + uint32_t(lane - my_head)] = r[i];
+  }
+}
+
+// The two corners of a plane coordinate in its tile's window, and their
+// weights (Cic2's).  A NaN coordinate has both corners at cell 0, as there.
+__device__ __forceinline__ void plane_corners(float u, int origin, int res, int l[2], float w[2]) {
+  const float f = floorf(u);
+  l[0] = plane_cell(u, res) - origin;
+  l[1] = u == u ? l[0] + 1 : l[0];
+  w[0] = 1.0f - fabsf(u - f);
+  w[1] = 1.0f - fabsf(u - (f + 1.0f));
+}
+
+__global__ void __launch_bounds__(512)
+plane_accum_kernel(const float2 *__restrict__ sorted, const ChunkDesc *__restrict__ desc,
+                   const uint32_t *__restrict__ nchunks, PlaneTiles t, float *__restrict__ partial) {
+  __shared__ double win[kPwCells];
+  if (blockIdx.x >= *nchunks) return;
+  const ChunkDesc d = desc[blockIdx.x];
+  const uint32_t tx = t.div_t.div(d.tile), ty = d.tile - tx * uint32_t(t.t);
+  for (int i = threadIdx.x; i < kPwCells; i += 512) win[i] = 0.0;
+  __syncthreads();
+  float2 next = sorted[d.start + (threadIdx.x < d.count ? threadIdx.x : 0u)];
+  for (uint32_t q = threadIdx.x; q < d.count; q += 512) {
+    const float2 r = next;
+    if (q + 512 < d.count) next = sorted[d.start + q + 512];
+    int lx[2], ly[2];
+    float wx[2], wy[2];
+    plane_corners(r.x, int(tx) * kPt, t.res, lx, wx);
+    plane_corners(r.y, int(ty) * kPt, t.res, ly, wy);
+#pragma unroll
+    for (int o = 0; o < 4; ++o)
+      unsafeAtomicAdd(&win[lx[o & 1] * kPw + ly[o >> 1]], double(wx[o & 1] * wy[o >> 1]));
+  }
+  __syncthreads();
+  float *out = partial + size_t(blockIdx.x) * kPwCells;
+  for (int i = threadIdx.x; i < kPwCells; i += 512) out[i] = float(win[i]);
+}
+
+// blockIdx.x: tile; blockIdx.y: 4 of its 64 rows, one pixel per thread.
+__global__ void __launch_bounds__(256)
+plane_reduce_kernel(const float *__restrict__ partial, const uint32_t *__restrict__ nchunk,
+                    const uint32_t *__restrict__ choff, PlaneTiles t, float norm, float *__restrict__ plane) {
+  const int tx = int(t.div_t.div(blockIdx.x)), ty = int(blockIdx.x) - tx * t.t;
+  const int a = int(blockIdx.y) * 4 + int(threadIdx.x >> 6), b = int(threadIdx.x & 63u);
+  if (a >= plane_len(tx, t) || b >= plane_len(ty, t)) return;
+  const int px = tx ? tx - 1 : t.t - 1, py = ty ? ty - 1 : t.t - 1;
+  double acc = 0.0;
+  for (int sx = 0; sx <= (a == 0 ? 1 : 0); ++sx)
+    for (int sy = 0; sy <= (b == 0 ? 1 : 0); ++sy) {
+      const uint32_t src = uint32_t(sx ? px : tx) * uint32_t(t.t) + uint32_t(sy ? py : ty);
+      const int la = sx ? plane_len(px, t) : a, lb = sy ? plane_len(py, t) : b;
+      const float *w = partial + size_t(choff[src]) * kPwCells + la * kPw + lb;
+      const uint32_t n = nchunk[src];
+      for (uint32_t k = 0; k < n; ++k) acc += double(w[size_t(k) * kPwCells]);
+    }
+  plane[uint32_t(tx * kPt + a) * uint32_t(t.res) + uint32_t(ty * kPt + b)] = float(acc) / norm;
 }
 
 // Adjoint of the density plane for a plane cotangent g (already divided by
@@ -203,8 +402,84 @@ static PlaneArgs plane_args(int box_nx, int box_ny, double center, double width,
   return a;
 }
 
+// Workspace of the sorted density plane (byte offsets); total 0 where one
+// float atomic per corner is used instead: few particles, or more tiles than
+// the LDS histogram holds.  A quarter of 64^3 particles takes 14-22 us by
+// atomics and 29-45 us sorted, of 96^3 31-67 against 34-55 us, of 128^3
+// 63-207 against 40-90 us (128^2 to 1024^2 pixels, both orders).
+struct PlaneWs {
+  uint32_t T, maxchunks;
+  size_t count, nsel, tstart, cursor, nchunk, choff, totals, desc, recs, sorted, partial, total;
+};
+
+static PlaneWs plane_ws(int64_t n, int res) {
+  PlaneWs w{};
+  if (n < kPlaneSortMin || n > int64_t(0xffffffffu) || res <= 0) return w;
+  const uint64_t t = uint64_t((res + kPt - 1) / kPt);
+  if (t * t > kPlaneMaxTiles) return w;
+  w.T = uint32_t(t * t);
+  w.maxchunks = uint32_t((uint64_t(n) + kPlaneChunk - 1) / kPlaneChunk + w.T);
+  size_t o = 0;
+  auto take = [&o](size_t bytes) {
+    const size_t at = o;
+    o += align_up(bytes);
+    return at;
+  };
+  w.count = take((size_t(w.T) + 1) * 4);
+  w.nsel = w.count + size_t(w.T) * 4;   // cleared with the counts
+  w.tstart = take(size_t(w.T) * 4);
+  w.cursor = take(size_t(w.T) * 4);
+  w.nchunk = take(size_t(w.T) * 4);
+  w.choff = take(size_t(w.T) * 4);
+  w.totals = take(16);
+  w.desc = take(size_t(w.maxchunks) * sizeof(ChunkDesc));
+  w.recs = take(size_t(n) * sizeof(float2));
+  w.sorted = take(size_t(n) * sizeof(float2));
+  w.partial = take(size_t(w.maxchunks) * kPwCells * sizeof(float));
+  w.total = o;
+  return w;
+}
+
+size_t density_plane_ws(int64_t n, int res) { return plane_ws(n, res).total; }
+
+static int density_plane_sorted(hipStream_t s, const float *pos, uint32_t n, float bnx, const PlaneArgs &a, int res,
+                                float *plane, char *base, const PlaneWs &w) {
+  PlaneTiles t;
+  t.res = res;
+  t.t = (res + kPt - 1) / kPt;
+  t.div_t = FastDiv(uint32_t(t.t));
+  auto *count = reinterpret_cast<uint32_t *>(base + w.count);
+  auto *nsel = reinterpret_cast<uint32_t *>(base + w.nsel);
+  auto *cursor = reinterpret_cast<uint32_t *>(base + w.cursor);
+  auto *nchunk = reinterpret_cast<uint32_t *>(base + w.nchunk);
+  auto *choff = reinterpret_cast<uint32_t *>(base + w.choff);
+  auto *totals = reinterpret_cast<uint32_t *>(base + w.totals);
+  auto *desc = reinterpret_cast<ChunkDesc *>(base + w.desc);
+  auto *recs = reinterpret_cast<float2 *>(base + w.recs);
+  auto *sorted = reinterpret_cast<float2 *>(base + w.sorted);
+  auto *partial = reinterpret_cast<float *>(base + w.partial);
+  const unsigned grid = unsigned((uint64_t(n) + kPlaneSelect - 1) / kPlaneSelect);
+  hipLaunchKernelGGL(plane_clear_kernel, dim3((w.T + 64) / 64), dim3(64), 0, s, count, w.T + 1);
+  JPM_LAUNCHED("plane_clear_kernel");
+  hipLaunchKernelGGL(plane_select_kernel, dim3(grid), dim3(256), size_t(w.T) * 4, s, pos, n, bnx, a.lo, a.hi, t, nsel,
+                     count, recs);
+  JPM_LAUNCHED("plane_select_kernel");
+  int rc = tile_table(s, count, w.T, kPlaneChunk, reinterpret_cast<uint32_t *>(base + w.tstart), cursor, nchunk, choff,
+                      totals, desc);
+  if (rc) return rc;
+  hipLaunchKernelGGL(plane_scatter_kernel, dim3(grid), dim3(512), size_t(w.T) * 4, s, recs, nsel, t, cursor, sorted);
+  JPM_LAUNCHED("plane_scatter_kernel");
+  hipLaunchKernelGGL(plane_accum_kernel, dim3(w.maxchunks), dim3(512), 0, s, sorted, desc, totals + 1, t, partial);
+  JPM_LAUNCHED("plane_accum_kernel");
+  hipLaunchKernelGGL(plane_reduce_kernel, dim3(w.T, kPt / 4), dim3(256), 0, s, partial, nchunk, choff, t, a.norm,
+                     plane);
+  JPM_LAUNCHED("plane_reduce_kernel");
+  return JPM_OK;
+}
+
+// ws: density_plane_ws(n, res) bytes, or null for the form without one.
 int density_plane(hipStream_t s, const float *pos, int64_t n, int box_nx, int box_ny, double center, double width,
-                  int res, float *plane) {
+                  int res, float *plane, void *ws, size_t ws_bytes) {
   JPM_REQUIRE(box_nx > 0 && box_ny > 0, "box shape must be positive");
   JPM_REQUIRE(res > 0 && int64_t(res) * res <= kMaxCells, "plane resolution %d out of range", res);
   JPM_REQUIRE(n >= 0 && n <= int64_t(0xffffffffu), "particle count %lld out of range", (long long)n);
@@ -212,6 +487,12 @@ int density_plane(hipStream_t s, const float *pos, int64_t n, int box_nx, int bo
   const PlaneArgs a = plane_args(box_nx, box_ny, center, width, res);
   const uint32_t m = uint32_t(res) * uint32_t(res);
   JPM_TIMED(s, "density_plane");
+  if (ws) {
+    const PlaneWs w = plane_ws(n, res);
+    JPM_REQUIRE(ws_bytes >= w.total, "the density plane needs %zu workspace bytes, got %zu", w.total, ws_bytes);
+    if (w.total)
+      return density_plane_sorted(s, pos, uint32_t(n), float(box_nx), a, res, plane, static_cast<char *>(ws), w);
+  }
   hipLaunchKernelGGL(plane_zero_kernel, dim3(grid_for(m, 256, 4096)), dim3(256), 0, s, plane, m);
   JPM_LAUNCHED("plane_zero_kernel");
   if (n > 0) {

@@ -118,6 +118,25 @@ __device__ __forceinline__ float4 load_global(const float4 *p) {
   return make_float4(q[0], q[1], q[2], q[3]);
 }
 
+// Runs of equal keys among the 64 lanes of a wavefront: `heads` has bit l set
+// when lane l starts a run (its key differs from lane l-1's, or l is lane 0);
+// a head's run ends where the next head begins or at the last active lane
+// (active lanes are always a prefix of the wavefront).
+__device__ __forceinline__ unsigned long long run_heads(uint32_t key, bool active) {
+  const int lane = threadIdx.x & 63;
+  const uint32_t prev = __shfl_up(key, 1);
+  const bool head = active && (lane == 0 || key != prev);
+  return __ballot(head);
+}
+
+__device__ __forceinline__ uint32_t run_length(unsigned long long heads, unsigned long long act) {
+  const int lane = threadIdx.x & 63;
+  const unsigned long long above = heads & ~((2ull << lane) - 1ull);
+  const int next = above ? __ffsll((long long)above) - 1 : 64;
+  const int last_active = 63 - __clzll((long long)act);
+  return uint32_t(min(next, last_active + 1) - lane);
+}
+
 struct TileGrid {
   int nx, ny, nz;   // mesh
   int tx, ty, tz;   // tiles per axis
@@ -171,6 +190,12 @@ __device__ __forceinline__ int floor_cell_rel(float p, int n) {
 struct ChunkDesc {
   uint32_t tile, start, count, pad;
 };
+
+// The tile table of at most 32768 tile counts (bin.hip): tile starts, scatter
+// cursors, chunks per tile and their offsets, totals [particles, chunks, 0]
+// and the chunk descriptors.
+int tile_table(hipStream_t s, const uint32_t *count, uint32_t K, uint32_t chunk, uint32_t *tstart, uint32_t *cursor,
+               uint32_t *nchunk, uint32_t *choff, uint32_t *totals, ChunkDesc *desc);
 
 // One simulation as the tile-sort kernels see it.  A batch concatenates its
 // simulations: particles [part0, part0 + n) of the positions, tiles
