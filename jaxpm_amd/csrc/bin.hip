@@ -521,12 +521,13 @@ __device__ __forceinline__ void window_corners(const float4 &rec, const TileGrid
     uint32_t i = t.div_ny.div(r);
     uint32_t j = r - i * uint32_t(t.ny);
     const float px = float(i) + x, py = float(j) + y, pz = float(k) + z;
-    lcorner_rel(px, 0.0f, t.nx, ox, lx[0], wx[0], gx[0]);
-    lcorner_rel(px, 1.0f, t.nx, ox, lx[1], wx[1], gx[1]);
-    lcorner_rel(py, 0.0f, t.ny, oy, ly[0], wy[0], gy[0]);
-    lcorner_rel(py, 1.0f, t.ny, oy, ly[1], wy[1], gy[1]);
-    lcorner_rel(pz, 0.0f, t.nz, oz, lz[0], wz[0], gz[0]);
-    lcorner_rel(pz, 1.0f, t.nz, oz, lz[1], wz[1], gz[1]);
+    float nd;
+    lcorner_rel(px, 0.0f, t.nx, ox, lx[0], wx[0], gx[0], nd);
+    lcorner_rel(px, 1.0f, t.nx, ox, lx[1], wx[1], gx[1], nd);
+    lcorner_rel(py, 0.0f, t.ny, oy, ly[0], wy[0], gy[0], nd);
+    lcorner_rel(py, 1.0f, t.ny, oy, ly[1], wy[1], gy[1], nd);
+    lcorner_rel(pz, 0.0f, t.nz, oz, lz[0], wz[0], gz[0], nd);
+    lcorner_rel(pz, 1.0f, t.nz, oz, lz[1], wz[1], gz[1], nd);
   } else {
     LAxis ax = laxis_abs(x, ox, t.nx), ay = laxis_abs(y, oy, t.ny), az = laxis_abs(z, oz, t.nz);
     lx[0] = ax.l0; lx[1] = ax.l1; wx[0] = ax.w0; wx[1] = ax.w1;

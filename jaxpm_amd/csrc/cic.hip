@@ -39,17 +39,9 @@ __device__ __forceinline__ Axis axis_abs(float x, int n) {
   return a;
 }
 
-__device__ __forceinline__ float jnp_mod(float x, float L) {
-  float m = fmodf(x, L);
-  if (m != 0.0f && m < 0.0f) m = m + L;
-  return m;
-}
-
 __device__ __forceinline__ void corner_rel(float p, float o, float L, int &idx, float &w, float &dw) {
-  float q = jnp_mod(p + o, L);
-  q = floorf(q);
-  float nd = p - q;
-  nd = nd - rintf(nd / L) * L;
+  const float q = floorf(jmod(p + o, L));
+  const float nd = fold_period(p - q, L);
   // Out-of-range corners (q == L after rounding, or NaN) carry zero weight at
   // a valid index, which is what dropping them does to a sum.
   bool ok = (q >= 0.0f) && (q < L);

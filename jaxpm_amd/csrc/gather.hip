@@ -42,12 +42,8 @@ __device__ __forceinline__ void corner_set(float4 rec, const TileGrid &t, uint32
     for (int a = 0; a < 3; ++a) {
 #pragma unroll
       for (int b = 0; b < 2; ++b) {
-        lcorner_rel(p[a], float(b), n[a], o[a], cs.l[a][b], cs.w[a][b], cs.g[a][b]);
-        // the same nd the weight came from gives the derivative sign
-        const float L = float(n[a]);
-        float q = floorf(jmod(p[a] + float(b), L));
-        float nd = p[a] - q;
-        nd = nd - rintf(nd / L) * L;
+        float nd;   // its sign is the derivative's
+        lcorner_rel(p[a], float(b), n[a], o[a], cs.l[a][b], cs.w[a][b], cs.g[a][b], nd);
         cs.d[a][b] = cs.l[a][b] == -2 ? 0.0f : (nd >= 0.0f ? -1.0f : 1.0f);
       }
     }

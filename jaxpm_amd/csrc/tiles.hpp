@@ -172,10 +172,26 @@ __device__ __forceinline__ int wrapi(int c, int n) {
 // or, when that corner is dropped, the high corner minus one.
 __device__ __forceinline__ int floor_cell_abs(float x, int n) { return wrapi(cell_int(floorf(x)), n); }
 
-__device__ __forceinline__ float jmod(float x, float L) {
+// jnp.remainder(x, L) for L > 0.  Inside [0, 2 L) and (-L, 0) fmodf is x, the
+// exact difference x - L (Sterbenz) or x, so nearly every lattice node plus
+// displacement skips its division loop; the rest, NaN among it, takes it.
+__host__ __device__ __forceinline__ float jmod(float x, float L) {
+  if (x >= 0.0f && x < L) return x;
+  if (x < 0.0f && x > -L) return x + L;
+  if (x >= L && x < 2.0f * L) return x - L;
   float m = fmodf(x, L);
   if (m != 0.0f && m < 0.0f) m = m + L;
   return m;
+}
+
+// nd - rint(nd / L) L for L > 0 (enmesh's periodic fold of a distance):
+// a quarter of a period around 0 or +-L the quotient rounds to 0 or +-1
+// without being formed.
+__host__ __device__ __forceinline__ float fold_period(float nd, float L) {
+  const float a = fabsf(nd);
+  if (a <= 0.25f * L) return nd;
+  if (a >= 0.75f * L && a <= 1.25f * L) return nd - copysignf(L, nd);
+  return nd - rintf(nd / L) * L;
 }
 
 __device__ __forceinline__ int floor_cell_rel(float p, int n) {
@@ -328,11 +344,11 @@ __device__ __forceinline__ LAxis laxis_abs(float x, int origin, int n) {
 // enmesh corner (painting_utils.py:48-69) mapped into the window; corners
 // that land outside [origin, origin + 16] (rounding edge cases) report -1 and
 // are deposited by the caller through the overflow path.
-__device__ __forceinline__ void lcorner_rel(float p, float o, int n, int origin, int &l, float &w, int &cell) {
+__device__ __forceinline__ void lcorner_rel(float p, float o, int n, int origin, int &l, float &w, int &cell,
+                                            float &nd) {
   const float L = float(n);
-  float q = floorf(jmod(p + o, L));
-  float nd = p - q;
-  nd = nd - rintf(nd / L) * L;
+  const float q = floorf(jmod(p + o, L));
+  nd = fold_period(p - q, L);
   const bool ok = (q >= 0.0f) && (q < L);
   cell = ok ? int(q) : -1;
   w = ok ? 1.0f - fabsf(nd) : 0.0f;
