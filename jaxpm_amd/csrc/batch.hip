@@ -44,7 +44,9 @@ int batch_create(int B, const int *dims, const int64_t *counts, uint32_t flags, 
   bt->B = B;
   bt->rel = rel;
   bt->chunk = tuned_chunk(flags);
-  bt->slice = tuned_slice(flags);
+  int64_t total = 0;
+  for (int b = 0; b < B; ++b) total += counts[b] > 0 ? counts[b] : 0;
+  bt->slice = tuned_slice(flags, total, true);
   bt->rho_lds = tuned_rho_lds(flags);
   bt->slabs = tuned_slabs(flags);
   uint64_t K = 0, N = 0, M = 0, H = 0, G = 0;

@@ -70,35 +70,54 @@ __device__ __forceinline__ void block_range(const SimRef &s, uint32_t blk, uint3
   p1 = min(s.part0 + s.n, p0 + slice);
 }
 
-// LDS histogram of the (simulation-local) tile keys of particles [p0, p1).
+// LDS histogram of the (simulation-local) tile keys of particles [p0, p1),
+// four positions of a thread in flight together.
 template <bool REL>
 __device__ __forceinline__ void slice_histogram(const float *__restrict__ pos, uint32_t p0, uint32_t p1,
                                                 const SimRef &s, uint32_t *sh) {
-  for (uint32_t b0 = p0; b0 < p1; b0 += blockDim.x) {
-    const uint32_t p = b0 + threadIdx.x;
-    const bool active = p < p1;
-    uint32_t key = 0xffffffffu;
-    if (active) {
-      int cx, cy, cz;
-      floor_cells<REL>(pos, p, p - s.part0, s.t, cx, cy, cz);
-      key = tile_key(cx, cy, cz, s.t);
+  constexpr int kPer = 4;
+  for (uint32_t b0 = p0; b0 < p1; b0 += kPer * blockDim.x) {
+    float x[kPer], y[kPer], z[kPer];
+#pragma unroll
+    for (int i = 0; i < kPer; ++i) {
+      const uint32_t p = b0 + uint32_t(i) * blockDim.x + threadIdx.x;
+      const size_t at = 3 * size_t(p < p1 ? p : p1 - 1);
+      x[i] = pos[at];
+      y[i] = pos[at + 1];
+      z[i] = pos[at + 2];
     }
-    const unsigned long long act = __ballot(active);
-    const unsigned long long heads = run_heads(key, active);
-    if (active && ((heads >> (threadIdx.x & 63)) & 1ull)) atomicAdd(&sh[key], run_length(heads, act));
+#pragma unroll
+    for (int i = 0; i < kPer; ++i) {
+      const uint32_t p = b0 + uint32_t(i) * blockDim.x + threadIdx.x;
+      const bool active = p < p1;
+      uint32_t key = 0xffffffffu;
+      if (active) {
+        int cx, cy, cz;
+        floor_cells_xyz<REL>(x[i], y[i], z[i], p - s.part0, s.t, cx, cy, cz);
+        key = tile_key(cx, cy, cz, s.t);
+      }
+      const unsigned long long act = __ballot(active);
+      const unsigned long long heads = run_heads(key, active);
+      if (active && ((heads >> (threadIdx.x & 63)) & 1ull)) atomicAdd(&sh[key], run_length(heads, act));
+    }
   }
 }
 
 template <bool REL, class G>
 __global__ void __launch_bounds__(kBinThreads)
-bin_count_kernel(const float *__restrict__ pos, uint32_t slice, G g, uint32_t *__restrict__ count) {
+bin_count_kernel(const float *__restrict__ pos, uint32_t slice, uint32_t shift, G g, uint32_t *__restrict__ count) {
   extern __shared__ uint32_t sh[];
-  const SimRef &s = g.block_sim(blockIdx.x);
+  // 2^shift workgroups share a slice, each an equal part of it
+  const uint32_t blk = blockIdx.x >> shift;
+  const SimRef &s = g.block_sim(blk);
   const uint32_t K = s.t.K, tile0 = s.tile0;
   for (uint32_t k = threadIdx.x; k < K; k += blockDim.x) sh[k] = 0;
   __syncthreads();
   uint32_t p0, p1;
-  block_range(s, blockIdx.x, slice, p0, p1);
+  block_range(s, blk, slice, p0, p1);
+  const uint32_t part = slice >> shift;
+  p0 += (blockIdx.x & ((1u << shift) - 1u)) * part;
+  p1 = min(p1, p0 + part);
   slice_histogram<REL>(pos, p0, p1, s, sh);
   __syncthreads();
   for (uint32_t k = threadIdx.x; k < K; k += blockDim.x)
@@ -372,8 +391,7 @@ bin_scatter_kernel(const float *__restrict__ pos, uint32_t slice, G g, uint32_t 
 // particles each (slice = THREADS PER), loaded and keyed once for both the
 // histogram and the scatter, so the positions are read once.  1024 x 8 and
 // 1024 x 16 hold one workgroup per CU (their registers); 512 x 8, three.
-constexpr int kScatterRegThreads = 1024;
-
+// (256 x 4 and 256 x 8 are for sorts of few particles, see tuned_slice.)
 template <bool REL, class G, int PER, int THREADS>
 __global__ void __launch_bounds__(THREADS)
 bin_scatter_reg_kernel(const float *__restrict__ pos, uint32_t slice, G g, uint32_t *__restrict__ cursor,
@@ -968,7 +986,7 @@ static SortDims one_dims(const TileGrid &t, int64_t n, uint32_t flags) {
   const uint64_t nn = uint64_t(n > 0 ? n : 1);
   d.K = t.K;
   d.n = uint32_t(n);
-  d.slice = tuned_slice(flags);
+  d.slice = tuned_slice(flags, n, flags & kSortOrdered);
   d.chunk = tuned_chunk(flags);
   d.G = uint32_t((nn + d.slice - 1) / d.slice);
   d.maxchunks = uint32_t((nn + d.chunk - 1) / d.chunk + t.K);
@@ -1061,6 +1079,27 @@ Bins bins_view(int nx, int ny, int nz, int64_t n, uint32_t flags, const void *ws
   return view_of(g, one_dims(t, n, flags), uint32_t(cells(nx, ny, nz)), flags & JPM_RELATIVE, ws);
 }
 
+// The scatter that holds its slice in registers, for slices of 1024 to 16384
+// particles.
+template <class G>
+struct ScatterReg {
+  void (*kern)(const float *, uint32_t, G, uint32_t *, float4 *);
+  unsigned threads;
+};
+
+static bool scatter_reg_ok(uint32_t slice) { return slice >= 1024u && slice <= 16384u; }
+
+template <class G>
+static ScatterReg<G> scatter_reg(uint32_t slice, bool rel) {
+  switch (slice) {
+    case 1024: return {rel ? bin_scatter_reg_kernel<true, G, 4, 256> : bin_scatter_reg_kernel<false, G, 4, 256>, 256};
+    case 2048: return {rel ? bin_scatter_reg_kernel<true, G, 8, 256> : bin_scatter_reg_kernel<false, G, 8, 256>, 256};
+    case 4096: return {rel ? bin_scatter_reg_kernel<true, G, 8, 512> : bin_scatter_reg_kernel<false, G, 8, 512>, 512};
+    case 8192: return {rel ? bin_scatter_reg_kernel<true, G, 8, 1024> : bin_scatter_reg_kernel<false, G, 8, 1024>, 1024};
+    default: return {rel ? bin_scatter_reg_kernel<true, G, 16, 1024> : bin_scatter_reg_kernel<false, G, 16, 1024>, 1024};
+  }
+}
+
 // Sort the particles of every simulation into its tiles (workspace of
 // sort_ws(d).total bytes).  counts_in: NULL, or the tile counts of these
 // positions already (d.K entries, e.g. from the kick that drifted them),
@@ -1094,7 +1133,14 @@ static int sort_into(hipStream_t s, const G &g, const SortDims &d, uint32_t M, b
       rc = set_lds(kern, lds_hist);
       if (rc) return rc;
       JPM_TIMED(s, "bin_count_kernel");
-      hipLaunchKernelGGL(kern, dim3(d.G), dim3(kBinThreads), lds_hist, s, pos, d.slice, g, count);
+      // Few slices are split between workgroups, down to one particle a
+      // thread: 256 workgroups fill the chip, and particles in no order make
+      // every workgroup add to every tile's counter, whose atomics then
+      // queue (96^3 random: paint 103 us with 1728 workgroups, 51 with 432).
+      uint32_t shift = 0;
+      while ((d.G << shift) < 256u && (d.slice >> (shift + 1)) >= uint32_t(kBinThreads))
+        ++shift;
+      hipLaunchKernelGGL(kern, dim3(d.G << shift), dim3(kBinThreads), lds_hist, s, pos, d.slice, shift, g, count);
       JPM_LAUNCHED("bin_count_kernel");
     } else {
       auto kern = rel ? bin_count_global_kernel<true, G> : bin_count_global_kernel<false, G>;
@@ -1125,17 +1171,12 @@ static int sort_into(hipStream_t s, const G &g, const SortDims &d, uint32_t M, b
     JPM_LAUNCHED("zero_u32_kernel");
   }
   // 3. scatter particles into tile order
-  if (lds && (d.slice == 4u * kScatterRegThreads || d.slice == 8u * kScatterRegThreads ||
-              d.slice == 16u * kScatterRegThreads)) {
-    const int v = d.slice == 4u * kScatterRegThreads ? 0 : d.slice == 8u * kScatterRegThreads ? 1 : 2;
-    auto kern = rel ? (v == 0 ? bin_scatter_reg_kernel<true, G, 8, 512>
-                              : v == 1 ? bin_scatter_reg_kernel<true, G, 8, 1024> : bin_scatter_reg_kernel<true, G, 16, 1024>)
-                    : (v == 0 ? bin_scatter_reg_kernel<false, G, 8, 512>
-                              : v == 1 ? bin_scatter_reg_kernel<false, G, 8, 1024> : bin_scatter_reg_kernel<false, G, 16, 1024>);
-    rc = set_lds(kern, lds_hist);
+  if (lds && scatter_reg_ok(d.slice)) {
+    const ScatterReg<G> v = scatter_reg<G>(d.slice, rel);
+    rc = set_lds(v.kern, lds_hist);
     if (rc) return rc;
     JPM_TIMED(s, "bin_scatter_kernel");
-    hipLaunchKernelGGL(kern, dim3(d.G), dim3(v == 0 ? 512 : kScatterRegThreads), lds_hist, s, pos, d.slice, g,
+    hipLaunchKernelGGL(v.kern, dim3(d.G), dim3(v.threads), lds_hist, s, pos, d.slice, g,
                        cursor, reinterpret_cast<float4 *>(base + w.spos));
     JPM_LAUNCHED("bin_scatter_reg_kernel");
   } else if (lds) {

@@ -13,7 +13,7 @@ constexpr int kWin = kTile + 1;                 // window edge (CIC +1 corner)
 constexpr int kWinCells = kWin * kWin * kWin;   // 4913
 constexpr int kChunk = 8192;                    // default max particles per chunk
 constexpr int kMaxKeysLds = 32768;              // LDS histogram limit (128 KiB)
-constexpr uint32_t kSlice = 8192;               // default particles per count / scatter workgroup
+constexpr uint32_t kSlice = 8192;               // particles per count / scatter workgroup of a large sort
 // Accumulation / force-gather workgroup size: their LDS windows (38-39 KiB)
 // allow 4 workgroups per CU, so 512 threads keep 32 waves resident.
 constexpr int kWindowThreads = 512;
@@ -75,10 +75,22 @@ __device__ __forceinline__ uint32_t gather_item(uint32_t b, uint32_t per, bool s
   const uint32_t blk = b / (8u * kXcdRun), r = b % (8u * kXcdRun);
   return blk * (8u * kXcdRun) + (r & 7u) * kXcdRun + (r >> 3);
 }
-inline uint32_t tuned_slice(uint32_t flags) {
+// Particles per count / scatter workgroup of a sort of n particles.  Slices
+// that narrow with n keep a few hundred workgroups on the chip (a slice of
+// 8192 is 4 workgroups at 32^3, which take 11 us for a 2 us scatter); wide
+// ones write longer runs per tile, which is what particles in no order need
+// (256^3 random: paint 471 us, 520 with slices of 4096).  A simulation's
+// particles (`ordered`) are in the order of their lattice or of their tiles,
+// and take slices of 4096 at every size (192^3 relative forces 420 -> 402 us).
+inline uint32_t tuned_slice(uint32_t flags, int64_t n, bool ordered = false) {
   const uint32_t v = (flags >> 20) & 0xfu;
-  return (v >= 1 && v <= 7) ? (1u << (11 + v)) : kSlice;
+  if (v >= 1 && v <= 7) return 1u << (11 + v);
+  if (n < (int64_t(1) << 17)) return 1024;
+  if (n < (int64_t(1) << 19)) return 2048;
+  return ordered || n < (int64_t(1) << 22) ? 4096 : kSlice;
 }
+// Bit 27, set inside the force pipelines: the particles are `ordered`.
+constexpr uint32_t kSortOrdered = 1u << 27;
 
 // A tile's low-face cells (lx = 0, or ly = 0, or lz = 0), numbered in face
 // order: the lx = 0 plane (ly * 16 + lz), then ly = 0 with lx > 0

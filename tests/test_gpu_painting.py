@@ -309,3 +309,27 @@ def test_sorted_read_matches_direct(gpu, shape, nc):
     close(srt.reshape(n, nc), ref)
     api = host(painting.cic_read(dev(meshes[0]), dev(pos), method="sorted"))
     np.testing.assert_array_equal(api, host(_ops.read(dev(meshes[0]), dev(pos))))
+
+
+@pytest.mark.parametrize("n", [1, 255, 256, 1025, 131071, 131072, 524287, 524289, 4194303, 4194305])
+def test_default_slices_give_the_same_bits(gpu, n):
+    """The sort's slice follows the particle count; the fixed-point paint is
+    the same bits whatever the slice (against slices of 16384), at the counts
+    where the default changes and in slices that end inside a wave."""
+    from jaxpm_amd import _lib
+    print(f"default slice n={n}", flush=True)
+    shape = (48, 33, 20)
+    r = np.random.default_rng(60)
+    pos = torch.as_tensor((r.uniform(-0.2, 1.2, (n, 3)) * shape).astype(np.float32), device="cuda")
+    w = torch.as_tensor(r.normal(size=n).astype(np.float32), device="cuda")
+    out = []
+    for flags in (_lib.ZERO_MESH, _lib.ZERO_MESH | _lib.tune_flags(slice_code=3)):
+        mesh = torch.empty(shape, device="cuda")
+        wsb = _lib.size("jpm_cic_paint_binned_workspace_size", *shape, n, 1, flags)
+        ws = torch.empty(wsb, dtype=torch.uint8, device="cuda")
+        _lib.call("jpm_cic_paint_binned_f32", _lib.stream(), *shape, _lib.ptr(pos), n, _lib.ptr(w), 1.0, 1,
+                  _lib.ptr(mesh), flags, _lib.ptr(ws), wsb)
+        out.append(mesh)
+    assert torch.equal(out[0], out[1])
+    m = float(w.double().sum())
+    assert abs(float(out[0].double().sum()) - m) < 1e-5 * float(w.double().abs().sum())
