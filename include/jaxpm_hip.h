@@ -287,6 +287,25 @@ int jpm_kspace_linear_field_f32(void *stream, int nx, int ny, int nz,
                                 const float *k_tab, const float *pk_tab,
                                 int ntab, float scale);
 
+/* out = C2R(c R2C(noise)) / M with jpm_kspace_linear_field_f32's multiplier
+ * c: the initial conditions of pm.py:129-144 in one call (noise and out may be
+ * the same array), in a workspace of jpm_linear_field_workspace_size bytes. */
+size_t jpm_linear_field_workspace_size(int nx, int ny, int nz);
+int jpm_linear_field_f32(void *stream, int nx, int ny, int nz,
+                         const float *noise, float *out, float Lx, float Ly,
+                         float Lz, const float *k_tab, const float *pk_tab,
+                         int ntab, void *ws, size_t ws_bytes);
+
+/* lpt (pm.py:61-126) of a real field: dx, p, f [n][3] from the growth
+ * coefficients coef (host): dx1 = coef[0] F1, p1 = coef[1] dx1, f1 = coef[2]
+ * F1 and, for order 2, dx2 = coef[3] F2, p2 = coef[4] dx2, f2 = coef[5] F2
+ * added to them, F1 and F2 the first- and second-order force fields at the
+ * lattice nodes (pos NULL, n = nx ny nz) or read at n absolute positions. */
+size_t jpm_lpt_workspace_size(int nx, int ny, int nz, int order);
+int jpm_lpt_f32(void *stream, int nx, int ny, int nz, const float *field,
+                const float *pos, int64_t n, int order, const float *coef,
+                float *dx, float *p, float *f, void *ws, size_t ws_bytes);
+
 /* Workspace bytes for jpm_kspace_linear_field_table_vjp_f32. */
 size_t jpm_linear_field_table_vjp_workspace_size(int ntab);
 

@@ -117,21 +117,21 @@ class LinearField(torch.autograd.Function):
 
     @staticmethod
     def forward(ctx, noise, box, ktab, pktab):
-        shape = tuple(noise.shape)
         noise = noise.contiguous()
-        fk = _ops.kspace_linear_field(_ops.r2c(noise), shape, box, ktab, pktab, 1.0 / noise.numel())
         ctx.save_for_backward(noise, ktab, pktab)
-        ctx.box, ctx.shape = box, shape
-        return _ops.c2r(fk, shape, clobber=True)
+        ctx.box, ctx.shape = box, tuple(noise.shape)
+        return _ops.linear_field(noise, box, ktab, pktab)
 
     @staticmethod
     def backward(ctx, g):
         noise, ktab, pktab = ctx.saved_tensors
+        if not ctx.needs_input_grad[3]:
+            gn = _ops.linear_field(g.contiguous(), ctx.box, ktab, pktab) if ctx.needs_input_grad[0] else None
+            return gn, None, None, None
         gk = _ops.r2c(g.contiguous())
-        gn = gt = None
-        if ctx.needs_input_grad[3]:
-            gt = _ops.linear_field_table_vjp(_ops.r2c(noise), gk, ctx.shape, ctx.box, ktab, pktab,
-                                             1.0 / g.numel()).to(pktab.dtype)
+        gn = None
+        gt = _ops.linear_field_table_vjp(_ops.r2c(noise), gk, ctx.shape, ctx.box, ktab, pktab,
+                                         1.0 / g.numel()).to(pktab.dtype)
         if ctx.needs_input_grad[0]:
             fk = _ops.kspace_linear_field(gk, ctx.shape, ctx.box, ktab, pktab, 1.0 / g.numel())
             gn = _ops.c2r(fk, ctx.shape, clobber=True)

@@ -74,6 +74,10 @@ SIGNATURES = {
     "jpm_fd4_gradient_f32": (_i, [_vp, _i, _i, _i, _vp, _f, _vp]),
     "jpm_fd4_divergence_f32": (_i, [_vp, _i, _i, _i, _vp, _f, _vp]),
     "jpm_kspace_linear_field_f32": (_i, [_vp, _i, _i, _i, _vp, _f, _f, _f, _vp, _vp, _i, _f]),
+    "jpm_linear_field_workspace_size": (_sz, [_i, _i, _i]),
+    "jpm_linear_field_f32": (_i, [_vp, _i, _i, _i, _vp, _vp, _f, _f, _f, _vp, _vp, _i, _vp, _sz]),
+    "jpm_lpt_workspace_size": (_sz, [_i, _i, _i, _i]),
+    "jpm_lpt_f32": (_i, [_vp, _i, _i, _i, _vp, _vp, _i64, _i, _vp, _vp, _vp, _vp, _vp, _sz]),
     "jpm_kspace_shear6_f32": (_i, [_vp, _i, _i, _i, _vp, _vp, _f, _u32]),
     "jpm_lpt2_source_f32": (_i, [_vp, _i64, _vp, _vp]),
     "jpm_kspace_shear6_adjoint_f32": (_i, [_vp, _i, _i, _i, _vp, _vp, _f, _u32]),

@@ -308,6 +308,41 @@ def kspace_linear_field(fk, shape, box, ktab, pktab, scale=1.0):
     return fk
 
 
+def linear_field(noise, box, ktab, pktab):
+    """C2R(sqrt(pk M / V) R2C(noise)) / M (jpm_linear_field_f32)."""
+    noise = _f32(noise, "noise")
+    nx, ny, nz = _dims(noise.shape)
+    ktab = _f32(ktab, "k table")
+    pktab = _f32(pktab, "pk table")
+    if ktab.numel() != pktab.numel():
+        raise ValueError("k and P(k) tables differ in length")
+    out = torch.empty_like(noise)
+    wsb = size("jpm_linear_field_workspace_size", nx, ny, nz)
+    ws = torch.empty(wsb, dtype=torch.uint8, device=noise.device)
+    call("jpm_linear_field_f32", stream(), nx, ny, nz, ptr(noise), ptr(out), float(box[0]), float(box[1]),
+         float(box[2]), ptr(ktab), ptr(pktab), ktab.numel(), ptr(ws), wsb)
+    return out
+
+
+def lpt(field, pos, coeffs):
+    """(dx, p, f) of jpm_lpt_f32 for 3 (first order) or 6 growth
+    coefficients: (nx, ny, nz, 3) at the lattice nodes (``pos`` None) or of
+    pos's shape (..., 3) at absolute positions."""
+    field = _f32(field, "initial conditions")
+    nx, ny, nz = _dims(field.shape)
+    order = len(coeffs) // 3
+    if pos is not None:
+        pos = _f32(pos, "positions")
+    shape = (nx, ny, nz, 3) if pos is None else tuple(pos.shape)
+    out = [torch.empty(shape, dtype=torch.float32, device=field.device) for _ in range(3)]
+    wsb = size("jpm_lpt_workspace_size", nx, ny, nz, order)
+    ws = torch.empty(wsb, dtype=torch.uint8, device=field.device)
+    carr = (ctypes.c_float * len(coeffs))(*[float(c) for c in coeffs])
+    call("jpm_lpt_f32", stream(), nx, ny, nz, ptr(field), ptr(pos), out[0].numel() // 3, order, carr, ptr(out[0]),
+         ptr(out[1]), ptr(out[2]), ptr(ws), wsb)
+    return tuple(out)
+
+
 def kspace_shear6(dk, shape, scale=1.0, flags=0):
     dk = _c64(dk, "delta_k")
     nx, ny, nz = _dims(shape)

@@ -25,8 +25,8 @@ int batch_kick(hipStream_t, const BatchBins &, const float *, const float *, flo
                float *, uint32_t *, float *);
 int kspace_force_batch(hipStream_t, int, int, int, int, const void *, void *, float, uint32_t);
 int kspace_force_adjoint_batch(hipStream_t, int, int, int, int, const void *, void *, float, uint32_t);
-int kspace_linear_field_batch(hipStream_t, int, int, int, int, void *, const float *, const float *, const float *, int,
-                              float);
+int linear_field(hipStream_t, int, int, int, int, const float *, float *, float, float, float, const float *,
+                 const float *, const float *, int, float, void *);
 int grad_pos_batch(hipStream_t, const SimRef *, int, bool, const float *, const float *, float *);
 int batch_grad(hipStream_t, const BatchBins &, const float *, const float *, const float *, const float *, float *,
                bool, const float *, float *, float *);
@@ -273,11 +273,10 @@ int batch_linear_field(hipStream_t s, const SimBatch &bt, const float *noise, fl
   int rc;
   for (const SimClass &c : bt.classes) {
     const float inv_m = float(1.0 / double(cells(c.nx, c.ny, c.nz)));
-    if ((rc = fft_r2c(s, c.nx, c.ny, c.nz, c.count, noise + c.cell0, spec + c.half0))) return rc;
-    if ((rc = kspace_linear_field_batch(s, c.nx, c.ny, c.nz, c.count, spec + c.half0, boxes + 3 * size_t(c.first), ktab,
-                                        pktabs + size_t(c.first) * ntab, ntab, inv_m)))
+    if ((rc = linear_field(s, c.nx, c.ny, c.nz, c.count, noise + c.cell0, out + c.cell0, 1.0f, 1.0f, 1.0f,
+                           boxes + 3 * size_t(c.first), ktab, pktabs + size_t(c.first) * ntab, ntab, inv_m,
+                           spec + c.half0)))
       return rc;
-    if ((rc = fft_c2r(s, c.nx, c.ny, c.nz, c.count, spec + c.half0, out + c.cell0))) return rc;
   }
   return JPM_OK;
 }

@@ -10,6 +10,8 @@
 #include <string>
 #include <vector>
 
+#include "kspace.hpp"
+#include "lpt.hpp"
 #include "tiles.hpp"
 
 namespace jpm {
@@ -125,6 +127,11 @@ int density_plane_vjp(hipStream_t, const float *, int64_t, int, int, double, dou
 size_t gaussian_smoothing_ws(int, int);
 int gaussian_smoothing(hipStream_t, int, int, const float *, float *, double, void *, size_t);
 int kspace_potential(hipStream_t, int, int, int, const void *, void *, float, float, uint32_t);
+int linear_field(hipStream_t, int, int, int, int, const float *, float *, float, float, float, const float *,
+                 const float *, const float *, int, float, void *);
+bool native_fft_ok(int, int, int);
+int native_lpt2(hipStream_t, int, int, int, const float *, void *, void *, float *, float *, const Tabs &, float);
+int zero_f32(hipStream_t, float *, int64_t);
 int fd4_gradient(hipStream_t, int, int, int, const float *, float, float *);
 int fd4_divergence(hipStream_t, int, int, int, const float *, float, float *);
 
@@ -502,6 +509,92 @@ static int pm_forces(hipStream_t s, int nx, int ny, int nz, const float *pos, in
   return cic_read(s, nx, ny, nz, meshes, 3, m, pos, n, forces, pflags & JPM_RELATIVE);
 }
 
+
+// Workspace of lpt: [half spectrum][7 half spectra, later the force meshes,
+// or first order the force meshes][potential 1][potential 2].
+struct LptSpace {
+  size_t spec, many, phi1, phi2, total;
+};
+
+static LptSpace lpt_space(int nx, int ny, int nz, int order) {
+  const size_t m = size_t(cells(nx, ny, nz)), h = size_t(half_cells(nx, ny, nz));
+  LptSpace w;
+  size_t o = 0;
+  w.spec = o; o += align_up(h * 8);
+  // second order: 7 spectra, or 6 and their 6 meshes, or 6 force meshes;
+  // first order: 3 force meshes (and the second half spectrum of a solve)
+  // and, on a mesh with an axis of one cell, 3 floats of displacement per cell
+  w.many = o;
+  o += order == 2 ? align_up(7 * h * 8) + align_up(6 * m * 4) : align_up(3 * m * 4) + align_up(h * 8);
+  if (nx == 1 || ny == 1 || nz == 1) o += align_up(3 * m * 4);
+  w.phi1 = o; o += align_up(m * 4);
+  w.phi2 = o; o += order == 2 ? align_up(m * 4) : 0;
+  w.total = o;
+  return w;
+}
+
+// (dx, p, f) of lpt (pm.py:61-126) for the real field ic: at the lattice
+// nodes (pos null) or at n absolute positions.
+static int lpt(hipStream_t s, int nx, int ny, int nz, const float *ic, const float *pos, int64_t n, int order,
+               const float *coef, float *dx, float *p, float *f, void *ws, size_t ws_bytes) {
+  int rc = check_dims(nx, ny, nz);
+  if (rc) return rc;
+  JPM_REQUIRE(order == 1 || order == 2, "order must be 1 or 2, got %d", order);
+  JPM_REQUIRE(ic && coef, "null pointer argument");
+  const int64_t m = cells(nx, ny, nz);
+  JPM_REQUIRE(n >= 0 && n <= kMaxCells && (pos || n == m), "particle count %lld out of range", (long long)n);
+  JPM_REQUIRE(n == 0 || (dx && p && f), "null pointer argument");
+  JPM_REQUIRE(3 * m <= (int64_t(1) << 32) && (order == 1 || 6 * half_cells(nx, ny, nz) <= (int64_t(1) << 32)),
+              "mesh too large");
+  const LptSpace w = lpt_space(nx, ny, nz, order);
+  JPM_REQUIRE(ws && ws_bytes >= w.total, "lpt needs %zu workspace bytes, got %zu", w.total, ws_bytes);
+  char *base = static_cast<char *>(ws);
+  void *spec = base + w.spec, *many = base + w.many;
+  float *phi1 = reinterpret_cast<float *>(base + w.phi1);
+  float *phi2 = order == 2 ? reinterpret_cast<float *>(base + w.phi2) : nullptr;
+  const float scale = float(1.0 / double(m));
+  if (order == 1) {
+    rc = potential_solve(s, nx, ny, nz, 1, ic, spec, many, phi1, 0.0f, scale, nullptr, 0);
+    if (rc) return rc;
+  } else {
+    const bool aligned = (reinterpret_cast<uintptr_t>(ic) & 7u) == 0;
+    if (native_fft_ok(nx, ny, nz) && nx >= 2 && aligned) {
+      Tabs t;
+      rc = get_tabs(s, nx, ny, nz, 0, t);
+      if (rc) return rc;
+      rc = native_lpt2(s, nx, ny, nz, ic, spec, many, phi1, phi2, t, scale);
+      if (rc) return rc;
+    } else {
+      float *phi6 = reinterpret_cast<float *>(static_cast<char *>(many) + align_up(7 * size_t(half_cells(nx, ny, nz)) * 8));
+      if ((rc = fft_r2c(s, nx, ny, nz, 1, ic, spec))) return rc;
+      if ((rc = kspace_potential(s, nx, ny, nz, spec, many, 0.0f, scale, 0))) return rc;
+      if ((rc = fft_c2r(s, nx, ny, nz, 1, many, phi1))) return rc;
+      if ((rc = kspace_shear6(s, nx, ny, nz, spec, many, scale, 0))) return rc;
+      if ((rc = fft_c2r(s, nx, ny, nz, 6, many, phi6))) return rc;
+      if ((rc = lpt2_source(s, m, phi6, phi2))) return rc;
+    }
+    // the second-order potential, over its source
+    rc = potential_solve(s, nx, ny, nz, 1, phi2, spec, many, phi2, 0.0f, scale, nullptr, 0);
+    if (rc) return rc;
+  }
+  LptCoef lc{};
+  for (int i = 0; i < 3 * order; ++i) lc.c[i] = coef[i];
+  // An axis of one cell gives a lattice particle both its corners there, each
+  // of weight 1: the read, not the node's value.
+  if (!pos && nx > 1 && ny > 1 && nz > 1) return lpt_lattice(s, nx, ny, nz, phi1, phi2, lc, dx, p, f);
+  float *f1 = static_cast<float *>(many), *f2 = phi2 ? f1 + 3 * m : nullptr;
+  if ((rc = fd4_gradient(s, nx, ny, nz, phi1, 1.0f, f1))) return rc;
+  if (phi2 && (rc = fd4_gradient(s, nx, ny, nz, phi2, 1.0f, f2))) return rc;
+  if (!pos) {
+    // lattice particles are zero displacements, held past the force meshes
+    float *zeros = f1 + 3 * order * m;
+    rc = zero_f32(s, zeros, 3 * n);
+    if (rc) return rc;
+    return lpt_read(s, nx, ny, nz, f1, f2, zeros, n, true, lc, dx, p, f);
+  }
+  return lpt_read(s, nx, ny, nz, f1, f2, pos, n, false, lc, dx, p, f);
+}
+
 }  // namespace jpm
 
 using namespace jpm;
@@ -654,6 +747,31 @@ int jpm_fd4_divergence_f32(void *stream, int nx, int ny, int nz, const float *g3
 
 int jpm_kspace_compensate_f32(void *stream, int nx, int ny, int nz, void *field_k, float scale) {
   JPM_GUARD(kspace_compensate(as_stream(stream), nx, ny, nz, field_k, scale));
+}
+
+size_t jpm_linear_field_workspace_size(int nx, int ny, int nz) {
+  return nx > 0 && ny > 0 && nz > 0 ? align_up(size_t(half_cells(nx, ny, nz)) * 8) : 0;
+}
+
+int jpm_linear_field_f32(void *stream, int nx, int ny, int nz, const float *noise, float *out, float Lx, float Ly,
+                         float Lz, const float *k_tab, const float *pk_tab, int ntab, void *ws, size_t ws_bytes) {
+  JPM_GUARD([&]() -> int {
+    int rc = check_dims(nx, ny, nz);
+    if (rc) return rc;
+    const size_t need = jpm_linear_field_workspace_size(nx, ny, nz);
+    JPM_REQUIRE(ws && ws_bytes >= need, "linear_field needs %zu workspace bytes, got %zu", need, ws_bytes);
+    return linear_field(as_stream(stream), nx, ny, nz, 1, noise, out, Lx, Ly, Lz, nullptr, k_tab, pk_tab, ntab,
+                        float(1.0 / double(cells(nx, ny, nz))), ws);
+  }());
+}
+
+size_t jpm_lpt_workspace_size(int nx, int ny, int nz, int order) {
+  return nx > 0 && ny > 0 && nz > 0 && (order == 1 || order == 2) ? lpt_space(nx, ny, nz, order).total : 0;
+}
+
+int jpm_lpt_f32(void *stream, int nx, int ny, int nz, const float *field, const float *pos, int64_t n, int order,
+                const float *coef, float *dx, float *p, float *f, void *ws, size_t ws_bytes) {
+  JPM_GUARD(lpt(as_stream(stream), nx, ny, nz, field, pos, n, order, coef, dx, p, f, ws, ws_bytes));
 }
 
 int jpm_kspace_linear_field_f32(void *stream, int nx, int ny, int nz, void *field_k, float Lx, float Ly, float Lz,

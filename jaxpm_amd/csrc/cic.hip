@@ -9,6 +9,7 @@
 //     0 <= q < L (scatter drops, gather mode='drop' reads 0).
 // The library is built with -ffp-contract=off so these sequences round as
 // written.
+#include "lpt.hpp"
 #include "tiles.hpp"
 
 namespace jpm {
@@ -773,6 +774,53 @@ permute_rows_kernel(const uint32_t *__restrict__ order, const float *__restrict_
   out0[dst] = a0;
   out0[dst + 1] = a1;
   out0[dst + 2] = a2;
+}
+
+// LPT at given positions: the three-component reads of the first- and (ORDER
+// 2) second-order force meshes, read_kernel's sums, and their growth-factor
+// products, without the force arrays and the elementwise passes over them.
+template <bool REL, int ORDER>
+__global__ void __launch_bounds__(256)
+lpt_read_kernel(const float *__restrict__ f1, const float *__restrict__ f2, uint32_t m, const float *__restrict__ pos,
+                uint32_t n, Grid g, LptCoef lc, float *__restrict__ dx, float *__restrict__ pp,
+                float *__restrict__ ff) {
+  for (uint32_t p = blockIdx.x * blockDim.x + threadIdx.x; p < n; p += gridDim.x * blockDim.x) {
+    Cic c;
+    particle_cic<REL>(pos, p, g, c);
+#pragma unroll
+    for (int comp = 0; comp < 3; ++comp) {
+      float s1 = 0.0f, s2 = 0.0f;
+#pragma unroll
+      for (int o = 0; o < 8; ++o) {
+        s1 += f1[size_t(comp) * m + c.idx[o]] * c.w[o];
+        if (ORDER == 2) s2 += f2[size_t(comp) * m + c.idx[o]] * c.w[o];
+      }
+      float a, b, d;
+      lpt_combine(lc, s1, ORDER == 2, s2, a, b, d);
+      const size_t e = 3 * size_t(p) + comp;
+      dx[e] = a;
+      pp[e] = b;
+      ff[e] = d;
+    }
+  }
+}
+
+int lpt_read(hipStream_t s, int nx, int ny, int nz, const float *f1, const float *f2, const float *pos, int64_t n,
+             bool rel, const LptCoef &lc, float *dx, float *p, float *f) {
+  const int64_t m = cells(nx, ny, nz);
+  JPM_REQUIRE(n >= 0 && n <= kMaxCells, "particle count %lld out of range", (long long)n);
+  JPM_REQUIRE(!rel || n == m, "relative mode needs one particle per lattice node (n=%lld, mesh %lld)", (long long)n,
+              (long long)m);
+  if (n == 0) return JPM_OK;
+  JPM_REQUIRE(f1 && pos && dx && p && f, "null pointer argument");
+  const Grid g = make_grid(nx, ny, nz);
+  auto kern = rel ? (f2 ? lpt_read_kernel<true, 2> : lpt_read_kernel<true, 1>)
+                  : (f2 ? lpt_read_kernel<false, 2> : lpt_read_kernel<false, 1>);
+  JPM_TIMED(s, "lpt_read_kernel");
+  hipLaunchKernelGGL(kern, dim3(grid_for(n, 256, 256 * 128)), dim3(256), 0, s, f1, f2, uint32_t(m), pos, uint32_t(n),
+                     g, lc, dx, p, f);
+  JPM_LAUNCHED("lpt_read_kernel");
+  return JPM_OK;
 }
 
 int permute_rows(hipStream_t s, int64_t n, const uint32_t *order, const float *in0, float *out0, const float *in1,

@@ -380,6 +380,117 @@ fft_cols_potential_kernel(float2 *__restrict__ data, int nzh, size_t lstride, si
   }
 }
 
+// The x pass of a linear field, in place: as fft_cols_potential_kernel with
+// the linear field's multiplier (linear_factor) between the transforms.
+// Bound by the multiplier's divisions, roots and table search (80 us at
+// 256^3, the potential's 44; with the P(k) table in LDS it took as long), in
+// place of two column passes and linear_field_kernel, 110 us.
+template <int L>
+__global__ void __launch_bounds__(kFftThreads)
+fft_cols_linear_kernel(float2 *__restrict__ data, int nzh, size_t lstride, size_t ostride, size_t bstride,
+                       const float2 *__restrict__ tw_all, uint32_t nkzb, uint32_t nouter, uint32_t nblk,
+                       uint32_t per, Tabs t, LinearArgs la) {
+  constexpr int KB = FftCols<L>::KB, total = L * KB;
+  __shared__ float2 buf[total];
+  __shared__ float2 tw[L];
+  const uint32_t item = (blockIdx.x & 7u) * per + (blockIdx.x >> 3);
+  if (item >= nblk) return;
+  const uint32_t kzb = item % nkzb, rest = item / nkzb, outer = rest % nouter, bi = rest / nouter;
+  float2 *base = data + size_t(bi) * bstride + size_t(outer) * ostride;
+  const int kz0 = int(kzb) * KB;
+  la.item(bi);
+  constexpr int iters = (total + kFftThreads - 1) / kFftThreads;
+  load_cols<L, KB>(base, lstride, kz0, nzh, buf, tw_all, tw);
+  __syncthreads();
+  lds_fft<L, KB, KB, false>(buf, tw);
+  const uint32_t jy = t.oy + outer;
+#pragma unroll
+  for (int it = 0; it < iters; ++it) {
+    const int f = threadIdx.x + it * kFftThreads;
+    if (total % kFftThreads != 0 && f >= total) break;
+    const int c = f & (KB - 1), l = f / KB;
+    if (kz0 + c < nzh) {
+      const float fac = linear_factor(t, uint32_t(l), jy, t.oz + uint32_t(kz0 + c), la);
+      const float2 v = buf[f];
+      buf[f] = make_float2(v.x * fac, v.y * fac);
+    }
+  }
+  __syncthreads();
+  lds_fft<L, KB, KB, true>(buf, tw);
+#pragma unroll
+  for (int it = 0; it < iters; ++it) {
+    const int f = threadIdx.x + it * kFftThreads;
+    if (total % kFftThreads != 0 && f >= total) break;
+    const int c = f & (KB - 1), l = f / KB;
+    if (kz0 + c < nzh) base[size_t(l) * lstride + kz0 + c] = buf[f];
+  }
+}
+
+// The x pass of second-order LPT: the columns of `in` (a spectrum whose z and
+// y passes are done) transformed forward once, then the inverse transforms of
+// G X and of the six -g_a g_b G X (aa = xx, yy, zz, xy, xz, yz) into the seven
+// spectra out + m H, the columns kept in registers between them.  One read and
+// seven writes of the spectrum, against two forward x passes, the potential
+// and shear passes and seven in-place inverse x passes; the same float
+// operations in the same order, so the same bits.  Bound by its eight LDS
+// transforms: 198 us at 256^3 for 540 MB (the passes it stands for, 340 us).
+template <int L>
+__global__ void __launch_bounds__(kFftThreads)
+fft_cols_shear_kernel(const float2 *__restrict__ in, float2 *__restrict__ out, int nzh, size_t lstride,
+                      size_t ostride, size_t H, const float2 *__restrict__ tw_all, uint32_t nkzb, uint32_t nblk,
+                      uint32_t per, Tabs t, float scale) {
+  constexpr int KB = FftCols<L>::KB, total = L * KB;
+  __shared__ float2 buf[total];
+  __shared__ float2 tw[L];
+  const uint32_t item = (blockIdx.x & 7u) * per + (blockIdx.x >> 3);
+  if (item >= nblk) return;
+  const uint32_t kzb = item % nkzb, outer = item / nkzb;
+  const int kz0 = int(kzb) * KB;
+  constexpr int iters = (total + kFftThreads - 1) / kFftThreads;
+  load_cols<L, KB>(in + size_t(outer) * ostride, lstride, kz0, nzh, buf, tw_all, tw);
+  __syncthreads();
+  lds_fft<L, KB, KB, false>(buf, tw);
+  const uint32_t jy = t.oy + outer;
+  const float gy = t.g[jy];
+  float2 v[iters];
+#pragma unroll
+  for (int it = 0; it < iters; ++it) {
+    const int f0 = threadIdx.x + it * kFftThreads;
+    const int f = (total % kFftThreads != 0 && f0 >= total) ? total - 1 : f0;
+    const int c = f & (KB - 1), l = f / KB;
+    const uint32_t kz = t.oz + uint32_t(kz0 + c < nzh ? kz0 + c : nzh - 1);
+    const float G = potential_factor(t, uint32_t(l), jy, kz, 0.0f, 0, scale);
+    v[it] = make_float2(buf[f].x * G, buf[f].y * G);
+  }
+  // every element of buf is read and, below, written by the thread that owns
+  // it; the barriers inside lds_fft separate those from its own accesses
+  for (int m = 0; m < 7; ++m) {
+    __syncthreads();
+#pragma unroll
+    for (int it = 0; it < iters; ++it) {
+      const int f = threadIdx.x + it * kFftThreads;
+      if (total % kFftThreads != 0 && f >= total) break;
+      const int c = f & (KB - 1), l = f / KB;
+      const float gx = t.g[l], gz = t.g[t.oz + uint32_t(kz0 + c < nzh ? kz0 + c : nzh - 1)];
+      // (i g_a)(i g_b) = -g_a g_b
+      const float a = m == 2 || m == 6 ? gy : (m == 3 ? gz : gx);
+      const float b = m == 1 ? gx : (m == 2 || m == 4 ? gy : gz);
+      const float cm = -(a * b);
+      buf[f] = m == 0 ? v[it] : make_float2(cm * v[it].x, cm * v[it].y);
+    }
+    __syncthreads();
+    lds_fft<L, KB, KB, true>(buf, tw);
+    float2 *dst = out + size_t(m) * H + size_t(outer) * ostride;
+#pragma unroll
+    for (int it = 0; it < iters; ++it) {
+      const int f = threadIdx.x + it * kFftThreads;
+      if (total % kFftThreads != 0 && f >= total) break;
+      const int c = f & (KB - 1), l = f / KB;
+      if (kz0 + c < nzh) dst[size_t(l) * lstride + kz0 + c] = buf[f];
+    }
+  }
+}
+
 // The three channels of a vector mesh whose divergence the R2C reads in
 // place of a scalar mesh: channel d of item b at g3 + b * 2 * in_bstride +
 // d * chan floats.
@@ -594,6 +705,86 @@ fft_c2r_rows_kernel(const float2 *__restrict__ in, float2 *__restrict__ out, int
 }
 
 
+// The z pass of six C2Rs whose meshes second-order LPT multiplies at once:
+// the rows of the shear spectra spec + m H (m = 0 .. 5: xx, yy, zz, xy, xz,
+// yz), each transformed as in fft_c2r_rows_kernel, and the source
+// (pm.py:92-109) of the six values in their accumulation order.  The six
+// meshes stay in LDS and registers: 164 us at 256^3, against 244 us for six
+// C2R row passes and lpt2_source_kernel (403 MB of meshes each way).
+template <int M>
+__global__ void __launch_bounds__(kC2rThreads)
+fft_c2r_source_kernel(const float2 *__restrict__ spec, size_t H, float2 *__restrict__ out, int nrows,
+                      const float2 *__restrict__ tw_all) {
+  constexpr int KB = C2rRows<M>::KB, PITCH = KB + 1, total = M * KB, nzh = M + 1;
+  __shared__ float2 buf[M * PITCH];
+  __shared__ float2 twM[M];
+  TwStage<M, kC2rThreads> tsM;
+  const float2 *twN = tw_all + tw_off(2 * M);
+  const int r0 = blockIdx.x * KB;
+  constexpr int iters = (total + kC2rThreads - 1) / kC2rThreads;
+  float2 d[iters], acc[iters], va[iters], vb[iters];
+  tsM.load(tw_all, tw_off(M));
+  tsM.store(twM);
+  auto load = [&](int m) {
+#pragma unroll
+    for (int it = 0; it < iters; ++it) {
+      const int f0 = threadIdx.x + it * kC2rThreads;
+      const int f = (total % kC2rThreads != 0 && f0 >= total) ? total - 1 : f0;
+      const int k = f % M, c = f / M;
+      const float2 *row = spec + size_t(m) * H + size_t(r0 + c < nrows ? r0 + c : nrows - 1) * nzh;
+      va[it] = row[k];
+      vb[it] = row[M - k];
+    }
+  };
+  // in the order the source takes them: xx, xy, xz, yy, yz, zz
+  constexpr int order[6] = {0, 3, 4, 1, 5, 2};
+  load(order[0]);
+#pragma unroll
+  for (int q = 0; q < 6; ++q) {
+#pragma unroll
+    for (int it = 0; it < iters; ++it) {
+      const int f = threadIdx.x + it * kC2rThreads;
+      if (total % kC2rThreads != 0 && f >= total) break;
+      const int k = f % M, c = f / M;
+      float2 a = va[it], b = vb[it];
+      if (k == 0) {
+        a.y = 0.0f;
+        b.y = 0.0f;
+      }
+      const float2 bc = conjf2(b);
+      const float2 E = cadd(a, bc);
+      const float2 O = cmul(csub(a, bc), conjf2(twN[k]));
+      buf[k * PITCH + c] = make_float2(E.x - O.y, E.y + O.x);
+    }
+    if (q < 5) load(order[q + 1]);   // in flight during the transform
+    __syncthreads();
+    lds_fft<M, KB, PITCH, true, kC2rThreads>(buf, twM);
+#pragma unroll
+    for (int it = 0; it < iters; ++it) {
+      const int f = threadIdx.x + it * kC2rThreads;
+      if (total % kC2rThreads != 0 && f >= total) break;
+      const float2 s = buf[(f % M) * PITCH + f / M];
+      if (q == 0) {
+        d[it] = make_float2(0.0f + s.x * 0.0f, 0.0f + s.y * 0.0f);
+        acc[it] = s;
+      } else if (q == 3 || q == 5) {
+        d[it] = make_float2(d[it].x + s.x * acc[it].x, d[it].y + s.y * acc[it].y);
+        acc[it] = cadd(acc[it], s);
+      } else {
+        d[it] = make_float2(d[it].x - s.x * s.x, d[it].y - s.y * s.y);
+      }
+    }
+    __syncthreads();
+  }
+#pragma unroll
+  for (int it = 0; it < iters; ++it) {
+    const int f = threadIdx.x + it * kC2rThreads;
+    if (total % kC2rThreads != 0 && f >= total) break;
+    const int l = f % M, c = f / M;
+    if (r0 + c < nrows) out[size_t(r0 + c) * M + l] = d[it];
+  }
+}
+
 // The native transforms cover meshes whose nx and ny are transform lengths
 // (powers of two 2 .. 1024 or 3 * 2^k 6 .. 768; nx = 1 too: 2-D images, no
 // x pass) and whose nz is twice one (the R2C's complex rows of nz / 2).
@@ -746,6 +937,93 @@ int native_potential(hipStream_t s, int nx, int ny, int nz, int batch, const flo
   JPM_LAUNCHED("fft_cols_potential_kernel");
   if ((rc = cols_pass(s, true, h, ny, nzh, nx, size_t(nzh), size_t(ny) * nzh, H, batch, tw))) return rc;
   return rows_c2r(s, nx, ny, nz, batch, h, out, tw);
+}
+
+// out = C2R(c(k) R2C(in)), c the linear field's multiplier, for a batch of
+// meshes (spec: H complex per mesh; in and out may be the same array).
+int native_linear(hipStream_t s, int nx, int ny, int nz, int batch, const float *in, void *spec, float *out,
+                  const Tabs &t, const LinearArgs &la) {
+  JPM_REQUIRE(native_fft_ok(nx, ny, nz) && nx >= 2 && batch >= 1 && batch <= 65535, "native FFT shape");
+  const float2 *tw;
+  int rc = twiddles(&tw);
+  if (rc) return rc;
+  const int nzh = nz / 2 + 1;
+  const size_t H = size_t(nx) * ny * nzh;
+  float2 *h = static_cast<float2 *>(spec);
+  if ((rc = rows_r2c(s, nx, ny, nz, batch, in, h, tw))) return rc;
+  if ((rc = cols_pass(s, false, h, ny, nzh, nx, size_t(nzh), size_t(ny) * nzh, H, batch, tw))) return rc;
+  {
+    JPM_TIMED(s, "fft_cols_linear_kernel");
+    switch (nx) {
+#define JPM_LIN(N)                                                                                        \
+    case N: {                                                                                             \
+      const uint32_t nkzb = (nzh + FftCols<N>::KB - 1) / FftCols<N>::KB;                                 \
+      const uint32_t nblk = nkzb * uint32_t(ny) * uint32_t(batch), per = (nblk + 7) / 8;                  \
+      hipLaunchKernelGGL(fft_cols_linear_kernel<N>, dim3(8 * per), dim3(kFftThreads), 0, s, h, nzh,       \
+                         size_t(ny) * nzh, size_t(nzh), H, tw, nkzb, uint32_t(ny), nblk, per, t, la);     \
+      break;                                                                                              \
+    }
+      JPM_FFT_LENGTHS(JPM_LIN)
+#undef JPM_LIN
+      default:
+        return fail(JPM_E_INVALID, "native FFT length %d", nx);
+    }
+  }
+  JPM_LAUNCHED("fft_cols_linear_kernel");
+  if ((rc = cols_pass(s, true, h, ny, nzh, nx, size_t(nzh), size_t(ny) * nzh, H, batch, tw))) return rc;
+  return rows_c2r(s, nx, ny, nz, batch, h, out, tw);
+}
+
+// The potential phi = C2R(scale G R2C(ic)) and the second-order LPT source of
+// the six shear fields C2R(-g_a g_b scale G R2C(ic)) (pm.py:88-112).  spec: H
+// complex, spec7: 7 H.
+int native_lpt2(hipStream_t s, int nx, int ny, int nz, const float *ic, void *spec, void *spec7, float *phi,
+                float *source, const Tabs &t, float scale) {
+  JPM_REQUIRE(native_fft_ok(nx, ny, nz) && nx >= 2, "native FFT shape");
+  const float2 *tw;
+  int rc = twiddles(&tw);
+  if (rc) return rc;
+  const int nzh = nz / 2 + 1, M = nz / 2, nrows = nx * ny;
+  const size_t H = size_t(nx) * ny * nzh;
+  float2 *h = static_cast<float2 *>(spec), *h7 = static_cast<float2 *>(spec7);
+  if ((rc = rows_r2c(s, nx, ny, nz, 1, ic, h, tw))) return rc;
+  if ((rc = cols_pass(s, false, h, ny, nzh, nx, size_t(nzh), size_t(ny) * nzh, H, 1, tw))) return rc;
+  {
+    JPM_TIMED(s, "fft_cols_shear_kernel");
+    switch (nx) {
+#define JPM_SHEAR(N)                                                                                      \
+    case N: {                                                                                             \
+      const uint32_t nkzb = (nzh + FftCols<N>::KB - 1) / FftCols<N>::KB;                                 \
+      const uint32_t nblk = nkzb * uint32_t(ny), per = (nblk + 7) / 8;                                    \
+      hipLaunchKernelGGL(fft_cols_shear_kernel<N>, dim3(8 * per), dim3(kFftThreads), 0, s, h, h7, nzh,    \
+                         size_t(ny) * nzh, size_t(nzh), H, tw, nkzb, nblk, per, t, scale);                \
+      break;                                                                                              \
+    }
+      JPM_FFT_LENGTHS(JPM_SHEAR)
+#undef JPM_SHEAR
+      default:
+        return fail(JPM_E_INVALID, "native FFT length %d", nx);
+    }
+  }
+  JPM_LAUNCHED("fft_cols_shear_kernel");
+  if ((rc = cols_pass(s, true, h7, ny, nzh, nx, size_t(nzh), size_t(ny) * nzh, H, 7, tw))) return rc;
+  if ((rc = rows_c2r(s, nx, ny, nz, 1, h7, phi, tw))) return rc;
+  {
+    JPM_TIMED(s, "fft_c2r_source_kernel");
+    switch (M) {
+#define JPM_SRC(N)                                                                                            \
+    case N:                                                                                                   \
+      hipLaunchKernelGGL(fft_c2r_source_kernel<N>, dim3((nrows + C2rRows<N>::KB - 1) / C2rRows<N>::KB),       \
+                         dim3(kC2rThreads), 0, s, h7 + H, H, reinterpret_cast<float2 *>(source), nrows, tw);  \
+      break;
+      JPM_FFT_LENGTHS(JPM_SRC)
+#undef JPM_SRC
+      default:
+        return fail(JPM_E_INVALID, "native FFT length %d", nz);
+    }
+  }
+  JPM_LAUNCHED("fft_c2r_source_kernel");
+  return JPM_OK;
 }
 
 }  // namespace jpm

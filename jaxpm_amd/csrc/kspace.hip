@@ -167,46 +167,15 @@ compensate_kernel(float2 *__restrict__ fk, HalfGrid hg, Tabs t, float scale) {
   }
 }
 
-// jnp.interp(x, xp, fp) with the default clamping (fp[0] left of xp[0],
-// fp[-1] right of xp[-1]).
-__device__ __forceinline__ float interp(float x, const float *__restrict__ xp, const float *__restrict__ fp,
-                                        int n) {
-  // i = clip(searchsorted(xp, x, side='right'), 1, n - 1)
-  int lo = 0, hi = n;
-  while (lo < hi) {
-    int mid = (lo + hi) >> 1;
-    if (xp[mid] <= x) lo = mid + 1; else hi = mid;
-  }
-  int i = lo < 1 ? 1 : (lo > n - 1 ? n - 1 : lo);
-  float df = fp[i] - fp[i - 1];
-  float dx = xp[i] - xp[i - 1];
-  float delta = x - xp[i - 1];
-  float f = (fabsf(dx) <= 0.0f) ? fp[i - 1] : fp[i - 1] + (delta / dx) * df;
-  if (x < xp[0]) f = fp[0];
-  if (x > xp[n - 1]) f = fp[n - 1];
-  return f;
-}
-
 __global__ void __launch_bounds__(256)
-linear_field_kernel(float2 *__restrict__ fk, HalfGrid hg, Tabs t, float3 box, float3 nm, float mcells, float vol,
-                    const float *__restrict__ ktab, const float *__restrict__ pktab, int ntab, float scale,
-                    const float *__restrict__ boxes) {
-  // blockIdx.y: spectrum of a batch of equal shapes (stride H) with its own
-  // box (boxes[3 y..3 y+2], when given) and P(k) table (pktab + y ntab)
+linear_field_kernel(float2 *__restrict__ fk, HalfGrid hg, Tabs t, LinearArgs la) {
+  // blockIdx.y: spectrum of a batch of equal shapes (stride H)
   fk += size_t(blockIdx.y) * hg.H;
-  pktab += size_t(blockIdx.y) * ntab;
-  if (boxes) {
-    box = make_float3(boxes[3 * blockIdx.y], boxes[3 * blockIdx.y + 1], boxes[3 * blockIdx.y + 2]);
-    vol = float(double(box.x) * double(box.y) * double(box.z));
-  }
+  la.item(blockIdx.y);
   for (uint32_t e = blockIdx.x * blockDim.x + threadIdx.x; e < hg.H; e += gridDim.x * blockDim.x) {
     uint32_t i, j, k;
     hg.coords(e, i, j, k);
-    // pm.py:137-138: (k_i / L_i * n_i)^2 summed, then ** 0.5
-    float ax = t.k[i] / box.x * nm.x, ay = t.k[t.oy + j] / box.y * nm.y, az = t.k[t.oz + k] / box.z * nm.z;
-    float kmesh = sqrtf((ax * ax + ay * ay) + az * az);
-    float pk = interp(kmesh, ktab, pktab, ntab);
-    float c = sqrtf(pk * mcells / vol) * scale;
+    const float c = linear_factor(t, i, t.oy + j, t.oz + k, la);
     float2 v = fk[e];
     fk[e] = make_float2(v.x * c, v.y * c);
   }
@@ -502,6 +471,8 @@ bool native_fft_ok(int nx, int ny, int nz);
 int native_potential(hipStream_t s, int nx, int ny, int nz, int batch, const float *in, void *spec, float *out,
                      const Tabs &t, float r2, float scale, const float *scale_dev, int deconv,
                      const float *g3 = nullptr, size_t chan = 0, const FaceCells *faces = nullptr);
+int native_linear(hipStream_t s, int nx, int ny, int nz, int batch, const float *in, void *spec, float *out,
+                  const Tabs &t, const LinearArgs &la);
 int fd4_divergence_batch(hipStream_t s, int nx, int ny, int nz, int batch, const float *g3, size_t chan_stride,
                          float scale, float *out);
 
@@ -585,6 +556,21 @@ int kspace_compensate(hipStream_t s, int nx, int ny, int nz, void *fk, float sca
   return JPM_OK;
 }
 
+static LinearArgs linear_args(int nx, int ny, int nz, float Lx, float Ly, float Lz, const float *ktab,
+                              const float *pktab, int ntab, float scale, const float *boxes) {
+  LinearArgs la;
+  la.box = make_float3(Lx, Ly, Lz);
+  la.nm = make_float3(float(nx), float(ny), float(nz));
+  la.mcells = float(cells(nx, ny, nz));
+  la.vol = float(double(Lx) * double(Ly) * double(Lz));
+  la.scale = scale;
+  la.ktab = ktab;
+  la.pktab = pktab;
+  la.ntab = ntab;
+  la.boxes = boxes;
+  return la;
+}
+
 int kspace_linear_field(hipStream_t s, int nx, int ny, int nz, void *fk, float Lx, float Ly, float Lz,
                         const float *ktab, const float *pktab, int ntab, float scale) {
   int rc = check_dims(nx, ny, nz);
@@ -596,18 +582,47 @@ int kspace_linear_field(hipStream_t s, int nx, int ny, int nz, void *fk, float L
   rc = get_tabs(s, nx, ny, nz, 0, t);
   if (rc) return rc;
   HalfGrid hg = make_half(nx, ny, nz);
-  const float3 box = make_float3(Lx, Ly, Lz);
-  const float3 nm = make_float3(float(nx), float(ny), float(nz));
-  const float mcells = float(cells(nx, ny, nz));
-  const float vol = float(double(Lx) * double(Ly) * double(Lz));
   {
     JPM_TIMED(s, "linear_field_kernel");
     hipLaunchKernelGGL(linear_field_kernel, dim3(grid_for(hg.H, 256, 256 * 128)), dim3(256), 0, s,
-                       static_cast<float2 *>(fk), hg, t, box, nm, mcells, vol, ktab, pktab, ntab, scale,
-                       static_cast<const float *>(nullptr));
+                       static_cast<float2 *>(fk), hg, t,
+                       linear_args(nx, ny, nz, Lx, Ly, Lz, ktab, pktab, ntab, scale, nullptr));
   }
   JPM_LAUNCHED("linear_field_kernel");
   return JPM_OK;
+}
+
+// out = C2R(c(k) R2C(in)) for a batch of equal meshes, c the linear field's
+// multiplier (pm.py:137-143): the initial conditions of white noise.  spec
+// holds H complex values per mesh.  The library's FFT applies c between the
+// x pass's forward and inverse transforms (256^3: 212 -> 182 us); other shapes
+// run hipFFT, linear_field_kernel, hipFFT.  boxes: per-item box sizes and
+// P(k) tables (pktab + item ntab), or null for one box.
+int linear_field(hipStream_t s, int nx, int ny, int nz, int batch, const float *in, float *out, float Lx, float Ly,
+                 float Lz, const float *boxes, const float *ktab, const float *pktab, int ntab, float scale,
+                 void *spec) {
+  int rc = check_dims(nx, ny, nz);
+  if (rc) return rc;
+  JPM_REQUIRE(in && out && spec && ktab && pktab, "null pointer argument");
+  JPM_REQUIRE(batch >= 1 && batch <= 65535, "batch of %d meshes", batch);
+  JPM_REQUIRE(ntab >= 2, "power-spectrum table needs at least 2 entries (got %d)", ntab);
+  JPM_REQUIRE(boxes || (Lx > 0 && Ly > 0 && Lz > 0), "box size must be positive");
+  const LinearArgs la = linear_args(nx, ny, nz, Lx, Ly, Lz, ktab, pktab, ntab, scale, boxes);
+  Tabs t;
+  rc = get_tabs(s, nx, ny, nz, 0, t);
+  if (rc) return rc;
+  const bool aligned = ((reinterpret_cast<uintptr_t>(in) | reinterpret_cast<uintptr_t>(out)) & 7u) == 0;
+  if (native_fft_ok(nx, ny, nz) && nx >= 2 && aligned)
+    return native_linear(s, nx, ny, nz, batch, in, spec, out, t, la);
+  if ((rc = fft_r2c(s, nx, ny, nz, batch, in, spec))) return rc;
+  HalfGrid hg = make_half(nx, ny, nz);
+  {
+    JPM_TIMED(s, "linear_field_kernel");
+    hipLaunchKernelGGL(linear_field_kernel, dim3(grid_for(hg.H, 256, 256 * 128 / batch + 1), batch), dim3(256), 0, s,
+                       static_cast<float2 *>(spec), hg, t, la);
+  }
+  JPM_LAUNCHED("linear_field_kernel");
+  return fft_c2r(s, nx, ny, nz, batch, spec, out);
 }
 
 // Batched forms over `batch` spectra of one shape (stride H; the force
@@ -643,25 +658,6 @@ int kspace_force_adjoint_batch(hipStream_t s, int nx, int ny, int nz, int batch,
                      static_cast<const float2 *>(in3), static_cast<float2 *>(out), hg, t, 0.0f, scale,
                      int((flags & JPM_K_DECONV) != 0));
   JPM_LAUNCHED("force_adjoint_kernel");
-  return JPM_OK;
-}
-
-int kspace_linear_field_batch(hipStream_t s, int nx, int ny, int nz, int batch, void *fk, const float *boxes,
-                              const float *ktab, const float *pktabs, int ntab, float scale) {
-  int rc = check_dims(nx, ny, nz);
-  if (rc) return rc;
-  JPM_REQUIRE(fk && boxes && ktab && pktabs && batch >= 1 && batch <= 65535, "bad batched linear field arguments");
-  JPM_REQUIRE(ntab >= 2, "power-spectrum table needs at least 2 entries (got %d)", ntab);
-  Tabs t;
-  rc = get_tabs(s, nx, ny, nz, 0, t);
-  if (rc) return rc;
-  HalfGrid hg = make_half(nx, ny, nz);
-  const float3 nm = make_float3(float(nx), float(ny), float(nz));
-  JPM_TIMED(s, "linear_field_kernel");
-  hipLaunchKernelGGL(linear_field_kernel, dim3(grid_for(hg.H, 256, 256 * 128 / batch + 1), batch), dim3(256), 0, s,
-                     static_cast<float2 *>(fk), hg, t, make_float3(1.0f, 1.0f, 1.0f), nm,
-                     float(cells(nx, ny, nz)), 1.0f, ktab, pktabs, ntab, scale, boxes);
-  JPM_LAUNCHED("linear_field_kernel");
   return JPM_OK;
 }
 

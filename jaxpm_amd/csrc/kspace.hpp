@@ -43,4 +43,48 @@ __device__ __forceinline__ float potential_factor(const Tabs &t, uint32_t i, uin
   return f * scale;
 }
 
+// jnp.interp(x, xp, fp) with the default clamping (fp[0] left of xp[0],
+// fp[-1] right of xp[-1]).
+__device__ __forceinline__ float interp(float x, const float *xp, const float *fp,
+                                        int n) {
+  // i = clip(searchsorted(xp, x, side='right'), 1, n - 1)
+  int lo = 0, hi = n;
+  while (lo < hi) {
+    int mid = (lo + hi) >> 1;
+    if (xp[mid] <= x) lo = mid + 1; else hi = mid;
+  }
+  int i = lo < 1 ? 1 : (lo > n - 1 ? n - 1 : lo);
+  float df = fp[i] - fp[i - 1];
+  float dx = xp[i] - xp[i - 1];
+  float delta = x - xp[i - 1];
+  float f = (fabsf(dx) <= 0.0f) ? fp[i - 1] : fp[i - 1] + (delta / dx) * df;
+  if (x < xp[0]) f = fp[0];
+  if (x > xp[n - 1]) f = fp[n - 1];
+  return f;
+}
+
+// The linear field's multiplier (pm.py:137-143): sqrt(P(|k|) M / V) scale.
+struct LinearArgs {
+  float3 box, nm;
+  float mcells, vol, scale;
+  const float *ktab, *pktab;
+  int ntab;
+  const float *boxes;   // per-item boxes (3 floats) and P(k) tables, or null
+  __device__ __forceinline__ void item(uint32_t b) {
+    if (!boxes) return;
+    pktab += size_t(b) * ntab;
+    box = make_float3(boxes[3 * b], boxes[3 * b + 1], boxes[3 * b + 2]);
+    vol = float(double(box.x) * double(box.y) * double(box.z));
+  }
+};
+
+__device__ __forceinline__ float linear_factor(const Tabs &t, uint32_t i, uint32_t jy, uint32_t kz,
+                                               const LinearArgs &a) {
+  // pm.py:137-138: (k_i / L_i * n_i)^2 summed, then ** 0.5
+  const float ax = t.k[i] / a.box.x * a.nm.x, ay = t.k[jy] / a.box.y * a.nm.y, az = t.k[kz] / a.box.z * a.nm.z;
+  const float kmesh = sqrtf((ax * ax + ay * ay) + az * az);
+  const float pk = interp(kmesh, a.ktab, a.pktab, a.ntab);
+  return sqrtf(pk * a.mcells / a.vol) * a.scale;
+}
+
 }  // namespace jpm

@@ -96,11 +96,13 @@ def lpt(cosmo, initial_conditions, particles=None, a=0.1, halo_size=0, sharding=
     ic = to_device(initial_conditions)
     shape = tuple(ic.shape)
     rel = particles is None
+    parts = None if rel else to_device(particles)
+    a = _coef(a)
+    if not _needs_grad(ic, parts):
+        out = _ops.lpt(ic, None if rel else parts.reshape(-1, 3), lpt_coefficients(cosmo, a, order))
+        return out if rel else tuple(t.reshape(parts.shape) for t in out)
     if rel:
         parts = torch.zeros((*shape, 3), dtype=torch.float32, device=ic.device)
-    else:
-        parts = to_device(particles)
-    a = _coef(a)
     E = _coef(np.sqrt(gr.Esqr(cosmo, a)))
     f1 = _forces_from_field(ic, parts.reshape(-1, 3), rel, 0.0, 0).reshape(parts.shape)
     d1 = _coef(gr.growth_factor(cosmo, a))

@@ -142,6 +142,58 @@ def test_lpt(gpu, config, a, order, absolute):
         assert rel_err(host(g), rr) < 3e-5
 
 
+@pytest.mark.parametrize("shape", [(2, 2, 4), (16, 24, 20), (48, 6, 96), (64, 32, 8), (33, 17, 34), (5, 7, 9), (1, 8, 10),
+                                   (9, 16, 64)])
+@pytest.mark.parametrize("order", [1, 2])
+@pytest.mark.parametrize("absolute", [True, False])
+def test_lpt_passes_give_the_bits_of_the_separate_steps(gpu, shape, order, absolute):
+    """lpt's fused passes (one forward transform, the shear fields' shared x
+    pass, the source formed in the inverse z pass, force and growth products in
+    one pass) against the entry points they stand for, one by one: the same
+    float operations, so the same bits.  Mesh axes of the library's own
+    transforms and of others, an axis of one cell, marches and waves that end
+    early."""
+    from jaxpm_amd import _ops, pm
+    print(f"lpt passes {shape} order={order} absolute={absolute}", flush=True)
+    pcos, _ = _pair_cosmo()
+    r = np.random.default_rng(28)
+    ic = dev(r.normal(size=shape))
+    parts = dev(lattice(shape) + r.normal(scale=0.4, size=(*shape, 3))) if absolute else None
+    got = pm.lpt(pcos, ic, parts, a=0.1, order=order)
+    m = ic.numel()
+    pos = parts.reshape(-1, 3) if absolute else torch.zeros((m, 3), device="cuda")
+
+    def force(field):
+        phi = _ops.c2r(_ops.kspace_potential(_ops.r2c(field), shape, 0.0, 1.0 / m), shape)
+        return _ops.read(_ops.fd4_gradient(phi), pos, relative=not absolute).reshape(*shape, 3)
+
+    c = [float(v) for v in pm.lpt_coefficients(pcos, 0.1, order)]
+    f1 = force(ic)
+    dx = c[0] * f1
+    p, f = c[1] * dx, c[2] * f1
+    if order == 2:
+        phi6 = _ops.c2r(_ops.kspace_shear6(_ops.r2c(ic), shape, 1.0 / m), shape)
+        f2 = force(_ops.lpt2_source(phi6))
+        dx2 = c[3] * f2
+        dx, p, f = dx + dx2, p + c[4] * dx2, f + c[5] * f2
+    for g, ref in zip(got, (dx, p, f)):
+        assert g.shape == ref.shape and torch.equal(g, ref)
+
+
+@pytest.mark.parametrize("shape", [(2, 2, 4), (16, 24, 96), (128, 6, 8), (33, 17, 34), (1, 8, 10)])
+@pytest.mark.parametrize("ntab", [2, 37])
+def test_linear_field_passes_give_the_bits_of_the_separate_steps(gpu, shape, ntab):
+    from jaxpm_amd import _ops
+    print(f"linear field passes {shape} ntab={ntab}", flush=True)
+    r = np.random.default_rng(29)
+    noise, box = dev(r.normal(size=shape)), [3.0 * s for s in shape]
+    k = np.linspace(0.05, 1.2, ntab)
+    ktab, pktab = dev(k), dev(np.exp(-k))
+    got = _ops.linear_field(noise, box, ktab, pktab)
+    fk = _ops.kspace_linear_field(_ops.r2c(noise), shape, box, ktab, pktab, 1.0 / noise.numel())
+    assert torch.equal(got, _ops.c2r(fk, shape))
+
+
 def test_linear_field_tabulated(gpu):
     from jaxpm_amd import cosmology as pc
     from jaxpm_amd import pm
