@@ -84,7 +84,10 @@ def paint_f64(mesh, pos, weight=None, wscalar=1.0, relative=False, zero=False):
     nx, ny, nz = _dims(mesh.shape)
     n = pos.shape[0]
     flags = (_lib.RELATIVE if relative else 0) | (_lib.ZERO_MESH if zero else 0)
-    call("jpm_cic_paint_f64", stream(), nx, ny, nz, ptr(pos), n, ptr(weight), float(wscalar), ptr(mesh), flags)
+    wsb = size("jpm_cic_paint_f64_workspace_size", nx, ny, nz, n)
+    ws = torch.empty(wsb, dtype=torch.uint8, device=mesh.device) if wsb else None
+    call("jpm_cic_paint_ws_f64", stream(), nx, ny, nz, ptr(pos), n, ptr(weight), float(wscalar), ptr(mesh), flags,
+         ptr(ws), wsb)
     return mesh
 
 

@@ -71,7 +71,9 @@ int kspace_linear_field(hipStream_t, int, int, int, void *, float, float, float,
                         int, float);
 int kspace_shear6(hipStream_t, int, int, int, const void *, void *, float, uint32_t);
 int lpt2_source(hipStream_t, int64_t, const float *, float *);
-int cic_paint_f64(hipStream_t, int, int, int, const double *, int64_t, const double *, double, double *, uint32_t);
+size_t cic_paint_f64_ws(int, int, int, int64_t);
+int cic_paint_f64(hipStream_t, int, int, int, const double *, int64_t, const double *, double, double *, uint32_t,
+                  void *, size_t);
 int cic_read_f64(hipStream_t, int, int, int, const double *, int, int64_t, const double *, int64_t, double *,
                  uint32_t);
 size_t pm_forces_f64_workspace_size(int, int, int);
@@ -694,7 +696,14 @@ int jpm_cic_read_f32(void *stream, int nx, int ny, int nz, const float *mesh, in
 
 int jpm_cic_paint_f64(void *stream, int nx, int ny, int nz, const double *pos, int64_t n, const double *weight,
                       double wscalar, double *mesh, uint32_t flags) {
-  JPM_GUARD(cic_paint_f64(as_stream(stream), nx, ny, nz, pos, n, weight, wscalar, mesh, flags));
+  JPM_GUARD(cic_paint_f64(as_stream(stream), nx, ny, nz, pos, n, weight, wscalar, mesh, flags, nullptr, 0));
+}
+
+size_t jpm_cic_paint_f64_workspace_size(int nx, int ny, int nz, int64_t n) { return cic_paint_f64_ws(nx, ny, nz, n); }
+
+int jpm_cic_paint_ws_f64(void *stream, int nx, int ny, int nz, const double *pos, int64_t n, const double *weight,
+                         double wscalar, double *mesh, uint32_t flags, void *ws, size_t ws_bytes) {
+  JPM_GUARD(cic_paint_f64(as_stream(stream), nx, ny, nz, pos, n, weight, wscalar, mesh, flags, ws, ws_bytes));
 }
 
 int jpm_cic_read_f64(void *stream, int nx, int ny, int nz, const double *mesh, int ncomp, int64_t comp_stride,

@@ -110,3 +110,60 @@ def test_float64_input_without_x64_runs_float32(gpu):
         out = painting.cic_paint(torch.zeros((8, 8, 8), device=gpu), pos)
     assert out.dtype == torch.float32
     assert any("jax_enable_x64" in str(w.message) for w in wl)
+
+
+@pytest.mark.parametrize("shape,n", [((16, 16, 16), 131072), ((33, 17, 70), 140000), ((1, 50, 33), 131073),
+                                     ((2, 2, 2), 150000), ((48, 40, 31), 262144)])
+def test_sorted_paint_f64(gpu, x64, shape, n):
+    """The paint of many particles (tile sort and LDS windows, several chunks
+    a tile): ragged tiles, axes of one tile and of one cell, positions past
+    both ends.  Sums of n deposits of |w| <= 1 in double: below 1e-13 of the
+    largest cell, as the atomic form's tests allow."""
+    from jaxpm_amd import painting
+    print(f"sorted paint f64 {shape} n={n}", flush=True)
+    r = np.random.default_rng(6)
+    pos = r.uniform(-1.2, 2.1, (n, 3)) * shape
+    w = r.uniform(0.5, 1.0, n)
+    mesh0 = r.normal(size=shape)
+    got = painting.cic_paint(torch.as_tensor(mesh0, device=gpu), torch.as_tensor(pos, device=gpu),
+                             torch.as_tensor(w, device=gpu))
+    assert rel(got.cpu().numpy(), op.cic_paint(mesh0, pos, w)) < 1e-13
+
+
+@pytest.mark.parametrize("shape", [(64, 64, 32), (66, 51, 40)])
+def test_sorted_relative_paint_and_forces_f64(gpu, x64, shape):
+    """Displacements that put corners on, just below and past the mesh ends
+    (dropped corners among them), and the forces that paint in their own
+    workspace, with one and with three particles per cell."""
+    from jaxpm_amd import painting, pm
+    print(f"sorted relative f64 {shape}", flush=True)
+    r = np.random.default_rng(7)
+    disp = r.normal(scale=1.3, size=(*shape, 3))
+    disp[0, :, :, 0] = -1e-17
+    disp[1, :, :, 1] = np.round(disp[1, :, :, 1])
+    disp[2, :, :, 2] = -2.5 * shape[2]
+    got = painting.cic_paint_dx(torch.as_tensor(disp, device=gpu))
+    assert rel(got.cpu().numpy(), op.cic_paint_dx(disp)) < 1e-13
+    got = pm.pm_forces(torch.as_tensor(disp, device=gpu), mesh_shape=shape, paint_absolute_pos=False)
+    assert rel(got.cpu().numpy(), opm.pm_forces(disp, mesh_shape=shape, paint_absolute_pos=False)) < 1e-12
+    pos = np.concatenate([(lattice(shape) + r.normal(scale=0.7, size=(*shape, 3))).reshape(-1, 3) for _ in range(3)])
+    got = pm.pm_forces(torch.as_tensor(pos, device=gpu), mesh_shape=shape)
+    assert rel(got.cpu().numpy(), opm.pm_forces(pos, mesh_shape=shape)) < 1e-12
+
+
+def test_sorted_paint_f64_nonfinite(gpu, x64):
+    """Non-finite positions and weights reach the cells that one atomic per
+    corner puts them in."""
+    from jaxpm_amd import _lib, painting
+    print("sorted paint f64 non-finite", flush=True)
+    shape, n = (32, 16, 20), 140000
+    r = np.random.default_rng(8)
+    pos, w = r.uniform(0, 16, (n, 3)), r.uniform(0.5, 1.0, n)
+    pos[3, 0], pos[500, 2], pos[7000, 1], w[20000] = np.nan, np.inf, -1e300, np.inf
+    p, wt = torch.as_tensor(pos, device=gpu), torch.as_tensor(w, device=gpu)
+    got = painting.cic_paint(torch.zeros(shape, dtype=torch.float64, device=gpu), p, wt)
+    ref = torch.zeros(shape, dtype=torch.float64, device=gpu)
+    _lib.call("jpm_cic_paint_f64", _lib.stream(), *shape, _lib.ptr(p), n, _lib.ptr(wt), 1.0, _lib.ptr(ref), 0)
+    assert torch.equal(torch.isnan(got), torch.isnan(ref)) and torch.equal(torch.isinf(got), torch.isinf(ref))
+    ok = torch.isfinite(ref)
+    assert not bool(ok.all()) and rel(got[ok].cpu().numpy(), ref[ok].cpu().numpy()) < 1e-13
