@@ -27,7 +27,7 @@ int kspace_force_batch(hipStream_t, int, int, int, int, const void *, void *, fl
 int kspace_force_adjoint_batch(hipStream_t, int, int, int, int, const void *, void *, float, uint32_t);
 int linear_field(hipStream_t, int, int, int, int, const float *, float *, float, float, float, const float *,
                  const float *, const float *, int, float, void *);
-int grad_pos_batch(hipStream_t, const SimRef *, int, bool, const float *, const float *, float *);
+int grad_pos_batch(hipStream_t, const SimRef *, int, bool, bool, const float *, const float *, float *);
 int batch_grad(hipStream_t, const BatchBins &, const float *, const float *, const float *, const float *, float *,
                bool, const float *, float *, float *);
 
@@ -382,7 +382,9 @@ int batch_paint_mesh(hipStream_t s, const SimBatch &bt, const float *pos, float 
 }
 
 int batch_paint_vjp(hipStream_t s, const SimBatch &bt, const float *pos, const float *gmesh, float *gpos) {
-  return grad_pos_batch(s, bt.dev, bt.B, bt.rel, gmesh, pos, gpos);
+  bool pair = true;
+  for (const SimClass &c : bt.classes) pair = pair && c.nz >= 2;
+  return grad_pos_batch(s, bt.dev, bt.B, bt.rel, pair, gmesh, pos, gpos);
 }
 
 // ------------------------------------------------- per-simulation vectors

@@ -101,6 +101,21 @@ __device__ __forceinline__ void corners_bit_order(const Axis &ax, const Axis &ay
   }
 }
 
+// sum_o v_o W_o of corner values v[bx | by << 1 | bz << 2], in the reference's
+// corner order: painting.py:24-25, or relative painting_utils.py:43-45.
+template <bool REL>
+__device__ __forceinline__ float corner_sum(const float v[8], const Axis &ax, const Axis &ay, const Axis &az) {
+  const int abs_order[8] = {0, 1, 2, 4, 3, 5, 6, 7};
+  float s = 0.0f;
+#pragma unroll
+  for (int q = 0; q < 8; ++q) {
+    const int o = REL ? q : abs_order[q];
+    const float wx = (o & 1) ? ax.w1 : ax.w0, wy = (o & 2) ? ay.w1 : ay.w0, wz = (o & 4) ? az.w1 : az.w0;
+    s += v[o] * (wx * wy * wz);
+  }
+  return s;
+}
+
 struct Grid {
   int nx, ny, nz;
   FastDiv div_nz, div_ny;
@@ -273,22 +288,26 @@ __global__ void __launch_bounds__(256) zero_f32_kernel(float *__restrict__ p, ui
 
 // ------------------------------------------------------------------- read
 
-template <bool REL, int NC>
+// The direct reads and their adjoint below are bound by vector-memory issue
+// and by the mesh lines their lanes touch: the z corners come in pairs, and
+// each XCD takes a contiguous run of particles.  9 million displaced particles
+// on 250 x 201 x 180 cells, single loads and dispatch order before: read 163
+// -> 109 us, gradient 196 -> 159 us; three meshes, 1.1 million particles: 76
+// -> 38 and 58 -> 39 us.
+template <bool REL, int NC, bool PAIR>
 __global__ void __launch_bounds__(256)
 read_kernel(const float *__restrict__ mesh, uint32_t cstride, const float *__restrict__ pos,
-            uint32_t n, Grid g, float *__restrict__ out) {
-  for (uint32_t p = blockIdx.x * blockDim.x + threadIdx.x; p < n; p += gridDim.x * blockDim.x) {
-    Cic c;
-    particle_cic<REL>(pos, p, g, c);
+            uint32_t n, Grid g, float *__restrict__ out, uint32_t per) {
+  const uint32_t p = ((blockIdx.x & 7u) * per + (blockIdx.x >> 3)) * blockDim.x + threadIdx.x;
+  if (p >= n) return;
+  Axis ax, ay, az;
+  particle_axes<REL>(pos, p, g, ax, ay, az);
+  const uint32_t ix[2] = {uint32_t(ax.i0), uint32_t(ax.i1)}, iy[2] = {uint32_t(ay.i0), uint32_t(ay.i1)},
+                 iz[2] = {uint32_t(az.i0), uint32_t(az.i1)};
+  float v[NC][8];
+  load_corners<PAIR, NC>(mesh, cstride, ix, iy, iz, uint32_t(g.ny), uint32_t(g.nz), v);
 #pragma unroll
-    for (int comp = 0; comp < NC; ++comp) {
-      const float *m = mesh + size_t(comp) * cstride;
-      float s = 0.0f;
-#pragma unroll
-      for (int o = 0; o < 8; ++o) s += m[c.idx[o]] * c.w[o];
-      out[size_t(p) * NC + comp] = s;
-    }
-  }
+  for (int comp = 0; comp < NC; ++comp) out[size_t(p) * NC + comp] = corner_sum<REL>(v[comp], ax, ay, az);
 }
 
 // Multi-channel paint: channel c of particle p deposits weight[p*nc + c]
@@ -342,56 +361,60 @@ paint_multi_fixed_kernel(const float *__restrict__ pos, const float *__restrict_
 // cot == NULL means cot = 1.  This is the position cotangent of both
 // cic_read (mesh = the sampled field, cot = output cotangent) and cic_paint
 // (mesh = cotangent of the painted mesh, w = particle weight).
-template <bool REL, int NC>
+template <bool REL, int NC, bool PAIR>
+__device__ __forceinline__ void grad_pos_of(const float *__restrict__ mesh, size_t cstride, const float *__restrict__ pos,
+                                            uint32_t p, const Grid &g, const float *__restrict__ cot, float out[3]) {
+  Axis ax, ay, az;
+  particle_axes<REL>(pos, p, g, ax, ay, az);
+  const uint32_t ix[2] = {uint32_t(ax.i0), uint32_t(ax.i1)}, iy[2] = {uint32_t(ay.i0), uint32_t(ay.i1)},
+                 iz[2] = {uint32_t(az.i0), uint32_t(az.i1)};
+  float v[NC][8];
+  load_corners<PAIR, NC>(mesh, cstride, ix, iy, iz, uint32_t(g.ny), uint32_t(g.nz), v);
+  const float wx[2] = {ax.w0, ax.w1}, wy[2] = {ay.w0, ay.w1}, wz[2] = {az.w0, az.w1};
+  const float dx[2] = {ax.d0, ax.d1}, dy[2] = {ay.d0, ay.d1}, dz[2] = {az.d0, az.d1};
+  out[0] = out[1] = out[2] = 0.0f;
+#pragma unroll
+  for (int comp = 0; comp < NC; ++comp) {
+    float sx = 0.0f, sy = 0.0f, sz = 0.0f;
+#pragma unroll
+    for (int o = 0; o < 8; ++o) {
+      const int bx = o & 1, by = (o >> 1) & 1, bz = (o >> 2) & 1;
+      sx += v[comp][o] * (dx[bx] * wy[by] * wz[bz]);
+      sy += v[comp][o] * (wx[bx] * dy[by] * wz[bz]);
+      sz += v[comp][o] * (wx[bx] * wy[by] * dz[bz]);
+    }
+    const float cc = cot ? cot[size_t(p) * NC + comp] : 1.0f;
+    out[0] += cc * sx;
+    out[1] += cc * sy;
+    out[2] += cc * sz;
+  }
+}
+
+template <bool REL, int NC, bool PAIR>
 __global__ void __launch_bounds__(256)
 grad_pos_kernel(const float *__restrict__ mesh, uint32_t cstride, const float *__restrict__ pos, uint32_t n,
                 Grid g, const float *__restrict__ cot, const float *__restrict__ weight, float wscalar,
-                int accumulate, float *__restrict__ gpos) {
-  for (uint32_t p = blockIdx.x * blockDim.x + threadIdx.x; p < n; p += gridDim.x * blockDim.x) {
-    Axis ax, ay, az;
-    particle_axes<REL>(pos, p, g, ax, ay, az);
-    const uint32_t ixs[2] = {uint32_t(ax.i0), uint32_t(ax.i1)};
-    const uint32_t iys[2] = {uint32_t(ay.i0), uint32_t(ay.i1)};
-    const uint32_t izs[2] = {uint32_t(az.i0), uint32_t(az.i1)};
-    const float wx[2] = {ax.w0, ax.w1}, wy[2] = {ay.w0, ay.w1}, wz[2] = {az.w0, az.w1};
-    const float dx[2] = {ax.d0, ax.d1}, dy[2] = {ay.d0, ay.d1}, dz[2] = {az.d0, az.d1};
-    float gx = 0.0f, gy = 0.0f, gz = 0.0f;
-#pragma unroll
-    for (int comp = 0; comp < NC; ++comp) {
-      const float *mc = mesh + size_t(comp) * cstride;
-      float sx = 0.0f, sy = 0.0f, sz = 0.0f;
-#pragma unroll
-      for (int o = 0; o < 8; ++o) {
-        const int bx = o & 1, by = (o >> 1) & 1, bz = (o >> 2) & 1;
-        const float v = mc[(ixs[bx] * uint32_t(g.ny) + iys[by]) * uint32_t(g.nz) + izs[bz]];
-        sx += v * (dx[bx] * wy[by] * wz[bz]);
-        sy += v * (wx[bx] * dy[by] * wz[bz]);
-        sz += v * (wx[bx] * wy[by] * dz[bz]);
-      }
-      const float cc = cot ? cot[size_t(p) * NC + comp] : 1.0f;
-      gx += cc * sx;
-      gy += cc * sy;
-      gz += cc * sz;
-    }
-    const float wp = weight ? weight[p] : wscalar;
-    gx *= wp;
-    gy *= wp;
-    gz *= wp;
-    float *o = gpos + 3 * size_t(p);
-    if (accumulate) {
-      gx += o[0];
-      gy += o[1];
-      gz += o[2];
-    }
-    o[0] = gx;
-    o[1] = gy;
-    o[2] = gz;
+                int accumulate, float *__restrict__ gpos, uint32_t per) {
+  const uint32_t p = ((blockIdx.x & 7u) * per + (blockIdx.x >> 3)) * blockDim.x + threadIdx.x;
+  if (p >= n) return;
+  float s[3];
+  grad_pos_of<REL, NC, PAIR>(mesh, cstride, pos, p, g, cot, s);
+  const float wp = weight ? weight[p] : wscalar;
+  float gx = s[0] * wp, gy = s[1] * wp, gz = s[2] * wp;
+  float *o = gpos + 3 * size_t(p);
+  if (accumulate) {
+    gx += o[0];
+    gy += o[1];
+    gz += o[2];
   }
+  o[0] = gx;
+  o[1] = gy;
+  o[2] = gz;
 }
 
 // Position cotangent of the batched paint: gpos_p = sum_o g[idx_o] dW_o/dx
 // over each simulation's particles and mesh (blockIdx.y: simulation).
-template <bool REL>
+template <bool REL, bool PAIR>
 __global__ void __launch_bounds__(256)
 grad_pos_batch_kernel(const SimRef *__restrict__ sims, const float *__restrict__ mesh_all,
                       const float *__restrict__ pos_all, float *__restrict__ gpos_all) {
@@ -405,38 +428,26 @@ grad_pos_batch_kernel(const SimRef *__restrict__ sims, const float *__restrict__
   const float *mesh = mesh_all + s.cell0;
   const float *pos = pos_all + 3 * size_t(s.part0);
   float *gpos = gpos_all + 3 * size_t(s.part0);
-  for (uint32_t p = blockIdx.x * blockDim.x + threadIdx.x; p < s.n; p += gridDim.x * blockDim.x) {
-    Axis ax, ay, az;
-    particle_axes<REL>(pos, p, g, ax, ay, az);
-    const uint32_t ixs[2] = {uint32_t(ax.i0), uint32_t(ax.i1)};
-    const uint32_t iys[2] = {uint32_t(ay.i0), uint32_t(ay.i1)};
-    const uint32_t izs[2] = {uint32_t(az.i0), uint32_t(az.i1)};
-    const float wx[2] = {ax.w0, ax.w1}, wy[2] = {ay.w0, ay.w1}, wz[2] = {az.w0, az.w1};
-    const float dx[2] = {ax.d0, ax.d1}, dy[2] = {ay.d0, ay.d1}, dz[2] = {az.d0, az.d1};
-    float sx = 0.0f, sy = 0.0f, sz = 0.0f;
-#pragma unroll
-    for (int o = 0; o < 8; ++o) {
-      const int bx = o & 1, by = (o >> 1) & 1, bz = (o >> 2) & 1;
-      const float v = mesh[(ixs[bx] * uint32_t(g.ny) + iys[by]) * uint32_t(g.nz) + izs[bz]];
-      sx += v * (dx[bx] * wy[by] * wz[bz]);
-      sy += v * (wx[bx] * dy[by] * wz[bz]);
-      sz += v * (wx[bx] * wy[by] * dz[bz]);
-    }
-    float *o = gpos + 3 * size_t(p);
-    o[0] = 1.0f * sx;
-    o[1] = 1.0f * sy;
-    o[2] = 1.0f * sz;
+  // each XCD's workgroups (blockIdx.x mod 8) walk one contiguous eighth
+  const uint32_t per = ((s.n + 255u) / 256u + 7u) / 8u;
+  for (uint32_t b = blockIdx.x >> 3; b < per; b += gridDim.x >> 3) {
+    const uint32_t p = ((blockIdx.x & 7u) * per + b) * 256u + threadIdx.x;
+    if (p >= s.n) continue;
+    float o[3];
+    grad_pos_of<REL, 1, PAIR>(mesh, 0, pos, p, g, nullptr, o);
+    gpos[3 * size_t(p)] = o[0];
+    gpos[3 * size_t(p) + 1] = o[1];
+    gpos[3 * size_t(p) + 2] = o[2];
   }
 }
 
-int grad_pos_batch(hipStream_t s, const SimRef *sims, int B, bool rel, const float *mesh, const float *pos,
+int grad_pos_batch(hipStream_t s, const SimRef *sims, int B, bool rel, bool pair, const float *mesh, const float *pos,
                    float *gpos) {
   JPM_REQUIRE(sims && mesh && pos && gpos && B >= 1, "null pointer argument");
   JPM_TIMED(s, "grad_pos_kernel");
-  if (rel)
-    hipLaunchKernelGGL(grad_pos_batch_kernel<true>, dim3(256, B), dim3(256), 0, s, sims, mesh, pos, gpos);
-  else
-    hipLaunchKernelGGL(grad_pos_batch_kernel<false>, dim3(256, B), dim3(256), 0, s, sims, mesh, pos, gpos);
+  auto kern = pair ? (rel ? grad_pos_batch_kernel<true, true> : grad_pos_batch_kernel<false, true>)
+                   : (rel ? grad_pos_batch_kernel<true, false> : grad_pos_batch_kernel<false, false>);
+  hipLaunchKernelGGL(kern, dim3(256, B), dim3(256), 0, s, sims, mesh, pos, gpos);
   JPM_LAUNCHED("grad_pos_batch_kernel");
   return JPM_OK;
 }
@@ -562,11 +573,12 @@ int cic_read(hipStream_t s, int nx, int ny, int nz, const float *mesh, int ncomp
   if (n == 0) return JPM_OK;
   JPM_REQUIRE(mesh && pos && out, "null pointer argument");
   Grid g = make_grid(nx, ny, nz);
-  const unsigned grid = grid_for(n, 256, 256 * 128);
   const uint32_t cs = uint32_t(comp_stride);
-#define JPM_READ(R, C)                                                                      \
-  hipLaunchKernelGGL((read_kernel<R, C>), dim3(grid), dim3(256), 0, s, mesh, cs, pos, uint32_t(n), g, \
-                     out)
+  uint32_t per;
+  const unsigned grid = xcd_blocks(n, 256, per);
+#define JPM_READ(R, C)                                                                                           \
+  hipLaunchKernelGGL((nz >= 2 ? read_kernel<R, C, true> : read_kernel<R, C, false>), dim3(grid), dim3(256), 0, s, \
+                     mesh, cs, pos, uint32_t(n), g, out, per)
 #define JPM_READ_NC(R)                 \
   switch (ncomp) {                     \
     case 1: JPM_READ(R, 1); break;     \
@@ -684,11 +696,12 @@ int cic_grad_pos(hipStream_t s, int nx, int ny, int nz, const float *mesh, int n
   if (n == 0) return JPM_OK;
   JPM_REQUIRE(mesh && pos && gpos, "null pointer argument");
   Grid g = make_grid(nx, ny, nz);
-  const unsigned grid = grid_for(n, 256, 256 * 128);
   const uint32_t cs = uint32_t(ncomp == 1 ? m : comp_stride);
-#define JPM_G(R, C)                                                                                          \
-  hipLaunchKernelGGL((grad_pos_kernel<R, C>), dim3(grid), dim3(256), 0, s, mesh, cs, pos, uint32_t(n), g, cot, \
-                     weight, wscalar, accumulate, gpos)
+  uint32_t per;
+  const unsigned grid = xcd_blocks(n, 256, per);
+#define JPM_G(R, C)                                                                                               \
+  hipLaunchKernelGGL((nz >= 2 ? grad_pos_kernel<R, C, true> : grad_pos_kernel<R, C, false>), dim3(grid), dim3(256), \
+                     0, s, mesh, cs, pos, uint32_t(n), g, cot, weight, wscalar, accumulate, gpos, per)
 #define JPM_G_NC(R)              \
   switch (ncomp) {               \
     case 1: JPM_G(R, 1); break;  \
@@ -733,22 +746,20 @@ __global__ void axpy_tail_kernel(float a, const float *__restrict__ x, float *__
 }
 
 // Kick fused into the 3-component read: vel[p] += gamma * sum_o phi[idx_o] W_o.
-template <bool REL>
+template <bool REL, bool PAIR>
 __global__ void __launch_bounds__(256)
 kick_kernel(const float *__restrict__ phi, uint32_t cstride, const float *__restrict__ pos, uint32_t n, Grid g,
-            float gamma, float *__restrict__ vel) {
-  for (uint32_t p = blockIdx.x * blockDim.x + threadIdx.x; p < n; p += gridDim.x * blockDim.x) {
-    Cic c;
-    particle_cic<REL>(pos, p, g, c);
+            float gamma, float *__restrict__ vel, uint32_t per) {
+  const uint32_t p = ((blockIdx.x & 7u) * per + (blockIdx.x >> 3)) * blockDim.x + threadIdx.x;
+  if (p >= n) return;
+  Axis ax, ay, az;
+  particle_axes<REL>(pos, p, g, ax, ay, az);
+  const uint32_t ix[2] = {uint32_t(ax.i0), uint32_t(ax.i1)}, iy[2] = {uint32_t(ay.i0), uint32_t(ay.i1)},
+                 iz[2] = {uint32_t(az.i0), uint32_t(az.i1)};
+  float v[3][8];
+  load_corners<PAIR, 3>(phi, cstride, ix, iy, iz, uint32_t(g.ny), uint32_t(g.nz), v);
 #pragma unroll
-    for (int comp = 0; comp < 3; ++comp) {
-      const float *m = phi + size_t(comp) * cstride;
-      float s = 0.0f;
-#pragma unroll
-      for (int o = 0; o < 8; ++o) s += m[c.idx[o]] * c.w[o];
-      vel[size_t(p) * 3 + comp] += gamma * s;
-    }
-  }
+  for (int comp = 0; comp < 3; ++comp) vel[size_t(p) * 3 + comp] += gamma * corner_sum<REL>(v[comp], ax, ay, az);
 }
 
 // Rows of 3 floats in another order, one or two arrays per launch:
@@ -779,29 +790,33 @@ permute_rows_kernel(const uint32_t *__restrict__ order, const float *__restrict_
 // LPT at given positions: the three-component reads of the first- and (ORDER
 // 2) second-order force meshes, read_kernel's sums, and their growth-factor
 // products, without the force arrays and the elementwise passes over them.
-template <bool REL, int ORDER>
+template <bool REL, int ORDER, bool PAIR>
 __global__ void __launch_bounds__(256)
 lpt_read_kernel(const float *__restrict__ f1, const float *__restrict__ f2, uint32_t m, const float *__restrict__ pos,
                 uint32_t n, Grid g, LptCoef lc, float *__restrict__ dx, float *__restrict__ pp,
-                float *__restrict__ ff) {
-  for (uint32_t p = blockIdx.x * blockDim.x + threadIdx.x; p < n; p += gridDim.x * blockDim.x) {
-    Cic c;
-    particle_cic<REL>(pos, p, g, c);
+                float *__restrict__ ff, uint32_t per) {
+  const uint32_t p = ((blockIdx.x & 7u) * per + (blockIdx.x >> 3)) * blockDim.x + threadIdx.x;
+  if (p >= n) return;
+  Axis ax, ay, az;
+  particle_axes<REL>(pos, p, g, ax, ay, az);
+  const uint32_t ix[2] = {uint32_t(ax.i0), uint32_t(ax.i1)}, iy[2] = {uint32_t(ay.i0), uint32_t(ay.i1)},
+                 iz[2] = {uint32_t(az.i0), uint32_t(az.i1)};
+  float F[2][3];
 #pragma unroll
-    for (int comp = 0; comp < 3; ++comp) {
-      float s1 = 0.0f, s2 = 0.0f;
+  for (int o = 0; o < ORDER; ++o) {
+    float v[3][8];
+    load_corners<PAIR, 3>(o ? f2 : f1, m, ix, iy, iz, uint32_t(g.ny), uint32_t(g.nz), v);
 #pragma unroll
-      for (int o = 0; o < 8; ++o) {
-        s1 += f1[size_t(comp) * m + c.idx[o]] * c.w[o];
-        if (ORDER == 2) s2 += f2[size_t(comp) * m + c.idx[o]] * c.w[o];
-      }
-      float a, b, d;
-      lpt_combine(lc, s1, ORDER == 2, s2, a, b, d);
-      const size_t e = 3 * size_t(p) + comp;
-      dx[e] = a;
-      pp[e] = b;
-      ff[e] = d;
-    }
+    for (int comp = 0; comp < 3; ++comp) F[o][comp] = corner_sum<REL>(v[comp], ax, ay, az);
+  }
+#pragma unroll
+  for (int comp = 0; comp < 3; ++comp) {
+    float a, b, d;
+    lpt_combine(lc, F[0][comp], ORDER == 2, F[ORDER - 1][comp], a, b, d);
+    const size_t e = 3 * size_t(p) + comp;
+    dx[e] = a;
+    pp[e] = b;
+    ff[e] = d;
   }
 }
 
@@ -814,11 +829,13 @@ int lpt_read(hipStream_t s, int nx, int ny, int nz, const float *f1, const float
   if (n == 0) return JPM_OK;
   JPM_REQUIRE(f1 && pos && dx && p && f, "null pointer argument");
   const Grid g = make_grid(nx, ny, nz);
-  auto kern = rel ? (f2 ? lpt_read_kernel<true, 2> : lpt_read_kernel<true, 1>)
-                  : (f2 ? lpt_read_kernel<false, 2> : lpt_read_kernel<false, 1>);
+  uint32_t per;
+  const unsigned grid = xcd_blocks(n, 256, per);
+#define JPM_LR(R, O) (nz >= 2 ? lpt_read_kernel<R, O, true> : lpt_read_kernel<R, O, false>)
+  auto kern = rel ? (f2 ? JPM_LR(true, 2) : JPM_LR(true, 1)) : (f2 ? JPM_LR(false, 2) : JPM_LR(false, 1));
+#undef JPM_LR
   JPM_TIMED(s, "lpt_read_kernel");
-  hipLaunchKernelGGL(kern, dim3(grid_for(n, 256, 256 * 128)), dim3(256), 0, s, f1, f2, uint32_t(m), pos, uint32_t(n),
-                     g, lc, dx, p, f);
+  hipLaunchKernelGGL(kern, dim3(grid), dim3(256), 0, s, f1, f2, uint32_t(m), pos, uint32_t(n), g, lc, dx, p, f, per);
   JPM_LAUNCHED("lpt_read_kernel");
   return JPM_OK;
 }
@@ -871,19 +888,14 @@ int kick(hipStream_t s, int nx, int ny, int nz, const float *phi3, const float *
   if (n == 0) return JPM_OK;
   JPM_REQUIRE(phi3 && pos && vel, "null pointer argument");
   Grid g = make_grid(nx, ny, nz);
-  const unsigned grid = grid_for(n, 256, 256 * 128);
-  if (rel)
-    {
-      JPM_TIMED(s, "kick_kernel");
-      hipLaunchKernelGGL(kick_kernel<true>, dim3(grid), dim3(256), 0, s, phi3, uint32_t(m), pos, uint32_t(n), g, gamma,
-                         vel);
-    }
-  else
-    {
-      JPM_TIMED(s, "kick_kernel");
-      hipLaunchKernelGGL(kick_kernel<false>, dim3(grid), dim3(256), 0, s, phi3, uint32_t(m), pos, uint32_t(n), g,
-                         gamma, vel);
-    }
+  uint32_t per;
+  const unsigned grid = xcd_blocks(n, 256, per);
+  auto kern = nz >= 2 ? (rel ? kick_kernel<true, true> : kick_kernel<false, true>)
+                      : (rel ? kick_kernel<true, false> : kick_kernel<false, false>);
+  {
+    JPM_TIMED(s, "kick_kernel");
+    hipLaunchKernelGGL(kern, dim3(grid), dim3(256), 0, s, phi3, uint32_t(m), pos, uint32_t(n), g, gamma, vel, per);
+  }
   JPM_LAUNCHED("kick_kernel");
   return JPM_OK;
 }

@@ -213,6 +213,12 @@ sort_f64_kernel(const double *__restrict__ pos, uint32_t n, GridD g, TileGrid t,
   }
 }
 
+// The corners are the (periodic) 2^3 block at the low corner.
+__device__ __forceinline__ bool block_corners(const AxisD &ax, const AxisD &ay, const AxisD &az, const GridD &g) {
+  return ax.i1 == (ax.i0 + 1 == g.nx ? 0 : ax.i0 + 1) && ay.i1 == (ay.i0 + 1 == g.ny ? 0 : ay.i0 + 1) &&
+         az.i1 == (az.i0 + 1 == g.nz ? 0 : az.i0 + 1);
+}
+
 // A particle whose corners are the 2^3 block at its low corner deposits in
 // the window; any other (a dropped or doubly rounded relative corner, a
 // non-finite position) adds its eight deposits to the mesh itself, as
@@ -235,9 +241,7 @@ accum_f64_kernel(const Rec64 *__restrict__ recs, const ChunkDesc *__restrict__ d
     const double wp = weight ? weight[r.p] : wscalar;
     AxisD ax, ay, az;
     axes_d<REL>(r.x, r.y, r.z, r.p, g, ax, ay, az);
-    const bool block = ax.i1 == (ax.i0 + 1 == g.nx ? 0 : ax.i0 + 1) && ay.i1 == (ay.i0 + 1 == g.ny ? 0 : ay.i0 + 1) &&
-                       az.i1 == (az.i0 + 1 == g.nz ? 0 : az.i0 + 1);
-    if (block) {
+    if (block_corners(ax, ay, az, g)) {
       double *w0 = win + ((ax.i0 - ox) * kWin + (ay.i0 - oy)) * kWin + (az.i0 - oz);
 #pragma unroll
       for (int o = 0; o < 8; ++o) {
@@ -296,21 +300,96 @@ reduce_f64_kernel(const double *__restrict__ partial, const uint32_t *__restrict
   }
 }
 
-template <bool REL>
+template <bool REL, int NC, bool PAIR>
 __global__ void __launch_bounds__(256)
-read_f64_kernel(const double *__restrict__ mesh, int nc, int64_t cstride, const double *__restrict__ pos, uint32_t n,
-                GridD g, double *__restrict__ out) {
-  for (uint32_t p = blockIdx.x * blockDim.x + threadIdx.x; p < n; p += gridDim.x * blockDim.x) {
-    int64_t idx[8];
-    double w[8];
-    corners_d<REL>(pos, p, g, idx, w);
-    for (int c = 0; c < nc; ++c) {
-      const double *m = mesh + c * cstride;
-      double s = 0.0;
+read_f64_kernel(const double *__restrict__ mesh, int64_t cstride, const double *__restrict__ pos, uint32_t n, GridD g,
+                double *__restrict__ out, uint32_t per) {
+  const uint32_t p = ((blockIdx.x & 7u) * per + (blockIdx.x >> 3)) * blockDim.x + threadIdx.x;
+  if (p >= n) return;
+  AxisD ax, ay, az;
+  axes_d<REL>(pos[3 * size_t(p)], pos[3 * size_t(p) + 1], pos[3 * size_t(p) + 2], p, g, ax, ay, az);
+  const uint32_t ix[2] = {uint32_t(ax.i0), uint32_t(ax.i1)}, iy[2] = {uint32_t(ay.i0), uint32_t(ay.i1)},
+                 iz[2] = {uint32_t(az.i0), uint32_t(az.i1)};
+  // the corner order of corners_of_d
+  const int abs_order[8] = {0, 1, 2, 4, 3, 5, 6, 7};
+  double v[NC][8];
+  load_corners<PAIR, NC>(mesh, size_t(cstride), ix, iy, iz, uint32_t(g.ny), uint32_t(g.nz), v);
 #pragma unroll
-      for (int o = 0; o < 8; ++o) s += m[idx[o]] * w[o];
-      out[size_t(p) * nc + c] = s;
+  for (int c = 0; c < NC; ++c) {
+    double s = 0.0;
+#pragma unroll
+    for (int q = 0; q < 8; ++q) {
+      const int o = REL ? q : abs_order[q];
+      s += v[c][o] * (((o & 1) ? ax.w1 : ax.w0) * ((o & 2) ? ay.w1 : ay.w0) * ((o & 4) ? az.w1 : az.w0));
     }
+    out[size_t(p) * NC + c] = s;
+  }
+}
+
+// read_f64_kernel<REL, 3> over a tile sort: each workgroup holds the three
+// meshes' 17^3 windows of its tile in LDS (115 KiB, one workgroup of 16 waves
+// a CU), so the particles of displaced lattices, whose lanes touch a cache line
+// each, read LDS instead.  A particle whose corners are no 2^3 block reads the
+// meshes.  The same sums in the same order.  128^3 particles displaced by 3
+// cells rms: 46 us, the direct read 122 (173 with single loads).
+template <bool REL>
+__global__ void __launch_bounds__(1024)
+read3_sorted_f64_kernel(const Rec64 *__restrict__ recs, const ChunkDesc *__restrict__ desc,
+                        const uint32_t *__restrict__ nchunks, const double *__restrict__ phi3, int64_t M, GridD g,
+                        TileGrid t, double *__restrict__ out) {
+  extern __shared__ double rwin[];
+  if (blockIdx.x >= *nchunks) return;
+  const ChunkDesc d = desc[blockIdx.x];
+  int itx, ity, itz;
+  tile_origin(d.tile, t, itx, ity, itz);
+  const int ox = itx * kTile, oy = ity * kTile, oz = itz * kTile;
+  constexpr int kPer = (kWinCells + 1023) / 1024;
+  double v[3][kPer];
+#pragma unroll
+  for (int i = 0; i < kPer; ++i) {
+    const int e0 = int(threadIdx.x) + i * 1024, e = e0 < kWinCells ? e0 : kWinCells - 1;
+    const int c = e % kWin, ab = e / kWin, b = ab % kWin, a = ab / kWin;
+    const size_t cell = (size_t((ox + a) % t.nx) * t.ny + size_t((oy + b) % t.ny)) * t.nz + size_t((oz + c) % t.nz);
+#pragma unroll
+    for (int f = 0; f < 3; ++f) v[f][i] = phi3[f * M + cell];
+  }
+#pragma unroll
+  for (int i = 0; i < kPer; ++i) {
+    const int e = int(threadIdx.x) + i * 1024;
+#pragma unroll
+    for (int f = 0; f < 3; ++f)
+      if (e < kWinCells) rwin[f * kWinCells + e] = v[f][i];
+  }
+  __syncthreads();
+  const int abs_order[8] = {0, 1, 2, 4, 3, 5, 6, 7};
+  for (uint32_t q = threadIdx.x; q < d.count; q += 1024) {
+    const Rec64 r = recs[d.start + q];
+    AxisD ax, ay, az;
+    axes_d<REL>(r.x, r.y, r.z, r.p, g, ax, ay, az);
+    double s[3] = {0.0, 0.0, 0.0};
+    if (block_corners(ax, ay, az, g)) {
+      const double *w0 = rwin + ((ax.i0 - ox) * kWin + (ay.i0 - oy)) * kWin + (az.i0 - oz);
+#pragma unroll
+      for (int k = 0; k < 8; ++k) {
+        const int o = REL ? k : abs_order[k];
+        const double w = ((o & 1) ? ax.w1 : ax.w0) * ((o & 2) ? ay.w1 : ay.w0) * ((o & 4) ? az.w1 : az.w0);
+        const int off = ((o & 1) * kWin + ((o >> 1) & 1)) * kWin + (o >> 2);
+#pragma unroll
+        for (int f = 0; f < 3; ++f) s[f] += w0[f * kWinCells + off] * w;
+      }
+    } else {
+      int64_t idx[8];
+      double w[8];
+      corners_of_d<REL>(ax, ay, az, g, idx, w);
+#pragma unroll
+      for (int k = 0; k < 8; ++k)
+#pragma unroll
+        for (int f = 0; f < 3; ++f) s[f] += phi3[f * M + idx[k]] * w[k];
+    }
+    double *o3 = out + 3 * size_t(r.p);
+    o3[0] = s[0];
+    o3[1] = s[1];
+    o3[2] = s[2];
   }
 }
 
@@ -392,7 +471,8 @@ GridD make_grid_d(int nx, int ny, int nz) {
 int fft_d2z(hipStream_t s, int nx, int ny, int nz, int batch, const double *in, void *out);
 int fft_z2d(hipStream_t s, int nx, int ny, int nz, int batch, void *in, double *out);
 
-// Workspace of the sorted paint (byte offsets); total 0 where the atomic form
+// Workspace of the sorted paint (byte offsets); the sort, which a read may reuse,
+// then the windows of the accumulation; total 0 where the atomic form
 // is used instead: few particles, or more tiles than the LDS histogram
 // holds.  48^3 random particles take 43 us by atomics and 42 us sorted, 64^3
 // 94 and 47 us, 128^3 727 and 120 us; in the order of an undisturbed lattice,
@@ -400,7 +480,7 @@ int fft_z2d(hipStream_t s, int nx, int ny, int nz, int batch, void *in, double *
 // 110 and 75 us.
 struct Paint64Ws {
   uint32_t maxchunks;
-  size_t count, tstart, cursor, nchunk, choff, totals, desc, recs, partial, total;
+  size_t count, tstart, cursor, nchunk, choff, totals, desc, recs, sort, partial, total;
 };
 
 static Paint64Ws paint64_ws(int nx, int ny, int nz, int64_t n) {
@@ -423,6 +503,7 @@ static Paint64Ws paint64_ws(int nx, int ny, int nz, int64_t n) {
   w.totals = take(16);
   w.desc = take(size_t(w.maxchunks) * sizeof(ChunkDesc));
   w.recs = take(size_t(n) * sizeof(Rec64));
+  w.sort = o;
   w.partial = take(size_t(w.maxchunks) * kWinCells * sizeof(double));
   w.total = o;
   return w;
@@ -430,14 +511,14 @@ static Paint64Ws paint64_ws(int nx, int ny, int nz, int64_t n) {
 
 size_t cic_paint_f64_ws(int nx, int ny, int nz, int64_t n) { return paint64_ws(nx, ny, nz, n).total; }
 
+// base: w.sort bytes for the sort; partial: the windows.
 static int paint_f64_sorted(hipStream_t s, int nx, int ny, int nz, const double *pos, uint32_t n, const double *weight,
-                            double wscalar, bool rel, double *mesh, char *base, const Paint64Ws &w) {
+                            double wscalar, bool rel, double *mesh, char *base, double *partial, const Paint64Ws &w) {
   const TileGrid t = make_tiles(nx, ny, nz);
   const GridD g = make_grid_d(nx, ny, nz);
   auto u32 = [base](size_t at) { return reinterpret_cast<uint32_t *>(base + at); };
   auto *desc = reinterpret_cast<ChunkDesc *>(base + w.desc);
   auto *recs = reinterpret_cast<Rec64 *>(base + w.recs);
-  auto *partial = reinterpret_cast<double *>(base + w.partial);
   const unsigned grid = unsigned((uint64_t(n) + kSort64Slice - 1) / kSort64Slice);
   const size_t lds = size_t(t.K) * 4;
   int rc = zero_u32(s, u32(w.count), t.K);
@@ -456,6 +537,22 @@ static int paint_f64_sorted(hipStream_t s, int nx, int ny, int nz, const double 
   JPM_LAUNCHED("accum_f64_kernel");
   hipLaunchKernelGGL(reduce_f64_kernel, dim3(t.K), dim3(1024), 0, s, partial, u32(w.choff), u32(w.nchunk), t, mesh);
   JPM_LAUNCHED("reduce_f64_kernel");
+  return JPM_OK;
+}
+
+// The three-component read at the particles of a sort that paint_f64_sorted
+// left in base.
+static int read3_f64_sorted(hipStream_t s, int nx, int ny, int nz, const double *phi3, bool rel, double *out,
+                            const char *base, const Paint64Ws &w) {
+  const TileGrid t = make_tiles(nx, ny, nz);
+  auto kern = rel ? read3_sorted_f64_kernel<true> : read3_sorted_f64_kernel<false>;
+  JPM_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(kern), hipFuncAttributeMaxDynamicSharedMemorySize,
+                              int(3 * kWinCells * sizeof(double))));
+  hipLaunchKernelGGL(kern, dim3(w.maxchunks), dim3(1024), 3 * kWinCells * sizeof(double), s,
+                     reinterpret_cast<const Rec64 *>(base + w.recs), reinterpret_cast<const ChunkDesc *>(base + w.desc),
+                     reinterpret_cast<const uint32_t *>(base + w.totals) + 1, phi3, cells(nx, ny, nz),
+                     make_grid_d(nx, ny, nz), t, out);
+  JPM_LAUNCHED("read3_sorted_f64_kernel");
   return JPM_OK;
 }
 
@@ -481,7 +578,8 @@ int cic_paint_f64(hipStream_t s, int nx, int ny, int nz, const double *pos, int6
   if (n == 0) return JPM_OK;
   JPM_REQUIRE(pos != nullptr, "positions are null");
   if (w.total)
-    return paint_f64_sorted(s, nx, ny, nz, pos, uint32_t(n), weight, wscalar, rel, mesh, static_cast<char *>(ws), w);
+    return paint_f64_sorted(s, nx, ny, nz, pos, uint32_t(n), weight, wscalar, rel, mesh, static_cast<char *>(ws),
+                            reinterpret_cast<double *>(static_cast<char *>(ws) + w.partial), w);
   const GridD g = make_grid_d(nx, ny, nz);
   const unsigned grid = grid_for(n, 256, 256 * 128);
   if (rel)
@@ -507,30 +605,49 @@ int cic_read_f64(hipStream_t s, int nx, int ny, int nz, const double *mesh, int 
   if (n == 0) return JPM_OK;
   JPM_REQUIRE(mesh && pos && out, "null pointer argument");
   const GridD g = make_grid_d(nx, ny, nz);
-  const unsigned grid = grid_for(n, 256, 256 * 128);
-  if (rel)
-    hipLaunchKernelGGL(read_f64_kernel<true>, dim3(grid), dim3(256), 0, s, mesh, ncomp, comp_stride, pos, uint32_t(n),
-                       g, out);
-  else
-    hipLaunchKernelGGL(read_f64_kernel<false>, dim3(grid), dim3(256), 0, s, mesh, ncomp, comp_stride, pos,
-                       uint32_t(n), g, out);
+  uint32_t per;
+  const unsigned grid = xcd_blocks(n, 256, per);
+#define JPM_R64(C)                                                                                                  \
+  case C: {                                                                                                         \
+    auto kern = nz >= 2 ? (rel ? read_f64_kernel<true, C, true> : read_f64_kernel<false, C, true>)                  \
+                        : (rel ? read_f64_kernel<true, C, false> : read_f64_kernel<false, C, false>);               \
+    hipLaunchKernelGGL(kern, dim3(grid), dim3(256), 0, s, mesh, comp_stride, pos, uint32_t(n), g, out, per);        \
+    break;                                                                                                          \
+  }
+  switch (ncomp) {
+    JPM_R64(1)
+    JPM_R64(2)
+    JPM_R64(3)
+    JPM_R64(4)
+  }
+#undef JPM_R64
   JPM_LAUNCHED("read_f64_kernel");
   return JPM_OK;
 }
 
 // Workspace of pm_forces_f64: the density mesh, its half spectrum, the three
-// force spectra and the three force meshes.
-size_t pm_forces_f64_workspace_size(int nx, int ny, int nz) {
-  if (nx <= 0 || ny <= 0 || nz <= 0) return 0;
+// force spectra, the three force meshes and, where one particle per cell would
+// be painted sorted, that sort, which the read takes up again.  The paint's
+// windows lie where the spectra follow.
+struct Forces64Ws {
+  size_t spec, spec3, phi3, sort, sort_bytes, total;
+};
+
+static Forces64Ws forces64_ws(int nx, int ny, int nz) {
   const size_t M = size_t(cells(nx, ny, nz)), H = size_t(half_cells(nx, ny, nz));
-  return align_up(M * 8) + align_up(H * 16) + align_up(3 * H * 16) + align_up(3 * M * 8);
+  Forces64Ws w;
+  w.spec = align_up(M * 8);
+  w.spec3 = w.spec + align_up(H * 16);
+  w.phi3 = w.spec3 + align_up(3 * H * 16);
+  w.sort = w.phi3 + align_up(3 * M * 8);
+  w.sort_bytes = paint64_ws(nx, ny, nz, int64_t(M)).sort;
+  w.total = w.sort + w.sort_bytes;
+  return w;
 }
 
-// The paint's workspace is free again before the spectra are written: it
-// takes their place where it fits (it does for up to about one particle per
-// cell), and the paint falls back to atomics where it does not.
-static size_t pm_forces_f64_paint_space(int nx, int ny, int nz) {
-  return pm_forces_f64_workspace_size(nx, ny, nz) - align_up(size_t(cells(nx, ny, nz)) * 8);
+size_t pm_forces_f64_workspace_size(int nx, int ny, int nz) {
+  if (nx <= 0 || ny <= 0 || nz <= 0) return 0;
+  return forces64_ws(nx, ny, nz).total;
 }
 
 int pm_forces_f64(hipStream_t s, int nx, int ny, int nz, const double *pos, int64_t n, const double *delta,
@@ -539,20 +656,34 @@ int pm_forces_f64(hipStream_t s, int nx, int ny, int nz, const double *pos, int6
   if (rc) return rc;
   JPM_REQUIRE(n >= 0 && n <= kMaxCells, "particle count %lld out of range", (long long)n);
   JPM_REQUIRE(out3 != nullptr && (n == 0 || pos != nullptr), "null pointer argument");
-  const size_t need = pm_forces_f64_workspace_size(nx, ny, nz);
-  JPM_REQUIRE(ws && ws_bytes >= need, "pm_forces_f64 needs %zu workspace bytes, got %zu", need, ws_bytes);
+  const Forces64Ws w = forces64_ws(nx, ny, nz);
+  JPM_REQUIRE(ws && ws_bytes >= w.total, "pm_forces_f64 needs %zu workspace bytes, got %zu", w.total, ws_bytes);
   const int64_t M = cells(nx, ny, nz), H = half_cells(nx, ny, nz);
+  const bool rel = flags & JPM_RELATIVE;
   char *base = static_cast<char *>(ws);
   double *rho = reinterpret_cast<double *>(base);
-  double2 *spec = reinterpret_cast<double2 *>(base + align_up(size_t(M) * 8));
-  double2 *spec3 = reinterpret_cast<double2 *>(base + align_up(size_t(M) * 8) + align_up(size_t(H) * 16));
-  double *phi3 = reinterpret_cast<double *>(base + align_up(size_t(M) * 8) + align_up(size_t(H) * 16) +
-                                            align_up(3 * size_t(H) * 16));
+  double2 *spec = reinterpret_cast<double2 *>(base + w.spec);
+  double2 *spec3 = reinterpret_cast<double2 *>(base + w.spec3);
+  double *phi3 = reinterpret_cast<double *>(base + w.phi3);
   const double *field = delta;
+  Paint64Ws p{};
   if (!field) {
-    const bool fits = cic_paint_f64_ws(nx, ny, nz, n) <= pm_forces_f64_paint_space(nx, ny, nz);
-    rc = cic_paint_f64(s, nx, ny, nz, pos, n, nullptr, 1.0, rho, (flags & JPM_RELATIVE) | JPM_ZERO_MESH,
-                       fits ? static_cast<void *>(spec) : nullptr, pm_forces_f64_paint_space(nx, ny, nz));
+    p = paint64_ws(nx, ny, nz, n);
+    if (p.total && (p.sort > w.sort_bytes || p.total - p.sort > w.sort - w.spec)) p = Paint64Ws{};
+    if (p.total) {
+      JPM_REQUIRE(!rel || n == M, "relative painting needs one particle per lattice node (n=%lld, mesh %lld)",
+                  (long long)n, (long long)M);
+      hipLaunchKernelGGL(zero_f64_kernel, dim3(grid_for(M, 256)), dim3(256), 0, s, rho, M);
+      JPM_LAUNCHED("zero_f64_kernel");
+      rc = paint_f64_sorted(s, nx, ny, nz, pos, uint32_t(n), nullptr, 1.0, rel, rho, base + w.sort,
+                            reinterpret_cast<double *>(spec), p);
+    } else {
+      // too many particles per cell for the sort's share of the workspace:
+      // the whole paint where the spectra follow, or atomics
+      const bool fits = cic_paint_f64_ws(nx, ny, nz, n) <= w.sort - w.spec;
+      rc = cic_paint_f64(s, nx, ny, nz, pos, n, nullptr, 1.0, rho, (flags & JPM_RELATIVE) | JPM_ZERO_MESH,
+                         fits ? static_cast<void *>(spec) : nullptr, w.sort - w.spec);
+    }
     if (rc) return rc;
     field = rho;
   }
@@ -561,6 +692,7 @@ int pm_forces_f64(hipStream_t s, int nx, int ny, int nz, const double *pos, int6
                      kflags, 1.0 / double(M), spec3);
   JPM_LAUNCHED("force_f64_kernel");
   if ((rc = fft_z2d(s, nx, ny, nz, 3, spec3, phi3))) return rc;
+  if (p.total) return read3_f64_sorted(s, nx, ny, nz, phi3, rel, out3, base + w.sort, p);
   return cic_read_f64(s, nx, ny, nz, phi3, 3, M, pos, n, out3, flags & JPM_RELATIVE);
 }
 

@@ -215,6 +215,73 @@ __device__ __forceinline__ int floor_cell_rel(float p, int n) {
   return 0;  // NaN: every corner is dropped, any tile will do
 }
 
+// Two neighbouring mesh values in one load, aligned to a single one.
+template <class T>
+struct PairOf {
+  typedef T type __attribute__((ext_vector_type(2), aligned(sizeof(T))));
+};
+
+// The 8 corner values of NC meshes (cstride apart) at cells {ix}, {iy}, {iz}
+// (per axis the low and the high corner), v[c][bx | by << 1 | bz << 2].  The
+// two z corners are neighbours in memory except across the periodic end and
+// where a relative corner was dropped, so they come in one load per (x, y) row
+// (PAIR; needs nz >= 2), at the low corner or, for the last cell, one before
+// it, with loads of their own for a high corner elsewhere.  Every mesh's pairs
+// are issued before the first is used.
+template <bool PAIR, int NC, class T>
+__device__ __forceinline__ void load_corners(const T *__restrict__ m, size_t cstride, const uint32_t ix[2],
+                                             const uint32_t iy[2], const uint32_t iz[2], uint32_t ny, uint32_t nz,
+                                             T v[NC][8]) {
+  if (PAIR) {
+    const uint32_t zc = iz[0] + 1 < nz ? iz[0] : nz - 2;
+    typename PairOf<T>::type p[NC][4];
+    uint32_t row[4];
+#pragma unroll
+    for (int q = 0; q < 4; ++q) row[q] = (ix[q & 1] * ny + iy[q >> 1]) * nz;
+#pragma unroll
+    for (int c = 0; c < NC; ++c)
+#pragma unroll
+      for (int q = 0; q < 4; ++q)
+        p[c][q] = *reinterpret_cast<const typename PairOf<T>::type *>(m + c * cstride + row[q] + zc);
+    if (iz[1] != zc + 1) {
+      // the low corner is the pair's second value in the last cell of a row
+      T hi[NC][4];
+#pragma unroll
+      for (int c = 0; c < NC; ++c)
+#pragma unroll
+        for (int q = 0; q < 4; ++q) hi[c][q] = m[c * cstride + row[q] + iz[1]];
+#pragma unroll
+      for (int c = 0; c < NC; ++c)
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          v[c][q] = iz[0] == zc ? p[c][q].x : p[c][q].y;
+          v[c][q | 4] = hi[c][q];
+        }
+    } else {
+#pragma unroll
+      for (int c = 0; c < NC; ++c)
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          v[c][q] = iz[0] == zc ? p[c][q].x : p[c][q].y;
+          v[c][q | 4] = p[c][q].y;
+        }
+    }
+  } else {
+#pragma unroll
+    for (int c = 0; c < NC; ++c)
+#pragma unroll
+      for (int o = 0; o < 8; ++o) v[c][o] = m[c * cstride + (ix[o & 1] * ny + iy[(o >> 1) & 1]) * nz + iz[o >> 2]];
+  }
+}
+
+// Workgroup b of a per-particle kernel takes the particles of block
+// (b mod 8) per + b / 8: each XCD walks one contiguous eighth of them, so the
+// mesh rows that neighbouring particles share come through one L2.
+inline unsigned xcd_blocks(int64_t n, int block, uint32_t &per) {
+  per = uint32_t(((n + block - 1) / block + 7) / 8);
+  return 8u * per;
+}
+
 struct ChunkDesc {
   uint32_t tile, start, count, pad;
 };

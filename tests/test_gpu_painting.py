@@ -333,3 +333,30 @@ def test_default_slices_give_the_same_bits(gpu, n):
     assert torch.equal(out[0], out[1])
     m = float(w.double().sum())
     assert abs(float(out[0].double().sum()) - m) < 1e-5 * float(w.double().abs().sum())
+
+
+@pytest.mark.parametrize("shape", [(3, 4, 1), (4, 3, 2), (2, 2, 3), (5, 1, 7), (1, 1, 64), (6, 5, 65)])
+def test_reads_at_the_ends_of_rows(gpu, shape):
+    """The reads and position cotangents that load both z corners at once:
+    rows of one to three cells, particles in the last cell of a row, on its
+    edge and wrapped past it, dropped relative corners.  Against the oracle's
+    float32 corners (reads) and float64 gradient, at the other reads'
+    tolerance."""
+    from jaxpm_amd import _ops
+    from oracle import adjoint as oa
+    print(f"row ends {shape}", flush=True)
+    r = np.random.default_rng(61)
+    meshes = r.normal(size=(3, *shape)).astype(np.float32)
+    pos = (r.uniform(-0.6, 1.7, (200, 3)) * shape).astype(np.float32)
+    pos[:60, 2] = shape[2] - 1 + r.uniform(0, 1, 60).astype(np.float32)
+    got = host(_ops.read(dev(meshes), dev(pos)))
+    close(got, np.stack([op.cic_read(x, pos, dtype=np.float32) for x in meshes], -1).astype(np.float64))
+    grad = host(_ops.grad_pos(dev(meshes[0]), dev(pos)))
+    close(grad, oa.cic_read_grad(meshes[0].astype(np.float64), pos.astype(np.float64)))
+    m = shape[0] * shape[1] * shape[2]
+    disp = r.uniform(-1.5, 1.5, (m, 3)).astype(np.float32)
+    disp[::5, 2] = np.float32(-1e-9)
+    disp[1::5] = 0
+    got = host(_ops.read(dev(meshes), dev(disp), relative=True))
+    close(got, np.stack([op.cic_read_dx(x, disp.reshape(*shape, 3), dtype=np.float32).reshape(-1) for x in meshes],
+                        -1).astype(np.float64))
