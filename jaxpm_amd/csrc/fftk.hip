@@ -174,15 +174,15 @@ __device__ __forceinline__ void dftR(float2 *a) {
 // 16 while at least 16 remain, then what is left (8, 4 or 2).
 constexpr int stage_radix(int rem) { return rem % 3 == 0 ? 3 : rem >= 16 ? 16 : rem; }
 
-// FFTs of KB columns of length L held in LDS as buf[l * PITCH + c]
-// (c < KB), in place; L, KB and PITCH are compile-time, so every index is
-// shifts and masks and the stage loop unrolls.  Stockham stage with span Ns
-// and radix R: butterfly j of a column reads elements j + r L/R, twiddles
-// them by W_L^{r k L/(Ns R)} (k = j mod Ns), and writes element
-// (j / Ns) Ns R + k + r Ns.  Every thread keeps its butterflies in registers
-// between the read and the write half of a stage.  L * KB <= 4096, so a
-// thread holds at most 16 points.  tw is the length-L table in LDS.
-template <int L, int KB, int PITCH, bool INV, int NS, int NT = kFftThreads>
+// FFTs of KB columns of length L held in LDS as buf[l * SL + c * SC]
+// (c < KB), in place; L, KB and the strides are compile-time, so every index
+// is shifts, masks and constant multiplies and the stage loop unrolls.
+// Stockham stage with span Ns and radix R: butterfly j of a column reads
+// elements j + r L/R, twiddles them by W_L^{r k L/(Ns R)} (k = j mod Ns), and
+// writes element (j / Ns) Ns R + k + r Ns.  Every thread keeps its butterflies
+// in registers between the read and the write half of a stage.  tw is the
+// length-L table in LDS.
+template <int L, int KB, int SL, bool INV, int NS, int NT = kFftThreads, int SC = 1>
 __device__ __forceinline__ void fft_stage(float2 *buf, const float2 *tw) {
   constexpr int R = stage_radix(L / NS);
   constexpr int nb = L / R, step = L / (NS * R), total = nb * KB;
@@ -193,10 +193,10 @@ __device__ __forceinline__ void fft_stage(float2 *buf, const float2 *tw) {
   for (int it = 0; it < per; ++it) {
     const int f = threadIdx.x + it * NT;
     if (total % NT == 0 || f < total) {
-      const int c = f & (KB - 1), j = f / KB, k = j % NS;
+      const int c = f % KB, j = f / KB, k = j % NS;
       float2 a[R];
 #pragma unroll
-      for (int r = 0; r < R; ++r) a[r] = buf[(j + r * nb) * PITCH + c];
+      for (int r = 0; r < R; ++r) a[r] = buf[(j + r * nb) * SL + c * SC];
       if constexpr (NS > 1) {
 #pragma unroll
         for (int r = 1; r < R; ++r) {
@@ -218,17 +218,17 @@ __device__ __forceinline__ void fft_stage(float2 *buf, const float2 *tw) {
     const int f = threadIdx.x + it * NT;
     if (total % NT == 0 || f < total) {
 #pragma unroll
-      for (int r = 0; r < R; ++r) buf[(dst[it] + r * NS) * PITCH + cc[it]] = x[it][r];
+      for (int r = 0; r < R; ++r) buf[(dst[it] + r * NS) * SL + cc[it] * SC] = x[it][r];
     }
   }
   __syncthreads();
   constexpr int next = NS * R;
-  if constexpr (next < L) fft_stage<L, KB, PITCH, INV, next, NT>(buf, tw);
+  if constexpr (next < L) fft_stage<L, KB, SL, INV, next, NT, SC>(buf, tw);
 }
 
-template <int L, int KB, int PITCH, bool INV, int NT = kFftThreads>
+template <int L, int KB, int SL, bool INV, int NT = kFftThreads, int SC = 1>
 __device__ __forceinline__ void lds_fft(float2 *buf, const float2 *tw) {
-  if constexpr (L > 1) fft_stage<L, KB, PITCH, INV, 1, NT>(buf, tw);
+  if constexpr (L > 1) fft_stage<L, KB, SL, INV, 1, NT, SC>(buf, tw);
 }
 
 // A twiddle table into LDS in two halves, so that its loads share their
@@ -534,6 +534,29 @@ __device__ __forceinline__ float2 divergence_pair(const float *__restrict__ g, s
   return make_float2((dx0 + dy0) + dz0, (dx1 + dy1) + dz1);
 }
 
+// Where the pair of cells (x, y, 2l), (x, y, 2l + 1) of a paint with its face
+// cells kept apart is: p (the mesh's pair) becomes the face buffer's in a
+// tile's lx = 0 or ly = 0 plane; otherwise, when true is returned, the first
+// cell is a tile's lz = 0 cell, whose value zf replaces the mesh's.
+__device__ __forceinline__ bool face_pair(const FaceCells &fc, uint32_t x, uint32_t y, uint32_t l, const float2 *&p,
+                                          float &zf) {
+  // tile (x/16, y/16, l/8), local (a, b, cz) and (a, b, cz + 1) with cz = 2 (l
+  // mod 8); face offsets in 32 bits (the host checks the buffer's size)
+  const uint32_t a = x & uint32_t(kTile - 1), b = y & uint32_t(kTile - 1), cz = (l & 7u) * 2u;
+  const uint32_t tile = ((x >> 4) * fc.ty + (y >> 4)) * fc.tz + (l >> 3);
+  // face_index(a, b, 0): in a plane (a == 0 or b == 0) the row's first cell,
+  // whose pair at cz is consecutive there; else the lz = 0 cell
+  const uint32_t row = a == 0 ? b * uint32_t(kTile)
+                              : (b == 0 ? uint32_t(kTile * kTile) + (a - 1u) * uint32_t(kTile)
+                                        : uint32_t(kTile * kTile + (kTile - 1) * kTile) +
+                                              (a - 1u) * uint32_t(kTile - 1) + (b - 1u));
+  const float *ft = fc.fb + (tile * uint32_t(kFaceStride) + row);
+  const bool plane = a == 0 || b == 0;
+  if (plane) p = reinterpret_cast<const float2 *>(ft + cz);
+  zf = *ft;
+  return !plane && cz == 0;
+}
+
 // z pass of the R2C: rows r = blockIdx.x * KB + c (< nrows) of item
 // blockIdx.y, each nz = 2M reals read as M complex points.  With DIV the
 // reals are the divergence of the vector mesh dv, formed as they load.
@@ -588,23 +611,8 @@ fft_r2c_rows_kernel(const float2 *__restrict__ in, float2 *__restrict__ out, int
       const float2 *p = src + size_t(r) * M + l;
       zsel[it] = false;
       if (fc.fb) {
-        // cells (x, y, 2l) and (x, y, 2l + 1): tile (x/16, y/16, l/8), local
-        // (a, b, cz) and (a, b, cz + 1) with cz = 2 (l mod 8); face offsets
-        // in 32 bits (the host checks the buffer's size)
-        const uint32_t x = fc.div_ny.div(r), y = r - x * fc.ny;
-        const uint32_t a = x & uint32_t(kTile - 1), b = y & uint32_t(kTile - 1), cz = (uint32_t(l) & 7u) * 2u;
-        const uint32_t tile = ((x >> 4) * fc.ty + (y >> 4)) * fc.tz + (uint32_t(l) >> 3);
-        // face_index(a, b, 0): in a plane (a == 0 or b == 0) the row's first
-        // cell, whose pair at cz is consecutive there; else the lz = 0 cell
-        const uint32_t row = a == 0 ? b * uint32_t(kTile)
-                                    : (b == 0 ? uint32_t(kTile * kTile) + (a - 1u) * uint32_t(kTile)
-                                              : uint32_t(kTile * kTile + (kTile - 1) * kTile) +
-                                                    (a - 1u) * uint32_t(kTile - 1) + (b - 1u));
-        const float *ft = fc.fb + (tile * uint32_t(kFaceStride) + row);
-        const bool plane = a == 0 || b == 0;
-        if (plane) p = reinterpret_cast<const float2 *>(ft + cz);
-        zf[it] = *ft;
-        zsel[it] = !plane && cz == 0;
+        const uint32_t x = fc.div_ny.div(r);
+        zsel[it] = face_pair(fc, x, r - x * fc.ny, uint32_t(l), p, zf[it]);
       }
       v[it] = *p;
     }
@@ -704,6 +712,155 @@ fft_c2r_rows_kernel(const float2 *__restrict__ in, float2 *__restrict__ out, int
   }
 }
 
+
+// The z and y passes of one x plane together, for planes of N x N cells whose
+// (N/2 + 1) x (N + 1) complex values fit LDS: the plane is read and written
+// once instead of twice, by one launch instead of two.  Held as buf[k * P +
+// y], P = N + 1: the z transform runs along k (stride P), the y transform along
+// y (stride 1), and the split between them in place on the pairs k, M - k.  The
+// float operations are those of the row and column passes, so the bits are.
+// Bound by LDS traffic and barriers between the stages (two workgroups fit a
+// CU at N = 128).  Four 128^3 meshes, both directions of the two passes: 58
+// -> 44 us; four 64^3: 22 -> 13; one 32^3: 15 -> 9.
+template <int N>
+struct PlaneFft {
+  static constexpr int M = N / 2, nzh = M + 1, P = N + 1;
+  static constexpr int NT = N >= 128 ? 1024 : N >= 64 ? 512 : 256;
+  static constexpr int points = nzh * P;
+  static constexpr size_t lds = size_t(points + M + (M + 1) + N) * sizeof(float2);
+};
+
+template <int N, bool DIV>
+__global__ void __launch_bounds__(PlaneFft<N>::NT)
+fft_plane_r2c_kernel(const float2 *__restrict__ in, float2 *__restrict__ out, int nx, uint32_t per, size_t in_bstride,
+                     size_t out_bstride, const float2 *__restrict__ tw_all, DivIn dv, FaceCells fc) {
+  using F = PlaneFft<N>;
+  constexpr int M = F::M, P = F::P, NT = F::NT, nzh = F::nzh, total = N * M;
+  extern __shared__ float2 buf[];
+  float2 *twM = buf + F::points, *twN = twM + M, *twY = twN + M + 1;
+  // planes in XCD slabs, so that a divergence's x neighbours share an L2
+  const uint32_t x = (blockIdx.x & 7u) * per + (blockIdx.x >> 3);
+  if (int(x) >= nx) return;
+  TwStage<M, NT> tsM;
+  TwStage<M + 1, NT> tsN;
+  TwStage<N, NT> tsY;
+  constexpr int iters = (total + NT - 1) / NT;
+  if constexpr (DIV) {
+    const float *g = dv.g3 + size_t(blockIdx.y) * 2 * in_bstride;
+#pragma unroll
+    for (int it = 0; it < iters; ++it) {
+      const int f = threadIdx.x + it * NT;
+      if (total % NT != 0 && f >= total) break;
+      buf[(f % M) * P + f / M] = divergence_pair<M>(g, dv.chan, dv.nx, dv.ny, x, uint32_t(f / M), f % M);
+    }
+    tsM.load(tw_all, tw_off(M));
+    tsN.load(tw_all, tw_off(2 * M));
+    tsY.load(tw_all, tw_off(N));
+  } else {
+    const float2 *src = in + size_t(blockIdx.y) * in_bstride + size_t(x) * total;
+    float2 v[iters];
+    float zf[iters];
+    bool zsel[iters];
+#pragma unroll
+    for (int it = 0; it < iters; ++it) {
+      const int f0 = threadIdx.x + it * NT;
+      const int f = (total % NT != 0 && f0 >= total) ? total - 1 : f0;
+      const float2 *p = src + f;
+      zsel[it] = false;
+      if (fc.fb) zsel[it] = face_pair(fc, x, uint32_t(f / M), uint32_t(f % M), p, zf[it]);
+      v[it] = *p;
+    }
+    tsM.load(tw_all, tw_off(M));
+    tsN.load(tw_all, tw_off(2 * M));
+    tsY.load(tw_all, tw_off(N));
+#pragma unroll
+    for (int it = 0; it < iters; ++it) {
+      const int f = threadIdx.x + it * NT;
+      if (total % NT != 0 && f >= total) break;
+      if (zsel[it]) v[it].x = zf[it];
+      buf[(f % M) * P + f / M] = v[it];
+    }
+  }
+  tsM.store(twM);
+  tsN.store(twN);
+  tsY.store(twY);
+  __syncthreads();
+  lds_fft<M, N, P, false, NT>(buf, twM);
+  // X[k] = E[k] + W_{2M}^k O[k] as in fft_r2c_rows_kernel, the pair (k, M - k)
+  // of a row by one thread; k = 0 gives X[0] and X[M], k = M / 2 its own pair
+  auto split = [&](float2 z, float2 zm, int k) {
+    const float2 E = make_float2(0.5f * (z.x + zm.x), 0.5f * (z.y - zm.y));
+    const float2 O = make_float2(0.5f * (z.y + zm.y), -0.5f * (z.x - zm.x));
+    return cadd(E, cmul(twN[k], O));
+  };
+  for (int f = threadIdx.x; f < (M / 2 + 1) * N; f += NT) {
+    const int k = f / N, y = f % N;
+    const float2 z = buf[k * P + y], zm = buf[((M - k) % M) * P + y];
+    buf[k * P + y] = split(z, zm, k);
+    if (2 * k != M) buf[(M - k) * P + y] = split(zm, z, M - k);
+  }
+  __syncthreads();
+  lds_fft<N, nzh, 1, false, NT, P>(buf, twY);
+  float2 *dst = out + size_t(blockIdx.y) * out_bstride + size_t(x) * (N * nzh);
+  for (int f = threadIdx.x; f < N * nzh; f += NT) dst[f] = buf[(f % nzh) * P + f / nzh];
+}
+
+template <int N>
+__global__ void __launch_bounds__(PlaneFft<N>::NT)
+fft_plane_c2r_kernel(const float2 *__restrict__ in, float2 *__restrict__ out, int nx, uint32_t per, size_t in_bstride,
+                     size_t out_bstride, const float2 *__restrict__ tw_all) {
+  using F = PlaneFft<N>;
+  constexpr int M = F::M, P = F::P, NT = F::NT, nzh = F::nzh, total = N * M, half = N * nzh;
+  extern __shared__ float2 buf[];
+  float2 *twM = buf + F::points, *twN = twM + M, *twY = twN + M + 1;
+  const uint32_t x = (blockIdx.x & 7u) * per + (blockIdx.x >> 3);
+  if (int(x) >= nx) return;
+  TwStage<M, NT> tsM;
+  TwStage<M + 1, NT> tsN;
+  TwStage<N, NT> tsY;
+  const float2 *src = in + size_t(blockIdx.y) * in_bstride + size_t(x) * half;
+  constexpr int iters = (half + NT - 1) / NT;
+  float2 v[iters];
+#pragma unroll
+  for (int it = 0; it < iters; ++it) {
+    const int f = threadIdx.x + it * NT;
+    v[it] = src[f < half ? f : half - 1];
+  }
+  tsM.load(tw_all, tw_off(M));
+  tsN.load(tw_all, tw_off(2 * M));
+  tsY.load(tw_all, tw_off(N));
+#pragma unroll
+  for (int it = 0; it < iters; ++it) {
+    const int f = threadIdx.x + it * NT;
+    if (f < half) buf[(f % nzh) * P + f / nzh] = v[it];
+  }
+  tsM.store(twM);
+  tsN.store(twN);
+  tsY.store(twY);
+  __syncthreads();
+  lds_fft<N, nzh, 1, true, NT, P>(buf, twY);
+  // Z'[k] as in fft_c2r_rows_kernel; X[0] and X[M] enter with their real parts
+  auto merge = [&](float2 a, float2 b, int k) {
+    const float2 bc = conjf2(b);
+    const float2 E = cadd(a, bc);
+    const float2 O = cmul(csub(a, bc), conjf2(twN[k]));
+    return make_float2(E.x - O.y, E.y + O.x);
+  };
+  for (int f = threadIdx.x; f < (M / 2 + 1) * N; f += NT) {
+    const int k = f / N, y = f % N;
+    float2 a = buf[k * P + y], b = buf[(M - k) * P + y];
+    if (k == 0) {
+      a.y = 0.0f;
+      b.y = 0.0f;
+    }
+    buf[k * P + y] = merge(a, b, k);
+    if (k > 0 && 2 * k != M) buf[(M - k) * P + y] = merge(b, a, M - k);
+  }
+  __syncthreads();
+  lds_fft<M, N, P, true, NT>(buf, twM);
+  float2 *dst = out + size_t(blockIdx.y) * out_bstride + size_t(x) * total;
+  for (int f = threadIdx.x; f < total; f += NT) dst[f] = buf[(f % M) * P + f / M];
+}
 
 // The z pass of six C2Rs whose meshes second-order LPT multiplies at once:
 // the rows of the shear spectra spec + m H (m = 0 .. 5: xx, yy, zz, xy, xz,
@@ -869,6 +1026,94 @@ static int rows_c2r(hipStream_t s, int nx, int ny, int nz, int batch, float2 *in
   return JPM_OK;
 }
 
+// The planes the z and y passes take together (PlaneFft).  One workgroup
+// does a whole plane, so few planes leave the chip idle for longer than the
+// launches saved: R2C and C2R of (planes, 128, 128) took 22.7 us together and
+// 21.5 apart at 8 planes, 26.4 and 26.6 at 32, 34.2 and 44.7 at 128.  Planes
+// of 96 and less gain at any count (20.0 and 21.6 at 2 planes, 29.0 and 33.6 at
+// 96).
+#define JPM_PLANES(X) X(16) X(24) X(32) X(48) X(64) X(96) X(128)
+
+static bool plane_fft_ok(int nx, int ny, int nz, int batch) {
+  if (nx < 2 || ny != nz || (ny > 96 && size_t(nx) * batch < 64)) return false;
+  switch (ny) {
+#define JPM_PLANE_CASE(N) case N:
+    JPM_PLANES(JPM_PLANE_CASE)
+#undef JPM_PLANE_CASE
+    return true;
+    default: return false;
+  }
+}
+
+template <typename K>
+static int plane_lds(K kern, size_t bytes) {
+  if (bytes > 65536)
+    JPM_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(kern), hipFuncAttributeMaxDynamicSharedMemorySize,
+                                int(bytes)));
+  return JPM_OK;
+}
+
+// The z and y passes of the R2C (of the divergence with dv.g3), together where
+// the plane allows.
+static int zy_r2c(hipStream_t s, int nx, int ny, int nz, int batch, const float *in, float2 *out, const float2 *tw,
+                  const DivIn &dv = DivIn{nullptr, 0, 0, 0, FastDiv(1)},
+                  const FaceCells &fc = FaceCells{nullptr, 0, 0, 0, 0, FastDiv(1)}) {
+  const int nzh = nz / 2 + 1;
+  const size_t H = size_t(nx) * ny * nzh, Mc = size_t(nx) * ny * (nz / 2);
+  int rc;
+  if (!plane_fft_ok(nx, ny, nz, batch)) {
+    if ((rc = rows_r2c(s, nx, ny, nz, batch, in, out, tw, dv, fc))) return rc;
+    return cols_pass(s, false, out, ny, nzh, nx, size_t(nzh), size_t(ny) * nzh, H, batch, tw);
+  }
+  JPM_REQUIRE(!fc.fb || (!dv.g3 && batch == 1 && nx % kTile == 0 && ny % kTile == 0 && fc.ny == uint32_t(ny) &&
+                         fc.ty == uint32_t(ny / kTile) && fc.tz == uint32_t(nz / kTile)),
+              "face cells apart need one mesh of full 16^3 tiles");
+  const uint32_t per = uint32_t((nx + 7) / 8);
+  const float2 *i2 = reinterpret_cast<const float2 *>(in);
+  JPM_TIMED(s, dv.g3 ? "fft_plane_r2c_kernel[div]" : "fft_plane_r2c_kernel");
+  switch (ny) {
+#define JPM_PLANE_R2C(N)                                                                                           \
+  case N: {                                                                                                        \
+    auto kern = dv.g3 ? fft_plane_r2c_kernel<N, true> : fft_plane_r2c_kernel<N, false>;                            \
+    if ((rc = plane_lds(kern, PlaneFft<N>::lds))) return rc;                                                       \
+    hipLaunchKernelGGL(kern, dim3(8 * per, batch), dim3(PlaneFft<N>::NT), PlaneFft<N>::lds, s, i2, out, nx, per,   \
+                       Mc, H, tw, dv, fc);                                                                         \
+    break;                                                                                                         \
+  }
+    JPM_PLANES(JPM_PLANE_R2C)
+#undef JPM_PLANE_R2C
+  }
+  JPM_LAUNCHED("fft_plane_r2c_kernel");
+  return JPM_OK;
+}
+
+// The inverse y and z passes of the C2R.
+static int yz_c2r(hipStream_t s, int nx, int ny, int nz, int batch, float2 *in, float *out, const float2 *tw) {
+  const int nzh = nz / 2 + 1;
+  const size_t H = size_t(nx) * ny * nzh, Mc = size_t(nx) * ny * (nz / 2);
+  int rc;
+  if (!plane_fft_ok(nx, ny, nz, batch)) {
+    if ((rc = cols_pass(s, true, in, ny, nzh, nx, size_t(nzh), size_t(ny) * nzh, H, batch, tw))) return rc;
+    return rows_c2r(s, nx, ny, nz, batch, in, out, tw);
+  }
+  const uint32_t per = uint32_t((nx + 7) / 8);
+  JPM_TIMED(s, "fft_plane_c2r_kernel");
+  switch (ny) {
+#define JPM_PLANE_C2R(N)                                                                                        \
+  case N: {                                                                                                     \
+    auto kern = fft_plane_c2r_kernel<N>;                                                                        \
+    if ((rc = plane_lds(kern, PlaneFft<N>::lds))) return rc;                                                    \
+    hipLaunchKernelGGL(kern, dim3(8 * per, batch), dim3(PlaneFft<N>::NT), PlaneFft<N>::lds, s, in,              \
+                       reinterpret_cast<float2 *>(out), nx, per, H, Mc, tw);                                    \
+    break;                                                                                                      \
+  }
+    JPM_PLANES(JPM_PLANE_C2R)
+#undef JPM_PLANE_C2R
+  }
+  JPM_LAUNCHED("fft_plane_c2r_kernel");
+  return JPM_OK;
+}
+
 int native_r2c(hipStream_t s, int nx, int ny, int nz, int batch, const float *in, void *out) {
   JPM_REQUIRE(native_fft_ok(nx, ny, nz) && batch >= 1 && batch <= 65535, "native FFT shape");
   const float2 *tw;
@@ -877,8 +1122,7 @@ int native_r2c(hipStream_t s, int nx, int ny, int nz, int batch, const float *in
   const int nzh = nz / 2 + 1;
   const size_t H = size_t(nx) * ny * nzh;
   float2 *o = static_cast<float2 *>(out);
-  if ((rc = rows_r2c(s, nx, ny, nz, batch, in, o, tw))) return rc;
-  if ((rc = cols_pass(s, false, o, ny, nzh, nx, size_t(nzh), size_t(ny) * nzh, H, batch, tw))) return rc;
+  if ((rc = zy_r2c(s, nx, ny, nz, batch, in, o, tw))) return rc;
   if (nx == 1) return JPM_OK;
   return cols_pass(s, false, o, nx, nzh, ny, size_t(ny) * nzh, size_t(nzh), H, batch, tw);
 }
@@ -892,8 +1136,7 @@ int native_c2r(hipStream_t s, int nx, int ny, int nz, int batch, void *in, float
   const size_t H = size_t(nx) * ny * nzh;
   float2 *h = static_cast<float2 *>(in);
   if (nx > 1 && (rc = cols_pass(s, true, h, nx, nzh, ny, size_t(ny) * nzh, size_t(nzh), H, batch, tw))) return rc;
-  if ((rc = cols_pass(s, true, h, ny, nzh, nx, size_t(nzh), size_t(ny) * nzh, H, batch, tw))) return rc;
-  return rows_c2r(s, nx, ny, nz, batch, h, out, tw);
+  return yz_c2r(s, nx, ny, nz, batch, h, out, tw);
 }
 
 // out = C2R(scale G . R2C(in)) for a batch of meshes, the spectrum in spec
@@ -914,8 +1157,7 @@ int native_potential(hipStream_t s, int nx, int ny, int nz, int batch, const flo
   float2 *h = static_cast<float2 *>(spec);
   DivIn dv{g3, chan, uint32_t(nx), uint32_t(ny), FastDiv(uint32_t(ny))};
   const FaceCells fc = faces ? *faces : FaceCells{nullptr, 0, 0, 0, 0, FastDiv(1)};
-  if ((rc = rows_r2c(s, nx, ny, nz, batch, in, h, tw, dv, fc))) return rc;
-  if ((rc = cols_pass(s, false, h, ny, nzh, nx, size_t(nzh), size_t(ny) * nzh, H, batch, tw))) return rc;
+  if ((rc = zy_r2c(s, nx, ny, nz, batch, in, h, tw, dv, fc))) return rc;
   {
     JPM_TIMED(s, "fft_cols_potential_kernel");
     switch (nx) {
@@ -935,8 +1177,7 @@ int native_potential(hipStream_t s, int nx, int ny, int nz, int batch, const flo
     }
   }
   JPM_LAUNCHED("fft_cols_potential_kernel");
-  if ((rc = cols_pass(s, true, h, ny, nzh, nx, size_t(nzh), size_t(ny) * nzh, H, batch, tw))) return rc;
-  return rows_c2r(s, nx, ny, nz, batch, h, out, tw);
+  return yz_c2r(s, nx, ny, nz, batch, h, out, tw);
 }
 
 // out = C2R(c(k) R2C(in)), c the linear field's multiplier, for a batch of
@@ -950,8 +1191,7 @@ int native_linear(hipStream_t s, int nx, int ny, int nz, int batch, const float 
   const int nzh = nz / 2 + 1;
   const size_t H = size_t(nx) * ny * nzh;
   float2 *h = static_cast<float2 *>(spec);
-  if ((rc = rows_r2c(s, nx, ny, nz, batch, in, h, tw))) return rc;
-  if ((rc = cols_pass(s, false, h, ny, nzh, nx, size_t(nzh), size_t(ny) * nzh, H, batch, tw))) return rc;
+  if ((rc = zy_r2c(s, nx, ny, nz, batch, in, h, tw))) return rc;
   {
     JPM_TIMED(s, "fft_cols_linear_kernel");
     switch (nx) {
@@ -970,8 +1210,7 @@ int native_linear(hipStream_t s, int nx, int ny, int nz, int batch, const float 
     }
   }
   JPM_LAUNCHED("fft_cols_linear_kernel");
-  if ((rc = cols_pass(s, true, h, ny, nzh, nx, size_t(nzh), size_t(ny) * nzh, H, batch, tw))) return rc;
-  return rows_c2r(s, nx, ny, nz, batch, h, out, tw);
+  return yz_c2r(s, nx, ny, nz, batch, h, out, tw);
 }
 
 // The potential phi = C2R(scale G R2C(ic)) and the second-order LPT source of
@@ -986,8 +1225,7 @@ int native_lpt2(hipStream_t s, int nx, int ny, int nz, const float *ic, void *sp
   const int nzh = nz / 2 + 1, M = nz / 2, nrows = nx * ny;
   const size_t H = size_t(nx) * ny * nzh;
   float2 *h = static_cast<float2 *>(spec), *h7 = static_cast<float2 *>(spec7);
-  if ((rc = rows_r2c(s, nx, ny, nz, 1, ic, h, tw))) return rc;
-  if ((rc = cols_pass(s, false, h, ny, nzh, nx, size_t(nzh), size_t(ny) * nzh, H, 1, tw))) return rc;
+  if ((rc = zy_r2c(s, nx, ny, nz, 1, ic, h, tw))) return rc;
   {
     JPM_TIMED(s, "fft_cols_shear_kernel");
     switch (nx) {
@@ -1006,8 +1244,8 @@ int native_lpt2(hipStream_t s, int nx, int ny, int nz, const float *ic, void *sp
     }
   }
   JPM_LAUNCHED("fft_cols_shear_kernel");
-  if ((rc = cols_pass(s, true, h7, ny, nzh, nx, size_t(nzh), size_t(ny) * nzh, H, 7, tw))) return rc;
-  if ((rc = rows_c2r(s, nx, ny, nz, 1, h7, phi, tw))) return rc;
+  if ((rc = yz_c2r(s, nx, ny, nz, 1, h7, phi, tw))) return rc;
+  if ((rc = cols_pass(s, true, h7 + H, ny, nzh, nx, size_t(nzh), size_t(ny) * nzh, H, 6, tw))) return rc;
   {
     JPM_TIMED(s, "fft_c2r_source_kernel");
     switch (M) {

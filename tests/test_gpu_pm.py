@@ -66,6 +66,34 @@ def test_native_fft_shapes(gpu, shape, batch):
     assert rel_err(got, want) < 3e-6
 
 
+@pytest.mark.parametrize("n", [16, 24, 32, 48, 64, 96, 128])
+@pytest.mark.parametrize("nx,batch", [(2, 1), (12, 3), (64, 1)])
+def test_plane_transforms(gpu, n, nx, batch):
+    """Meshes whose (y, z) planes fit LDS take the z and y passes together:
+    against numpy in float64 on both sides of every rule on the plane count,
+    and a mesh of a batch has the bits of the mesh alone (planes of 128 take
+    one route in the batch of 108 planes and the other alone)."""
+    from jaxpm_amd import _ops
+    shape = (nx, n, n)
+    print(f"plane fft {shape} batch={batch}", flush=True)
+    r = np.random.default_rng(31)
+    x = r.normal(size=(batch, *shape)).astype(np.float32)
+    got = _ops.r2c(dev(x))
+    ref = np.fft.rfftn(x.astype(np.float64), axes=(1, 2, 3))
+    assert rel_err(host(got), ref) < 3e-6
+    z = (r.normal(size=ref.shape) + 1j * r.normal(size=ref.shape)).astype(np.complex64)
+    back = _ops.c2r(dev(z, torch.complex64), shape)
+    want = np.fft.irfftn(z.astype(np.complex128), s=shape, axes=(1, 2, 3)) * np.prod(shape)
+    assert rel_err(host(back), want) < 3e-6
+    if nx == 12:
+        many = np.concatenate([x, x, x])
+        assert torch.equal(_ops.r2c(dev(many))[:batch], got)
+        assert torch.equal(_ops.c2r(dev(np.concatenate([z, z, z]), torch.complex64), shape)[:batch], back)
+    if batch > 1:
+        assert torch.equal(_ops.r2c(dev(x[1])), got[1])
+        assert torch.equal(_ops.c2r(dev(z[1], torch.complex64), shape), back[1])
+
+
 @pytest.mark.parametrize("order,fd,r_split,deconv", [(1, False, 0.0, False), (0, False, 0.0, False),
                                                      (1, True, 0.0, False), (1, False, 1.5, False),
                                                      (1, False, 0.0, True)])
