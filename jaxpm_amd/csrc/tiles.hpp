@@ -420,6 +420,49 @@ __device__ __forceinline__ LAxis laxis_abs(float x, int origin, int n) {
   return a;
 }
 
+// A tile as floats, for the floor cells of its absolute positions: origin,
+// length - 1 and mesh edge per axis (exact below 2^22 cells; a longer axis
+// gets a NaN origin, which sends every position to the general path).
+struct TileFrame {
+  float o[3], last[3], n[3];
+};
+
+__device__ __forceinline__ float window_edge(int n) { return n <= (1 << 22) ? float(n) : __builtin_nanf(""); }
+
+// Window index (lx * kWin + ly) * kWin + lz of the floor cell f of an absolute
+// position that the sort put in this tile.  Nearly all floors lie in the tile
+// as they are, some one period away (a particle that left the box), and what
+// is left (non-finite, far away) takes the wrap of floor_cell_abs; every path
+// gives that cell.  far: set when the last path was taken; otherwise the
+// position is finite, at most two periods from the box.
+__device__ __forceinline__ uint32_t window_cell(const float f[3], const TileFrame &F, const TileGrid &t, int ox,
+                                                int oy, int oz, bool &far) {
+  float l[3];
+  bool in = true;
+#pragma unroll
+  for (int a = 0; a < 3; ++a) {
+    l[a] = f[a] - F.o[a];
+    in = in && __builtin_amdgcn_fmed3f(l[a], 0.0f, F.last[a]) == l[a];
+  }
+  far = false;
+  if (!in) {
+    bool one = true;
+#pragma unroll
+    for (int a = 0; a < 3; ++a) {
+      if (l[a] < 0.0f) l[a] += F.n[a];
+      else if (l[a] > F.last[a]) l[a] -= F.n[a];
+      one = one && __builtin_amdgcn_fmed3f(l[a], 0.0f, F.last[a]) == l[a];
+    }
+    if (!one) {
+      far = true;
+      l[0] = float(wrapi(cell_int(f[0]), t.nx) - ox);
+      l[1] = float(wrapi(cell_int(f[1]), t.ny) - oy);
+      l[2] = float(wrapi(cell_int(f[2]), t.nz) - oz);
+    }
+  }
+  return uint32_t(fmaf(l[0], float(kWin * kWin), fmaf(l[1], float(kWin), l[2])));
+}
+
 // enmesh corner (painting_utils.py:48-69) mapped into the window; corners
 // that land outside [origin, origin + 16] (rounding edge cases) report -1 and
 // are deposited by the caller through the overflow path.
@@ -451,6 +494,18 @@ __device__ __forceinline__ void tile_origin(uint32_t tile, const TileGrid &t, in
   itz = int(tile - txy * uint32_t(t.tz));
   itx = int(t.div_ty.div(txy));
   ity = int(txy - uint32_t(itx) * uint32_t(t.ty));
+}
+
+__device__ __forceinline__ TileFrame tile_frame(const TileGrid &t, int itx, int ity, int itz) {
+  TileFrame F;
+  const int n[3] = {t.nx, t.ny, t.nz}, it[3] = {itx, ity, itz}, T[3] = {t.tx, t.ty, t.tz};
+#pragma unroll
+  for (int a = 0; a < 3; ++a) {
+    F.n[a] = window_edge(n[a]);
+    F.o[a] = float(it[a] * kTile) + 0.0f * F.n[a];
+    F.last[a] = float(tile_len(it[a], T[a], n[a]) - 1);
+  }
+  return F;
 }
 
 }  // namespace jpm

@@ -360,3 +360,38 @@ def test_reads_at_the_ends_of_rows(gpu, shape):
     got = host(_ops.read(dev(meshes), dev(disp), relative=True))
     close(got, np.stack([op.cic_read_dx(x, disp.reshape(*shape, 3), dtype=np.float32).reshape(-1) for x in meshes],
                         -1).astype(np.float64))
+
+
+@pytest.mark.parametrize("shape", [(16, 16, 16), (20, 33, 17), (5, 40, 64), (48, 16, 9), (1, 1, 4194352)])
+def test_paint_cells_in_and_out_of_the_box(gpu, shape):
+    """The window index of a floor cell, by its three rules: inside the tile,
+    one period away, farther away, on full and partial tiles and on an axis
+    whose cells a float cannot number exactly; with lanes that share a cell,
+    whose corners go in another order per lane.  Coordinates are multiples of
+    1/8 (1/2 on the long axis) and weights small integers, so every sum is
+    exact in float32 and the mesh has to equal the float64 sum."""
+    from jaxpm_amd import _ops
+    print(f"paint cells {shape}", flush=True)
+    r = np.random.default_rng(41)
+    n = 6000
+    L = np.array(shape, dtype=np.float64)
+    step = np.where(L > 1e6, 2, 8)
+    pos = r.integers(0, (L * step).astype(np.int64), size=(n, 3)) / step
+    pos[: n // 3] = pos[0] + r.integers(-8, 9, size=(n // 3, 3)) / step     # many lanes in a few cells
+    periods = r.choice([0, 0, 0, 1, -1, 2, -3], size=(n, 3)) * np.where(L > 1e6, 0, 1)
+    pos = pos + periods * L
+    w = r.integers(-4, 5, size=n).astype(np.float32)
+    assert np.array_equal(pos.astype(np.float32), pos)
+    ref = np.zeros(shape)
+    f = np.floor(pos)
+    for o in range(8):
+        b = np.array([o & 1, (o >> 1) & 1, (o >> 2) & 1])
+        cell = (f + b).astype(np.int64) % np.array(shape)
+        wt = np.prod(1.0 - np.abs(pos - (f + b)), axis=1) * w
+        np.add.at(ref, tuple(cell.T), wt)
+    got = _ops.paint(torch.zeros(shape, device="cuda"), dev(pos), weight=dev(w))
+    assert np.array_equal(host(got), ref)
+    bad = dev(pos).clone()
+    bad[7, 1] = float("nan")
+    bad[11, 2] = float("inf")
+    assert torch.isnan(_ops.paint(torch.zeros(shape, device="cuda"), bad, weight=dev(w))).any()
