@@ -560,16 +560,17 @@ __device__ __forceinline__ void window_corners(const float4 &rec, const TileGrid
 // scatter's atomic order, so only exact sums across its chunks are
 // reproducible bit for bit.  slot: the window's index in the partial buffer;
 // dst: the channel's mesh at the simulation's first cell.
-template <bool REL>
 __device__ __forceinline__ void write_window(const unsigned long long *win, const ChunkDesc &d, const TileGrid &t,
                                              int itx, int ity, int itz, double scale, size_t slot,
                                              float *__restrict__ partial, float *__restrict__ dst, int accumulate) {
   const int ox = itx * kTile, oy = ity * kTile, oz = itz * kTile;
-  if (!REL && d.pad == 0) {
-    // Absolute positions never leave the window, so the cells of a
-    // single-chunk tile hold their own deposits complete: they go straight
-    // to the mesh, and only the +1 halo (the low faces of the upper
-    // neighbours) is kept for the reduce.
+  if (d.pad == 0) {
+    // The cells of a single-chunk tile hold their own deposits complete (the
+    // rare relative corners outside the window are added last, by the
+    // reduce): they go straight to the mesh, and only the +1 halo (the low
+    // faces of the upper neighbours) is kept for the reduce.  Relative
+    // positions used to store whole windows for it: at 192^3 the reduce took
+    // 68 us and takes 21, the accumulation 77 and 81.
     const double inv = 1.0 / scale;
     const int Lx = tile_len(itx, t.tx, t.nx), Ly = tile_len(ity, t.ty, t.ny), Lz = tile_len(itz, t.tz, t.nz);
     float *out = partial + slot * 2;
@@ -623,10 +624,6 @@ __device__ __forceinline__ void write_window(const unsigned long long *win, cons
         }
       }
     }
-  } else if (d.pad == 0) {
-    const double inv = 1.0 / scale;
-    float *out = partial + slot * 2;
-    for (int i = threadIdx.x; i < kWinCells; i += blockDim.x) out[i] = float(double((long long)win[i]) * inv);
   } else {
     unsigned long long *out = reinterpret_cast<unsigned long long *>(partial) + slot;
     for (int i = threadIdx.x; i < kWinCells; i += blockDim.x) out[i] = win[i];
@@ -651,7 +648,7 @@ bin_accum_kernel(const float4 *__restrict__ spos, const float *__restrict__ weig
                  const ChunkDesc *__restrict__ desc, const uint32_t *__restrict__ nchunks_total, G g, uint32_t M,
                  const float *__restrict__ wmax_dev, float wmax_host, uint32_t n, float *__restrict__ partial,
                  float *__restrict__ overflow, int accumulate, float *__restrict__ mesh, uint32_t per, bool slabs,
-                 uint32_t *__restrict__ nonfinite) {
+                 uint32_t *__restrict__ nonfinite, uint32_t *__restrict__ outside) {
   __shared__ unsigned long long win[kWinCells];
   // (chunk, channel) of this workgroup: the nc channels of one chunk go to
   // one XCD back to back (workgroups b, b + 8, ...), so their reads of the
@@ -756,14 +753,17 @@ bin_accum_kernel(const float4 *__restrict__ spos, const float *__restrict__ weig
         atomicAdd(&win[(Lx * kWin + Ly) * kWin + Lz], fixed_point_q(v, scale));
       } else {
         // rounding put a relative corner outside the window: global path
-        const uint32_t cell = (uint32_t(gx[bx]) * uint32_t(t.ny) + uint32_t(gy[by])) * uint32_t(t.nz) + uint32_t(gz[bz]);
+        // (its tile's reduce adds it)
+        const uint32_t x = uint32_t(gx[bx]), y = uint32_t(gy[by]), z = uint32_t(gz[bz]);
+        const uint32_t cell = (x * uint32_t(t.ny) + y) * uint32_t(t.nz) + z;
+        outside[sim.tile0 + (x / kTile * uint32_t(t.ty) + y / kTile) * uint32_t(t.tz) + z / kTile] = 1u;
         atomicAdd(&overflow[size_t(ch) * M + cell0 + cell], v);
       }
     }
   }
   if (hit) atomicOr(nonfinite, 1u);
   __syncthreads();
-  write_window<REL>(win, d, t, itx, ity, itz, scale, (size_t(c) * nc + ch) * kWinCells, partial,
+  write_window(win, d, t, itx, ity, itz, scale, (size_t(c) * nc + ch) * kWinCells, partial,
                     mesh + size_t(ch) * M + cell0, accumulate);
 }
 
@@ -774,9 +774,11 @@ bin_accum_kernel(const float4 *__restrict__ spos, const float *__restrict__ weig
 // faces, the +1 halo of the lower neighbour(s): along an axis where the local
 // coordinate is 0, the neighbour at -1 (periodic) contributes at its own
 // local index = its tile length.  The (up to 8) sources and each tile's
-// chunks are summed in a fixed order.  With DIRECT, a single-chunk tile's
-// own deposits are already in the mesh (the accumulation wrote them), and
-// only its low-face cells take the neighbours' halos, in the same order.
+// chunks are summed in a fixed order.  A single-chunk tile's own deposits
+// are already in the mesh (the accumulation wrote them), and only its
+// low-face cells take the neighbours' halos, in the same order.  Relative
+// corners outside their window are added to the finished cells from the
+// overflow mesh, in the tiles where the accumulation marked any.
 //
 // When the accumulation flagged a non-finite deposit, the workgroup then
 // walks the particles of the same (up to 8) source tiles and adds their
@@ -784,13 +786,14 @@ bin_accum_kernel(const float4 *__restrict__ spos, const float *__restrict__ weig
 // floats (only this workgroup writes them, so nothing races).
 constexpr int kReduceThreads = 256;
 
-template <class G, bool DIRECT>
+template <class G, bool REL>
 __global__ void __launch_bounds__(kReduceThreads)
 bin_reduce_kernel(const float *__restrict__ partial, const uint32_t *__restrict__ chunk_off,
                   const uint32_t *__restrict__ nchunk, G g, uint32_t M, int nc, const float *__restrict__ overflow,
-                  int has_overflow, const float *__restrict__ wmax_dev, float wmax_host, int has_w, uint32_t n,
+                  const float *__restrict__ wmax_dev, float wmax_host, int has_w, uint32_t n,
                   int accumulate, float *__restrict__ mesh, uint32_t K, uint32_t per, bool slabs,
-                  const uint32_t *__restrict__ nonfinite, const float4 *__restrict__ spos,
+                  const uint32_t *__restrict__ nonfinite, const uint32_t *__restrict__ outside,
+                  const float4 *__restrict__ spos,
                   const ChunkDesc *__restrict__ desc, const float *__restrict__ weight, float wscalar,
                   FaceCells fc) {
   const uint32_t gtile = slab_item(blockIdx.x, per, slabs);
@@ -824,7 +827,7 @@ bin_reduce_kernel(const float *__restrict__ partial, const uint32_t *__restrict_
     src_id[q] = src;
   }
   __syncthreads();
-  const bool faces_only = DIRECT && src_cnt[0] == 1;
+  const bool faces_only = src_cnt[0] == 1;
   const bool full = Lx == kTile && Ly == kTile && Lz == kTile;
   // faces: the a = 0 plane, then b = 0 with a > 0, then c = 0 with a, b > 0
   const int nf0 = Ly * Lz, nf1 = (Lx - 1) * Lz, nf2 = (Lx - 1) * (Ly - 1);
@@ -919,8 +922,8 @@ bin_reduce_kernel(const float *__restrict__ partial, const uint32_t *__restrict_
             const int li = (la * kWin + lb) * kWin + lc;
             const uint32_t c0 = src_off[q], cn = src_cnt[q];
             if (cn == 1) {
-              // a full single-chunk source (absolute mode) holds its halo compactly
-              const bool compact = DIRECT && (sx ? PLx : Lx) == kTile && (sy ? PLy : Ly) == kTile &&
+              // a full single-chunk source holds its halo compactly
+              const bool compact = (sx ? PLx : Lx) == kTile && (sy ? PLy : Ly) == kTile &&
                                    (sz ? PLz : Lz) == kTile;
               acc += partial[((size_t(c0) * nc + ch) * kWinCells) * 2 + (compact ? halo_index(la, lb, lc) : li)];
             } else if (cn > 1) {
@@ -936,18 +939,26 @@ bin_reduce_kernel(const float *__restrict__ partial, const uint32_t *__restrict_
           *dst = acc;
         continue;
       }
-      float v = acc;
-      if (has_overflow) v += overflow[size_t(ch) * M + cell];
       if (fbt && (a == 0 || b == 0 || c == 0))
-        fbt[face_index(a, b, c)] = v;
+        fbt[face_index(a, b, c)] = acc;
       else
-        *dst = accumulate ? *dst + v : v;
+        *dst = accumulate ? *dst + acc : acc;
+    }
+  }
+  float *meshc = mesh + size_t(ch) * M + cell0;
+  if (REL && outside[gtile] != 0u) {
+    __threadfence();
+    __syncthreads();
+    for (int e = threadIdx.x; e < Lx * Ly * Lz; e += blockDim.x) {
+      const int c = e % Lz, ab = e / Lz;
+      const uint32_t cell = (uint32_t(itx * kTile + ab / Ly) * uint32_t(t.ny) + uint32_t(ity * kTile + ab % Ly)) *
+                                uint32_t(t.nz) + uint32_t(itz * kTile + c);
+      meshc[cell] += overflow[size_t(ch) * M + cell0 + cell];
     }
   }
   if (*nonfinite == 0u) return;
   __threadfence();
   __syncthreads();
-  float *meshc = mesh + size_t(ch) * M + cell0;
   for (int q = 0; q < 8; ++q) {
     bool dup = false;
     for (int r = 0; r < q; ++r) dup |= src_id[r] == src_id[q];
@@ -962,13 +973,13 @@ bin_reduce_kernel(const float *__restrict__ partial, const uint32_t *__restrict_
         const float wp = weight ? weight[size_t(__float_as_uint(rec.w)) * nc + ch] : wscalar;
         int lx[2], ly[2], lz[2], gx[2], gy[2], gz[2];
         float wx[2], wy[2], wz[2];
-        window_corners<!DIRECT>(rec, t, sim.part0, ox, oy, oz, lx, ly, lz, gx, gy, gz, wx, wy, wz);
+        window_corners<REL>(rec, t, sim.part0, ox, oy, oz, lx, ly, lz, gx, gy, gz, wx, wy, wz);
         for (int o = 0; o < 8; ++o) {
           const int bx = o & 1, by = (o >> 1) & 1, bz = (o >> 2) & 1;
           const float v = wp * (wx[bx] * wy[by] * wz[bz]);
           if (isfinite(v)) continue;
           int cx, cy, cz;
-          if (DIRECT) {
+          if (!REL) {
             cx = ox + lx[bx];
             cy = oy + ly[by];
             cz = oz + lz[bz];
@@ -1060,7 +1071,8 @@ static size_t accum_ws(const SortDims &d, size_t M, int nc, bool rel, size_t *pa
                        size_t *wmax) {
   size_t o = 0;
   *partial = o;  o += align_up(size_t(d.maxchunks) * nc * kWinCells * 8);
-  *overflow = o; o += rel ? align_up(size_t(nc) * M * 4) : 0;
+  // the overflow mesh and a word per tile whether it holds anything there
+  *overflow = o; o += rel ? align_up((size_t(nc) * M + d.K) * 4) : 0;
   *wmax = o;     o += align_up(4);
   return o;
 }
@@ -1279,6 +1291,7 @@ static int paint_sorted(hipStream_t s, const BinsT<G> &b, const float *weight, f
                         const FaceCells *faces = nullptr) {
   SortDims d{};
   d.maxchunks = b.maxchunks;
+  d.K = b.K;
   JPM_REQUIRE(nc == 1 || nc == 3, "binned paint supports 1 or 3 channels (got %d)", nc);
   JPM_REQUIRE(mesh != nullptr, "mesh is null");
   const int64_t M = b.M;
@@ -1293,7 +1306,10 @@ static int paint_sorted(hipStream_t s, const BinsT<G> &b, const float *weight, f
   char *base = static_cast<char *>(ws);
   int rc;
   if (b.rel) {
-    rc = zero_f32(s, reinterpret_cast<float *>(base + oover), nc * M);
+    // one launch for both while its 32-bit count allows
+    const bool both = nc * M + b.K < (int64_t(1) << 32);
+    rc = zero_f32(s, reinterpret_cast<float *>(base + oover), both ? nc * M + b.K : nc * M);
+    if (!rc && !both) rc = zero_f32(s, reinterpret_cast<float *>(base + oover) + nc * M, b.K);
     if (rc) return rc;
   }
   const float wmax_host = finite_abs(wscalar);
@@ -1304,6 +1320,7 @@ static int paint_sorted(hipStream_t s, const BinsT<G> &b, const float *weight, f
   auto *partial = reinterpret_cast<float *>(base + opart);
   const float *wmax_dev = wmax_in ? wmax_in : reinterpret_cast<const float *>(base + owmax);
   float *overflow = reinterpret_cast<float *>(base + oover);
+  uint32_t *outside = reinterpret_cast<uint32_t *>(overflow + (b.rel ? nc * M : 0));
   {
     JPM_TIMED(s, nc == 1 ? "bin_accum_kernel[nc=1]" : "bin_accum_kernel[nc=3]");
     auto kern = b.rel ? bin_accum_kernel<true, G> : bin_accum_kernel<false, G>;
@@ -1312,21 +1329,20 @@ static int paint_sorted(hipStream_t s, const BinsT<G> &b, const float *weight, f
     const unsigned grid = 8u * per * unsigned(nc);
     hipLaunchKernelGGL(kern, dim3(grid), dim3(kWindowThreads), 0, s, b.spos, weight, nc, wscalar, b.desc,
                        b.total_chunks, b.g, b.M, wmax_dev, wmax_host, b.n, partial, overflow, int(accumulate), mesh,
-                       per, b.slabs, b.nonfinite);
+                       per, b.slabs, b.nonfinite, outside);
   }
   JPM_LAUNCHED("bin_accum_kernel");
   {
     JPM_TIMED(s, nc == 1 ? "bin_reduce_kernel[nc=1]" : "bin_reduce_kernel[nc=3]");
-    // absolute positions: single-chunk tiles wrote their own cells already
-    auto kern = b.rel ? bin_reduce_kernel<G, false> : bin_reduce_kernel<G, true>;
+    auto kern = b.rel ? bin_reduce_kernel<G, true> : bin_reduce_kernel<G, false>;
     // always in XCD slabs: tiles consecutive in z then run on one XCD, and
     // their low-z faces, single floats a tile apart along each mesh row,
     // share that XCD's L2 lines (0.14 -> 0.10 ms for 3 channels at 256^3)
     uint32_t per;
     const unsigned grid = slab_grid(b.K, true, per);
     hipLaunchKernelGGL(kern, dim3(grid, nc), dim3(kReduceThreads), 0, s, partial, b.choff, b.nchunk, b.g, b.M, nc, overflow,
-                       int(b.rel), wmax_dev, wmax_host, int(weight != nullptr), b.n, int(accumulate), mesh, b.K, per,
-                       true, b.nonfinite, b.spos, b.desc, weight, wscalar, fc);
+                       wmax_dev, wmax_host, int(weight != nullptr), b.n, int(accumulate), mesh, b.K, per,
+                       true, b.nonfinite, outside, b.spos, b.desc, weight, wscalar, fc);
   }
   JPM_LAUNCHED("bin_reduce_kernel");
   return JPM_OK;

@@ -395,3 +395,31 @@ def test_paint_cells_in_and_out_of_the_box(gpu, shape):
     bad[7, 1] = float("nan")
     bad[11, 2] = float("inf")
     assert torch.isnan(_ops.paint(torch.zeros(shape, device="cuda"), bad, weight=dev(w))).any()
+
+
+@pytest.mark.parametrize("shape", [(16, 16, 16), (32, 32, 48), (40, 24, 20), (48, 17, 33)])
+def test_relative_paint_writes_cells_directly(gpu, shape):
+    """Relative paints on full and partial tiles: added to a mesh and into a
+    fresh one, on tiles of one chunk, of several and of none, with corners that
+    float rounding puts one cell outside their window (node + displacement one
+    ulp below 16, where adding 1 rounds up to 17); and three weighted channels
+    against the atomic kernel.  Tolerances are those of the paints above."""
+    from jaxpm_amd import _ops
+    print(f"relative paint {shape}", flush=True)
+    r = np.random.default_rng(45)
+    disp = r.normal(scale=2.0, size=(*shape, 3)).astype(np.float32)
+    node = lattice(shape)
+    edge = np.nextafter(np.float32(16.0), np.float32(0.0))
+    if shape[0] > 16:
+        disp[5, :, :, 0] = edge - np.float32(5.0)
+        assert np.float32(np.float32(5.0) + disp[5, 0, 0, 0]) == edge
+    if shape[0] == 32:   # most particles in one tile, which takes several chunks
+        disp[8:] = (np.float32(4.0) + r.uniform(0, 8, size=disp[8:].shape).astype(np.float32)) - node[8:]
+    base = r.normal(size=shape).astype(np.float32)
+    w = r.normal(size=shape).astype(np.float32)
+    ref = op.cic_paint_dx(disp, weight=w, dtype=np.float32)
+    close(host(_ops.paint(dev(np.full(shape, 7.0)), dev(disp), weight=dev(w), relative=True, zero=True)), ref)
+    close(host(_ops.paint(dev(base), dev(disp), weight=dev(w), relative=True)), base + ref)
+    w3 = dev(r.normal(size=(int(np.prod(shape)), 3)))
+    close(host(_ops.paint_multi(shape, dev(disp), w3, relative=True)),
+          host(_ops.paint_multi(shape, dev(disp), w3, relative=True, method="atomic")), rel=1e-5)
