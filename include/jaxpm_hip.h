@@ -452,6 +452,16 @@ int jpm_cic_read_sorted_f32(void *stream, int nx, int ny, int nz,
                             const float *pos, int64_t n, float *out,
                             uint32_t flags, void *ws, size_t ws_bytes);
 
+/* Both cotangents of jpm_cic_read_f32 of 1 or 3 contiguous meshes at absolute
+ * positions, from one tile sort: gmesh[c] = the paint of cot[:, c], and
+ * gpos[n][3] bit for bit that of jpm_cic_grad_pos_f32.  Workspace of
+ * jpm_cic_paint_binned_workspace_size(nx, ny, nz, n, ncomp, flags) bytes. */
+int jpm_cic_read_vjp_f32(void *stream, int nx, int ny, int nz,
+                         const float *mesh, int ncomp, const float *pos,
+                         int64_t n, const float *cot, float *gmesh,
+                         float *gpos, uint32_t flags, void *ws,
+                         size_t ws_bytes);
+
 /* Workspace bytes for jpm_force_kick_f32 (0 when three meshes exceed 2^32
  * cells or flags ask for the exact gradient / atomic paint, which the sorted
  * pipeline does not cover). */

@@ -51,6 +51,10 @@ class CicRead(torch.autograd.Function):
         meshes, pos = ctx.saved_tensors
         g = g.contiguous()
         gm = gp = None
+        if ctx.needs_input_grad[0] and ctx.needs_input_grad[1] and not ctx.relative and \
+                meshes.shape[0] in (1, 3) and _ops.binned_ok(meshes.shape[1:]):
+            gm, gp = _ops.read_vjp(meshes, pos, g, deterministic=ctx.deterministic)
+            return gm, gp.reshape(pos.shape), None, None, None
         if ctx.needs_input_grad[0]:
             gm = _ops.paint_multi(meshes.shape[1:], pos, g, relative=ctx.relative,
                                   deterministic=ctx.deterministic)

@@ -169,6 +169,24 @@ def read(meshes, pos, relative=False, method="direct"):
     return out.reshape(n) if single else out
 
 
+def read_vjp(meshes, pos, cot, deterministic=False):
+    """(gmesh (nc,nx,ny,nz), gpos (n,3)) of ``read`` at absolute positions from
+    one tile sort: the values of paint_multi and grad_pos (nc 1 or 3)."""
+    m4 = _f32(meshes, "mesh")
+    nc = m4.shape[0]
+    nx, ny, nz = _dims(m4.shape[1:])
+    pos = _f32(pos, "positions").reshape(-1, 3)
+    n = pos.shape[0]
+    cot = _f32(cot, "cotangent").reshape(n, nc)
+    gmesh, gpos = torch.empty_like(m4), torch.empty_like(pos)
+    flags = (_lib.DETERMINISTIC if deterministic else 0) | _lib.ZERO_MESH
+    wsb = size("jpm_cic_paint_binned_workspace_size", nx, ny, nz, n, nc, flags)
+    ws = torch.empty(wsb, dtype=torch.uint8, device=pos.device)
+    call("jpm_cic_read_vjp_f32", stream(), nx, ny, nz, ptr(m4), nc, ptr(pos), n, ptr(cot), ptr(gmesh), ptr(gpos),
+         flags, ptr(ws), wsb)
+    return gmesh, gpos
+
+
 def grad_pos(meshes, pos, cot=None, weight=None, wscalar=1.0, relative=False, out=None):
     """Position cotangent (n,3) of CIC sampling (see jpm_cic_grad_pos_f32)."""
     meshes = _f32(meshes, "mesh")

@@ -197,6 +197,7 @@ int bins_kick(hipStream_t, const Bins &, const float *, float, float *, int, flo
 int bins_grad(hipStream_t, const Bins &, const float *, const float *, const float *, float, float *, bool, float,
               float *, float *);
 int bins_read(hipStream_t, const Bins &, const float *, int, uint32_t, float *);
+int bins_grad_pos(hipStream_t, const Bins &, const float *, int, uint32_t, const float *, float *);
 
 // ------------------------------------------------------ sorted pipelines
 //
@@ -310,6 +311,41 @@ static int cic_read_sorted(hipStream_t s, int nx, int ny, int nz, const float *m
   rc = bin_sort(s, nx, ny, nz, pos, n, 0, ws, ws_bytes, b);
   if (rc) return rc;
   return bins_read(s, b, mesh, ncomp, uint32_t(ncomp == 1 ? m : comp_stride), out);
+}
+
+// Both cotangents of cic_read of 1 or 3 meshes at absolute positions from one
+// tile sort: gmesh = the cotangents painted, gpos = the positions' cotangent.
+// The latter reads LDS windows of the sorted particles unless they are so few
+// that most of a window would be loaded for nothing: with the paint, in us,
+// windows against direct loads for N / r particles on a mesh of N = 200^3 took,
+// for particles in lattice order and in none, one mesh, r = 1: 245 and 264, 651
+// and 872; r = 4: 109 and 108, 202 and 269; r = 8: 92 and 88, 134 and 165; three
+// meshes, r = 1: 401 and 520, 847 and 2277; r = 8: 183 and 198, 227 and 392.
+static int cic_read_vjp(hipStream_t s, int nx, int ny, int nz, const float *mesh, int ncomp, const float *pos,
+                        int64_t n, const float *cot, float *gmesh, float *gpos, uint32_t flags, void *ws,
+                        size_t ws_bytes) {
+  int rc = check_dims(nx, ny, nz);
+  if (rc) return rc;
+  JPM_REQUIRE(!(flags & JPM_RELATIVE), "the read's sorted cotangents take absolute positions");
+  JPM_REQUIRE(binned_paint_supported(nx, ny, nz), "mesh too large for the tile sort");
+  JPM_REQUIRE(ncomp == 1 || ncomp == 3, "ncomp=%d must be 1 or 3", ncomp);
+  JPM_REQUIRE(n >= 0 && n <= kMaxCells, "particle count %lld out of range", (long long)n);
+  JPM_REQUIRE(gmesh != nullptr, "gmesh is null");
+  flags |= JPM_ZERO_MESH;
+  const int64_t m = cells(nx, ny, nz);
+  const size_t need = binned_paint_workspace_size(nx, ny, nz, n, ncomp, flags);
+  JPM_REQUIRE(ws && ws_bytes >= need, "the read's cotangents need %zu workspace bytes, got %zu", need, ws_bytes);
+  if (n == 0) return zero_f32(s, gmesh, ncomp * m);
+  JPM_REQUIRE(mesh && pos && cot && gpos, "null pointer argument");
+  const size_t sort_bytes = align_up(bin_sort_workspace_size(nx, ny, nz, n, flags));
+  Bins b;
+  if ((rc = bin_sort(s, nx, ny, nz, pos, n, flags, ws, sort_bytes, b))) return rc;
+  if ((rc = bins_paint(s, b, cot, 1.0f, ncomp, gmesh, flags, static_cast<char *>(ws) + sort_bytes,
+                       ws_bytes - sort_bytes, nullptr)))
+    return rc;
+  if (n < (ncomp == 1 ? m / 2 : m / 8))
+    return cic_grad_pos(s, nx, ny, nz, mesh, ncomp, m, pos, n, cot, nullptr, 1.0f, gpos, 0, 0);
+  return bins_grad_pos(s, b, mesh, ncomp, uint32_t(m), cot, gpos);
 }
 
 static int tile_order(hipStream_t s, int nx, int ny, int nz, const float *pos, int64_t n, uint32_t *order, void *ws,
@@ -1108,6 +1144,12 @@ int jpm_cic_read_sorted_f32(void *stream, int nx, int ny, int nz, const float *m
                             const float *pos, int64_t n, float *out, uint32_t flags, void *ws, size_t ws_bytes) {
   JPM_GUARD(cic_read_sorted(as_stream(stream), nx, ny, nz, mesh, ncomp, comp_stride, pos, n, out, flags, ws,
                             ws_bytes));
+}
+
+int jpm_cic_read_vjp_f32(void *stream, int nx, int ny, int nz, const float *mesh, int ncomp, const float *pos,
+                         int64_t n, const float *cot, float *gmesh, float *gpos, uint32_t flags, void *ws,
+                         size_t ws_bytes) {
+  JPM_GUARD(cic_read_vjp(as_stream(stream), nx, ny, nz, mesh, ncomp, pos, n, cot, gmesh, gpos, flags, ws, ws_bytes));
 }
 
 size_t jpm_cic_paint_binned_workspace_size(int nx, int ny, int nz, int64_t n, int nc, uint32_t flags) {

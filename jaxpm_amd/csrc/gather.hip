@@ -740,6 +740,100 @@ bin_read_kernel(BinsT<G> bins, const float *__restrict__ mesh_all, uint32_t cstr
   }
 }
 
+// Position cotangent of cic_read over the tile-sorted particles: gpos[p] =
+// sum_c cot[p, c] sum_o mesh_c[idx_o] dW_o/dx, the corners from the tile's 17^3
+// windows in LDS, in the order and float operations of the direct kernel
+// (cic.hip), so both give the same bits.  Absolute positions only.
+template <int NC>
+constexpr int grad_pos_threads() { return NC == 1 ? kWindowThreads : 1024; }
+
+template <int NC>
+__global__ void __launch_bounds__(grad_pos_threads<NC>())
+bin_grad_pos_kernel(Bins bins, const float *__restrict__ mesh, uint32_t cstride, const float *__restrict__ cot,
+                    float *__restrict__ gpos, uint32_t per, uint32_t parts) {
+  constexpr int T = grad_pos_threads<NC>();
+  __shared__ float win[NC * kWinCells];
+  const uint32_t c = gather_item(blockIdx.x, per, bins.slabs);
+  if (c >= *bins.total_chunks) return;
+  const ChunkDesc d = bins.desc[c];
+  uint32_t start, cnt;
+  if (!chunk_part<true>(d, parts, start, cnt)) return;
+  const TileGrid &t = bins.g.s.t;
+  int itx, ity, itz;
+  tile_origin(d.tile, t, itx, ity, itz);
+  const int ox = itx * kTile, oy = ity * kTile, oz = itz * kTile;
+  // as in the kick: particle q computes while the cotangent of q + T and the
+  // record of q + 2T load
+  const float4 zero4 = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+  float4 rec1 = threadIdx.x < cnt ? load_global(bins.spos + (start + threadIdx.x)) : zero4;
+  float4 rec2 = threadIdx.x + T < cnt ? load_global(bins.spos + (start + threadIdx.x + T)) : zero4;
+  float nu[NC] = {};
+  if (threadIdx.x < cnt) {
+    const float *u = cot + NC * size_t(__float_as_uint(rec1.w));
+#pragma unroll
+    for (int k = 0; k < NC; ++k) nu[k] = u[k];
+  }
+#pragma unroll
+  for (int k = 0; k < NC; ++k)
+    load_window_t<kWin, 0, T>(mesh + size_t(k) * cstride, t, ox, oy, oz, win + k * kWinCells);
+  __syncthreads();
+  for (uint32_t q = threadIdx.x; q < cnt; q += T) {
+    const float4 rec = rec1;
+    float u[NC];
+#pragma unroll
+    for (int k = 0; k < NC; ++k) u[k] = nu[k];
+    rec1 = rec2;
+    if (q + T < cnt) {
+      const float *v = cot + NC * size_t(__float_as_uint(rec1.w));
+#pragma unroll
+      for (int k = 0; k < NC; ++k) nu[k] = v[k];
+    }
+    if (q + 2 * T < cnt) rec2 = load_global(bins.spos + (start + q + 2 * T));
+    CornerSet cs;
+    corner_set<false>(rec, t, 0u, ox, oy, oz, cs);
+    const float *w0 = win + (cs.l[0][0] * kWin + cs.l[1][0]) * kWin + cs.l[2][0];
+    // a coordinate without a next cell (not finite, or too large for floor + 1
+    // to differ) has both corners at its floor cell, as in the direct kernel
+    auto next = [](float x, int step) { return floorf(x) + 1.0f > floorf(x) ? step : 0; };
+    const int sx = next(rec.x, kWin * kWin), sy = next(rec.y, kWin), sz = next(rec.z, 1);
+    float out[3] = {0.0f, 0.0f, 0.0f};
+#pragma unroll
+    for (int k = 0; k < NC; ++k) {
+      float s[3] = {0.0f, 0.0f, 0.0f};
+#pragma unroll
+      for (int o = 0; o < 8; ++o) {
+        const int bx = o & 1, by = (o >> 1) & 1, bz = (o >> 2) & 1;
+        const float v = w0[k * kWinCells + bx * sx + by * sy + bz * sz];
+        s[0] += v * (cs.d[0][bx] * cs.w[1][by] * cs.w[2][bz]);
+        s[1] += v * (cs.w[0][bx] * cs.d[1][by] * cs.w[2][bz]);
+        s[2] += v * (cs.w[0][bx] * cs.w[1][by] * cs.d[2][bz]);
+      }
+#pragma unroll
+      for (int a = 0; a < 3; ++a) out[a] += u[k] * s[a];
+    }
+    float *g = gpos + 3 * size_t(__float_as_uint(rec.w));
+    g[0] = out[0];
+    g[1] = out[1];
+    g[2] = out[2];
+  }
+}
+
+int bins_grad_pos(hipStream_t s, const Bins &b, const float *mesh, int nc, uint32_t cstride, const float *cot,
+                  float *gpos) {
+  JPM_REQUIRE(mesh && cot && gpos, "null pointer argument");
+  JPM_REQUIRE(!b.rel && (nc == 1 || nc == 3), "the sorted position cotangent takes absolute positions, 1 or 3 meshes");
+  uint32_t per;
+  const uint32_t parts = gather_parts(b.n, b.K, nc == 1 ? grad_pos_threads<1>() : grad_pos_threads<3>());
+  const dim3 grid(gather_grid(b.maxchunks, b.K, b.slabs, per), 1u << parts);
+  JPM_TIMED(s, "bin_grad_pos_kernel");
+  if (nc == 1)
+    hipLaunchKernelGGL(bin_grad_pos_kernel<1>, grid, dim3(grad_pos_threads<1>()), 0, s, b, mesh, cstride, cot, gpos, per, parts);
+  else
+    hipLaunchKernelGGL(bin_grad_pos_kernel<3>, grid, dim3(grad_pos_threads<3>()), 0, s, b, mesh, cstride, cot, gpos, per, parts);
+  JPM_LAUNCHED("bin_grad_pos_kernel");
+  return JPM_OK;
+}
+
 template <class G>
 static int kick_sorted(hipStream_t s, const BinsT<G> &b, const float *phi, float gamma, const float *gamma_dev,
                        float *vel, int mode, DriftArgs dr) {

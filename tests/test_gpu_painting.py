@@ -423,3 +423,28 @@ def test_relative_paint_writes_cells_directly(gpu, shape):
     w3 = dev(r.normal(size=(int(np.prod(shape)), 3)))
     close(host(_ops.paint_multi(shape, dev(disp), w3, relative=True)),
           host(_ops.paint_multi(shape, dev(disp), w3, relative=True, method="atomic")), rel=1e-5)
+
+
+@pytest.mark.parametrize("nc", [1, 3])
+@pytest.mark.parametrize("shape,n", [((16, 16, 16), 5000), ((20, 33, 17), 11220), ((32, 32, 48), 40000),
+                                     ((64, 48, 40), 61441), ((48, 48, 48), 13000), ((9, 40, 64), 1)])
+def test_read_cotangents_from_one_sort(gpu, shape, n, nc):
+    """The cotangents of a read from one tile sort: both equal those of the
+    paint and of the direct kernel bit for bit, on full and partial tiles, at
+    counts on both sides of the rules on particles per cell and per tile, with
+    positions out of the box and one that is not finite."""
+    from jaxpm_amd import _ops
+    print(f"read vjp {shape} n={n} nc={nc}", flush=True)
+    r = np.random.default_rng(47)
+    pos = (r.uniform(-0.6, 1.7, size=(n, 3)) * np.array(shape)).astype(np.float32)
+    pos[: n // 4] = np.floor(pos[: n // 4])
+    meshes, cot = dev(r.normal(size=(nc, *shape))), dev(r.normal(size=(n, nc)))
+    p = dev(pos)
+    gm, gp = _ops.read_vjp(meshes, p, cot)
+    assert torch.equal(gm, _ops.paint_multi(shape, p, cot))
+    assert torch.equal(gp, _ops.grad_pos(meshes, p, cot=cot))
+    p[n // 2, 1] = float("nan")
+    gm, gp = _ops.read_vjp(meshes, p, cot)
+    direct = _ops.grad_pos(meshes, p, cot=cot)
+    assert torch.equal(gp.isnan(), direct.isnan()) and torch.equal(gp.nan_to_num(), direct.nan_to_num())
+    assert torch.equal(gm.isnan(), _ops.paint_multi(shape, p, cot).isnan())
