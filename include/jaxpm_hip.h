@@ -192,6 +192,13 @@ int jpm_cic_paint_binned_f32(void *stream, int nx, int ny, int nz,
                              float wscalar, int nc, float *mesh,
                              uint32_t flags, void *ws, size_t ws_bytes);
 
+/* mesh = base + the paint of jpm_cic_paint_binned_f32 (one channel, same
+ * workspace), bit for bit a copy of base painted in place; base may be mesh. */
+int jpm_cic_paint_onto_f32(void *stream, int nx, int ny, int nz,
+                           const float *base, const float *pos, int64_t n,
+                           const float *weights, float wscalar, float *mesh,
+                           uint32_t flags, void *ws, size_t ws_bytes);
+
 /* Bytes of device scratch the allocation-free paint holds per GPU (64 MiB). */
 #define JPM_NOALLOC_SCRATCH_BYTES ((size_t)64 << 20)
 

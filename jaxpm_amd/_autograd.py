@@ -16,8 +16,8 @@ class CicPaint(torch.autograd.Function):
 
     @staticmethod
     def forward(ctx, mesh, pos, weight, wscalar, relative, deterministic):
-        out = mesh.clone()
-        _ops.paint(out, pos, weight=weight, wscalar=wscalar, relative=relative, deterministic=deterministic)
+        out = _ops.paint_onto(mesh, pos, weight=weight, wscalar=wscalar, relative=relative,
+                              deterministic=deterministic)
         ctx.save_for_backward(pos, weight)
         ctx.wscalar, ctx.relative, ctx.shape = wscalar, relative, pos.shape
         return out

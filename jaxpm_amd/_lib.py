@@ -55,6 +55,7 @@ SIGNATURES = {
     "jpm_cic_paint_f32": (_i, [_vp, _i, _i, _i, _vp, _i64, _vp, _f, _vp, _u32, _vp, _sz]),
     "jpm_cic_read_f32": (_i, [_vp, _i, _i, _i, _vp, _i, _i64, _vp, _i64, _vp, _u32]),
     "jpm_cic_read_sorted_workspace_size": (_sz, [_i, _i, _i, _i64]),
+    "jpm_cic_paint_onto_f32": (_i, [_vp, _i, _i, _i, _vp, _vp, _i64, _vp, _f, _vp, _u32, _vp, _sz]),
     "jpm_cic_read_vjp_f32": (_i, [_vp, _i, _i, _i, _vp, _i, _vp, _i64, _vp, _vp, _vp, _u32, _vp, _sz]),
     "jpm_cic_read_sorted_f32": (_i, [_vp, _i, _i, _i, _vp, _i, _i64, _vp, _i64, _vp, _u32, _vp, _sz]),
     "jpm_cic_paint_multi_workspace_size": (_sz, [_i, _i, _i, _i, _u32]),

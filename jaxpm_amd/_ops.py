@@ -79,6 +79,28 @@ def paint(mesh, pos, weight=None, wscalar=1.0, relative=False, deterministic=Fal
     return mesh
 
 
+def paint_onto(base, pos, weight=None, wscalar=1.0, relative=False, deterministic=False):
+    """A new mesh: ``base`` plus the deposits of ``paint``, the bits of
+    painting a copy of it."""
+    base = _f32(base, "mesh")
+    if not binned_ok(base.shape):
+        return paint(base.clone(), pos, weight, wscalar, relative, deterministic)
+    pos = _f32(pos, "positions").reshape(-1, 3)
+    nx, ny, nz = _dims(base.shape)
+    n = pos.shape[0]
+    if weight is not None:
+        weight = _f32(weight, "weight").reshape(-1)
+        if weight.numel() != n:
+            raise ValueError(f"weight has {weight.numel()} entries for {n} particles")
+    out = torch.empty_like(base)
+    flags = (_lib.RELATIVE if relative else 0) | (_lib.DETERMINISTIC if deterministic else 0)
+    wsb = size("jpm_cic_paint_binned_workspace_size", nx, ny, nz, n, 1, flags)
+    ws = torch.empty(wsb, dtype=torch.uint8, device=base.device)
+    call("jpm_cic_paint_onto_f32", stream(), nx, ny, nz, ptr(base), ptr(pos), n, ptr(weight), float(wscalar),
+         ptr(out), flags, ptr(ws), wsb)
+    return out
+
+
 def paint_f64(mesh, pos, weight=None, wscalar=1.0, relative=False, zero=False):
     """Float64 paint into ``mesh`` (float64, updated in place)."""
     nx, ny, nz = _dims(mesh.shape)

@@ -105,7 +105,8 @@ __device__ __forceinline__ void slice_histogram(const float *__restrict__ pos, u
 
 template <bool REL, class G>
 __global__ void __launch_bounds__(kBinThreads)
-bin_count_kernel(const float *__restrict__ pos, uint32_t slice, uint32_t shift, G g, uint32_t *__restrict__ count) {
+bin_count_kernel(const float *__restrict__ pos, uint32_t slice, uint32_t shift, G g, uint32_t *__restrict__ count,
+                 uint32_t gstride) {
   extern __shared__ uint32_t sh[];
   // 2^shift workgroups share a slice, each an equal part of it
   const uint32_t blk = blockIdx.x >> shift;
@@ -121,7 +122,7 @@ bin_count_kernel(const float *__restrict__ pos, uint32_t slice, uint32_t shift, 
   slice_histogram<REL>(pos, p0, p1, s, sh);
   __syncthreads();
   for (uint32_t k = threadIdx.x; k < K; k += blockDim.x)
-    if (sh[k]) atomicAdd(&count[tile0 + k], sh[k]);
+    if (sh[k]) atomicAdd(&count[(blk & 7u) * gstride + tile0 + k], sh[k]);
 }
 
 // Tile counts for meshes of more than kMaxKeysLds tiles, where no LDS
@@ -251,6 +252,7 @@ chunk_desc_kernel(const uint32_t *__restrict__ tile_start, const uint32_t *__res
   }
 }
 
+constexpr uint32_t kSortGroups = 8;   // see sort_groups
 // The whole tile table of a sort of at most kTableMaxK tiles in one launch
 // of ceil(K / 1024) workgroups: tile starts and scatter cursors (exclusive
 // scan of the counts), chunks per tile and their offsets (exclusive scan),
@@ -262,8 +264,8 @@ constexpr int kTableThreads = 1024;
 constexpr uint32_t kTableMaxK = 32768;
 
 __global__ void __launch_bounds__(kTableThreads)
-tile_table_kernel(const uint32_t *__restrict__ count, uint32_t K, uint32_t chunk, uint32_t *__restrict__ tstart,
-                  uint32_t *__restrict__ cursor, uint32_t *__restrict__ nchunk, uint32_t *__restrict__ choff,
+tile_table_kernel(const uint32_t *__restrict__ count, uint32_t K, uint32_t groups, uint32_t chunk,
+                  uint32_t *__restrict__ tstart, uint32_t *__restrict__ cursor, uint32_t *__restrict__ nchunk, uint32_t *__restrict__ choff,
                   uint32_t *__restrict__ totals, ChunkDesc *__restrict__ desc) {
   // workgroup b owns tiles [b T, (b + 1) T), one per thread, T = kTableThreads
   __shared__ uint32_t sp[kTableThreads / 64], sc[kTableThreads / 64];
@@ -272,12 +274,19 @@ tile_table_kernel(const uint32_t *__restrict__ count, uint32_t K, uint32_t chunk
   // particles and chunks of the tiles before this workgroup's (summed by
   // every workgroup for itself: at most K counts, read from L2)
   uint32_t bp = 0, bc = 0;
+  auto tile_count = [&](uint32_t j) {
+    uint32_t c = count[j];
+    if (groups > 1)   // kSortGroups; unrolled, the loads in flight together
+#pragma unroll
+      for (uint32_t g = 1; g < kSortGroups; ++g) c += count[g * K + j];
+    return c;
+  };
   for (uint32_t j = t; j < first; j += kTableThreads) {
-    const uint32_t c = count[j];
+    const uint32_t c = tile_count(j);
     bp += c;
     bc += (c + chunk - 1) / chunk;
   }
-  const uint32_t np = k < K ? count[k] : 0u, nc = (np + chunk - 1) / chunk;
+  const uint32_t np = k < K ? tile_count(k) : 0u, nc = (np + chunk - 1) / chunk;
   // one pass of wavefront shuffles: the base sums reduced, this
   // workgroup's (np, nc) scanned inclusively
   uint32_t xp = np, xc = nc;
@@ -318,6 +327,13 @@ tile_table_kernel(const uint32_t *__restrict__ count, uint32_t K, uint32_t chunk
   if (k < K) {
     tstart[k] = pb;
     cursor[k] = pb;
+    if (groups > 1) {
+      uint32_t c[kSortGroups], at = pb;
+#pragma unroll
+      for (uint32_t g = 0; g < kSortGroups; ++g) c[g] = count[g * K + k];
+#pragma unroll
+      for (uint32_t g = 1; g < kSortGroups; ++g) cursor[g * K + k] = at += c[g - 1];
+    }
     nchunk[k] = nc;
     choff[k] = cb;
     for (uint32_t o = 0; o < np; o += chunk, ++cb) {
@@ -332,10 +348,10 @@ tile_table_kernel(const uint32_t *__restrict__ count, uint32_t K, uint32_t chunk
 }
 
 int tile_table(hipStream_t s, const uint32_t *count, uint32_t K, uint32_t chunk, uint32_t *tstart, uint32_t *cursor,
-               uint32_t *nchunk, uint32_t *choff, uint32_t *totals, ChunkDesc *desc) {
+               uint32_t *nchunk, uint32_t *choff, uint32_t *totals, ChunkDesc *desc, uint32_t groups) {
   JPM_REQUIRE(K >= 1 && K <= kTableMaxK, "%u tiles exceed the tile table's %u", K, kTableMaxK);
   hipLaunchKernelGGL(tile_table_kernel, dim3((K + kTableThreads - 1) / kTableThreads), dim3(kTableThreads), 0, s,
-                     count, K, chunk, tstart, cursor, nchunk, choff, totals, desc);
+                     count, K, groups, chunk, tstart, cursor, nchunk, choff, totals, desc);
   JPM_LAUNCHED("tile_table_kernel");
   return JPM_OK;
 }
@@ -395,8 +411,9 @@ bin_scatter_kernel(const float *__restrict__ pos, uint32_t slice, G g, uint32_t 
 template <bool REL, class G, int PER, int THREADS>
 __global__ void __launch_bounds__(THREADS)
 bin_scatter_reg_kernel(const float *__restrict__ pos, uint32_t slice, G g, uint32_t *__restrict__ cursor,
-                       float4 *__restrict__ spos) {
+                       float4 *__restrict__ spos, uint32_t gstride) {
   extern __shared__ uint32_t cur[];
+  cursor += (blockIdx.x & 7u) * gstride;
   const SimRef &s = g.block_sim(blockIdx.x);
   const uint32_t K = s.t.K, tile0 = s.tile0;
   for (uint32_t k = threadIdx.x; k < K; k += blockDim.x) cur[k] = 0;
@@ -562,7 +579,8 @@ __device__ __forceinline__ void window_corners(const float4 &rec, const TileGrid
 // dst: the channel's mesh at the simulation's first cell.
 __device__ __forceinline__ void write_window(const unsigned long long *win, const ChunkDesc &d, const TileGrid &t,
                                              int itx, int ity, int itz, double scale, size_t slot,
-                                             float *__restrict__ partial, float *__restrict__ dst, int accumulate) {
+                                             float *__restrict__ partial, float *__restrict__ dst,
+                                             const float *base) {
   const int ox = itx * kTile, oy = ity * kTile, oz = itz * kTile;
   if (d.pad == 0) {
     // The cells of a single-chunk tile hold their own deposits complete (the
@@ -582,12 +600,15 @@ __device__ __forceinline__ void write_window(const unsigned long long *win, cons
       const int lx0 = int(threadIdx.x) >> 8, ly = (int(threadIdx.x) >> 4) & 15, lz = int(threadIdx.x) & 15;
       const unsigned long long *w = win + (lx0 * kWin + ly) * kWin + lz;
       const uint32_t plane = uint32_t(t.ny) * uint32_t(t.nz);
-      float *cellp = dst + uint32_t(ox + lx0) * plane + uint32_t(oy + ly) * uint32_t(t.nz) + uint32_t(oz + lz);
+      const uint32_t at = uint32_t(ox + lx0) * plane + uint32_t(oy + ly) * uint32_t(t.nz) + uint32_t(oz + lz);
+      float b[kTile / kStep];
+      if (base)
+#pragma unroll
+        for (int i = 0; i < kTile / kStep; ++i) b[i] = base[at + size_t(i * kStep) * plane];
 #pragma unroll
       for (int i = 0; i < kTile / kStep; ++i) {
         const float v = float(double((long long)w[i * kStep * kWin * kWin]) * inv);
-        float *c = cellp + size_t(i * kStep) * plane;
-        *c = accumulate ? *c + v : v;
+        dst[at + size_t(i * kStep) * plane] = base ? b[i] + v : v;
       }
       // halo, compact (halo_index): the lx = 16 plane, then ly = 16 (lx <
       // 16), then lz = 16 (lx, ly < 16), so both this write and the reduce's
@@ -606,7 +627,7 @@ __device__ __forceinline__ void write_window(const unsigned long long *win, cons
         out[e] = float(double((long long)win[(lx * kWin + ly) * kWin + lz]) * inv);
       }
       // own face cells (face_cell order), the same floats the mesh received
-      if (!accumulate)
+      if (!base)
         for (int e = threadIdx.x; e < kFaces; e += blockDim.x) {
           int a, b, c;
           face_cell(e, a, b, c);
@@ -617,8 +638,8 @@ __device__ __forceinline__ void write_window(const unsigned long long *win, cons
         const int lz = i % kWin, lxy = i / kWin, ly = lxy % kWin, lx = lxy / kWin;
         const float v = float(double((long long)win[i]) * inv);
         if (lx < Lx && ly < Ly && lz < Lz) {
-          float *cellp = dst + (uint32_t(ox + lx) * uint32_t(t.ny) + uint32_t(oy + ly)) * uint32_t(t.nz) + uint32_t(oz + lz);
-          *cellp = accumulate ? *cellp + v : v;
+          const uint32_t at = (uint32_t(ox + lx) * uint32_t(t.ny) + uint32_t(oy + ly)) * uint32_t(t.nz) + uint32_t(oz + lz);
+          dst[at] = base ? base[at] + v : v;
         } else {
           out[i] = v;
         }
@@ -647,7 +668,7 @@ __global__ void __launch_bounds__(kWindowThreads)
 bin_accum_kernel(const float4 *__restrict__ spos, const float *__restrict__ weight, int nc, float wscalar,
                  const ChunkDesc *__restrict__ desc, const uint32_t *__restrict__ nchunks_total, G g, uint32_t M,
                  const float *__restrict__ wmax_dev, float wmax_host, uint32_t n, float *__restrict__ partial,
-                 float *__restrict__ overflow, int accumulate, float *__restrict__ mesh, uint32_t per, bool slabs,
+                 float *__restrict__ overflow, const float *base, float *mesh, uint32_t per, bool slabs,
                  uint32_t *__restrict__ nonfinite, uint32_t *__restrict__ outside) {
   __shared__ unsigned long long win[kWinCells];
   // (chunk, channel) of this workgroup: the nc channels of one chunk go to
@@ -764,7 +785,7 @@ bin_accum_kernel(const float4 *__restrict__ spos, const float *__restrict__ weig
   if (hit) atomicOr(nonfinite, 1u);
   __syncthreads();
   write_window(win, d, t, itx, ity, itz, scale, (size_t(c) * nc + ch) * kWinCells, partial,
-                    mesh + size_t(ch) * M + cell0, accumulate);
+                    mesh + size_t(ch) * M + cell0, base ? base + size_t(ch) * M + cell0 : nullptr);
 }
 
 // --------------------------------------------------------------- reduce
@@ -791,7 +812,7 @@ __global__ void __launch_bounds__(kReduceThreads)
 bin_reduce_kernel(const float *__restrict__ partial, const uint32_t *__restrict__ chunk_off,
                   const uint32_t *__restrict__ nchunk, G g, uint32_t M, int nc, const float *__restrict__ overflow,
                   const float *__restrict__ wmax_dev, float wmax_host, int has_w, uint32_t n,
-                  int accumulate, float *__restrict__ mesh, uint32_t K, uint32_t per, bool slabs,
+                  const float *base, float *mesh, uint32_t K, uint32_t per, bool slabs,
                   const uint32_t *__restrict__ nonfinite, const uint32_t *__restrict__ outside,
                   const float4 *__restrict__ spos,
                   const ChunkDesc *__restrict__ desc, const float *__restrict__ weight, float wscalar,
@@ -859,7 +880,7 @@ bin_reduce_kernel(const float *__restrict__ partial, const uint32_t *__restrict_
       dsts[i] = mesh + size_t(ch) * M + cell;
       // the tile's own deposits: from its slot, or, when the paint adds to
       // the mesh, the mesh value the accumulation already added them to
-      h[i][0] = accumulate ? *dsts[i] : own[e];
+      h[i][0] = base ? *dsts[i] : own[e];
 #pragma unroll
       for (int k = 1; k < 8; ++k) {
         const int sx = k >> 2, sy = (k >> 1) & 1, sz = k & 1;
@@ -911,7 +932,7 @@ bin_reduce_kernel(const float *__restrict__ partial, const uint32_t *__restrict_
       // a full single-chunk tile keeps its own face cells in its slot too
       float acc = 0.0f;
       if (faces_only)
-        acc = full && !accumulate ? partial[(size_t(src_off[0]) * nc + ch) * kWinCells * 2 + kH + e] : *dst;
+        acc = full && !base ? partial[(size_t(src_off[0]) * nc + ch) * kWinCells * 2 + kH + e] : *dst;
       const int nxs = a == 0 ? 2 : 1, nys = b == 0 ? 2 : 1, nzs = c == 0 ? 2 : 1;
       for (int sx = 0; sx < nxs; ++sx)
         for (int sy = 0; sy < nys; ++sy)
@@ -942,7 +963,7 @@ bin_reduce_kernel(const float *__restrict__ partial, const uint32_t *__restrict_
       if (fbt && (a == 0 || b == 0 || c == 0))
         fbt[face_index(a, b, c)] = acc;
       else
-        *dst = accumulate ? *dst + acc : acc;
+        *dst = base ? base[size_t(ch) * M + cell] + acc : acc;
     }
   }
   float *meshc = mesh + size_t(ch) * M + cell0;
@@ -1024,9 +1045,21 @@ static int set_lds(K kernel, size_t bytes) {
 // workgroups of `slice` particles, chunk-table capacity, and the largest
 // per-simulation tile count (the LDS histogram size).
 struct SortDims {
-  uint32_t K, n, G, slice, chunk, maxchunks, maxK, B;
+  uint32_t K, n, G, slice, chunk, maxchunks, maxK, B, groups = 1;
   bool slabs;
 };
+
+// Ranges of a tile's records that the slices of one XCD (workgroup index mod
+// 8) fill each.  Particles in no order leave a tile two records a slice, and
+// with one range for all, neighbouring records of a cache line came from
+// different XCDs, whose L2s each wrote a part of it.  256^3
+// particles: scatter 259 -> 212 us, count 84 -> 69 (its atomics meet less),
+// tile table 5 -> 8; paint of 2^22 on 164^3 127 -> 115 us.  In lattice order,
+// with long runs per tile, 2^22 on 200^3 119 and 121.
+constexpr uint32_t kGroupMaxK = 8192;
+static uint32_t sort_groups(uint32_t flags, int64_t n, uint32_t K) {
+  return !(flags & kSortOrdered) && n >= (int64_t(1) << 22) && K <= kGroupMaxK ? kSortGroups : 1u;
+}
 
 static SortDims one_dims(const TileGrid &t, int64_t n, uint32_t flags) {
   SortDims d;
@@ -1040,6 +1073,7 @@ static SortDims one_dims(const TileGrid &t, int64_t n, uint32_t flags) {
   d.maxK = t.K;
   d.B = 1;
   d.slabs = tuned_slabs(flags);
+  d.groups = sort_groups(flags, n, t.K);
   return d;
 }
 
@@ -1053,9 +1087,9 @@ static SortWs sort_ws(const SortDims &d) {
   const size_t nn = size_t(d.n > 0 ? d.n : 1);
   const size_t nsums = (size_t(d.K) + kScanBlock - 1) / kScanBlock + 1;
   size_t o = 0;
-  w.count = o;    o += align_up(size_t(d.K) * 4);
+  w.count = o;    o += align_up(size_t(d.K) * d.groups * 4);
   w.tstart = o;   o += align_up(size_t(d.K) * 4);
-  w.cursor = o;   o += align_up(size_t(d.K) * 4);
+  w.cursor = o;   o += align_up(size_t(d.K) * d.groups * 4);
   w.nchunk = o;   o += align_up(size_t(d.K) * 4);
   w.choff = o;    o += align_up(size_t(d.K) * 4);
   w.sums = o;     o += align_up(nsums * 4);
@@ -1066,13 +1100,19 @@ static SortWs sort_ws(const SortDims &d) {
   return w;
 }
 
+// Whether the marks of the tiles with relative corners outside their window (a
+// word per tile) fit the windows of the last chunk, which no chunk has: the
+// tiles' chunks, each less than its particles over the chunk size plus one,
+// add up to less than maxchunks.
+static bool marks_fit(uint32_t K, int nc) { return size_t(K) * 4 + 256 <= size_t(nc) * kWinCells * 8; }
+
 // Workspace of the window accumulation that follows a sort.
 static size_t accum_ws(const SortDims &d, size_t M, int nc, bool rel, size_t *partial, size_t *overflow,
                        size_t *wmax) {
   size_t o = 0;
   *partial = o;  o += align_up(size_t(d.maxchunks) * nc * kWinCells * 8);
-  // the overflow mesh and a word per tile whether it holds anything there
-  *overflow = o; o += rel ? align_up((size_t(nc) * M + d.K) * 4) : 0;
+  // the overflow mesh; the marks right before it, or else behind it
+  *overflow = o; o += rel ? align_up((size_t(nc) * M + (marks_fit(d.K, nc) ? 0 : d.K)) * 4) : 0;
   *wmax = o;     o += align_up(4);
   return o;
 }
@@ -1131,7 +1171,7 @@ Bins bins_view(int nx, int ny, int nz, int64_t n, uint32_t flags, const void *ws
 // particles.
 template <class G>
 struct ScatterReg {
-  void (*kern)(const float *, uint32_t, G, uint32_t *, float4 *);
+  void (*kern)(const float *, uint32_t, G, uint32_t *, float4 *, uint32_t);
   unsigned threads;
 };
 
@@ -1168,13 +1208,15 @@ static int sort_into(hipStream_t s, const G &g, const SortDims &d, uint32_t M, b
   uint32_t *sums = reinterpret_cast<uint32_t *>(base + w.sums);
   uint32_t *totals = reinterpret_cast<uint32_t *>(base + w.totals);  // [0] particles, [1] chunks
   const size_t lds_hist = size_t(d.maxK) * 4;
+  const uint32_t groups = lds && !counts_in && scatter_reg_ok(d.slice) && d.K <= kTableMaxK ? d.groups : 1u;
+  const uint32_t gstride = groups > 1 ? d.K : 0u;
   int rc;
 
   // 1. tile counts
   if (counts_in) {
     count = const_cast<uint32_t *>(counts_in);   // only read below
   } else {
-    hipLaunchKernelGGL(zero_u32_kernel, dim3(grid_for(d.K, 256)), dim3(256), 0, s, count, d.K);
+    hipLaunchKernelGGL(zero_u32_kernel, dim3(grid_for(d.K * groups, 256)), dim3(256), 0, s, count, d.K * groups);
     JPM_LAUNCHED("zero_u32_kernel");
     if (lds) {
       auto kern = rel ? bin_count_kernel<true, G> : bin_count_kernel<false, G>;
@@ -1188,7 +1230,8 @@ static int sort_into(hipStream_t s, const G &g, const SortDims &d, uint32_t M, b
       uint32_t shift = 0;
       while ((d.G << shift) < 256u && (d.slice >> (shift + 1)) >= uint32_t(kBinThreads))
         ++shift;
-      hipLaunchKernelGGL(kern, dim3(d.G << shift), dim3(kBinThreads), lds_hist, s, pos, d.slice, shift, g, count);
+      hipLaunchKernelGGL(kern, dim3(d.G << shift), dim3(kBinThreads), lds_hist, s, pos, d.slice, shift, g, count,
+                         gstride);
       JPM_LAUNCHED("bin_count_kernel");
     } else {
       auto kern = rel ? bin_count_global_kernel<true, G> : bin_count_global_kernel<false, G>;
@@ -1200,7 +1243,7 @@ static int sort_into(hipStream_t s, const G &g, const SortDims &d, uint32_t M, b
   // 2. tile starts, scatter cursors, chunk table
   if (d.K <= kTableMaxK) {
     rc = tile_table(s, count, d.K, d.chunk, tstart, cursor, nchunk, choff, totals,
-                    reinterpret_cast<ChunkDesc *>(base + w.desc));
+                    reinterpret_cast<ChunkDesc *>(base + w.desc), groups);
     if (rc) return rc;
   } else {
     JPM_HIP(hipMemcpyAsync(tstart, count, size_t(d.K) * 4, hipMemcpyDeviceToDevice, s));
@@ -1225,7 +1268,7 @@ static int sort_into(hipStream_t s, const G &g, const SortDims &d, uint32_t M, b
     if (rc) return rc;
     JPM_TIMED(s, "bin_scatter_kernel");
     hipLaunchKernelGGL(v.kern, dim3(d.G), dim3(v.threads), lds_hist, s, pos, d.slice, g,
-                       cursor, reinterpret_cast<float4 *>(base + w.spos));
+                       cursor, reinterpret_cast<float4 *>(base + w.spos), gstride);
     JPM_LAUNCHED("bin_scatter_reg_kernel");
   } else if (lds) {
     auto kern = rel ? bin_scatter_kernel<true, G> : bin_scatter_kernel<false, G>;
@@ -1288,7 +1331,7 @@ template int bins_order<SimTable>(hipStream_t, const BatchBins &, uint32_t *);
 template <class G>
 static int paint_sorted(hipStream_t s, const BinsT<G> &b, const float *weight, float wscalar, int nc, float *mesh,
                         uint32_t flags, void *ws, size_t ws_bytes, const float *wmax_in = nullptr,
-                        const FaceCells *faces = nullptr) {
+                        const FaceCells *faces = nullptr, const float *base_mesh = nullptr) {
   SortDims d{};
   d.maxchunks = b.maxchunks;
   d.K = b.K;
@@ -1299,17 +1342,23 @@ static int paint_sorted(hipStream_t s, const BinsT<G> &b, const float *weight, f
   size_t opart, oover, owmax;
   const size_t need = accum_ws(d, size_t(M), nc, b.rel, &opart, &oover, &owmax);
   JPM_REQUIRE(ws && ws_bytes >= need, "binned paint needs %zu workspace bytes, got %zu", need, ws_bytes);
-  const bool accumulate = !(flags & JPM_ZERO_MESH);
+  // what the deposits are added to: nothing, or a mesh (the output by default)
+  const float *onto = (flags & JPM_ZERO_MESH) ? nullptr : base_mesh ? base_mesh : mesh;
   const FaceCells fc = faces ? *faces : FaceCells{nullptr, 0, 0, 0, 0, FastDiv(1)};
-  JPM_REQUIRE(!fc.fb || (!b.rel && !accumulate && size_t(b.K) * kFaceStride <= fc.chan),
+  JPM_REQUIRE(!fc.fb || (!b.rel && !onto && size_t(b.K) * kFaceStride <= fc.chan),
               "face cells apart need absolute positions, a replaced mesh and room for every tile");
   char *base = static_cast<char *>(ws);
+  float *overflow = reinterpret_cast<float *>(base + oover);
+  const bool outside_before = marks_fit(b.K, nc);
+  uint32_t *outside =
+      reinterpret_cast<uint32_t *>(b.rel ? (outside_before ? overflow - b.K : overflow + nc * M) : overflow);
   int rc;
   if (b.rel) {
     // one launch for both while its 32-bit count allows
     const bool both = nc * M + b.K < (int64_t(1) << 32);
-    rc = zero_f32(s, reinterpret_cast<float *>(base + oover), both ? nc * M + b.K : nc * M);
-    if (!rc && !both) rc = zero_f32(s, reinterpret_cast<float *>(base + oover) + nc * M, b.K);
+    float *first = outside_before ? overflow - b.K : overflow;
+    rc = zero_f32(s, both ? first : overflow, both ? nc * M + b.K : nc * M);
+    if (!rc && !both) rc = zero_f32(s, reinterpret_cast<float *>(outside), b.K);
     if (rc) return rc;
   }
   const float wmax_host = finite_abs(wscalar);
@@ -1319,8 +1368,6 @@ static int paint_sorted(hipStream_t s, const BinsT<G> &b, const float *weight, f
   }
   auto *partial = reinterpret_cast<float *>(base + opart);
   const float *wmax_dev = wmax_in ? wmax_in : reinterpret_cast<const float *>(base + owmax);
-  float *overflow = reinterpret_cast<float *>(base + oover);
-  uint32_t *outside = reinterpret_cast<uint32_t *>(overflow + (b.rel ? nc * M : 0));
   {
     JPM_TIMED(s, nc == 1 ? "bin_accum_kernel[nc=1]" : "bin_accum_kernel[nc=3]");
     auto kern = b.rel ? bin_accum_kernel<true, G> : bin_accum_kernel<false, G>;
@@ -1328,7 +1375,7 @@ static int paint_sorted(hipStream_t s, const BinsT<G> &b, const float *weight, f
     (void)slab_grid(b.maxchunks, b.slabs, per);
     const unsigned grid = 8u * per * unsigned(nc);
     hipLaunchKernelGGL(kern, dim3(grid), dim3(kWindowThreads), 0, s, b.spos, weight, nc, wscalar, b.desc,
-                       b.total_chunks, b.g, b.M, wmax_dev, wmax_host, b.n, partial, overflow, int(accumulate), mesh,
+                       b.total_chunks, b.g, b.M, wmax_dev, wmax_host, b.n, partial, overflow, onto, mesh,
                        per, b.slabs, b.nonfinite, outside);
   }
   JPM_LAUNCHED("bin_accum_kernel");
@@ -1341,7 +1388,7 @@ static int paint_sorted(hipStream_t s, const BinsT<G> &b, const float *weight, f
     uint32_t per;
     const unsigned grid = slab_grid(b.K, true, per);
     hipLaunchKernelGGL(kern, dim3(grid, nc), dim3(kReduceThreads), 0, s, partial, b.choff, b.nchunk, b.g, b.M, nc, overflow,
-                       wmax_dev, wmax_host, int(weight != nullptr), b.n, int(accumulate), mesh, b.K, per,
+                       wmax_dev, wmax_host, int(weight != nullptr), b.n, onto, mesh, b.K, per,
                        true, b.nonfinite, outside, b.spos, b.desc, weight, wscalar, fc);
   }
   JPM_LAUNCHED("bin_reduce_kernel");
@@ -1349,12 +1396,13 @@ static int paint_sorted(hipStream_t s, const BinsT<G> &b, const float *weight, f
 }
 
 int bins_paint(hipStream_t s, const Bins &b, const float *weight, float wscalar, int nc, float *mesh, uint32_t flags,
-               void *ws, size_t ws_bytes, const float *wmax_in, const FaceCells *faces) {
-  return paint_sorted(s, b, weight, wscalar, nc, mesh, flags, ws, ws_bytes, wmax_in, faces);
+               void *ws, size_t ws_bytes, const float *wmax_in, const FaceCells *faces, const float *base_mesh) {
+  return paint_sorted(s, b, weight, wscalar, nc, mesh, flags, ws, ws_bytes, wmax_in, faces, base_mesh);
 }
 
 int binned_paint(hipStream_t s, int nx, int ny, int nz, const float *pos, int64_t n, const float *weight,
-                 float wscalar, int nc, float *mesh, uint32_t flags, void *ws, size_t ws_bytes) {
+                 float wscalar, int nc, float *mesh, uint32_t flags, void *ws, size_t ws_bytes,
+                 const float *base_mesh) {
   int rc = check_dims(nx, ny, nz);
   if (rc) return rc;
   JPM_REQUIRE(nc == 1 || nc == 3, "binned paint supports 1 or 3 channels (got %d)", nc);
@@ -1366,6 +1414,8 @@ int binned_paint(hipStream_t s, int nx, int ny, int nz, const float *pos, int64_
   JPM_REQUIRE(ws && ws_bytes >= need, "binned paint needs %zu workspace bytes, got %zu", need, ws_bytes);
   if (n == 0) {
     if (flags & JPM_ZERO_MESH) return zero_f32(s, mesh, nc * M);
+    if (base_mesh && base_mesh != mesh)
+      JPM_HIP(hipMemcpyAsync(mesh, base_mesh, size_t(nc) * M * 4, hipMemcpyDeviceToDevice, s));
     return JPM_OK;
   }
   const size_t sort_bytes = align_up(bin_sort_workspace_size(nx, ny, nz, n, flags));
@@ -1373,7 +1423,7 @@ int binned_paint(hipStream_t s, int nx, int ny, int nz, const float *pos, int64_
   rc = bin_sort(s, nx, ny, nz, pos, n, flags, ws, sort_bytes, b);
   if (rc) return rc;
   return bins_paint(s, b, weight, wscalar, nc, mesh, flags, static_cast<char *>(ws) + sort_bytes, ws_bytes - sort_bytes,
-                    nullptr);
+                    nullptr, nullptr, base_mesh);
 }
 
 // ------------------------------------------------------------- batches

@@ -159,7 +159,7 @@ static int force_meshes(hipStream_t s, int nx, int ny, int nz, const void *delta
   return fd4_gradient(s, nx, ny, nz, tmp_mesh, 1.0f, phi3);
 }
 int binned_paint(hipStream_t, int, int, int, const float *, int64_t, const float *, float, int, float *, uint32_t,
-                 void *, size_t);
+                 void *, size_t, const float * = nullptr);
 size_t binned_paint_workspace_size(int, int, int, int64_t, int, uint32_t);
 bool binned_paint_supported(int, int, int);
 
@@ -1159,6 +1159,14 @@ size_t jpm_cic_paint_binned_workspace_size(int nx, int ny, int nz, int64_t n, in
 int jpm_cic_paint_binned_f32(void *stream, int nx, int ny, int nz, const float *pos, int64_t n, const float *weights,
                              float wscalar, int nc, float *mesh, uint32_t flags, void *ws, size_t ws_bytes) {
   JPM_GUARD(binned_paint(as_stream(stream), nx, ny, nz, pos, n, weights, wscalar, nc, mesh, flags, ws, ws_bytes));
+}
+
+int jpm_cic_paint_onto_f32(void *stream, int nx, int ny, int nz, const float *base, const float *pos, int64_t n,
+                           const float *weights, float wscalar, float *mesh, uint32_t flags, void *ws,
+                           size_t ws_bytes) {
+  if (!base) return fail(JPM_E_INVALID, "base is null");
+  JPM_GUARD(binned_paint(as_stream(stream), nx, ny, nz, pos, n, weights, wscalar, 1, mesh, flags & ~JPM_ZERO_MESH, ws,
+                         ws_bytes, base));
 }
 
 int jpm_pm_forces_f32(void *stream, int nx, int ny, int nz, const float *pos, int64_t n, const void *delta_k,

@@ -9,7 +9,7 @@
 namespace jpm {
 
 int binned_paint(hipStream_t, int, int, int, const float *, int64_t, const float *, float, int, float *, uint32_t,
-                 void *, size_t);
+                 void *, size_t, const float * = nullptr);
 size_t binned_paint_workspace_size(int, int, int, int64_t, int, uint32_t);
 bool binned_paint_supported(int, int, int);
 

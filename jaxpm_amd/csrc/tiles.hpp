@@ -297,7 +297,7 @@ struct ChunkDesc {
 // cursors, chunks per tile and their offsets, totals [particles, chunks, 0]
 // and the chunk descriptors.
 int tile_table(hipStream_t s, const uint32_t *count, uint32_t K, uint32_t chunk, uint32_t *tstart, uint32_t *cursor,
-               uint32_t *nchunk, uint32_t *choff, uint32_t *totals, ChunkDesc *desc);
+               uint32_t *nchunk, uint32_t *choff, uint32_t *totals, ChunkDesc *desc, uint32_t groups = 1);
 
 // One simulation as the tile-sort kernels see it.  A batch concatenates its
 // simulations: particles [part0, part0 + n) of the positions, tiles
@@ -394,7 +394,8 @@ int batch_sort(hipStream_t s, const SimBatch &bt, const float *pos, void *ws, si
                const uint32_t *counts_in = nullptr);
 int zero_u32(hipStream_t s, uint32_t *p, uint32_t n);
 int bins_paint(hipStream_t s, const Bins &b, const float *weight, float wscalar, int nc, float *mesh, uint32_t flags,
-               void *ws, size_t ws_bytes, const float *wmax_in = nullptr, const FaceCells *faces = nullptr);
+               void *ws, size_t ws_bytes, const float *wmax_in = nullptr, const FaceCells *faces = nullptr,
+               const float *base_mesh = nullptr);
 // The potential solves (kspace.hip); faces: the painted mesh's face cells
 // kept apart, on the shapes potential_faces_ok accepts, for a one-mesh solve.
 bool potential_faces_ok(int nx, int ny, int nz);

@@ -448,3 +448,49 @@ def test_read_cotangents_from_one_sort(gpu, shape, n, nc):
     direct = _ops.grad_pos(meshes, p, cot=cot)
     assert torch.equal(gp.isnan(), direct.isnan()) and torch.equal(gp.nan_to_num(), direct.nan_to_num())
     assert torch.equal(gm.isnan(), _ops.paint_multi(shape, p, cot).isnan())
+
+
+@pytest.mark.parametrize("n", [(1 << 22) - 1, (1 << 22) + 4097])
+def test_paint_of_many_particles_is_exact(gpu, n):
+    """Both sides of the count from which each XCD's slices fill their own part
+    of a tile: coordinates are multiples of 1/8 and weights small integers, so
+    the mesh has to equal the float64 sum."""
+    from jaxpm_amd import _ops
+    shape = (40, 33, 50)
+    print(f"many particles {n}", flush=True)
+    r = np.random.default_rng(48)
+    pos = r.integers(0, np.array(shape) * 8, size=(n, 3), dtype=np.int32)
+    w = r.integers(-4, 5, size=n).astype(np.float32)
+    f, u = pos >> 3, (pos & 7) / 8.0
+    ref = np.zeros(int(np.prod(shape)))
+    for o in range(8):
+        b = np.array([o & 1, (o >> 1) & 1, (o >> 2) & 1])
+        c = (f + b) % np.array(shape)
+        wt = np.prod(np.where(b, u, 1.0 - u), axis=1) * w
+        ref += np.bincount((c[:, 0] * shape[1] + c[:, 1]) * shape[2] + c[:, 2], wt, ref.size)
+    p = dev(pos / 8.0)
+    got = _ops.paint(torch.empty(shape, device="cuda"), p, weight=dev(w), zero=True)
+    assert np.array_equal(host(got).reshape(-1), ref)
+    vals = dev(r.normal(size=shape))
+    assert torch.equal(_ops.read(vals, p, method="sorted"), _ops.read(vals, p))
+
+
+@pytest.mark.parametrize("shape,n", [((16, 16, 16), 4096), ((20, 33, 17), 3000), ((64, 48, 40), 60000),
+                                     ((32, 32, 32), 0)])
+@pytest.mark.parametrize("relative", [False, True])
+def test_paint_onto_a_mesh(gpu, shape, n, relative):
+    """mesh + paint in one pass has the bits of painting a copy, and leaves the
+    mesh; tiles of no, one and several chunks, full and partial."""
+    from jaxpm_amd import _ops
+    if relative and n != int(np.prod(shape)):
+        n = int(np.prod(shape))
+    print(f"paint onto {shape} n={n} relative={relative}", flush=True)
+    r = np.random.default_rng(49)
+    pos = (r.uniform(0, 1, size=(n, 3)) * np.array(shape)).astype(np.float32)
+    if shape[0] == 64 and not relative:
+        pos[:40000] = 20 + r.uniform(0, 8, size=(40000, 3))
+    base, p, w = dev(r.normal(size=shape)), dev(pos), dev(r.normal(size=n))
+    keep = base.clone()
+    got = _ops.paint_onto(base, p, weight=w, relative=relative)
+    assert torch.equal(base, keep)
+    assert torch.equal(got, _ops.paint(keep, p, weight=w, relative=relative))
