@@ -568,6 +568,11 @@ int jpm_dot_f32(void *stream, int64_t n, const float *x, const float *y,
  * of the leapfrog built on make_ode_fn (ode.py:139-140) and its adjoint. */
 int jpm_axpy_f32(void *stream, int64_t n, float a, const float *x, float *y);
 
+/* jpm_axpy_f32, then ykeep = y and xkeep = x: a drift whose positions and
+ * velocities an adjoint keeps. */
+int jpm_axpy_keep_f32(void *stream, int64_t n, float a, const float *x,
+                      float *y, float *ykeep, float *xkeep);
+
 /* ------------------------------------------------------- lens planes */
 
 /* mesh[nx][ny] += the weighted 2-D CIC deposits of n particles whose (x, y)

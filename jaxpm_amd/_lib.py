@@ -132,6 +132,7 @@ SIGNATURES = {
     "jpm_tile_count": (_sz, [_i, _i, _i]),
     "jpm_force_vjp_pot_drift_f32": (_i, [_vp, _i, _i, _i, _vp, _vp, _i64, _vp, _f, _f, _vp, _f, _u32, _vp, _sz, _vp,
                                          _sz, _vp, _vp]),
+    "jpm_axpy_keep_f32": (_i, [_vp, _i64, _f, _vp, _vp, _vp, _vp]),
     "jpm_axpy_f32": (_i, [_vp, _i64, _f, _vp, _vp]),
     "jpm_cic_paint_2d_f32": (_i, [_vp, _i, _i, _vp, _i64, _i, _vp, _vp]),
     "jpm_cic_paint_2d_vjp_f32": (_i, [_vp, _i, _i, _vp, _i64, _i, _vp, _vp, _vp, _i, _vp]),

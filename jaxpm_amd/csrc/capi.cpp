@@ -119,6 +119,7 @@ int power_spectrum(hipStream_t, int, int, int, const void *, const void *, doubl
                    int, const int *, int, double, double, double, double *, void *, size_t);
 
 int axpy(hipStream_t, int64_t, float, const float *, float *);
+int axpy_keep(hipStream_t, int64_t, float, const float *, float *, float *, float *);
 int permute_rows(hipStream_t, int64_t, const uint32_t *, const float *, float *, const float *, float *, int);
 int paint_2d(hipStream_t, int, int, const float *, int64_t, int, const float *, float *);
 int paint_2d_vjp(hipStream_t, int, int, const float *, int64_t, int, const float *, const float *, float *, int,
@@ -1022,6 +1023,10 @@ int jpm_force_vjp_f32(void *stream, int nx, int ny, int nz, const float *phi3, c
 
 int jpm_axpy_f32(void *stream, int64_t n, float a, const float *x, float *y) {
   JPM_GUARD(axpy(as_stream(stream), n, a, x, y));
+}
+
+int jpm_axpy_keep_f32(void *stream, int64_t n, float a, const float *x, float *y, float *ykeep, float *xkeep) {
+  JPM_GUARD(axpy_keep(as_stream(stream), n, a, x, y, ykeep, xkeep));
 }
 
 int jpm_cic_paint_2d_f32(void *stream, int nx, int ny, const float *pos, int64_t n, int stride,

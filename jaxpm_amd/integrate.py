@@ -252,6 +252,11 @@ class Stepper:
     def axpy(self, a, x, y):
         self._timed("axpy", "jpm_axpy_f32", stream(), 3 * self.n, float(a), ptr(x), ptr(y))
 
+    def drift_keep(self, a, v, x, xkeep, vkeep):
+        """x += a v, then copies of the new x and of v, in one launch."""
+        self._timed("axpy", "jpm_axpy_keep_f32", stream(), 3 * self.n, float(a), ptr(v), ptr(x), ptr(xkeep),
+                    ptr(vkeep))
+
     def vjp(self, phi, x, cot, scale, gpos):
         self._ensure_ws("jpm_force_vjp_workspace_size")
         self._timed("vjp", "jpm_force_vjp_f32", stream(), self.nx, self.ny, self.nz, ptr(phi), ptr(x), self.n,
@@ -282,16 +287,17 @@ def _run(stepper, x, v, k0, beta, gamma, start, stop, phi, keep=None, forces=Fal
     forces it kicked with (v += gamma F as forces-then-axpy, the same float
     operations as the fused kick)."""
     for i in range(start, stop):
+        if keep is not None and forces:
+            kp = keep[i - start]
+            stepper.drift_keep(beta[i], v, x, kp[0], kp[2])
+            stepper.forces(x, kp[3], kp[1])
+            stepper.axpy(gamma[i], kp[3], v)
+            continue
         stepper.axpy(beta[i], v, x)
         if keep is not None:
             kp = keep[i - start]
             kp[0].copy_(x)
             phi = kp[1]
-            if forces:
-                kp[2].copy_(v)
-                stepper.forces(x, kp[3], phi)
-                stepper.axpy(gamma[i], kp[3], v)
-                continue
         stepper.field_kick(x, v, gamma[i], phi)
 
 

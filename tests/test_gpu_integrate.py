@@ -309,3 +309,17 @@ def test_kick_drift_velocity_out_and_field_only(gpu):
     torch.cuda.synchronize()
     assert torch.equal(f_c[0], f_d[0])
     assert not torch.equal(v_d, v_in)
+
+
+@pytest.mark.parametrize("n", [1, 3, 4, 1023, 4096])
+def test_axpy_keep(gpu, n):
+    """The drift that keeps its operands: the bits of an axpy and two copies,
+    with and without a tail of fewer than four floats."""
+    from jaxpm_amd import _ops
+    from jaxpm_amd._lib import call, ptr, stream
+    r = np.random.default_rng(70)
+    x, y = [torch.as_tensor(r.normal(size=n).astype(np.float32), device="cuda") for _ in range(2)]
+    want = _ops.axpy(0.37, x, y.clone())
+    xk, yk = torch.full_like(x, 7.0), torch.full_like(x, 7.0)
+    call("jpm_axpy_keep_f32", stream(), n, 0.37, ptr(x), ptr(y), ptr(yk), ptr(xk))
+    assert torch.equal(y, want) and torch.equal(yk, want) and torch.equal(xk, x)
