@@ -847,7 +847,8 @@ def main():
                                f"2LPT IC at a=0.1, {args.steps} steps to a=1, checkpoint every {args.checkpoint}",
                    "mesh": n, "particles": N, "checkpoint_every": args.checkpoint,
                    "sort_tuning": {"chunk": 2 ** (9 + tuning[0]) if tuning[0] else 8192,
-                                   "slice": 2 ** (11 + tuning[1]) if tuning[1] else 8192,
+                                   "slice": 2 ** (11 + tuning[1]) if tuning[1] else
+                                   (4096 if N >= 2 ** 19 else 2048 if N >= 2 ** 17 else 1024),
                                    "vjp_density_window": "caches" if len(tuning) > 2 and tuning[2] else "lds",
                                    "xcd_placement": "slabs" if len(tuning) > 3 and tuning[3] else
                                    "round-robin (accumulation), runs of 32 chunks (gathers)"}},
