@@ -1055,10 +1055,12 @@ struct SortDims {
 // different XCDs, whose L2s each wrote a part of it.  256^3
 // particles: scatter 259 -> 212 us, count 84 -> 69 (its atomics meet less),
 // tile table 5 -> 8; paint of 2^22 on 164^3 127 -> 115 us.  In lattice order,
-// with long runs per tile, 2^22 on 200^3 119 and 121.
+// with long runs per tile, 2^22 on 200^3 119 and 121.  pm_forces of 256^3
+// particles (slices of 4096): in no order 989 -> 879 us, in their lattice's 522
+// and 522.
 constexpr uint32_t kGroupMaxK = 8192;
-static uint32_t sort_groups(uint32_t flags, int64_t n, uint32_t K) {
-  return !(flags & kSortOrdered) && n >= (int64_t(1) << 22) && K <= kGroupMaxK ? kSortGroups : 1u;
+static uint32_t sort_groups(int64_t n, uint32_t K) {
+  return n >= (int64_t(1) << 22) && K <= kGroupMaxK ? kSortGroups : 1u;
 }
 
 static SortDims one_dims(const TileGrid &t, int64_t n, uint32_t flags) {
@@ -1066,14 +1068,14 @@ static SortDims one_dims(const TileGrid &t, int64_t n, uint32_t flags) {
   const uint64_t nn = uint64_t(n > 0 ? n : 1);
   d.K = t.K;
   d.n = uint32_t(n);
-  d.slice = tuned_slice(flags, n, flags & kSortOrdered);
+  d.slice = tuned_slice(flags, n, flags & kSortForces);
   d.chunk = tuned_chunk(flags);
   d.G = uint32_t((nn + d.slice - 1) / d.slice);
   d.maxchunks = uint32_t((nn + d.chunk - 1) / d.chunk + t.K);
   d.maxK = t.K;
   d.B = 1;
   d.slabs = tuned_slabs(flags);
-  d.groups = sort_groups(flags, n, t.K);
+  d.groups = sort_groups(n, t.K);
   return d;
 }
 

@@ -259,7 +259,7 @@ static int force_kick(hipStream_t s, int nx, int ny, int nz, const float *pos, i
   if (rc) return rc;
   JPM_REQUIRE(!xout || !write_forces, "the fused drift follows a kick, not a force write");
   JPM_REQUIRE(!counts_out || (xout && !(flags & JPM_RELATIVE)), "tile counts of drifted absolute positions only");
-  const uint32_t pflags = paint_flags(flags) | kSortOrdered, kflags = kspace_flags(flags);
+  const uint32_t pflags = paint_flags(flags) | kSortForces, kflags = kspace_flags(flags);
   JPM_REQUIRE(sorted_supported(nx, ny, nz, flags), "the sorted pipeline needs the 4-point gradient, the binned paint and 3 meshes within 2^32 cells");
   JPM_REQUIRE(n >= 1, "no particles");
   JPM_REQUIRE(pos && phi, "null pointer argument");
@@ -371,7 +371,7 @@ static int force_vjp_pot(hipStream_t s, int nx, int ny, int nz, const float *phi
                          float *cot_out = nullptr, const float *cot_max_in = nullptr, float *cot_max_out = nullptr) {
   int rc = check_dims(nx, ny, nz);
   if (rc) return rc;
-  const uint32_t pflags = paint_flags(flags) | kSortOrdered, kflags = kspace_flags(flags);
+  const uint32_t pflags = paint_flags(flags) | kSortForces, kflags = kspace_flags(flags);
   JPM_REQUIRE(sorted_supported(nx, ny, nz, flags), "the sorted pipeline needs the 4-point gradient, the binned paint and 3 meshes within 2^32 cells");
   JPM_REQUIRE(n >= 1, "no particles");
   JPM_REQUIRE(phi && pos && cot && gpos, "null pointer argument");

@@ -85,19 +85,21 @@ __device__ __forceinline__ uint32_t gather_item(uint32_t b, uint32_t per, bool s
 // Particles per count / scatter workgroup of a sort of n particles.  Slices
 // that narrow with n keep a few hundred workgroups on the chip (a slice of
 // 8192 is 4 workgroups at 32^3, which take 11 us for a 2 us scatter); wide
-// ones write longer runs per tile, which is what particles in no order need
-// (256^3 random: paint 471 us, 520 with slices of 4096).  A simulation's
-// particles (`ordered`) are in the order of their lattice or of their tiles,
-// and take slices of 4096 at every size (192^3 relative forces 420 -> 402 us).
-inline uint32_t tuned_slice(uint32_t flags, int64_t n, bool ordered = false) {
+// ones write longer runs per tile, which is what a paint of particles in no
+// order needs.  The force pipelines (`forces`), whose particles are mostly in
+// the order of their lattice or of their tiles, take slices of 4096 from 2^19
+// particles on (192^3 relative forces 420 -> 402 us; pm_forces at 164^3, 224^3
+// and 256^3, slices of 8192 and 4096 us: lattice order 457 and 442, 521 and
+// 510, 538 and 522, no order 536 and 521, 739 and 729, 866 and 879).
+inline uint32_t tuned_slice(uint32_t flags, int64_t n, bool forces = false) {
   const uint32_t v = (flags >> 20) & 0xfu;
   if (v >= 1 && v <= 7) return 1u << (11 + v);
   if (n < (int64_t(1) << 17)) return 1024;
   if (n < (int64_t(1) << 19)) return 2048;
-  return ordered || n < (int64_t(1) << 22) ? 4096 : kSlice;
+  return forces || n < (int64_t(1) << 22) ? 4096 : kSlice;
 }
-// Bit 27, set inside the force pipelines: the particles are `ordered`.
-constexpr uint32_t kSortOrdered = 1u << 27;
+// Bit 27, set inside the force pipelines.
+constexpr uint32_t kSortForces = 1u << 27;
 
 // A tile's low-face cells (lx = 0, or ly = 0, or lz = 0), numbered in face
 // order: the lx = 0 plane (ly * 16 + lz), then ly = 0 with lx > 0

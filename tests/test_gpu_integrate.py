@@ -323,3 +323,49 @@ def test_axpy_keep(gpu, n):
     xk, yk = torch.full_like(x, 7.0), torch.full_like(x, 7.0)
     call("jpm_axpy_keep_f32", stream(), n, 0.37, ptr(x), ptr(y), ptr(yk), ptr(xk))
     assert torch.equal(y, want) and torch.equal(yk, want) and torch.equal(xk, x)
+
+
+@pytest.mark.parametrize("relative", [False, True])
+def test_force_sort_fills_tiles_by_xcd(gpu, relative):
+    """From 2^22 particles the sort of a force evaluation, which cannot know
+    their order, gives the slices of each XCD (4096 particles, slice index
+    mod 8) a run of their own in every tile; its kept sort serves the force
+    VJP as a sort of the VJP's own does, and neither changes a bit."""
+    from jaxpm_amd import _lib, integrate
+    shape = (164, 164, 156)
+    n = int(np.prod(shape))
+    print(f"force sort by XCD, relative={relative}", flush=True)
+    assert n >= 2 ** 22
+    gen = torch.Generator(device="cuda").manual_seed(5)
+    dims = torch.tensor(shape, dtype=torch.float32, device="cuda")
+    if relative:
+        # eighths of a cell: exact sums, no corner dropped by rounding
+        x = torch.round(24.0 * torch.randn((n, 3), generator=gen, device="cuda")) / 8
+        lat = torch.as_tensor(lattice(shape).astype(np.float32), device="cuda")
+        cell = torch.floor((lat + x).remainder(dims)).to(torch.int64)
+    else:
+        x = torch.rand((n, 3), generator=gen, device="cuda") * (dims - 0.01)
+        cell = torch.floor(x).to(torch.int64)
+    st = integrate.Stepper(shape, n, relative=relative)
+    v, field = torch.zeros_like(x), st.new_field(keep_sort=True)
+    st.field_kick(x, v, 1.0, field)
+    # the kept sort ends with its records (x, y, z, particle)
+    size = _lib.size("jpm_bin_sort_size", *shape, n, st.flags)
+    at = size - (16 * n + 255) // 256 * 256
+    p = field[1][at:at + 16 * n].view(torch.int32).reshape(n, 4)[:, 3].to(torch.int64)
+    assert torch.equal(torch.sort(p).values, torch.arange(n, device="cuda"))
+    t = (cell // 16)[p]
+    tile = (t[:, 0] * ((shape[1] + 15) // 16) + t[:, 1]) * ((shape[2] + 15) // 16) + t[:, 2]
+    run = 8 * tile + (p // 4096) % 8
+    assert bool((run[1:] >= run[:-1]).all())
+    # the same forces, particle by particle, from the particles in another order
+    if not relative:
+        perm = torch.randperm(n, generator=gen, device="cuda")
+        v2 = torch.zeros_like(x)
+        st.field_kick(x[perm].contiguous(), v2, 1.0, st.new_field())
+        assert torch.equal(v2, v[perm])
+    cot = torch.randn((n, 3), generator=gen, device="cuda")
+    g1, g2 = torch.zeros_like(x), torch.zeros_like(x)
+    st.vjp_field(field, x, cot, 0.5, g1)
+    st.vjp_field((field[0], None), x, cot, 0.5, g2)
+    assert torch.equal(g1, g2)
