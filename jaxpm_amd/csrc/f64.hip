@@ -137,16 +137,20 @@ paint_f64_kernel(const double *__restrict__ pos, const double *__restrict__ weig
 }
 
 // The paint of many particles: a counting sort into 16^3-cell tiles (count,
-// the tile table, scatter of 32-byte records), float64 sums of each chunk of
-// a tile in a 17^3 LDS window (ds_add_f64), and a reduce that adds the
-// windows covering each cell to the mesh.  One global float64 atomic per
-// corner runs at some 23 G/s (lines shared by the 8 XCDs' L2s).  128^3
-// displaced particles on 128^3 cells: 721 -> 87 us.
-constexpr int kSort64Threads = 256, kSort64Per = 8;
-constexpr uint32_t kSort64Slice = kSort64Threads * kSort64Per;
-constexpr uint32_t kChunk64 = 8192;
+// scatter of 32-byte records) and float64 sums of each chunk of a tile in a
+// 17^3 LDS window (ds_add_f64), added to the mesh by atomics, rows of
+// neighbouring cells.  One global float64 atomic per corner instead runs at some
+// 23 G/s (lines shared by the 8 XCDs' L2s).  128^3 displaced particles on 128^3
+// cells: 743 us by atomics, 82 with the windows stored for a reduce, now 73; the
+// small counts are bound by the launches: 64^3 95, 46 (seven launches), now 28
+// (four).
+constexpr int kSort64Threads = 256;
 constexpr int64_t kPaint64SortMin = 1 << 17;
 constexpr uint32_t kMaxTiles64 = 16384;   // the LDS histogram is 64 KiB
+// More tiles take the tile table's launch: the scan costs every workgroup, and
+// at 160^3 cells, 1000 tiles, 4 million particles in no order took 250 us with
+// it and 207 without.
+constexpr uint32_t kScanTiles64 = 512;
 
 struct Rec64 {
   double x, y, z;
@@ -158,17 +162,56 @@ __device__ __forceinline__ uint32_t tile_key_d(const AxisD &ax, const AxisD &ay,
          uint32_t(az.i0 / kTile);
 }
 
-template <bool REL, bool SCATTER>
-__global__ void __launch_bounds__(kSort64Threads)
-sort_f64_kernel(const double *__restrict__ pos, uint32_t n, GridD g, TileGrid t, uint32_t *__restrict__ table,
-                Rec64 *__restrict__ recs) {
-  extern __shared__ uint32_t cur[];
-  const uint32_t p0 = blockIdx.x * kSort64Slice;
-  for (uint32_t k = threadIdx.x; k < t.K; k += kSort64Threads) cur[k] = 0;
-  double x[kSort64Per], y[kSort64Per], z[kSort64Per];
-  uint32_t key[kSort64Per];
+// The eight deposits of a particle as atomics on the mesh.
+template <bool REL>
+__device__ __forceinline__ void deposit_d(const AxisD &ax, const AxisD &ay, const AxisD &az, const GridD &g, double wp,
+                                          double *__restrict__ mesh) {
+  int64_t idx[8];
+  double w[8];
+  corners_of_d<REL>(ax, ay, az, g, idx, w);
 #pragma unroll
-  for (int i = 0; i < kSort64Per; ++i) {
+  for (int o = 0; o < 8; ++o) unsafeAtomicAdd(&mesh[idx[o]], wp * w[o]);
+}
+
+// The eight corner values of three meshes (M apart), weighted.
+template <bool REL>
+__device__ __forceinline__ void read3_d(const AxisD &ax, const AxisD &ay, const AxisD &az, const GridD &g,
+                                        const double *__restrict__ phi3, int64_t M, double s[3]) {
+  int64_t idx[8];
+  double w[8];
+  corners_of_d<REL>(ax, ay, az, g, idx, w);
+#pragma unroll
+  for (int k = 0; k < 8; ++k)
+#pragma unroll
+    for (int f = 0; f < 3; ++f) s[f] += phi3[f * M + idx[k]] * w[k];
+}
+
+// The tile table as its arrays: the tiles' counts, starts or cursors, chunks.
+struct Table64 {
+  uint32_t *count, *cursor, *totals;
+  ChunkDesc *desc;
+  uint32_t chunk;
+};
+
+// One pass over the particles, kPer of a thread.  kCount64 adds to the tiles'
+// counts and clears mesh[0, zero).  The scatters write the records in tile
+// order: kScatter64 from the cursors of a tile table, kScanScatter64 scans the
+// counts itself, its cursors counting each tile's records from zero, and its
+// first workgroup leaves the chunks and their number (a launch of their own
+// otherwise: 64^3 4 us).
+enum { kCount64, kScatter64, kScanScatter64 };
+
+template <bool REL, int PASS, int kPer>
+__global__ void __launch_bounds__(kSort64Threads)
+sort_f64_kernel(const double *__restrict__ pos, uint32_t n, GridD g, TileGrid t, Table64 tab,
+                Rec64 *__restrict__ recs, double *__restrict__ mesh, int64_t zero) {
+  extern __shared__ uint32_t cur[];
+  const uint32_t p0 = blockIdx.x * uint32_t(kSort64Threads * kPer);
+  for (uint32_t k = threadIdx.x; k < t.K; k += kSort64Threads) cur[k] = 0;
+  double x[kPer], y[kPer], z[kPer];
+  uint32_t key[kPer];
+#pragma unroll
+  for (int i = 0; i < kPer; ++i) {
     const uint32_t p = p0 + uint32_t(i) * kSort64Threads + threadIdx.x;
     const size_t at = 3 * size_t(p < n ? p : n - 1);
     x[i] = pos[at];
@@ -176,7 +219,7 @@ sort_f64_kernel(const double *__restrict__ pos, uint32_t n, GridD g, TileGrid t,
     z[i] = pos[at + 2];
   }
 #pragma unroll
-  for (int i = 0; i < kSort64Per; ++i) {
+  for (int i = 0; i < kPer; ++i) {
     const uint32_t p = p0 + uint32_t(i) * kSort64Threads + threadIdx.x;
     AxisD ax, ay, az;
     axes_d<REL>(x[i], y[i], z[i], p < n ? p : n - 1, g, ax, ay, az);
@@ -185,22 +228,71 @@ sort_f64_kernel(const double *__restrict__ pos, uint32_t n, GridD g, TileGrid t,
   __syncthreads();
   const int lane = int(threadIdx.x & 63u);
 #pragma unroll
-  for (int i = 0; i < kSort64Per; ++i) {
+  for (int i = 0; i < kPer; ++i) {
     const bool active = key[i] != 0xffffffffu;
     const unsigned long long act = __ballot(active), heads = run_heads(key[i], active);
     if (active && ((heads >> lane) & 1ull)) atomicAdd(&cur[key[i]], run_length(heads, act));
   }
   __syncthreads();
-  // table: the tile counts, or, for the scatter, the tiles' cursors
-  for (uint32_t k = threadIdx.x; k < t.K; k += kSort64Threads)
-    if (cur[k]) {
-      const uint32_t at = atomicAdd(&table[k], cur[k]);
-      if (SCATTER) cur[k] = at;
+  if constexpr (PASS == kCount64) {
+    for (int64_t i = blockIdx.x * int64_t(kSort64Threads) + threadIdx.x; i < zero;
+         i += int64_t(gridDim.x) * kSort64Threads)
+      mesh[i] = 0.0;
+    for (uint32_t k = threadIdx.x; k < t.K; k += kSort64Threads)
+      if (cur[k]) atomicAdd(&tab.count[k], cur[k]);
+    return;
+  }
+  if constexpr (PASS == kScatter64) {
+    for (uint32_t k = threadIdx.x; k < t.K; k += kSort64Threads)
+      if (cur[k]) cur[k] = atomicAdd(&tab.cursor[k], cur[k]);
+  } else {
+    // particles and chunks of the tiles before this thread's, neighbours each
+    constexpr int kOwn = kScanTiles64 / kSort64Threads;
+    __shared__ uint32_t first[kScanTiles64], wave_p[kSort64Threads / 64], wave_c[kSort64Threads / 64];
+    const uint32_t k0 = threadIdx.x * kOwn;
+    uint32_t c[kOwn], np = 0, nc = 0;
+#pragma unroll
+    for (int i = 0; i < kOwn; ++i) c[i] = k0 + i < t.K ? tab.count[k0 + i] : 0u;
+#pragma unroll
+    for (int i = 0; i < kOwn; ++i) {
+      np += c[i];
+      nc += (c[i] + tab.chunk - 1) / tab.chunk;
     }
-  if (!SCATTER) return;
+    uint32_t xp = np, xc = nc;
+#pragma unroll
+    for (int off = 1; off < 64; off <<= 1) {
+      const uint32_t up = __shfl_up(xp, off), uc = __shfl_up(xc, off);
+      if (lane >= off) {
+        xp += up;
+        xc += uc;
+      }
+    }
+    if (lane == 63) {
+      wave_p[threadIdx.x >> 6] = xp;
+      wave_c[threadIdx.x >> 6] = xc;
+    }
+    __syncthreads();
+    for (uint32_t w = 0; w < threadIdx.x >> 6; ++w) {
+      xp += wave_p[w];
+      xc += wave_c[w];
+    }
+    if (blockIdx.x == 0 && threadIdx.x == kSort64Threads - 1) tab.totals[1] = xc;
+    uint32_t at = xp - np, ch = xc - nc;
+#pragma unroll
+    for (int i = 0; i < kOwn; ++i) {
+      first[k0 + i] = at;
+      if (blockIdx.x == 0)
+        for (uint32_t o = 0; o < c[i]; o += tab.chunk, ++ch)
+          tab.desc[ch] = ChunkDesc{k0 + i, at + o, min(tab.chunk, c[i] - o), 0u};
+      at += c[i];
+    }
+    __syncthreads();
+    for (uint32_t k = threadIdx.x; k < t.K; k += kSort64Threads)
+      if (cur[k]) cur[k] = first[k] + atomicAdd(&tab.cursor[k], cur[k]);
+  }
   __syncthreads();
 #pragma unroll
-  for (int i = 0; i < kSort64Per; ++i) {
+  for (int i = 0; i < kPer; ++i) {
     const uint32_t p = p0 + uint32_t(i) * kSort64Threads + threadIdx.x;
     const bool active = key[i] != 0xffffffffu;
     const unsigned long long act = __ballot(active), heads = run_heads(key[i], active);
@@ -222,12 +314,13 @@ __device__ __forceinline__ bool block_corners(const AxisD &ax, const AxisD &ay, 
 // A particle whose corners are the 2^3 block at its low corner deposits in
 // the window; any other (a dropped or doubly rounded relative corner, a
 // non-finite position) adds its eight deposits to the mesh itself, as
-// paint_f64_kernel does, before the reduce adds the windows.
+// paint_f64_kernel does.  The window is then added to the mesh but for its
+// zeros, among them the cells past a short tile's halo.
 template <bool REL>
 __global__ void __launch_bounds__(kWindowThreads)
 accum_f64_kernel(const Rec64 *__restrict__ recs, const ChunkDesc *__restrict__ desc,
                  const uint32_t *__restrict__ nchunks, const double *__restrict__ weight, double wscalar, GridD g,
-                 TileGrid t, double *__restrict__ partial, double *__restrict__ mesh) {
+                 TileGrid t, double *__restrict__ mesh) {
   __shared__ double win[kWinCells];
   if (blockIdx.x >= *nchunks) return;
   const ChunkDesc d = desc[blockIdx.x];
@@ -250,53 +343,16 @@ accum_f64_kernel(const Rec64 *__restrict__ recs, const ChunkDesc *__restrict__ d
         unsafeAtomicAdd(w0 + (bx * kWin + by) * kWin + bz, wp * w);
       }
     } else {
-      int64_t idx[8];
-      double w[8];
-      corners_of_d<REL>(ax, ay, az, g, idx, w);
-#pragma unroll
-      for (int o = 0; o < 8; ++o) unsafeAtomicAdd(&mesh[idx[o]], wp * w[o]);
+      deposit_d<REL>(ax, ay, az, g, wp, mesh);
     }
   }
   __syncthreads();
-  double *out = partial + size_t(blockIdx.x) * kWinCells;
-  for (int i = int(threadIdx.x); i < kWinCells; i += kWindowThreads) out[i] = win[i];
-}
-
-// One workgroup per tile: each of its cells adds its tile's windows and, on a
-// low face, the +1 halos of the lower neighbours.  1024 threads, four cells
-// each, and the sources' chunk ranges in LDS: the loads wait on nothing but
-// one another's issue (with 256 threads and the ranges read per cell, 40 us
-// whatever the mesh).
-__global__ void __launch_bounds__(1024)
-reduce_f64_kernel(const double *__restrict__ partial, const uint32_t *__restrict__ choff,
-                  const uint32_t *__restrict__ nchunk, TileGrid t, double *__restrict__ mesh) {
-  int itx, ity, itz;
-  tile_origin(blockIdx.x, t, itx, ity, itz);
-  const int Lx = tile_len(itx, t.tx, t.nx), Ly = tile_len(ity, t.ty, t.ny), Lz = tile_len(itz, t.tz, t.nz);
-  const int px = itx ? itx - 1 : t.tx - 1, py = ity ? ity - 1 : t.ty - 1, pz = itz ? itz - 1 : t.tz - 1;
-  const int PLx = tile_len(px, t.tx, t.nx), PLy = tile_len(py, t.ty, t.ny), PLz = tile_len(pz, t.tz, t.nz);
-  __shared__ uint32_t off[8], cnt[8];
-  if (threadIdx.x < 8) {
-    const int q = int(threadIdx.x);
-    const uint32_t src = (uint32_t(q & 4 ? px : itx) * uint32_t(t.ty) + uint32_t(q & 2 ? py : ity)) * uint32_t(t.tz) +
-                         uint32_t(q & 1 ? pz : itz);
-    off[q] = choff[src];
-    cnt[q] = nchunk[src];
-  }
-  __syncthreads();
-#pragma unroll
-  for (int i = 0; i < kTile * kTile * kTile / 1024; ++i) {
-    const int e = int(threadIdx.x) + i * 1024;
-    const int a = e >> 8, b = (e >> 4) & 15, c = e & 15;
-    if (a >= Lx || b >= Ly || c >= Lz) continue;
-    double acc = 0.0;
-    for (int q = 0; q < 8; ++q) {
-      if (((q & 4) && a) || ((q & 2) && b) || ((q & 1) && c)) continue;
-      const int li = ((q & 4 ? PLx : a) * kWin + (q & 2 ? PLy : b)) * kWin + (q & 1 ? PLz : c);
-      const double *w = partial + size_t(off[q]) * kWinCells + li;
-      for (uint32_t k = 0; k < cnt[q]; ++k) acc += w[size_t(k) * kWinCells];
-    }
-    mesh[(size_t(itx * kTile + a) * t.ny + size_t(ity * kTile + b)) * t.nz + size_t(itz * kTile + c)] += acc;
+  for (int i = int(threadIdx.x); i < kWinCells; i += kWindowThreads) {
+    const double v = win[i];
+    if (v == 0.0) continue;
+    const int c = i % kWin, ab = i / kWin, b = ab % kWin, a = ab / kWin;
+    const int x = ox + a < t.nx ? ox + a : 0, y = oy + b < t.ny ? oy + b : 0, z = oz + c < t.nz ? oz + c : 0;
+    unsafeAtomicAdd(&mesh[(size_t(x) * t.ny + y) * t.nz + z], v);
   }
 }
 
@@ -378,13 +434,7 @@ read3_sorted_f64_kernel(const Rec64 *__restrict__ recs, const ChunkDesc *__restr
         for (int f = 0; f < 3; ++f) s[f] += w0[f * kWinCells + off] * w;
       }
     } else {
-      int64_t idx[8];
-      double w[8];
-      corners_of_d<REL>(ax, ay, az, g, idx, w);
-#pragma unroll
-      for (int k = 0; k < 8; ++k)
-#pragma unroll
-        for (int f = 0; f < 3; ++f) s[f] += phi3[f * M + idx[k]] * w[k];
+      read3_d<REL>(ax, ay, az, g, phi3, M, s);
     }
     double *o3 = out + 3 * size_t(r.p);
     o3[0] = s[0];
@@ -471,16 +521,22 @@ GridD make_grid_d(int nx, int ny, int nz) {
 int fft_d2z(hipStream_t s, int nx, int ny, int nz, int batch, const double *in, void *out);
 int fft_z2d(hipStream_t s, int nx, int ny, int nz, int batch, void *in, double *out);
 
-// Workspace of the sorted paint (byte offsets); the sort, which a read may reuse,
-// then the windows of the accumulation; total 0 where the atomic form
-// is used instead: few particles, or more tiles than the LDS histogram
-// holds.  48^3 random particles take 43 us by atomics and 42 us sorted, 64^3
-// 94 and 47 us, 128^3 727 and 120 us; in the order of an undisturbed lattice,
-// where neighbouring lanes share their cells' lines, 64^3 15 and 44 us, 128^3
-// 110 and 75 us.
+// Workspace of the sorted paint (byte offsets): the sort, which a read may
+// reuse.  total 0 where the atomic form is used instead: few particles, or more
+// tiles than the LDS histogram holds.
+// Paint in us by atomics and sorted, for particles in the order of an
+// undisturbed lattice (whose neighbouring lanes share their cells' lines), of a
+// smooth displacement of 0.3 and of 3 cells, and in none:
+//   51^3, one per cell   11  23  54  53     21  21  23  25
+//   64^3                 16  38 100  94     26  27  28  34
+//   80^3                 29  69 179 181     34  36  39  46
+//   100^3                55 116 297 347     44  47  52  71
+//   128^3               114 214 595 725     66  68  73 106
+// (An undisturbed lattice of fewer than some 90^3 particles would be better off
+// with atomics, but the least displacement turns that over.)
 struct Paint64Ws {
-  uint32_t maxchunks;
-  size_t count, tstart, cursor, nchunk, choff, totals, desc, recs, sort, partial, total;
+  uint32_t maxchunks, chunk;
+  size_t count, tstart, cursor, nchunk, choff, totals, desc, recs, total;
 };
 
 static Paint64Ws paint64_ws(int nx, int ny, int nz, int64_t n) {
@@ -488,55 +544,68 @@ static Paint64Ws paint64_ws(int nx, int ny, int nz, int64_t n) {
   if (nx <= 0 || ny <= 0 || nz <= 0 || n < kPaint64SortMin || n > kMaxCells) return w;
   const TileGrid t = make_tiles(nx, ny, nz);
   if (uint64_t(t.tx) * t.ty * t.tz > kMaxTiles64) return w;
-  w.maxchunks = uint32_t((n + kChunk64 - 1) / kChunk64 + t.K);
+  for (w.chunk = 1024; w.chunk < 8192 && int64_t(w.chunk) * 128 < n;) w.chunk *= 2;
+  w.maxchunks = uint32_t((n + w.chunk - 1) / w.chunk + t.K);
   size_t o = 0;
   auto take = [&o](size_t bytes) {
     const size_t at = o;
     o += align_up(bytes);
     return at;
   };
-  w.count = take(size_t(t.K) * 4);
+  w.count = take(2 * size_t(t.K) * 4);
+  w.cursor = w.count + size_t(t.K) * 4;   // cleared with the counts
   w.tstart = take(size_t(t.K) * 4);
-  w.cursor = take(size_t(t.K) * 4);
   w.nchunk = take(size_t(t.K) * 4);
   w.choff = take(size_t(t.K) * 4);
   w.totals = take(16);
   w.desc = take(size_t(w.maxchunks) * sizeof(ChunkDesc));
   w.recs = take(size_t(n) * sizeof(Rec64));
-  w.sort = o;
-  w.partial = take(size_t(w.maxchunks) * kWinCells * sizeof(double));
   w.total = o;
   return w;
 }
 
 size_t cic_paint_f64_ws(int nx, int ny, int nz, int64_t n) { return paint64_ws(nx, ny, nz, n).total; }
 
-// base: w.sort bytes for the sort; partial: the windows.
+template <int PASS>
+static int sort_pass(hipStream_t s, const double *pos, uint32_t n, bool rel, const GridD &g, const TileGrid &t,
+                     const Table64 &tab, Rec64 *recs, double *mesh, int64_t zero) {
+  // Few particles in slices of 1024, so that every CU has one; slices of 2048
+  // add less often to the tiles' counters, of which particles in no order meet
+  // all (paint in us, slices of 1024 and 2048, lattice and no order: 64^3 25.8
+  // and 27.0, 33.6 and 32.4, 80^3 33.6 and 35.0, 54.6 and 46.3)
+  const int per = n < (1u << 19) && t.K <= kScanTiles64 ? 4 : 8;
+  auto kern = per == 4 ? (rel ? sort_f64_kernel<true, PASS, 4> : sort_f64_kernel<false, PASS, 4>)
+                       : (rel ? sort_f64_kernel<true, PASS, 8> : sort_f64_kernel<false, PASS, 8>);
+  const uint32_t slice = uint32_t(kSort64Threads * per);
+  hipLaunchKernelGGL(kern, dim3((n + slice - 1) / slice), dim3(kSort64Threads), size_t(t.K) * 4, s, pos, n, g, t, tab,
+                     recs, mesh, zero);
+  JPM_LAUNCHED("sort_f64_kernel");
+  return JPM_OK;
+}
+
+// mesh (cleared first if `zero`) += the paint.
 static int paint_f64_sorted(hipStream_t s, int nx, int ny, int nz, const double *pos, uint32_t n, const double *weight,
-                            double wscalar, bool rel, double *mesh, char *base, double *partial, const Paint64Ws &w) {
+                            double wscalar, bool rel, double *mesh, bool zero, char *base, const Paint64Ws &w) {
   const TileGrid t = make_tiles(nx, ny, nz);
   const GridD g = make_grid_d(nx, ny, nz);
   auto u32 = [base](size_t at) { return reinterpret_cast<uint32_t *>(base + at); };
-  auto *desc = reinterpret_cast<ChunkDesc *>(base + w.desc);
   auto *recs = reinterpret_cast<Rec64 *>(base + w.recs);
-  const unsigned grid = unsigned((uint64_t(n) + kSort64Slice - 1) / kSort64Slice);
-  const size_t lds = size_t(t.K) * 4;
-  int rc = zero_u32(s, u32(w.count), t.K);
+  const Table64 tab{u32(w.count), u32(w.cursor), u32(w.totals), reinterpret_cast<ChunkDesc *>(base + w.desc), w.chunk};
+  const int64_t m = zero ? cells(nx, ny, nz) : 0;
+  int rc = zero_u32(s, tab.count, 2 * t.K);
+  if (!rc) rc = sort_pass<kCount64>(s, pos, n, rel, g, t, tab, recs, mesh, m);
   if (rc) return rc;
-  hipLaunchKernelGGL(rel ? (sort_f64_kernel<true, false>) : (sort_f64_kernel<false, false>), dim3(grid),
-                     dim3(kSort64Threads), lds, s, pos, n, g, t, u32(w.count), recs);
-  JPM_LAUNCHED("sort_f64_kernel");
-  rc = tile_table(s, u32(w.count), t.K, kChunk64, u32(w.tstart), u32(w.cursor), u32(w.nchunk), u32(w.choff),
-                  u32(w.totals), desc);
+  if (t.K <= kScanTiles64) {
+    rc = sort_pass<kScanScatter64>(s, pos, n, rel, g, t, tab, recs, nullptr, 0);
+  } else {
+    rc = tile_table(s, tab.count, t.K, w.chunk, u32(w.tstart), tab.cursor, u32(w.nchunk), u32(w.choff), tab.totals,
+                    tab.desc);
+    if (!rc) rc = sort_pass<kScatter64>(s, pos, n, rel, g, t, tab, recs, nullptr, 0);
+  }
   if (rc) return rc;
-  hipLaunchKernelGGL(rel ? (sort_f64_kernel<true, true>) : (sort_f64_kernel<false, true>), dim3(grid),
-                     dim3(kSort64Threads), lds, s, pos, n, g, t, u32(w.cursor), recs);
-  JPM_LAUNCHED("sort_f64_kernel");
   hipLaunchKernelGGL(rel ? accum_f64_kernel<true> : accum_f64_kernel<false>, dim3(w.maxchunks), dim3(kWindowThreads), 0,
-                     s, recs, desc, u32(w.totals) + 1, weight, wscalar, g, t, partial, mesh);
+                     s, recs, tab.desc, tab.totals + 1, weight, wscalar, g, t, mesh);
   JPM_LAUNCHED("accum_f64_kernel");
-  hipLaunchKernelGGL(reduce_f64_kernel, dim3(t.K), dim3(1024), 0, s, partial, u32(w.choff), u32(w.nchunk), t, mesh);
-  JPM_LAUNCHED("reduce_f64_kernel");
   return JPM_OK;
 }
 
@@ -571,15 +640,15 @@ int cic_paint_f64(hipStream_t s, int nx, int ny, int nz, const double *pos, int6
               (long long)n, (long long)m);
   const Paint64Ws w = ws ? paint64_ws(nx, ny, nz, n) : Paint64Ws{};
   JPM_REQUIRE(ws_bytes >= w.total, "the float64 paint needs %zu workspace bytes, got %zu", w.total, ws_bytes);
+  JPM_REQUIRE(n == 0 || pos != nullptr, "positions are null");
+  if (w.total)
+    return paint_f64_sorted(s, nx, ny, nz, pos, uint32_t(n), weight, wscalar, rel, mesh, flags & JPM_ZERO_MESH,
+                            static_cast<char *>(ws), w);
   if (flags & JPM_ZERO_MESH) {
     hipLaunchKernelGGL(zero_f64_kernel, dim3(grid_for(m, 256)), dim3(256), 0, s, mesh, m);
     JPM_LAUNCHED("zero_f64_kernel");
   }
   if (n == 0) return JPM_OK;
-  JPM_REQUIRE(pos != nullptr, "positions are null");
-  if (w.total)
-    return paint_f64_sorted(s, nx, ny, nz, pos, uint32_t(n), weight, wscalar, rel, mesh, static_cast<char *>(ws),
-                            reinterpret_cast<double *>(static_cast<char *>(ws) + w.partial), w);
   const GridD g = make_grid_d(nx, ny, nz);
   const unsigned grid = grid_for(n, 256, 256 * 128);
   if (rel)
@@ -627,8 +696,7 @@ int cic_read_f64(hipStream_t s, int nx, int ny, int nz, const double *mesh, int 
 
 // Workspace of pm_forces_f64: the density mesh, its half spectrum, the three
 // force spectra, the three force meshes and, where one particle per cell would
-// be painted sorted, that sort, which the read takes up again.  The paint's
-// windows lie where the spectra follow.
+// be painted sorted, that sort, which the read takes up again.
 struct Forces64Ws {
   size_t spec, spec3, phi3, sort, sort_bytes, total;
 };
@@ -640,7 +708,7 @@ static Forces64Ws forces64_ws(int nx, int ny, int nz) {
   w.spec3 = w.spec + align_up(H * 16);
   w.phi3 = w.spec3 + align_up(3 * H * 16);
   w.sort = w.phi3 + align_up(3 * M * 8);
-  w.sort_bytes = paint64_ws(nx, ny, nz, int64_t(M)).sort;
+  w.sort_bytes = cic_paint_f64_ws(nx, ny, nz, int64_t(M));
   w.total = w.sort + w.sort_bytes;
   return w;
 }
@@ -669,14 +737,11 @@ int pm_forces_f64(hipStream_t s, int nx, int ny, int nz, const double *pos, int6
   Paint64Ws p{};
   if (!field) {
     p = paint64_ws(nx, ny, nz, n);
-    if (p.total && (p.sort > w.sort_bytes || p.total - p.sort > w.sort - w.spec)) p = Paint64Ws{};
+    if (p.total > w.sort_bytes) p = Paint64Ws{};
     if (p.total) {
       JPM_REQUIRE(!rel || n == M, "relative painting needs one particle per lattice node (n=%lld, mesh %lld)",
                   (long long)n, (long long)M);
-      hipLaunchKernelGGL(zero_f64_kernel, dim3(grid_for(M, 256)), dim3(256), 0, s, rho, M);
-      JPM_LAUNCHED("zero_f64_kernel");
-      rc = paint_f64_sorted(s, nx, ny, nz, pos, uint32_t(n), nullptr, 1.0, rel, rho, base + w.sort,
-                            reinterpret_cast<double *>(spec), p);
+      rc = paint_f64_sorted(s, nx, ny, nz, pos, uint32_t(n), nullptr, 1.0, rel, rho, true, base + w.sort, p);
     } else {
       // too many particles per cell for the sort's share of the workspace:
       // the whole paint where the spectra follow, or atomics

@@ -167,3 +167,63 @@ def test_sorted_paint_f64_nonfinite(gpu, x64):
     assert torch.equal(torch.isnan(got), torch.isnan(ref)) and torch.equal(torch.isinf(got), torch.isinf(ref))
     ok = torch.isfinite(ref)
     assert not bool(ok.all()) and rel(got[ok].cpu().numpy(), ref[ok].cpu().numpy()) < 1e-13
+
+
+def _concentrated(kind, shape, n, r):
+    """Positions of which most share few tiles, in many chunks each."""
+    pos = r.uniform(0, 1, (n, 3)) * shape
+    part = slice(None) if kind == "one tile" else slice(None, None, 2)
+    pos[part] = np.minimum(17.0, np.array(shape) / 2) + r.uniform(-3, 9, pos[part].shape)
+    return pos
+
+
+@pytest.mark.parametrize("kind", ["one tile", "half"])
+@pytest.mark.parametrize("shape,n", [((40, 33, 64), 131072), ((64, 64, 64), 300001)])
+def test_clustered_paint_and_forces_f64(gpu, x64, kind, shape, n):
+    """Most particles in the 2^3 tiles that a cluster of 12^3 cells touches, in
+    chunks of 1024 and 2048: sums of some 10^3 deposits of at most 1 a cell,
+    below 1e-13 of the largest."""
+    from jaxpm_amd import painting, pm
+    print(f"clustered f64: {kind} {shape} n={n}", flush=True)
+    r = np.random.default_rng(11)
+    pos = _concentrated(kind, shape, n, r)
+    w = r.uniform(0.5, 1.0, n)
+    pt = torch.as_tensor(pos, device=gpu)
+    got = painting.cic_paint(torch.zeros(shape, dtype=torch.float64, device=gpu), pt, torch.as_tensor(w, device=gpu))
+    assert rel(got.cpu().numpy(), op.cic_paint(np.zeros(shape), pos, w)) < 1e-13
+    got = pm.pm_forces(pt, mesh_shape=shape)
+    assert rel(got.cpu().numpy(), opm.pm_forces(pos, mesh_shape=shape)) < 1e-12
+
+
+def test_clustered_relative_f64(gpu, x64):
+    """Displacements that bring every second particle to one tile."""
+    from jaxpm_amd import painting, pm
+    shape = (66, 51, 40)
+    print(f"clustered relative f64 {shape}", flush=True)
+    r = np.random.default_rng(12)
+    disp = r.normal(scale=1.3, size=(*shape, 3))
+    disp[::2] = r.uniform(18, 30, disp[::2].shape) - lattice(shape)[::2]
+    got = painting.cic_paint_dx(torch.as_tensor(disp, device=gpu))
+    assert rel(got.cpu().numpy(), op.cic_paint_dx(disp)) < 1e-13
+    got = pm.pm_forces(torch.as_tensor(disp, device=gpu), mesh_shape=shape, paint_absolute_pos=False)
+    assert rel(got.cpu().numpy(), opm.pm_forces(disp, mesh_shape=shape, paint_absolute_pos=False)) < 1e-12
+
+
+@pytest.mark.parametrize("shape,n", [((32, 32, 32), 2 ** 17 - 1), ((32, 32, 32), 2 ** 17), ((48, 33, 32), 2 ** 19 - 1),
+                                     ((48, 33, 32), 2 ** 19), ((128, 128, 128), 2 ** 18), ((128, 128, 129), 2 ** 18),
+                                     ((256, 256, 256), 2 ** 18), ((1, 512, 700), 2 ** 17),
+                                     ((2048, 2048, 1), 2 ** 18), ((2064, 2048, 1), 2 ** 18), ((17, 16, 16), 2 ** 20)])
+def test_f64_paint_on_each_side_of_its_rules(gpu, x64, shape, n):
+    """Counts and tiles on each side of the sort's rules and
+    of its passes', against the atomic form: the same deposits in another
+    order, up to some 10^4 a cell."""
+    from jaxpm_amd import _lib, _ops
+    print(f"f64 paint rules {shape} n={n}", flush=True)
+    gen = torch.Generator(device=gpu).manual_seed(9)
+    pos = (torch.rand((n, 3), generator=gen, device=gpu, dtype=torch.float64) * 1.5 - 0.2) * \
+        torch.tensor(shape, dtype=torch.float64, device=gpu)
+    base = torch.randn(shape, generator=gen, device=gpu, dtype=torch.float64)
+    got = _ops.paint_f64(base.clone(), pos)
+    ref = base.clone()
+    _lib.call("jpm_cic_paint_f64", _lib.stream(), *shape, _lib.ptr(pos), n, None, 1.0, _lib.ptr(ref), 0)
+    assert float((got - ref).abs().max()) <= 1e-13 * float(ref.abs().max())
