@@ -138,7 +138,8 @@ int jpm_cic_paint_f64(void *stream, int nx, int ny, int nz, const double *pos,
 /* jpm_cic_paint_f64 with a workspace of jpm_cic_paint_f64_workspace_size
  * bytes (some 32 a particle), in which many particles are sorted by tile
  * and summed in LDS windows instead of one global atomic per corner.  Where that
- * size is 0 ws may be NULL and the call is jpm_cic_paint_f64. */
+ * size is 0 (few particles, in all or per cell) ws may be NULL and the call is
+ * jpm_cic_paint_f64. */
 size_t jpm_cic_paint_f64_workspace_size(int nx, int ny, int nz, int64_t n);
 int jpm_cic_paint_ws_f64(void *stream, int nx, int ny, int nz,
                          const double *pos, int64_t n, const double *weight,

@@ -522,8 +522,8 @@ int fft_d2z(hipStream_t s, int nx, int ny, int nz, int batch, const double *in, 
 int fft_z2d(hipStream_t s, int nx, int ny, int nz, int batch, void *in, double *out);
 
 // Workspace of the sorted paint (byte offsets): the sort, which a read may
-// reuse.  total 0 where the atomic form is used instead: few particles, or more
-// tiles than the LDS histogram holds.
+// reuse.  total 0 where the atomic form is used instead: few particles, few per
+// cell, or more tiles than the LDS histogram holds.
 // Paint in us by atomics and sorted, for particles in the order of an
 // undisturbed lattice (whose neighbouring lanes share their cells' lines), of a
 // smooth displacement of 0.3 and of 3 cells, and in none:
@@ -532,6 +532,10 @@ int fft_z2d(hipStream_t s, int nx, int ny, int nz, int batch, void *in, double *
 //   80^3                 29  69 179 181     34  36  39  46
 //   100^3                55 116 297 347     44  47  52  71
 //   128^3               114 214 595 725     66  68  73 106
+// and in lattice order and in none:
+//   256^3, 1/64 a cell  109 111    55  96
+//   256^3, 1/128         66  67    49  76
+//   400^3, 1/64         430 472   256 380
 // (An undisturbed lattice of fewer than some 90^3 particles would be better off
 // with atomics, but the least displacement turns that over.)
 struct Paint64Ws {
@@ -542,6 +546,7 @@ struct Paint64Ws {
 static Paint64Ws paint64_ws(int nx, int ny, int nz, int64_t n) {
   Paint64Ws w{};
   if (nx <= 0 || ny <= 0 || nz <= 0 || n < kPaint64SortMin || n > kMaxCells) return w;
+  if (n < cells(nx, ny, nz) / 64) return w;
   const TileGrid t = make_tiles(nx, ny, nz);
   if (uint64_t(t.tx) * t.ty * t.tz > kMaxTiles64) return w;
   for (w.chunk = 1024; w.chunk < 8192 && int64_t(w.chunk) * 128 < n;) w.chunk *= 2;

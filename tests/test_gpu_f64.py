@@ -211,10 +211,10 @@ def test_clustered_relative_f64(gpu, x64):
 
 @pytest.mark.parametrize("shape,n", [((32, 32, 32), 2 ** 17 - 1), ((32, 32, 32), 2 ** 17), ((48, 33, 32), 2 ** 19 - 1),
                                      ((48, 33, 32), 2 ** 19), ((128, 128, 128), 2 ** 18), ((128, 128, 129), 2 ** 18),
-                                     ((256, 256, 256), 2 ** 18), ((1, 512, 700), 2 ** 17),
+                                     ((256, 256, 256), 2 ** 18 - 1), ((256, 256, 256), 2 ** 18), ((1, 512, 700), 2 ** 17),
                                      ((2048, 2048, 1), 2 ** 18), ((2064, 2048, 1), 2 ** 18), ((17, 16, 16), 2 ** 20)])
 def test_f64_paint_on_each_side_of_its_rules(gpu, x64, shape, n):
-    """Counts and tiles on each side of the sort's rules and
+    """Counts, particles per cell and tiles on each side of the sort's rules and
     of its passes', against the atomic form: the same deposits in another
     order, up to some 10^4 a cell."""
     from jaxpm_amd import _lib, _ops
