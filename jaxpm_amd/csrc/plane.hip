@@ -120,6 +120,9 @@ constexpr uint32_t kPlaneSelect = 4096;     // particles per select workgroup, r
 constexpr uint32_t kPlaneChunk = 8192;      // records per window
 constexpr uint32_t kPlaneMaxTiles = 4096;   // 4096^2 pixels: the LDS histogram is 16 KiB
 constexpr int64_t kPlaneSortMin = 3 << 18;
+// Particles of one sort: more take it in turns, in the workspace of one (1.07 GB
+// of records, which all of them may fill), their sums kept in float64.
+constexpr int64_t kPlanePass = 1 << 26;
 
 struct PlaneTiles {
   int res, t;   // pixels and tiles per axis
@@ -280,15 +283,19 @@ plane_accum_kernel(const float2 *__restrict__ sorted, const ChunkDesc *__restric
   for (int i = threadIdx.x; i < kPwCells; i += 512) out[i] = float(win[i]);
 }
 
-// blockIdx.x: tile; blockIdx.y: 4 of its 64 rows, one pixel per thread.
+// blockIdx.x: tile; blockIdx.y: 4 of its 64 rows, one pixel per thread.  The
+// pixels start from `before` (null: zero) and go to `after` or, when that is
+// null, divided by the normalisation to the plane.
 __global__ void __launch_bounds__(256)
 plane_reduce_kernel(const float *__restrict__ partial, const uint32_t *__restrict__ nchunk,
-                    const uint32_t *__restrict__ choff, PlaneTiles t, float norm, float *__restrict__ plane) {
+                    const uint32_t *__restrict__ choff, PlaneTiles t, float norm, const double *before, double *after,
+                    float *__restrict__ plane) {
   const int tx = int(t.div_t.div(blockIdx.x)), ty = int(blockIdx.x) - tx * t.t;
   const int a = int(blockIdx.y) * 4 + int(threadIdx.x >> 6), b = int(threadIdx.x & 63u);
   if (a >= plane_len(tx, t) || b >= plane_len(ty, t)) return;
   const int px = tx ? tx - 1 : t.t - 1, py = ty ? ty - 1 : t.t - 1;
-  double acc = 0.0;
+  const uint32_t pixel = uint32_t(tx * kPt + a) * uint32_t(t.res) + uint32_t(ty * kPt + b);
+  double acc = before ? before[pixel] : 0.0;
   for (int sx = 0; sx <= (a == 0 ? 1 : 0); ++sx)
     for (int sy = 0; sy <= (b == 0 ? 1 : 0); ++sy) {
       const uint32_t src = uint32_t(sx ? px : tx) * uint32_t(t.t) + uint32_t(sy ? py : ty);
@@ -297,7 +304,10 @@ plane_reduce_kernel(const float *__restrict__ partial, const uint32_t *__restric
       const uint32_t n = nchunk[src];
       for (uint32_t k = 0; k < n; ++k) acc += double(w[size_t(k) * kPwCells]);
     }
-  plane[uint32_t(tx * kPt + a) * uint32_t(t.res) + uint32_t(ty * kPt + b)] = float(acc) / norm;
+  if (after)
+    after[pixel] = acc;
+  else
+    plane[pixel] = float(acc) / norm;
 }
 
 // Adjoint of the density plane for a plane cotangent g (already divided by
@@ -409,7 +419,7 @@ static PlaneArgs plane_args(int box_nx, int box_ny, double center, double width,
 // 63-207 against 40-90 us (128^2 to 1024^2 pixels, both orders).
 struct PlaneWs {
   uint32_t T, maxchunks;
-  size_t count, nsel, tstart, cursor, nchunk, choff, totals, desc, recs, sorted, partial, total;
+  size_t count, nsel, tstart, cursor, nchunk, choff, totals, desc, recs, sorted, partial, sums, total;
 };
 
 static PlaneWs plane_ws(int64_t n, int res) {
@@ -418,7 +428,8 @@ static PlaneWs plane_ws(int64_t n, int res) {
   const uint64_t t = uint64_t((res + kPt - 1) / kPt);
   if (t * t > kPlaneMaxTiles) return w;
   w.T = uint32_t(t * t);
-  w.maxchunks = uint32_t((uint64_t(n) + kPlaneChunk - 1) / kPlaneChunk + w.T);
+  const int64_t one = n < kPlanePass ? n : kPlanePass;
+  w.maxchunks = uint32_t((uint64_t(one) + kPlaneChunk - 1) / kPlaneChunk + w.T);
   size_t o = 0;
   auto take = [&o](size_t bytes) {
     const size_t at = o;
@@ -433,17 +444,19 @@ static PlaneWs plane_ws(int64_t n, int res) {
   w.choff = take(size_t(w.T) * 4);
   w.totals = take(16);
   w.desc = take(size_t(w.maxchunks) * sizeof(ChunkDesc));
-  w.recs = take(size_t(n) * sizeof(float2));
-  w.sorted = take(size_t(n) * sizeof(float2));
+  w.recs = take(size_t(one) * sizeof(float2));
+  w.sorted = take(size_t(one) * sizeof(float2));
   w.partial = take(size_t(w.maxchunks) * kPwCells * sizeof(float));
+  w.sums = take(one < n ? size_t(res) * size_t(res) * sizeof(double) : 0);
   w.total = o;
   return w;
 }
 
 size_t density_plane_ws(int64_t n, int res) { return plane_ws(n, res).total; }
 
+// The n particles of one sort; before, after: as for plane_reduce_kernel.
 static int density_plane_sorted(hipStream_t s, const float *pos, uint32_t n, float bnx, const PlaneArgs &a, int res,
-                                float *plane, char *base, const PlaneWs &w) {
+                                const double *before, double *after, float *plane, char *base, const PlaneWs &w) {
   PlaneTiles t;
   t.res = res;
   t.t = (res + kPt - 1) / kPt;
@@ -472,7 +485,7 @@ static int density_plane_sorted(hipStream_t s, const float *pos, uint32_t n, flo
   hipLaunchKernelGGL(plane_accum_kernel, dim3(w.maxchunks), dim3(512), 0, s, sorted, desc, totals + 1, t, partial);
   JPM_LAUNCHED("plane_accum_kernel");
   hipLaunchKernelGGL(plane_reduce_kernel, dim3(w.T, kPt / 4), dim3(256), 0, s, partial, nchunk, choff, t, a.norm,
-                     plane);
+                     before, after, plane);
   JPM_LAUNCHED("plane_reduce_kernel");
   return JPM_OK;
 }
@@ -490,8 +503,17 @@ int density_plane(hipStream_t s, const float *pos, int64_t n, int box_nx, int bo
   if (ws) {
     const PlaneWs w = plane_ws(n, res);
     JPM_REQUIRE(ws_bytes >= w.total, "the density plane needs %zu workspace bytes, got %zu", w.total, ws_bytes);
-    if (w.total)
-      return density_plane_sorted(s, pos, uint32_t(n), float(box_nx), a, res, plane, static_cast<char *>(ws), w);
+    if (w.total) {
+      double *sums = reinterpret_cast<double *>(static_cast<char *>(ws) + w.sums);
+      for (int64_t p0 = 0; p0 < n; p0 += kPlanePass) {
+        const int64_t left = n - p0;
+        const int rc = density_plane_sorted(s, pos + 3 * p0, uint32_t(left < kPlanePass ? left : kPlanePass),
+                                            float(box_nx), a, res, p0 ? sums : nullptr,
+                                            left > kPlanePass ? sums : nullptr, plane, static_cast<char *>(ws), w);
+        if (rc) return rc;
+      }
+      return JPM_OK;
+    }
   }
   hipLaunchKernelGGL(plane_zero_kernel, dim3(grid_for(m, 256, 4096)), dim3(256), 0, s, plane, m);
   JPM_LAUNCHED("plane_zero_kernel");

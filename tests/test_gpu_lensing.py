@@ -141,3 +141,20 @@ def test_sorted_density_plane_nonfinite(gpu):
     assert torch.equal(torch.isnan(got), torch.isnan(ref)) and bool(torch.isnan(ref).any())
     ok = ~torch.isnan(ref)
     assert rel_err(got[ok].cpu().numpy(), ref[ok].double().cpu().numpy()) < 3e-6
+
+
+def test_density_plane_of_more_particles_than_one_sort(gpu):
+    """2^26 particles and a few more are sorted in two turns.  The plane is
+    linear in the particles: against the sum of the planes of its two turns,
+    each rounded to float32 as windows, as a pixel and by the normalisation."""
+    from jaxpm_amd import _ops
+    n, res = 2 ** 26 + 900001, 200
+    print(f"density plane n={n}", flush=True)
+    gen = torch.Generator(device="cuda").manual_seed(21)
+    pos = torch.rand((n, 3), generator=gen, device="cuda") * 64
+    args = ((64, 64, 64), 32.0, 16.0, res)
+    whole = _ops.density_plane(pos, *args)
+    first, rest = _ops.density_plane(pos[:2 ** 26], *args), _ops.density_plane(pos[2 ** 26:], *args)
+    ref = first.double() + rest.double()
+    assert float(whole.double().sum()) > 0
+    assert float(((whole.double() - ref).abs() / ref).max()) < 6 * 2.0 ** -24
