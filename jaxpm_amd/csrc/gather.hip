@@ -777,6 +777,9 @@ bin_grad_pos_kernel(Bins bins, const float *__restrict__ mesh, uint32_t cstride,
   for (int k = 0; k < NC; ++k)
     load_window_t<kWin, 0, T>(mesh + size_t(k) * cstride, t, ox, oy, oz, win + k * kWinCells);
   __syncthreads();
+  // from 2^24 on floor + 1 may round two cells up, out of the window
+  auto skips = [](const float4 &r) { return fmaxf(fmaxf(fabsf(r.x), fabsf(r.y)), fabsf(r.z)) >= 16777216.0f; };
+  bool far = false;
   for (uint32_t q = threadIdx.x; q < cnt; q += T) {
     const float4 rec = rec1;
     float u[NC];
@@ -796,6 +799,7 @@ bin_grad_pos_kernel(Bins bins, const float *__restrict__ mesh, uint32_t cstride,
     // to differ) has both corners at its floor cell, as in the direct kernel
     auto next = [](float x, int step) { return floorf(x) + 1.0f > floorf(x) ? step : 0; };
     const int sx = next(rec.x, kWin * kWin), sy = next(rec.y, kWin), sz = next(rec.z, 1);
+    far |= skips(rec);
     float out[3] = {0.0f, 0.0f, 0.0f};
 #pragma unroll
     for (int k = 0; k < NC; ++k) {
@@ -815,6 +819,32 @@ bin_grad_pos_kernel(Bins bins, const float *__restrict__ mesh, uint32_t cstride,
     g[0] = out[0];
     g[1] = out[1];
     g[2] = out[2];
+  }
+  if (!far) return;
+  // those particles of this thread again, from the meshes
+  for (uint32_t q = threadIdx.x; q < cnt; q += T) {
+    const float4 rec = load_global(bins.spos + (start + q));
+    if (!skips(rec)) continue;
+    CornerSet cs;
+    corner_set<false>(rec, t, 0u, ox, oy, oz, cs);
+    const float f[3] = {floorf(rec.x), floorf(rec.y), floorf(rec.z)};
+    const uint32_t p = __float_as_uint(rec.w);
+    float out[3] = {0.0f, 0.0f, 0.0f};
+    for (int k = 0; k < NC; ++k) {
+      float s[3] = {0.0f, 0.0f, 0.0f};
+#pragma unroll
+      for (int o = 0; o < 8; ++o) {
+        const int bx = o & 1, by = (o >> 1) & 1, bz = (o >> 2) & 1;
+        const uint32_t x = wrapi(cell_int(f[0] + float(bx)), t.nx), y = wrapi(cell_int(f[1] + float(by)), t.ny),
+                       z = wrapi(cell_int(f[2] + float(bz)), t.nz);
+        const float v = mesh[size_t(k) * cstride + (x * uint32_t(t.ny) + y) * uint32_t(t.nz) + z];
+        s[0] += v * (cs.d[0][bx] * cs.w[1][by] * cs.w[2][bz]);
+        s[1] += v * (cs.w[0][bx] * cs.d[1][by] * cs.w[2][bz]);
+        s[2] += v * (cs.w[0][bx] * cs.w[1][by] * cs.d[2][bz]);
+      }
+      for (int a = 0; a < 3; ++a) out[a] += cot[size_t(NC) * p + k] * s[a];
+    }
+    for (int a = 0; a < 3; ++a) gpos[3 * size_t(p) + a] = out[a];
   }
 }
 

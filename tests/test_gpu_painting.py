@@ -494,3 +494,24 @@ def test_paint_onto_a_mesh(gpu, shape, n, relative):
     got = _ops.paint_onto(base, p, weight=w, relative=relative)
     assert torch.equal(base, keep)
     assert torch.equal(got, _ops.paint(keep, p, weight=w, relative=relative))
+
+
+@pytest.mark.parametrize("nc,n", [(1, 6000), (1, 900), (3, 6000)])
+def test_read_cotangents_where_floor_plus_one_skips_a_cell(gpu, nc, n):
+    """From 2^24 on a coordinate's floor + 1 rounds to itself or two cells up;
+    both kernels of the position cotangent take the cell it rounds to."""
+    from jaxpm_amd import _ops
+    shape = (20, 18, 17)
+    print(f"read vjp past 2^24 nc={nc} n={n}", flush=True)
+    r = np.random.default_rng(48)
+    pos = (r.uniform(0, 1, size=(n, 3)) * np.array(shape)).astype(np.float32)
+    far = np.float32([16777216, 16777218, -16777218, -16777216, 16777214.0, 33554430, -33554430, 33554434, 2147483520,
+                      -2147483648, 3e9, np.inf, -np.inf])
+    for a in range(3):
+        at = slice(a * len(far), (a + 1) * len(far))
+        pos[at, a] = far
+    pos[100:200] = r.choice(far[:6], (100, 3))
+    meshes, cot = dev(r.normal(size=(nc, *shape))), dev(r.normal(size=(n, nc)))
+    p = dev(pos)
+    gp, direct = _ops.read_vjp(meshes, p, cot)[1], _ops.grad_pos(meshes, p, cot=cot)
+    assert torch.equal(gp.isnan(), direct.isnan()) and torch.equal(gp.nan_to_num(), direct.nan_to_num())
