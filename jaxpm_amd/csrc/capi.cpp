@@ -549,6 +549,9 @@ static int pm_forces(hipStream_t s, int nx, int ny, int nz, const float *pos, in
 }
 
 
+// Second-order LPT by the library's FFT alone (native_lpt2).
+static bool lpt2_native(int nx, int ny, int nz) { return native_fft_ok(nx, ny, nz) && nx >= 2; }
+
 // Workspace of lpt: [half spectrum][7 half spectra, later the force meshes,
 // or first order the force meshes][potential 1][potential 2].
 struct LptSpace {
@@ -560,11 +563,14 @@ static LptSpace lpt_space(int nx, int ny, int nz, int order) {
   LptSpace w;
   size_t o = 0;
   w.spec = o; o += align_up(h * 8);
-  // second order: 7 spectra, or 6 and their 6 meshes, or 6 force meshes;
-  // first order: 3 force meshes (and the second half spectrum of a solve)
-  // and, on a mesh with an axis of one cell, 3 floats of displacement per cell
+  // second order: 7 spectra, then 6 force meshes in their place, and behind
+  // them the 6 shear meshes where the library's FFT does not form their source
+  // directly; first order: 3 force meshes (a solve's second half spectrum
+  // before them); and, on a mesh with an axis of one cell, 3 floats of
+  // displacement per cell behind the force meshes
   w.many = o;
-  o += order == 2 ? align_up(7 * h * 8) + align_up(6 * m * 4) : align_up(3 * m * 4) + align_up(h * 8);
+  o += order == 2 ? align_up(7 * h * 8) : align_up(3 * m * 4);
+  if (order == 2 && !lpt2_native(nx, ny, nz)) o += align_up(6 * m * 4);
   if (nx == 1 || ny == 1 || nz == 1) o += align_up(3 * m * 4);
   w.phi1 = o; o += align_up(m * 4);
   w.phi2 = o; o += order == 2 ? align_up(m * 4) : 0;
@@ -596,11 +602,15 @@ static int lpt(hipStream_t s, int nx, int ny, int nz, const float *ic, const flo
     rc = potential_solve(s, nx, ny, nz, 1, ic, spec, many, phi1, 0.0f, scale, nullptr, 0);
     if (rc) return rc;
   } else {
-    const bool aligned = (reinterpret_cast<uintptr_t>(ic) & 7u) == 0;
-    if (native_fft_ok(nx, ny, nz) && nx >= 2 && aligned) {
+    if (lpt2_native(nx, ny, nz)) {
       Tabs t;
       rc = get_tabs(s, nx, ny, nz, 0, t);
       if (rc) return rc;
+      if (reinterpret_cast<uintptr_t>(ic) & 7u) {
+        // the transforms load pairs: through the second potential's place
+        JPM_HIP(hipMemcpyAsync(phi2, ic, size_t(m) * 4, hipMemcpyDeviceToDevice, s));
+        ic = phi2;
+      }
       rc = native_lpt2(s, nx, ny, nz, ic, spec, many, phi1, phi2, t, scale);
       if (rc) return rc;
     } else {

@@ -300,3 +300,22 @@ def test_kspace_potential(gpu):
     kv = ok.fftk(shape)
     ref = np.fft.ifftn(np.fft.fftn(rho) * ok.invlaplace_kernel(kv) * ok.longrange_kernel(kv, 1.2)).real
     assert rel_err(pot, ref) < 5e-6
+
+
+@pytest.mark.parametrize("absolute", [False, True])
+def test_lpt2_of_a_field_at_an_odd_offset(gpu, absolute):
+    """Initial conditions that start 4 bytes past an 8-byte boundary give the
+    bits of an aligned copy, in the workspace of the shape."""
+    from jaxpm_amd import cosmology as pc
+    from jaxpm_amd import pm
+    shape = (32, 16, 48)
+    print(f"lpt2 odd offset {shape} absolute={absolute}", flush=True)
+    r = np.random.default_rng(52)
+    ic = dev(r.normal(size=shape))
+    odd = torch.empty(ic.numel() + 1, device="cuda")[1:].reshape(shape)
+    odd.copy_(ic)
+    assert odd.data_ptr() % 8 == 4
+    parts = dev(r.uniform(0, 16, size=(700, 3))) if absolute else None
+    got = pm.lpt(pc.Cosmology(), odd, parts, a=0.1, order=2)
+    ref = pm.lpt(pc.Cosmology(), ic, parts, a=0.1, order=2)
+    assert all(torch.equal(g, w) for g, w in zip(got, ref))

@@ -37,3 +37,16 @@ def test_density_plane_workspace_is_bounded(size, n, res):
     tiles = ((res + 63) // 64) ** 2
     windows = (2 ** 26 // 8192 + tiles) * (65 * 65 * 4 + 16)
     assert size("jpm_density_plane_workspace_size", n, res) <= 16 * 2 ** 26 + windows + 8 * res * res + 32 * tiles + 4096
+
+
+@pytest.mark.parametrize("shape,native", [((256, 256, 256), True), ((64, 96, 48), True), ((512, 512, 512), True),
+                                          ((100, 125, 90), False), ((64, 64, 63), False)])
+def test_lpt_workspace_holds_what_the_shape_needs(size, shape, native):
+    """First order: a half spectrum, three force meshes, a potential.  Second:
+    seven more spectra and a second potential, and the six shear meshes only on
+    shapes that the library's own FFT does not take."""
+    nx, ny, nz = shape
+    m, h = nx * ny * nz, nx * ny * (nz // 2 + 1)
+    slack = 8 * 256
+    assert size("jpm_lpt_workspace_size", *shape, 1) <= 8 * h + 4 * 3 * m + 4 * m + slack
+    assert size("jpm_lpt_workspace_size", *shape, 2) <= 8 * 8 * h + 2 * 4 * m + (0 if native else 4 * 6 * m) + slack
