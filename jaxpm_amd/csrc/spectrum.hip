@@ -152,7 +152,9 @@ __global__ __launch_bounds__(kPkMaxWaves * 64) void pk_bin_kernel(const float2 *
 #pragma unroll
         for (int q = 0; q < NP; ++q) {
           re[q] = pair ? 2.0 * xr : xr;
-          im[q] = pair ? 0.0 : xi;
+          // 0 but for a mode that is not finite, whose imaginary part and its
+          // mirror's cancel to NaN
+          im[q] = pair ? 0.0 * xi : xi;
         }
       } else {
         const double tx = kx * p.los[0], ty = ky * p.los[1], tz = kz * p.los[2];

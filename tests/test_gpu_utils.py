@@ -128,3 +128,26 @@ def _bin_count(n, L, k, b):
     dk = 4 * np.pi / L
     edges = np.arange(dk, np.pi * n / L, dk) + dk / 2
     return int(np.sum(np.digitize(kk.reshape(-1), edges) == b + 1))
+
+
+@pytest.mark.parametrize("poles", [[0], [0, 0], [0, 1, 2]])
+def test_cross_spectrum_of_modes_that_are_not_finite(gpu, poles):
+    """A mode of infinite product and its mirror, the conjugate, sum to an
+    infinite real and an undefined imaginary part, in the monopole of an
+    isotropic call as among other poles; the other bins stay finite."""
+    from jaxpm_amd import _ops
+    print(f"cross spectrum not finite {poles}", flush=True)
+    shape = (16, 12, 20)
+    gen = torch.Generator(device="cuda").manual_seed(31)
+    s1 = torch.randn((16, 12, 11), generator=gen, device="cuda", dtype=torch.complex64)
+    s2 = torch.randn((16, 12, 11), generator=gen, device="cuda", dtype=torch.complex64)
+    s1[1, 2, 3] = complex(float("inf"), 1.0)
+    s2[1, 2, 3] = complex(1.0, 1.0)
+    edges = np.linspace(0.3, 3.0, 10)
+    fac = [2 * np.pi] * 3
+    out = _ops.power_spectrum_sums(s1, s2, shape, fac, edges, poles, (0.0, 0.0, 1.0)).cpu().numpy()
+    k = 2 * np.pi * np.sqrt((1 / 16) ** 2 + (2 / 12) ** 2 + (3 / 20) ** 2)
+    hit = int(np.digitize(np.float32(k), edges))
+    rest = np.arange(out.shape[1]) != hit
+    assert np.isfinite(out[:, rest]).all()
+    assert np.isposinf(out[2, hit]) and np.isnan(out[2 + len(poles), hit])
