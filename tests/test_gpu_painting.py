@@ -515,3 +515,45 @@ def test_read_cotangents_where_floor_plus_one_skips_a_cell(gpu, nc, n):
     p = dev(pos)
     gp, direct = _ops.read_vjp(meshes, p, cot)[1], _ops.grad_pos(meshes, p, cot=cot)
     assert torch.equal(gp.isnan(), direct.isnan()) and torch.equal(gp.nan_to_num(), direct.nan_to_num())
+
+
+def _one_ulp_below(shape, edge):
+    """Displacements of a lattice at rest but for the plane x = 5, one float
+    below ``edge`` (2^-20 below 16, 2^-19 below 32), where adding 1 rounds up:
+    its high corner is the cell edge + 1, outside its tile's window, with the
+    weight -2^-20; and the mesh that this paints, exactly."""
+    disp = np.zeros((*shape, 3), np.float32)
+    x = np.nextafter(np.float32(edge), np.float32(0))
+    disp[5, :, :, 0] = x - np.float32(5)
+    assert np.float32(5) + disp[5, 0, 0, 0] == x and x + np.float32(1) == edge + 1
+    mesh = np.ones(shape, np.float32)
+    mesh[5] -= 1
+    mesh[edge - 1] += np.float32(edge) - x
+    mesh[edge + 1] -= np.float32(edge) - x
+    return disp, mesh
+
+
+def test_relative_batch_paints_corners_outside_their_windows(gpu):
+    """Corners outside their windows in the second and third simulations of a
+    batch: the marks of their tiles and their cells lie past the first's."""
+    from jaxpm_amd import integrate
+    shapes, edges = [(32, 32, 32), (32, 32, 32), (48, 17, 40), (48, 17, 40)], [None, 16, 32, 16]
+    print("relative batch, corners outside windows", flush=True)
+    want = [(np.zeros((*s, 3), np.float32), np.ones(s, np.float32)) if e is None else _one_ulp_below(s, e)
+            for s, e in zip(shapes, edges)]
+    st = integrate.BatchStepper(shapes, [int(np.prod(s)) for s in shapes], relative=True)
+    got = host(st.paint(dev(np.concatenate([d.reshape(-1, 3) for d, _ in want])))).reshape(-1)
+    assert np.array_equal(got, np.concatenate([m.reshape(-1) for _, m in want]))
+
+
+def test_relative_paint_of_many_tiles_marks_corners_outside_their_windows(gpu):
+    """More tiles than their marks fit in the last chunk's windows: they lie
+    behind the overflow mesh."""
+    from jaxpm_amd import _ops
+    shape = (352, 352, 352)
+    print(f"relative paint {shape}, corners outside windows", flush=True)
+    disp, mesh = _one_ulp_below(shape, 16)
+    d, m = dev(disp), dev(mesh)
+    assert torch.equal(_ops.paint(torch.full(shape, 7.0, device="cuda"), d, relative=True, zero=True), m)
+    assert torch.equal(_ops.paint(torch.full(shape, 2.0, device="cuda"), d, relative=True), m + 2.0)
+    assert torch.equal(_ops.paint(torch.zeros(shape, device="cuda"), d, relative=True, method="atomic"), m)
