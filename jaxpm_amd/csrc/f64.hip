@@ -42,27 +42,9 @@ __device__ __forceinline__ AxisD axis_abs_d(double x, int n) {
 // painting_utils.py:48-69 in double: q = (p + o) mod L (jnp.remainder),
 // floor, nd = p - q, nd -= rint(nd / L) L, weight 1 - |nd|; the corner is
 // dropped (zero weight at a valid index) unless 0 <= q < L.
-// The exact shortcuts of jmod and fold_period (tiles.hpp) skip fmod's loop
-// and the division for nearly every corner.
-__device__ __forceinline__ double jmod_d(double x, double L) {
-  if (x >= 0.0 && x < L) return x;
-  if (x < 0.0 && x > -L) return x + L;
-  if (x >= L && x < 2.0 * L) return x - L;
-  double m = fmod(x, L);
-  if (m != 0.0 && m < 0.0) m = m + L;
-  return m;
-}
-
-__device__ __forceinline__ double fold_period_d(double nd, double L) {
-  const double a = fabs(nd);
-  if (a <= 0.25 * L) return nd;
-  if (a >= 0.75 * L && a <= 1.25 * L) return nd - copysign(L, nd);
-  return nd - rint(nd / L) * L;
-}
-
 __device__ __forceinline__ void corner_rel_d(double p, double o, double L, int &idx, double &w) {
-  const double q = floor(jmod_d(p + o, L));
-  const double nd = fold_period_d(p - q, L);
+  const double q = floor(jmod(p + o, L));
+  const double nd = fold_period(p - q, L);
   const bool ok = (q >= 0.0) && (q < L);
   idx = ok ? int(q) : 0;
   w = ok ? 1.0 - fabs(nd) : 0.0;

@@ -193,26 +193,39 @@ __device__ __forceinline__ int wrapi(int c, int n) {
 // or, when that corner is dropped, the high corner minus one.
 __device__ __forceinline__ int floor_cell_abs(float x, int n) { return wrapi(cell_int(floorf(x)), n); }
 
-// jnp.remainder(x, L) for L > 0.  Inside [0, 2 L) and (-L, 0) fmodf is x, the
+// The exact expressions below in float and double (and on the host, for their
+// test).
+__host__ __device__ __forceinline__ float fmod_of(float x, float L) { return fmodf(x, L); }
+__host__ __device__ __forceinline__ double fmod_of(double x, double L) { return fmod(x, L); }
+__host__ __device__ __forceinline__ float abs_of(float x) { return fabsf(x); }
+__host__ __device__ __forceinline__ double abs_of(double x) { return fabs(x); }
+__host__ __device__ __forceinline__ float rint_of(float x) { return rintf(x); }
+__host__ __device__ __forceinline__ double rint_of(double x) { return rint(x); }
+__host__ __device__ __forceinline__ float copysign_of(float x, float y) { return copysignf(x, y); }
+__host__ __device__ __forceinline__ double copysign_of(double x, double y) { return copysign(x, y); }
+
+// jnp.remainder(x, L) for L > 0.  Inside [0, 2 L) and (-L, 0) fmod is x, the
 // exact difference x - L (Sterbenz) or x, so nearly every lattice node plus
 // displacement skips its division loop; the rest, NaN among it, takes it.
-__host__ __device__ __forceinline__ float jmod(float x, float L) {
-  if (x >= 0.0f && x < L) return x;
-  if (x < 0.0f && x > -L) return x + L;
-  if (x >= L && x < 2.0f * L) return x - L;
-  float m = fmodf(x, L);
-  if (m != 0.0f && m < 0.0f) m = m + L;
+template <class T>
+__host__ __device__ __forceinline__ T jmod(T x, T L) {
+  if (x >= T(0) && x < L) return x;
+  if (x < T(0) && x > -L) return x + L;
+  if (x >= L && x < T(2) * L) return x - L;
+  T m = fmod_of(x, L);
+  if (m != T(0) && m < T(0)) m = m + L;
   return m;
 }
 
 // nd - rint(nd / L) L for L > 0 (enmesh's periodic fold of a distance):
 // a quarter of a period around 0 or +-L the quotient rounds to 0 or +-1
 // without being formed.
-__host__ __device__ __forceinline__ float fold_period(float nd, float L) {
-  const float a = fabsf(nd);
-  if (a <= 0.25f * L) return nd;
-  if (a >= 0.75f * L && a <= 1.25f * L) return nd - copysignf(L, nd);
-  return nd - rintf(nd / L) * L;
+template <class T>
+__host__ __device__ __forceinline__ T fold_period(T nd, T L) {
+  const T a = abs_of(nd);
+  if (a <= T(0.25) * L) return nd;
+  if (a >= T(0.75) * L && a <= T(1.25) * L) return nd - copysign_of(L, nd);
+  return nd - rint_of(nd / L) * L;
 }
 
 __device__ __forceinline__ int floor_cell_rel(float p, int n) {
