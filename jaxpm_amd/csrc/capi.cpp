@@ -1179,9 +1179,13 @@ int jpm_cic_paint_binned_f32(void *stream, int nx, int ny, int nz, const float *
 int jpm_cic_paint_onto_f32(void *stream, int nx, int ny, int nz, const float *base, const float *pos, int64_t n,
                            const float *weights, float wscalar, float *mesh, uint32_t flags, void *ws,
                            size_t ws_bytes) {
-  if (!base) return fail(JPM_E_INVALID, "base is null");
-  JPM_GUARD(binned_paint(as_stream(stream), nx, ny, nz, pos, n, weights, wscalar, 1, mesh, flags & ~JPM_ZERO_MESH, ws,
-                         ws_bytes, base));
+  JPM_GUARD([&]() -> int {
+    const int rc = check_dims(nx, ny, nz);
+    if (rc) return rc;
+    JPM_REQUIRE(base, "base is null");
+    return binned_paint(as_stream(stream), nx, ny, nz, pos, n, weights, wscalar, 1, mesh, flags & ~JPM_ZERO_MESH, ws,
+                        ws_bytes, base);
+  }());
 }
 
 int jpm_pm_forces_f32(void *stream, int nx, int ny, int nz, const float *pos, int64_t n, const void *delta_k,

@@ -64,3 +64,18 @@ def test_product_fails_loudly_without_gpu():
     from jaxpm_amd import painting
     with pytest.raises(RuntimeError, match="no CPU fallback"):
         painting.cic_paint(torch.zeros(4, 4, 4), torch.zeros(10, 3))
+
+
+def test_paint_onto_names_the_bad_shape():
+    """An empty mesh has no address either: its shape is what is wrong."""
+    import torch
+    if torch.cuda.is_available():
+        pytest.skip("host-validation test runs without a GPU")
+    from jaxpm_amd import _lib
+    if not os.path.exists(_lib.LIB_PATH):
+        pytest.skip("libjaxpm_hip.so not built")
+    lib = _lib.load()
+    assert lib.jpm_cic_paint_onto_f32(None, 0, 8, 8, None, None, 0, None, 1.0, None, 0, None, 0) == -1
+    assert b"must be positive" in lib.jpm_last_error()
+    assert lib.jpm_cic_paint_onto_f32(None, 8, 8, 8, None, None, 0, None, 1.0, None, 0, None, 0) == -1
+    assert b"base is null" in lib.jpm_last_error()
