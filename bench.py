@@ -675,14 +675,15 @@ def main():
         "fft_cols_potential_kernel": 16 * H,           # in place
         "fft_c2r_rows_kernel": 8 * H + 4 * M,
         # aggregates of the passes above (not kernels; never the roofline kernel)
-        "potential_solve (5 passes)": 8 * M + 64 * H,
-        "potential_solve[div] (5 passes)": 16 * M + 64 * H,
-        "native_r2c (3 passes)": 4 * M + 40 * H,
-        "native_c2r (3 passes)": 40 * H + 4 * M,
+        "potential_solve": 8 * M + 64 * H,
+        "potential_solve[div]": 16 * M + 64 * H,
+        "native_r2c": 4 * M + 40 * H,
+        "native_c2r": 40 * H + 4 * M,
         "abs_max_kernel": 12 * N,
         "permute_rows_kernel": 2 * 24 * N,             # two (N, 3) arrays, read and written
         "record_order_kernel": 16 * N + 4 * N,
     }
+    aggregates = {"potential_solve", "potential_solve[div]", "native_r2c", "native_c2r"}
     kinfo = {}
     groups = {}
     for name, (cnt, tot) in per_kernel.items():
@@ -692,7 +693,7 @@ def main():
         if name in algo:
             gbs = algo[name] / (avg * 1e-3) / 1e9
             entry.update({"GB_s": round(gbs, 1), "frac_hbm": round(gbs / HBM_PEAK_GBS, 4)})
-            if " (" not in name:
+            if name not in aggregates:
                 g = groups.setdefault(name.split("[")[0], {"launches": 0, "ms": 0.0, "bytes": 0.0, "variants": {}})
                 g["launches"] += cnt
                 g["ms"] += tot

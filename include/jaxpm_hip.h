@@ -53,9 +53,10 @@ extern "C" {
  * flags in bits 0..7, k-space flags shifted left by 8, and the tile sort's
  * tuning in bits 16..26 -- JPM_TUNE_CHUNK(c): at most 2^(9+c) particles per
  * accumulation/gather chunk (c = 1..6, default 8192), JPM_TUNE_SLICE(s):
- * 2^(11+s) particles per counting/scatter workgroup (s = 1..7, default
- * 8192).  The choice changes speed, never results beyond float rounding;
- * a kept sort must be read with the flags it was built with. */
+ * 2^(11+s) particles per counting/scatter workgroup (s = 1..7; by default 1024
+ * below 2^17 particles, 2048 below 2^19, then 4096 and, in a paint, read or
+ * order of 2^22 on, 8192).  The choice changes speed, never results beyond
+ * float rounding; a kept sort must be read with the flags it was built with. */
 #define JPM_TUNE_CHUNK(c) ((uint32_t)(c) << 16)
 #define JPM_TUNE_SLICE(s) ((uint32_t)(s) << 20)
 #define JPM_TUNE_RHO_GLOBAL (1u << 24)  /* force-VJP gather: density adjoint

@@ -368,10 +368,10 @@ constexpr int kick_threads() { return REL ? 768 : 1024; }
 template <bool REL, int MODE, bool PARTS, class G>
 __global__ void __launch_bounds__(kick_threads<REL>(), REL ? 6 : 8)
 bin_kick_kernel(BinsT<G> bins, const float *__restrict__ phi_all, float gamma_s, const float *__restrict__ gamma_dev,
-                float *__restrict__ vel, uint32_t per, uint32_t parts, DriftArgs dr) {
+                float *__restrict__ vel, uint32_t place, uint32_t parts, DriftArgs dr) {
   __shared__ float win[3 * kWinCells];   // the potential window, then the force window
   __shared__ uint32_t ncount[27];   // drifted particles per neighbour tile
-  const uint32_t c = gather_item(blockIdx.x, per, bins.slabs);
+  const uint32_t c = gather_item(blockIdx.x, place, bins.slabs);
   if (c >= *bins.total_chunks) return;
   const bool count_next = MODE == 2 && !REL && dr.next_count;
   const ChunkDesc d = bins.desc[c];
@@ -523,13 +523,13 @@ template <bool REL, class G, bool RLDS, bool PARTS>
 __global__ void __launch_bounds__((grad_threads<REL, RLDS>()), ((grad_threads<REL, RLDS>()) == 768 ? 6 : 1))
 bin_grad_kernel(BinsT<G> bins, const float *__restrict__ phi_all, const float *__restrict__ rho_all,
                 const float *cot, float scale_s, const float *__restrict__ scale_dev,
-                float *__restrict__ gpos, uint32_t per, uint32_t parts, float beta_s, const float *__restrict__ beta_dev,
+                float *__restrict__ gpos, uint32_t place, uint32_t parts, float beta_s, const float *__restrict__ beta_dev,
                 float *cot_out, float *__restrict__ cot_max) {
   __shared__ float win[3 * kWinCells];   // the potential window, then the force window
   __shared__ float rwin[RLDS ? kWinCells : 1];
   constexpr int T = grad_threads<REL, RLDS>();
   __shared__ float wmax[T / 64];
-  const uint32_t c = gather_item(blockIdx.x, per, bins.slabs);
+  const uint32_t c = gather_item(blockIdx.x, place, bins.slabs);
   if (c >= *bins.total_chunks) return;
   const ChunkDesc d = bins.desc[c];
   uint32_t start, cnt;
@@ -702,9 +702,9 @@ bin_grad_kernel(BinsT<G> bins, const float *__restrict__ phi_all, const float *_
 template <int NC, class G>
 __global__ void __launch_bounds__(kWindowThreads)
 bin_read_kernel(BinsT<G> bins, const float *__restrict__ mesh_all, uint32_t cstride, float *__restrict__ out,
-                uint32_t per) {
+                uint32_t place) {
   __shared__ float win[NC * kWinCells];
-  const uint32_t c = gather_item(blockIdx.x, per, bins.slabs);
+  const uint32_t c = gather_item(blockIdx.x, place, bins.slabs);
   if (c >= *bins.total_chunks) return;
   const ChunkDesc d = bins.desc[c];
   const SimRef &sim = bins.g.tile_sim(d.tile);
@@ -750,10 +750,10 @@ constexpr int grad_pos_threads() { return NC == 1 ? kWindowThreads : 1024; }
 template <int NC>
 __global__ void __launch_bounds__(grad_pos_threads<NC>())
 bin_grad_pos_kernel(Bins bins, const float *__restrict__ mesh, uint32_t cstride, const float *__restrict__ cot,
-                    float *__restrict__ gpos, uint32_t per, uint32_t parts) {
+                    float *__restrict__ gpos, uint32_t place, uint32_t parts) {
   constexpr int T = grad_pos_threads<NC>();
   __shared__ float win[NC * kWinCells];
-  const uint32_t c = gather_item(blockIdx.x, per, bins.slabs);
+  const uint32_t c = gather_item(blockIdx.x, place, bins.slabs);
   if (c >= *bins.total_chunks) return;
   const ChunkDesc d = bins.desc[c];
   uint32_t start, cnt;
@@ -852,14 +852,14 @@ int bins_grad_pos(hipStream_t s, const Bins &b, const float *mesh, int nc, uint3
                   float *gpos) {
   JPM_REQUIRE(mesh && cot && gpos, "null pointer argument");
   JPM_REQUIRE(!b.rel && (nc == 1 || nc == 3), "the sorted position cotangent takes absolute positions, 1 or 3 meshes");
-  uint32_t per;
+  uint32_t place;
   const uint32_t parts = gather_parts(b.n, b.K, nc == 1 ? grad_pos_threads<1>() : grad_pos_threads<3>());
-  const dim3 grid(gather_grid(b.maxchunks, b.K, b.slabs, per), 1u << parts);
+  const dim3 grid(gather_grid(b.maxchunks, b.K, b.slabs, place), 1u << parts);
   JPM_TIMED(s, "bin_grad_pos_kernel");
   if (nc == 1)
-    hipLaunchKernelGGL(bin_grad_pos_kernel<1>, grid, dim3(grad_pos_threads<1>()), 0, s, b, mesh, cstride, cot, gpos, per, parts);
+    hipLaunchKernelGGL(bin_grad_pos_kernel<1>, grid, dim3(grad_pos_threads<1>()), 0, s, b, mesh, cstride, cot, gpos, place, parts);
   else
-    hipLaunchKernelGGL(bin_grad_pos_kernel<3>, grid, dim3(grad_pos_threads<3>()), 0, s, b, mesh, cstride, cot, gpos, per, parts);
+    hipLaunchKernelGGL(bin_grad_pos_kernel<3>, grid, dim3(grad_pos_threads<3>()), 0, s, b, mesh, cstride, cot, gpos, place, parts);
   JPM_LAUNCHED("bin_grad_pos_kernel");
   return JPM_OK;
 }
@@ -874,10 +874,10 @@ static int kick_sorted(hipStream_t s, const BinsT<G> &b, const float *phi, float
     int rc = zero_u32(s, dr.next_count, b.K);
     if (rc) return rc;
   }
-  uint32_t per;
+  uint32_t place;
   const int threads = b.rel ? kick_threads<true>() : kick_threads<false>();
   const uint32_t parts = gather_parts(b.n, b.K, threads);
-  const dim3 grid(gather_grid(b.maxchunks, b.K, b.slabs, per), 1u << parts), block(threads);
+  const dim3 grid(gather_grid(b.maxchunks, b.K, b.slabs, place), 1u << parts), block(threads);
   JPM_TIMED(s, mode == 2 ? "bin_kick_kernel[drift]" : mode == 1 ? "bin_kick_kernel[forces]" : "bin_kick_kernel");
   auto pick = [&](auto split) {
     constexpr bool P = decltype(split)::value;
@@ -887,7 +887,7 @@ static int kick_sorted(hipStream_t s, const BinsT<G> &b, const float *phi, float
                                                                             : bin_kick_kernel<false, 0, P, G>);
   };
   auto kern = parts ? pick(std::true_type{}) : pick(std::false_type{});
-  hipLaunchKernelGGL(kern, grid, block, 0, s, b, phi, gamma, gamma_dev, vel, per, parts, dr);
+  hipLaunchKernelGGL(kern, grid, block, 0, s, b, phi, gamma, gamma_dev, vel, place, parts, dr);
   JPM_LAUNCHED("bin_kick_kernel");
   return JPM_OK;
 }
@@ -905,11 +905,11 @@ static int grad_sorted(hipStream_t s, const BinsT<G> &b, const float *phi, const
     int rc = zero_f32(s, cot_max, 1);
     if (rc) return rc;
   }
-  uint32_t per;
+  uint32_t place;
   const int threads = b.rel ? (rho_lds ? grad_threads<true, true>() : grad_threads<true, false>())
                             : (rho_lds ? grad_threads<false, true>() : grad_threads<false, false>());
   const uint32_t parts = gather_parts(b.n, b.K, threads);
-  const dim3 grid(gather_grid(b.maxchunks, b.K, b.slabs, per), 1u << parts), block(threads);
+  const dim3 grid(gather_grid(b.maxchunks, b.K, b.slabs, place), 1u << parts), block(threads);
   JPM_TIMED(s, cot_out ? "bin_grad_kernel[drift]" : "bin_grad_kernel");
   auto pick = [&](auto split) {
     constexpr bool P = decltype(split)::value;
@@ -917,7 +917,7 @@ static int grad_sorted(hipStream_t s, const BinsT<G> &b, const float *phi, const
                  : (rho_lds ? bin_grad_kernel<false, G, true, P> : bin_grad_kernel<false, G, false, P>);
   };
   auto kern = parts ? pick(std::true_type{}) : pick(std::false_type{});
-  hipLaunchKernelGGL(kern, grid, block, 0, s, b, phi, rho_bar, cot, scale, scale_dev, gpos, per, parts, beta,
+  hipLaunchKernelGGL(kern, grid, block, 0, s, b, phi, rho_bar, cot, scale, scale_dev, gpos, place, parts, beta,
                      beta_dev, cot_out, cot_max);
   JPM_LAUNCHED("bin_grad_kernel");
   return JPM_OK;
@@ -952,11 +952,11 @@ int bins_read(hipStream_t s, const Bins &b, const float *mesh, int nc, uint32_t 
   JPM_REQUIRE(mesh && out, "null pointer argument");
   JPM_REQUIRE(!b.rel, "the tile-sorted read takes absolute positions");
   JPM_REQUIRE(nc >= 1 && nc <= 3, "the tile-sorted read takes 1 to 3 meshes (got %d)", nc);
-  uint32_t per;
-  const dim3 grid(gather_grid(b.maxchunks, b.K, b.slabs, per)), block(kWindowThreads);
+  uint32_t place;
+  const dim3 grid(gather_grid(b.maxchunks, b.K, b.slabs, place)), block(kWindowThreads);
   JPM_TIMED(s, "bin_read_kernel");
   auto kern = nc == 1 ? bin_read_kernel<1, OneSim> : nc == 2 ? bin_read_kernel<2, OneSim> : bin_read_kernel<3, OneSim>;
-  hipLaunchKernelGGL(kern, grid, block, 0, s, b, mesh, cstride, out, per);
+  hipLaunchKernelGGL(kern, grid, block, 0, s, b, mesh, cstride, out, place);
   JPM_LAUNCHED("bin_read_kernel");
   return JPM_OK;
 }

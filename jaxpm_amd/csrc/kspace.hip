@@ -513,7 +513,7 @@ int potential_solve(hipStream_t s, int nx, int ny, int nz, int batch, const floa
     Tabs t;
     rc = get_tabs(s, nx, ny, nz, flags, t);
     if (rc) return rc;
-    JPM_TIMED(s, "potential_solve (5 passes)");
+    JPM_TIMED(s, "potential_solve");
     return native_potential(s, nx, ny, nz, batch, in, spec, out, t, r_split * r_split, scale, scale_dev,
                             int((flags & JPM_K_DECONV) != 0), nullptr, 0, faces);
   }
@@ -540,7 +540,7 @@ int potential_solve_div(hipStream_t s, int nx, int ny, int nz, int batch, const 
     Tabs t;
     rc = get_tabs(s, nx, ny, nz, flags, t);
     if (rc) return rc;
-    JPM_TIMED(s, "potential_solve[div] (5 passes)");
+    JPM_TIMED(s, "potential_solve[div]");
     return native_potential(s, nx, ny, nz, batch, nullptr, spec, out, t, r_split * r_split, scale, scale_dev,
                             int((flags & JPM_K_DECONV) != 0), g3, chan);
   }

@@ -68,19 +68,22 @@ __device__ __forceinline__ uint32_t slab_item(uint32_t b, uint32_t per, bool sla
 // eighth of their tiles), so that every XCD has some: runs of 32 put the 8
 // tiles of a 32^3 mesh on one XCD and the 64 of a 64^3 mesh on two (its kick
 // 15.0 -> 13.6 us, its force VJP 19.8 -> 18.8).
+// `place` says which item a workgroup takes: with slabs the items per XCD,
+// without them log2 of the run.
 constexpr uint32_t kXcdRun = 32;
-inline unsigned gather_grid(uint32_t items, uint32_t tiles, bool slabs, uint32_t &per) {
-  const unsigned g = slab_grid(items, slabs, per);
+inline unsigned gather_grid(uint32_t items, uint32_t tiles, bool slabs, uint32_t &place) {
+  const unsigned g = slab_grid(items, slabs, place);
   if (slabs) return g;
-  per = 0;   // log2 of the run
-  while ((16u << per) <= tiles && (1u << per) < kXcdRun) ++per;
-  return ((g + (8u << per) - 1u) >> (3u + per)) << (3u + per);
+  uint32_t run = 0;
+  while ((16u << run) <= tiles && (1u << run) < kXcdRun) ++run;
+  place = run;
+  return ((g + (8u << run) - 1u) >> (3u + run)) << (3u + run);
 }
 
-__device__ __forceinline__ uint32_t gather_item(uint32_t b, uint32_t per, bool slabs) {
-  if (slabs) return slab_item(b, per, true);
-  const uint32_t block = b >> (3u + per) << (3u + per), r = b - block;
-  return block + ((r & 7u) << per) + (r >> 3);
+__device__ __forceinline__ uint32_t gather_item(uint32_t b, uint32_t place, bool slabs) {
+  if (slabs) return slab_item(b, place, true);
+  const uint32_t run = place, block = b >> (3u + run) << (3u + run), r = b - block;
+  return block + ((r & 7u) << run) + (r >> 3);
 }
 // Particles per count / scatter workgroup of a sort of n particles.  Slices
 // that narrow with n keep a few hundred workgroups on the chip (a slice of
