@@ -609,7 +609,7 @@ int jpm_density_plane_f32(void *stream, const float *pos, int64_t n,
 
 /* jpm_density_plane_f32 with a workspace of
  * jpm_density_plane_workspace_size(n, res) bytes (16 a particle, for at most
- * 2^26 of them, and some per pixel), in which many particles are sorted by plane
+ * 2^27 of them, and some per pixel), in which many particles are sorted by plane
  * tile and summed without atomics on the pixels.  Where that
  * size is 0 (few particles, or a plane of more than 4096^2 pixels) ws may be
  * NULL and the call is jpm_density_plane_f32. */

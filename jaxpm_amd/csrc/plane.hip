@@ -120,9 +120,10 @@ constexpr uint32_t kPlaneSelect = 4096;     // particles per select workgroup, r
 constexpr uint32_t kPlaneChunk = 8192;      // records per window
 constexpr uint32_t kPlaneMaxTiles = 4096;   // 4096^2 pixels: the LDS histogram is 16 KiB
 constexpr int64_t kPlaneSortMin = 3 << 18;
-// Particles of one sort: more take it in turns, in the workspace of one (1.07 GB
-// of records, which all of them may fill), their sums kept in float64.
-constexpr int64_t kPlanePass = 1 << 26;
+// Particles of one sort: more take it in turns, in the workspace of one (2.1 GB
+// of records, which all of them may fill), their sums kept in float64.  A turn
+// costs 46 us beyond its particles: 2^27 take 1067 us in one and 1113 in two.
+constexpr int64_t kPlanePass = 1 << 27;
 
 struct PlaneTiles {
   int res, t;   // pixels and tiles per axis

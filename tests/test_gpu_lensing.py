@@ -144,17 +144,17 @@ def test_sorted_density_plane_nonfinite(gpu):
 
 
 def test_density_plane_of_more_particles_than_one_sort(gpu):
-    """2^26 particles and a few more are sorted in two turns.  The plane is
+    """2^27 particles and a few more are sorted in two turns.  The plane is
     linear in the particles: against the sum of the planes of its two turns,
     each rounded to float32 as windows, as a pixel and by the normalisation."""
     from jaxpm_amd import _ops
-    n, res = 2 ** 26 + 900001, 200
+    n, res = 2 ** 27 + 900001, 200
     print(f"density plane n={n}", flush=True)
     gen = torch.Generator(device="cuda").manual_seed(21)
     pos = torch.rand((n, 3), generator=gen, device="cuda") * 64
     args = ((64, 64, 64), 32.0, 16.0, res)
     whole = _ops.density_plane(pos, *args)
-    first, rest = _ops.density_plane(pos[:2 ** 26], *args), _ops.density_plane(pos[2 ** 26:], *args)
+    first, rest = _ops.density_plane(pos[:2 ** 27], *args), _ops.density_plane(pos[2 ** 27:], *args)
     ref = first.double() + rest.double()
     assert float(whole.double().sum()) > 0
     assert float(((whole.double() - ref).abs() / ref).max()) < 6 * 2.0 ** -24

@@ -29,14 +29,14 @@ def test_f64_paint_workspace_follows_the_particles(size, shape, n):
     assert size("jpm_cic_paint_f64_workspace_size", *shape, n) <= 48 * n
 
 
-@pytest.mark.parametrize("n", [2 ** 26, 2 ** 26 + 1, 2 ** 27, 2 ** 30, 2 ** 32 - 1])
+@pytest.mark.parametrize("n", [2 ** 27, 2 ** 27 + 1, 2 ** 28, 2 ** 30, 2 ** 32 - 1])
 @pytest.mark.parametrize("res", [64, 1000, 1024, 4096])
 def test_density_plane_workspace_is_bounded(size, n, res):
-    """The records of 2^26 particles and the windows and sums of the plane,
+    """The records of 2^27 particles and the windows and sums of the plane,
     however many particles there are."""
     tiles = ((res + 63) // 64) ** 2
-    windows = (2 ** 26 // 8192 + tiles) * (65 * 65 * 4 + 16)
-    assert size("jpm_density_plane_workspace_size", n, res) <= 16 * 2 ** 26 + windows + 8 * res * res + 32 * tiles + 4096
+    windows = (2 ** 27 // 8192 + tiles) * (65 * 65 * 4 + 16)
+    assert size("jpm_density_plane_workspace_size", n, res) <= 16 * 2 ** 27 + windows + 8 * res * res + 32 * tiles + 4096
 
 
 @pytest.mark.parametrize("shape,native", [((256, 256, 256), True), ((64, 96, 48), True), ((512, 512, 512), True),
