@@ -291,6 +291,13 @@ __device__ __forceinline__ void load_corners(const T *__restrict__ m, size_t cst
           v[c][q | 4] = p[c][q].y;
         }
     }
+  } else if (nz == 1) {
+    // both z corners are the one cell: four loads (2^20 particles in no order on
+    // 512 x 512 x 1: 23.4 -> 14.8 us, float64 29.7 -> 15.4)
+#pragma unroll
+    for (int c = 0; c < NC; ++c)
+#pragma unroll
+      for (int q = 0; q < 4; ++q) v[c][q] = v[c][q | 4] = m[c * cstride + ix[q & 1] * ny + iy[q >> 1]];
   } else {
 #pragma unroll
     for (int c = 0; c < NC; ++c)

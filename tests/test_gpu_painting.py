@@ -557,3 +557,24 @@ def test_relative_paint_of_many_tiles_marks_corners_outside_their_windows(gpu):
     assert torch.equal(_ops.paint(torch.full(shape, 7.0, device="cuda"), d, relative=True, zero=True), m)
     assert torch.equal(_ops.paint(torch.full(shape, 2.0, device="cuda"), d, relative=True), m + 2.0)
     assert torch.equal(_ops.paint(torch.zeros(shape, device="cuda"), d, relative=True, method="atomic"), m)
+
+
+@pytest.mark.parametrize("nc", [1, 3])
+@pytest.mark.parametrize("shape", [(40, 33, 1), (1, 1, 1), (1, 30, 1), (2, 1, 1)])
+def test_reads_of_one_z_plane(gpu, shape, nc):
+    """Meshes of one cell along z, whose two z corners are that cell: the read
+    and its position cotangent against the mesh repeated along z (nz 2), where
+    the general corners hold the same values."""
+    from jaxpm_amd import _ops
+    print(f"one z plane {shape} nc={nc}", flush=True)
+    r = np.random.default_rng(53)
+    n = 3000
+    pos = (r.uniform(-1.2, 2.3, size=(n, 3)) * np.array(shape)).astype(np.float32)
+    pos[:500] = np.floor(pos[:500])
+    flat = dev(r.normal(size=(nc, *shape)))
+    two = flat.expand(nc, *shape[:2], 2).contiguous()
+    p, cot = dev(pos), dev(r.normal(size=(n, nc)))
+    assert torch.equal(_ops.read(flat, p), _ops.read(two, p))
+    assert torch.equal(_ops.grad_pos(flat, p, cot=cot), _ops.grad_pos(two, p, cot=cot))
+    f64, p64 = flat.double(), p.double()
+    assert torch.equal(_ops.read_f64(f64, p64), _ops.read_f64(two.double(), p64))
