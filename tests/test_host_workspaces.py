@@ -50,3 +50,18 @@ def test_lpt_workspace_holds_what_the_shape_needs(size, shape, native):
     slack = 8 * 256
     assert size("jpm_lpt_workspace_size", *shape, 1) <= 8 * h + 4 * 3 * m + 4 * m + slack
     assert size("jpm_lpt_workspace_size", *shape, 2) <= 8 * 8 * h + 2 * 4 * m + (0 if native else 4 * 6 * m) + slack
+
+
+def test_counts_below_which_no_workspace_is_asked_for(size):
+    """The Python layer's constants are the library's."""
+    from jaxpm_amd import _ops
+    n = _ops.PAINT_F64_WS_MIN
+    assert size("jpm_cic_paint_f64_workspace_size", 50, 50, 50, n) > 0
+    n = _ops.DENSITY_PLANE_WS_MIN
+    assert size("jpm_density_plane_workspace_size", n, 100) > 0
+    for shape in ((1, 1, 1), (16, 16, 16), (50, 50, 50), (256, 256, 256)):
+        for less in (1, 1000, 10 ** 5):
+            assert size("jpm_cic_paint_f64_workspace_size", *shape, _ops.PAINT_F64_WS_MIN - less) == 0
+    for res in (1, 64, 1000, 4096, 20000):
+        for less in (1, 1000, 10 ** 5):
+            assert size("jpm_density_plane_workspace_size", _ops.DENSITY_PLANE_WS_MIN - less, res) == 0
